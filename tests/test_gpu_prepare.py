@@ -53,3 +53,16 @@ def test_zero_points_moe(dev):
     got = moe_awq_to_marlin_zero_points(packed.to(dev), groups, n, 4)
     want = torch.stack([ml.marlin_zero_points(zp[i], groups, n) for i in range(e)])
     assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("rows,n,group", [(2, 64, 128), (33, 192, 128), (1, 4160, -1), (3, 64, -1)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_permute_scales_alignment(dev, rows, n, group, offset):
+    """16-byte pieces, and the element-wise form for a source that starts off a 16-byte boundary."""
+    from vllm_amd.marlin_utils import marlin_permute_scales
+    k = rows * 128 if group != -1 else 512
+    rows = rows if group != -1 else 1
+    flat = torch.randn(offset + rows * n, generator=torch.Generator().manual_seed(n)).half()
+    s = flat[offset:].view(rows, n)
+    got = marlin_permute_scales(flat.to(dev)[offset:].view(rows, n), k, n, group)
+    assert torch.equal(got.cpu(), ml.marlin_permute_scales(s, k, n, k if group == -1 else group))

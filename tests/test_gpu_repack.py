@@ -110,3 +110,23 @@ def test_moe_repack_wrappers(ops, dev, num_bits):
     got = ops.awq_marlin_moe_repack(packed.to(dev), perm.to(dev), size_k, size_n, num_bits)
     for i in range(e):
         assert torch.equal(got[i].cpu(), layout(q[i]))
+
+
+@pytest.mark.parametrize("size_k,size_n,experts,stack_rows", [(64, 576, 3, 1 << 23), (128, 512, 5, 256), (48, 64, 4, 100),
+                                                              (128, 1088, 7, 1)])
+def test_moe_repack_stacks(ops, dev, monkeypatch, size_k, size_n, experts, stack_rows):
+    """Experts repacked as one tall weight, in one or several launches, with and without act-order."""
+    from vllm_amd import _custom_ops
+    monkeypatch.setattr(_custom_ops, "_STACK_ROWS", stack_rows)
+    g = torch.Generator().manual_seed(size_n)
+    q = torch.randint(-2**31, 2**31 - 1, (experts, size_k // 8, size_n), generator=g, dtype=torch.int32)
+    perm = torch.stack([torch.randperm(size_k, generator=g) for _ in range(experts)]).to(torch.int32)
+    none = torch.empty((experts, 0), dtype=torch.int32)
+    for order in (none, perm):
+        got = ops.gptq_marlin_moe_repack(q.to(dev), order.to(dev), size_k, size_n, 4)
+        want = torch.stack([ml.gptq_marlin_repack(q[e], order[e] if order.numel() else None, size_k, size_n, 4)
+                            for e in range(experts)])
+        assert torch.equal(got.cpu(), want)
+    aq = q.reshape(experts, size_k, size_n // 8)
+    got = ops.awq_marlin_moe_repack(aq.to(dev), none.to(dev), size_k, size_n, 4)
+    assert torch.equal(got.cpu(), torch.stack([ml.awq_marlin_repack(aq[e], size_k, size_n, 4) for e in range(experts)]))
