@@ -1,4 +1,5 @@
-"""Compile the gfx950 HIP sources into vllm_amd/libw4a16_gfx950.so (in-tree).
+"""Compile the gfx950 HIP sources into vllm_amd/libw4a16_gfx950.so and the PyTorch operators on top of it into
+vllm_amd/_torch_ops.so (both in-tree).
 
 Usage: python -m vllm_amd.build
 """
@@ -24,6 +25,35 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]
+
+
+# the operators PyTorch sees: host code on torch's headers, linked against the C-ABI library beside it
+TORCH_SOURCE = os.path.join(CSRC, "torch_ops.cpp")
+TORCH_LIB_PATH = os.path.join(HERE, "_torch_ops.so")
+
+
+def _torch_ops_command(out: str) -> list:
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    inc = ["-isystem" + p for p in [*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]]
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc, TORCH_SOURCE, "-o", out, f"-L{lib}", f"-L{HERE}",
+            f"-l:{LIB_NAME}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{lib}"]
+
+
+def build_torch_ops(verbose: bool = False) -> str:
+    """Compiles and links _torch_ops.so (after the C-ABI library, which it links against)."""
+    tmp = TORCH_LIB_PATH + ".tmp"
+    cmd = _torch_ops_command(tmp)
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("compiling %s failed: %s\n%s" % (TORCH_SOURCE, " ".join(cmd), r.stdout))
+    os.replace(tmp, TORCH_LIB_PATH)
+    return TORCH_LIB_PATH
 
 
 def hipcc_path() -> str:
@@ -84,6 +114,7 @@ def build(verbose: bool = False, extra_flags: tuple = (), check_hazards: bool = 
     if r.returncode != 0:
         raise RuntimeError("link failed: %s\n%s" % (" ".join(cmd), r.stdout))
     os.replace(tmp, LIB_PATH)
+    build_torch_ops(verbose)
     return LIB_PATH
 
 

@@ -13,7 +13,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _custom_ops as ops
-from .marlin_utils import (MARLIN_SUPPORTED_GROUP_SIZES, apply_gptq_marlin_linear, check_marlin_supports_shape,
+from .marlin_utils import (MARLIN_SUPPORTED_GROUP_SIZES, USE_FP32_REDUCE_DEFAULT, apply_gptq_marlin_linear, check_marlin_supports_shape,
                            marlin_is_k_full, marlin_make_workspace_new, marlin_permute_bias, marlin_permute_scales,
                            marlin_sort_g_idx, marlin_zero_points_from_packed, query_marlin_supported_quant_types)
 from .scalar_type import ScalarType
@@ -169,10 +169,21 @@ class MarlinLinearKernel(MPLinearKernel):
             layer.bias.data = marlin_permute_bias(layer.bias.data)
 
     def apply_weights(self, layer: torch.nn.Module, x: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
-        size_k, size_n = self.config.partition_weight_shape
+        c = self.config
+        size_k, size_n = c.partition_weight_shape
+        if not torch.compiler.is_compiling():
+            p = layer._parameters  # (Module.__getattr__ costs half a microsecond per name)
+            try:
+                operands = (p[self.w_q_name], p[self.w_s_name], p[self.w_zp_name], p[self.w_gidx_name], p["g_idx_sort_indices"])
+            except KeyError:
+                operands = None  # a caller replaced a parameter by something else: the ordinary lookup below finds it
+            y = operands and ops.eager_linear(x, *operands, self.workspace, c.weight_type.id, size_n, size_k, self.is_k_full,
+                                              bias, USE_FP32_REDUCE_DEFAULT)
+            if y is not None:
+                return y
         w_q, w_s, w_zp, w_gidx = self._get_weight_params(layer)
         return apply_gptq_marlin_linear(x, w_q, w_s, w_zp, w_gidx, layer.g_idx_sort_indices, self.workspace,
-                                        self.config.weight_type, size_n, size_k, self.is_k_full, bias)
+                                        c.weight_type, size_n, size_k, self.is_k_full, bias)
 
 
 _POSSIBLE_KERNELS: list[type[MPLinearKernel]] = [MarlinLinearKernel]

@@ -26,15 +26,18 @@ class ScalarType:
     def size_bits(self) -> int:
         return self.exponent + self.mantissa + int(self.signed)
 
-    @property
-    def id(self) -> int:
+    def __post_init__(self):
         fields = ((self.exponent, 8), (self.mantissa, 8), (int(self.signed), 1), (self.bias, 32),
                   (int(self._finite_values_only), 1), (self.nan_repr, 8))
         val, off = 0, 0
         for member, width in fields:
             val |= (int(member) & ((1 << width) - 1)) << off
             off += width
-        return val
+        object.__setattr__(self, "_id", val)  # read on every GEMM call
+
+    @property
+    def id(self) -> int:
+        return self._id
 
     @classmethod
     def from_id(cls, type_id: int) -> "ScalarType":
