@@ -486,3 +486,16 @@ def test_moe_gemm_never_uses_memory_past_sorted_ids(dev, bs):
     want = call(s)
     got = call(big[:s.numel()])
     assert torch.equal(got, want)
+
+
+# one, two, four and sixteen experts per lane; as many picks as lanes and one more
+@pytest.mark.parametrize("e,topk", [(1, 1), (64, 64), (65, 8), (128, 128), (129, 65), (256, 8), (257, 9), (1024, 64)])
+def test_topk_softmax_lane_edges(dev, e, topk):
+    from vllm_amd.fused_moe import fused_topk
+    logits = (torch.randn(5, e, generator=torch.Generator().manual_seed(e)) * 2).to(torch.float16)
+    w, ids, src = fused_topk(torch.empty(5, 4, device=dev), logits.to(dev), topk, True)
+    ow, oi, osrc = mr.topk_softmax(logits, topk, True)
+    # (probabilities whose exponentials round differently may swap neighbours)
+    assert (ids.cpu() == oi).float().mean() > 0.99
+    torch.testing.assert_close(w.cpu(), ow, rtol=2e-5, atol=1e-7)
+    assert torch.equal(src.cpu(), osrc)
