@@ -499,3 +499,45 @@ def test_topk_softmax_lane_edges(dev, e, topk):
     assert (ids.cpu() == oi).float().mean() > 0.99
     torch.testing.assert_close(w.cpu(), ow, rtol=2e-5, atol=1e-7)
     assert torch.equal(src.cpu(), osrc)
+
+
+# blocks of 128 slots: one and several live tiles cut along K on the device, whole tiles in front of split ones, foreign
+# experts, a column strip that is not full, every form of scales, act-order
+@pytest.mark.parametrize("m,k,n,variant,foreign", [(1, 256, 192, "gptq_f16_g128", False), (300, 4096, 1024, "gptq_f16_g128", True),
+                                                   (700, 2048, 576, "awq_bf16_g32", False), (260, 1024, 512, "gptq_bf16_chan", False),
+                                                   (333, 512, 640, "awq_f16_chan", False), (150, 256, 192, "gptq_f16_g32_act", False),
+                                                   (8300, 4096, 1024, "awq_f16_g128", False)])
+def test_moe_gemm_blocks_of_128(dev, m, k, n, variant, foreign):
+    import vllm_amd.ops as ops
+    from vllm_amd.marlin_utils import marlin_make_workspace_new
+    from vllm_amd.moe_align_block_size import moe_align_block_size
+    from vllm_amd.scalar_type import scalar_types
+    print(f"blocks of 128: {m} {k} {n} {variant} {foreign}", flush=True)
+    topk, e, bs = 2, 4, 128
+    dtype = torch.bfloat16 if "bf16" in variant else torch.float16
+    group = -1 if "chan" in variant else 32 if "g32" in variant else 128
+    has_zp = variant.startswith("awq")
+    layers, mq, ms, mz, gi, perm = make_experts(e, k, n, group, dtype, has_zp, variant.endswith("act"), seed=90)
+    a = torch.randn(m, k, generator=torch.Generator().manual_seed(5)).to(dtype)
+    ids = rand_topk(m, topk, e, seed=6)
+    tw = torch.rand(m, topk, generator=torch.Generator().manual_seed(7))
+    emap = torch.tensor([0, -1, 1, 2], dtype=torch.int32) if foreign else None
+    local = [0, 2, 3] if foreign else [0, 1, 2, 3]
+    s, x, t = moe_align_block_size(ids.to(dev), bs, e, expert_map=emap.to(dev) if foreign else None)
+    c = torch.full((m * topk, n), 7.0, dtype=dtype, device=dev)
+    out = ops.moe_wna16_marlin_gemm(
+        a.to(dev), c, mq[local].to(dev), None, ms[local].to(dev), None, mz[local].to(dev) if has_zp else None, gi[local].to(dev),
+        perm[local].to(dev), marlin_make_workspace_new(dev, 4), s, x, t, tw.to(dev), moe_block_size=bs, top_k=topk,
+        mul_topk_weights=True, is_ep=foreign, b_q_type=scalar_types.uint4 if has_zp else scalar_types.uint4b8, size_m=m,
+        size_n=n, size_k=k, is_k_full=True, use_atomic_add=False, use_fp32_reduce=True, is_zp_float=False).cpu()
+    flat = ids.flatten().long()
+    for ex in range(e):
+        rows = torch.nonzero(flat == ex).flatten()
+        if foreign and ex == 1:
+            assert (out[rows] == 7.0).all()
+            continue
+        if rows.numel() == 0:
+            continue
+        ref = (a[rows // topk].float() @ layers[ex].w_ref.float()) * tw.flatten()[rows].unsqueeze(1)
+        mtr = gr.error_metrics(out[rows], ref)
+        assert mtr["max_rel"] <= tol_for(dtype) and mtr["mean_rel"] < 0.04, (ex, mtr)

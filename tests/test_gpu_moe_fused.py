@@ -197,3 +197,26 @@ def test_fused_marlin_moe_falls_back_when_the_fused_epilogues_do_not_apply(dev, 
     w2 = torch.stack([l.w_ref.t() for l in l2])
     ref = mr.torch_experts(a, w1, w2, tw, ti)
     torch.testing.assert_close(res.cpu().float(), ref.float(), atol=5e-2, rtol=0)
+
+
+@pytest.mark.parametrize("m,k,d", [(333, 256, 192), (1500, 2048, 512)])
+@pytest.mark.parametrize("variant", ["gptq_bf16_chan", "awq_f16_g128"])
+def test_epilogues_on_blocks_of_128(dev, m, k, d, variant):
+    """The prefill kernel's two epilogues, unsplit and through the pass that adds K pieces."""
+    import vllm_amd.ops as ops
+    topk, bs = 2, 128
+    dtype, a, tw, align, w, ws = _setup(dev, m, topk, 4, bs, variant, k, 2 * d, seed=30)
+    h = _plain(ops, a, w, ws, align, tw, bs, topk, False, m, 2 * d, k)
+    want = torch.empty(m * topk, d, dtype=dtype, device=dev)
+    ops.silu_and_mul(want, h)
+    got = torch.full((m * topk, d), 7.0, dtype=dtype, device=dev)
+    _fused(ops, a, got, w, ws, align, tw, bs, topk, False, m, 2 * d, k, silu_and_mul=True)
+    assert torch.equal(got, want) and float(want.float().abs().max()) > 0
+    _, _, tw, align, w, ws = _setup(dev, m, topk, 4, bs, variant, d if d % 128 == 0 else 256, k, seed=31)
+    act = want if d % 128 == 0 else torch.randn(m * topk, 256, device=dev, dtype=dtype)
+    y = _plain(ops, act, w, ws, align, tw, bs, 1, True, m * topk, k, act.size(1))
+    want = torch.empty(m, k, dtype=dtype, device=dev)
+    ops.moe_sum(y.view(m, topk, k), want)
+    got = torch.zeros(m, k, dtype=dtype, device=dev)
+    _fused(ops, act, got, w, ws, align, tw, bs, 1, True, m * topk, k, act.size(1), sum_top_k=2)
+    assert torch.equal(got, want)

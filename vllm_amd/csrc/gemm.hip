@@ -99,7 +99,7 @@ static int validate(const w4a16_gemm_args* a) {
   if (a->flags & W4A16_F_MOE) {
     W4A16_CHECK(a->sorted_token_ids && a->expert_ids && a->num_tokens_past_padded, "null MoE index pointer");
     W4A16_CHECK(a->moe_block_size == 8 || (a->moe_block_size % 16 == 0 && a->moe_block_size >= 16 &&
-                                           a->moe_block_size <= 64),
+                                           a->moe_block_size <= 64) || a->moe_block_size == 128,
                 "unsupported moe_block_size=%d", a->moe_block_size);
     W4A16_CHECK(a->top_k >= 1, "top_k must be >= 1");
     W4A16_CHECK(a->lda == a->size_k, "A is not contiguous");
@@ -144,6 +144,29 @@ static int make_plan(const w4a16_gemm_args* a, Plan& pl) {
   // the 64-row kernel has instantiations for all of them
   const bool mid_ok = !general_only || a->wtype == W4A16_WTYPE_FE2M1 || w8 || ((a->flags & W4A16_F_ZP_FLOAT) && !moe);
   const bool pow2_group = (pl.group_ksteps & (pl.group_ksteps - 1)) == 0;  // prefill / 64-row kernels shift
+  if (moe && a->moe_block_size == 128) {
+    // blocks of 128 slots: the prefill kernel.  One workgroup per compute unit; the tiles of the last, partly filled round of
+    // the live ones are cut along K on the device (tail_split), at most one piece per compute unit.
+    W4A16_CHECK(!general_only && pow2_group && pl.gm != GM_GIDX && a->size_k % 128 == 0,
+                "moe_block_size=128 needs integer 4-bit weights, power-of-two groups, size_k a multiple of 128");
+    pl.kind = 2;
+    pl.tn = 512;
+    pl.mb = 8;
+    pl.bm = 128;
+    pl.total_ksteps = (int)(a->size_k / 32);
+    pl.mtiles = (int)ceil_div(a->n_sorted, 128);
+    pl.ncp = (int)ceil_div(a->size_n, 512);
+    const int64_t tiles = (int64_t)pl.mtiles * pl.ncp;
+    W4A16_CHECK(tiles < (1LL << 31) / 64, "too many tiles");
+    pl.tiles = (int)tiles;
+    pl.splits = 1;
+    pl.kps = pl.total_ksteps;
+    pl.xcd_map = 0;
+    pl.dyn_slots = num_cus();
+    pl.ctmp_bytes = mid_tail_pieces(tiles, pl.dyn_slots) * 128 * 512 * 4;
+    pl.atmp_bytes = act_order ? a->n_sorted * a->size_k * 2 : 0;  // one gathered row per sorted slot
+    return 0;
+  }
   if (moe) {
     const int bs = a->moe_block_size;
     pl.mb = bs <= 16 ? 1 : bs <= 32 ? 2 : 4;

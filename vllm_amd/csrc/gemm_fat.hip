@@ -14,7 +14,9 @@
 // of dequantisation (about 105 instructions per 64 MFMAs for fp16) is interleaved with them: the MFMAs run
 // word-major (16 per Marlin word), and as soon as a word's operands are dead the next k-step's word is
 // dequantised into the same registers.
-// Requirements (host-checked; otherwise the skinny kernel runs): dense op, K % 128 == 0, no per-row g_idx.
+// MoE blocks of 128 sorted slots run here too when experts are large and full (pick_block_size): the 64-row kernel dequantises
+// every weight once per 64 rows (8 experts of 4096 x 14336, top-2, 4096 tokens, bf16: GEMM1 2129 -> 1815 us, GEMM2 1011 -> 874).
+// Requirements (host-checked; otherwise the skinny kernel runs): K % 128 == 0, no per-row g_idx.
 #include <type_traits>
 
 #include "gemm_kernels.h"
@@ -25,41 +27,97 @@ constexpr int FB_MB = 8;     // m-blocks per wavefront
 constexpr int FB_BM = 128;   // rows per workgroup tile
 constexpr int FB_D = 4;      // weight k-steps in flight per wavefront
 constexpr int FB_ABUF = 2 * FB_MB * 64 * 16;  // bytes of one A buffer: 2 k-steps x 8 m-blocks x 64 lanes x 16 B
-constexpr int FB_SMEM = (2 * FB_ABUF > 4 * 16 * RED_RS * 4) ? 2 * FB_ABUF : 4 * 16 * RED_RS * 4;
+constexpr int FB_MIN_SPLIT = 2;  // tail tiles are cut in K pieces as soon as two of each fit the compute units
+constexpr int FB_SLABS = 4 * 16 * RED_RS * 4;                // four wavefront slabs of the epilogue
+constexpr int FB_SMEM = (2 * FB_ABUF > FB_SLABS ? 2 * FB_ABUF : FB_SLABS) + FB_BM * 8;  // + C row and routing weight of each tile row
 
 // BITS = 8: uint8b128 or (FP8) float8_e4m3fn weights in the 8-bit Marlin layout: twice the words per lane, the same 64
 // MFMAs per k-step; no zero points.
 // FP4 = 1 / 2: float4_e2m1f weights (4-bit layout) with NVFP4 / MXFP4 scale records, one 16-byte record per lane and
 // k-step / two k-steps (the host sets the group to 1 / 2 k-steps); NVFP4's global scale is applied to the accumulator.
 // ZPF: uint4 weights with fp16 zero points laid out like the scales (HQQ): operand = fma(q, s, -half(zp * s)).
-template <int DT, bool ZP, bool CHANNEL, int BITS = 4, bool FP8 = false, int FP4 = 0, bool ZPF = false>
+// MOE: blocks of 128 sorted token slots (integer 4-bit weights); rows are gathered through sorted_token_ids while staging.
+template <int DT, bool ZP, bool CHANNEL, int BITS = 4, bool FP8 = false, int FP4 = 0, bool ZPF = false, bool MOE = false>
 __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
   static_assert(!ZPF || (DT == DT_F16 && !ZP && !CHANNEL && BITS == 4 && FP4 == 0), "float zero points: fp16 uint4 grouped");
   static_assert(BITS == 4 || (BITS == 8 && !ZP), "8-bit weights have no zero points");
   static_assert(!FP8 || BITS == 8, "fp8 weights use the 8-bit layout");
   static_assert(FP4 == 0 || (BITS == 4 && !ZP && !CHANNEL), "fp4 weights: grouped scale records, no zero points");
+  static_assert(!MOE || (BITS == 4 && FP4 == 0 && !ZPF), "MoE: integer 4-bit weights");
   constexpr bool UNIT = CHANNEL;
   extern __shared__ __align__(16) unsigned char smem[];
+  int* s_crow = (int*)(smem + FB_SMEM - FB_BM * 8);
+  float* s_tw = (float*)(smem + FB_SMEM - FB_BM * 4);
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int c = lane & 7, h = (lane >> 3) & 1, g = lane >> 4;
 
-  // tile order: consecutive workgroups walk M first, so workgroups resident together share weight strips
-  const int mtiles = (p.M + FB_BM - 1) / FB_BM;
-  const int mt = blockIdx.x % mtiles, nt4 = blockIdx.x / mtiles;
+  // tile order: M first, so workgroups resident together share weight strips (MoE: neighbouring blocks mostly belong to
+  // the same expert)
+  int mtiles = MOE ? (p.n_sorted + FB_BM - 1) / FB_BM : (p.M + FB_BM - 1) / FB_BM;
+  int ks_b = 0, ks_e = p.total_ksteps, split = 0, nsplit = 1, part = 0;
+  int j = blockIdx.x;
+  if constexpr (MOE) {
+    zero_fill_side_job(p);
+    mtiles = min((*p.ntpp + FB_BM - 1) / FB_BM, mtiles);
+    if (mtiles == 0) return;
+    // live tiles; those of the last, partly filled round in K pieces (see tail_split), which walk the tiles first, then K
+    const TailSplit d = tail_split(mtiles * p.ncp, p.dyn_slots, p.total_ksteps, FB_MIN_SPLIT);
+    if (j < d.F) {
+      // workgroup b runs on XCD b mod 8: every XCD gets a contiguous run of tiles, so that the ones it holds at a time share
+      // their expert's weight strips and activation rows in its L2
+      if ((d.F & 7) == 0) j = (j & 7) * (d.F >> 3) + (j >> 3);
+    } else {
+      const int u = j - d.F;
+      if (u >= d.R * d.S) return;
+      part = u % d.R, split = u / d.R, nsplit = d.S;
+      ks_b = split * d.kps, ks_e = min(ks_b + d.kps, p.total_ksteps);
+      j = d.F + part;
+    }
+  }
+  const int mt = j % mtiles, nt4 = j / mtiles;
   const int cp = nt4 * 4 + wv;                 // column pair of this wavefront
   const bool wave_on = cp * 128 < p.N;         // N not a multiple of 512: trailing wavefronts only help staging
   const int row0 = mt * FB_BM;
 
+  const uint32_t* Bq = p.B;
+  const uint16_t* Sc = (const uint16_t*)p.S;
+  const uint32_t* Zp = p.Z;
+  const uint16_t* bias = (const uint16_t*)p.bias;
+  if constexpr (MOE) {
+    const int e = p.expert_ids[mt];
+    if (e < 0) return;  // expert of another rank
+    Bq += e * p.b_estride;
+    Sc += e * p.s_estride;
+    if (ZP) Zp += e * p.z_estride;
+    if (bias) bias += e * p.n_estride;
+  }
+  // which A row feeds tile row r and which C row receives it (-1: none)
+  auto tile_row_ids = [&](int r, int& src, int& dst) {
+    src = dst = -1;
+    const int id = p.sorted_ids[row0 + r];
+    if ((unsigned)id < (unsigned)p.c_rows) {
+      src = p.a_by_slot ? row0 + r : id / p.top_k;
+      dst = id;
+    }
+  };
+  if (MOE && t < FB_BM) {
+    int src, dst;
+    tile_row_ids(t, src, dst);
+    s_crow[t] = dst;
+    if (p.mul_topk) s_tw[t] = dst >= 0 ? p.topk_w[dst] : 0.f;
+  }
+
   // ---- weights of this wavefront
-  const int nt = (wave_on && (2 * cp + h) * 64 < p.N) ? 2 * cp + h : 0;
+  // (fused SiLU-and-mul: gate n-tile cp paired with the up n-tile of the same output columns, N/128 + cp)
+  const int nt = !wave_on ? 0 : (MOE && p.act) ? (h ? (p.N >> 7) + cp : cp) : ((2 * cp + h) * 64 < p.N ? 2 * cp + h : 0);
   // 4-bit: 32 u32x4 per n-tile and k-tile, one per Marlin thread; 8-bit: 64, two per thread (words 2w + half)
   const int64_t b_row = (BITS == 4) ? (p.N >> 1) : p.N;
-  const u32x4* bp = (const u32x4*)p.B + nt * (8 * BITS) + (4 * c + g) * (BITS / 4);
+  const u32x4* bp = (const u32x4*)Bq + nt * (8 * BITS) + (4 * c + g) * (BITS / 4);
   const int64_t s_row = p.N >> 3;
-  const u32x4* sp = (const u32x4*)p.S + nt * 8 + c;
-  const uint32_t* zp = ZP ? p.Z + nt * 8 + c : nullptr;
+  const u32x4* sp = (const u32x4*)Sc + nt * 8 + c;
+  const uint32_t* zp = ZP ? Zp + nt * 8 + c : nullptr;
   const u32x4* zfp = ZPF ? (const u32x4*)p.Z + nt * 8 + c : nullptr;  // fp16 zero points: indexed like the scales
 
   // ---- activation staging: thread t loads piece (t & 7) of rows (t >> 3) + 32 i, i = 0..3
@@ -68,7 +126,13 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     int r = row0 + (t >> 3) + 32 * i;
-    if (r >= p.M) r = p.M - 1;  // rows past the end replicate the last row; never stored
+    if constexpr (MOE) {
+      int dst;
+      tile_row_ids((t >> 3) + 32 * i, r, dst);
+      if (r < 0) r = 0;  // slots without a token read row 0; never stored
+    } else if (r >= p.M) {
+      r = p.M - 1;  // rows past the end replicate the last row; never stored
+    }
     arow[i] = (const uint16_t*)p.A + (int64_t)r * p.lda + piece * 8;
   }
   // LDS A layout: [buffer][k-step 2][m-block 8][lane 64][4 dwords]; the 16 bytes of (row, piece) are the K
@@ -83,8 +147,8 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
   u32x4 areg[4];
   // (chunk and k-step indices are clamped instead of guarded: the last iteration re-reads its own data, which
   //  keeps the main loop free of branches, so the compiler can overlap LDS reads and dequantisation with MFMAs)
-  auto load_a = [&](int chunk) {
-    chunk = min(chunk, p.total_ksteps / 2 - 1);
+  auto load_a = [&](int chunk) {  // chunk, k-step: relative to ks_b
+    chunk = min(ks_b / 2 + chunk, ks_e / 2 - 1);
 #pragma unroll
     for (int i = 0; i < 4; ++i) areg[i] = *(const u32x4*)(arow[i] + chunk * 64);
   };
@@ -105,7 +169,7 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
   };
   Stage st[FB_D];
   auto issue = [&](Stage& s, int ks) {
-    ks = min(ks, p.total_ksteps - 1);
+    ks = min(ks_b + ks, ks_e - 1);
     int gi = 0;
     if (!CHANNEL) gi = ks >> p.group_shift;  // the host only picks this kernel for power-of-two group sizes
     if (!CHANNEL) s.sc = sp[(int64_t)gi * s_row];
@@ -156,8 +220,7 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
       acc[mb][w][1] = f32x4{0, 0, 0, 0};
     }
 
-  const int total = p.total_ksteps;  // multiple of 4 (K % 128 == 0)
-  const int nchunks = total / 2;
+  const int nchunks = (ks_e - ks_b) / 2;  // even: K % 128 == 0, pieces are multiples of 4 k-steps
 
   // ---- prologue
   load_a(0);
@@ -320,13 +383,13 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
   // per wavefront and m-block: accumulators -> private LDS slab [16 rows][RED_RS] -> 8-byte row stores
   float* slab = (float*)smem + wv * (16 * RED_RS);
-  const uint16_t* Sc = (const uint16_t*)p.S;
-  const uint16_t* bias = (const uint16_t*)p.bias;
   const int fc4 = (lane & 31) * 4;
   const int fpos = fc4 + (fc4 >= 64 ? 8 : 0);
   const int ncol = cp * 128 + fc4;
   const bool fcol_ok = wave_on && ncol < p.N;
-  float cs[4] = {1.f, 1.f, 1.f, 1.f}, bs[4] = {0.f, 0.f, 0.f, 0.f};
+  const bool act = MOE && p.act;
+  // cs / bs: channel (and global) scale and bias of the thread's four columns; cu / bu: of the up half's columns
+  float cs[4] = {1.f, 1.f, 1.f, 1.f}, bs[4] = {0.f, 0.f, 0.f, 0.f}, cu[4] = {1.f, 1.f, 1.f, 1.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
   if constexpr (FP4 == 1) {
     // NVFP4 global scale: stored times 2^7 (fp16) / 2^119 (bf16) by the reference's load-time processing
     const uint16_t gv = *(const uint16_t*)p.gscale;
@@ -334,19 +397,31 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) cs[j] = gs;
   }
-  if (fcol_ok) {
-    const int base = ncol & ~31, cl = ncol & 31;
+  auto col_consts = [&](int col, float* sc_out, float* b_out) {
+    const int base = col & ~31, cl = col & 31;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if (CHANNEL) {
         const uint16_t sv = Sc[base + single_perm_pos(cl + j)];
-        cs[j] = ((DT == DT_F16) ? f16_lo_f32(sv) : bf16_lo_f32(sv)) * (FP8 ? fp8_scale_unbias<DT>() : 1.0f);
+        sc_out[j] = ((DT == DT_F16) ? f16_lo_f32(sv) : bf16_lo_f32(sv)) * (FP8 ? fp8_scale_unbias<DT>() : 1.0f);
       }
       if (bias) {
         const uint16_t bv = bias[base + single_perm_pos(cl + j)];
-        bs[j] = (DT == DT_F16) ? f16_lo_f32(bv) : bf16_lo_f32(bv);
+        b_out[j] = (DT == DT_F16) ? f16_lo_f32(bv) : bf16_lo_f32(bv);
       }
     }
+  };
+  // fused SiLU-and-mul, unsplit: lane -> row (lane >> 4) + 4 i, gate columns 4 (lane & 15) .. + 3 and the up columns of
+  // the same outputs, so that all 64 lanes take part
+  const int ac4 = (lane & 15) * 4;
+  const int ocol = cp * 64 + ac4;
+  if (act) {
+    if (wave_on) {
+      col_consts(ocol, cs, bs);
+      col_consts((p.N >> 1) + ocol, cu, bu);
+    }
+  } else if (fcol_ok) {
+    col_consts(ncol, cs, bs);
   }
 #pragma unroll
   for (int mb = 0; mb < FB_MB; ++mb) {
@@ -357,21 +432,44 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) slab[(4 * g + r) * RED_RS + 72 * h + 16 * w + 8 * hf + c] = acc[mb][w][hf][r];
     __builtin_amdgcn_wave_barrier();
+    if (act && nsplit == 1) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r16 = (lane >> 4) + 4 * i;
+        const int crow = s_crow[mb * 16 + r16];
+        if (crow < 0 || !wave_on) continue;
+        f32x4 v = *(const f32x4*)(slab + r16 * RED_RS + ac4);
+        f32x4 u = *(const f32x4*)(slab + r16 * RED_RS + ac4 + 72);
+        const float tw = p.mul_topk ? s_tw[mb * 16 + r16] : 1.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v[j] = (v[j] * cs[j] + bs[j]) * tw;
+          u[j] = (u[j] * cu[j] + bu[j]) * tw;
+        }
+        store_row4_silu_mul<DT>(p, crow, ocol, v, u);
+      }
+      __builtin_amdgcn_wave_barrier();
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int r16 = (lane >> 5) + 2 * i;
-      const int grow = row0 + mb * 16 + r16;
+      const int crow = MOE ? s_crow[mb * 16 + r16] : row0 + mb * 16 + r16;
       f32x4 v = *(const f32x4*)(slab + r16 * RED_RS + fpos);
-      if (fcol_ok && grow < p.M) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = v[j] * cs[j] + bs[j];
-        u32x2 o;
-        if constexpr (DT == DT_F16)
-          o = u32x2{pack_f16(v[0], v[1]), pack_f16(v[2], v[3])};
-        else
-          o = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
-        *(u32x2*)((uint16_t*)p.C + (int64_t)grow * p.N + ncol) = o;
+      if (!fcol_ok || (MOE ? crow < 0 : crow >= p.M)) continue;
+      if (MOE && nsplit > 1) {
+        // a K piece: the fp32 partial tile [row 128][column 512] goes to scratch; the pass launched behind finishes the rows
+        *(f32x4*)(p.ctmp + (((int64_t)part * nsplit + split) * FB_BM + mb * 16 + r16) * 512 + wv * 128 + fc4) = v;
+        continue;
       }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = v[j] * cs[j] + bs[j];
+      if (MOE && p.mul_topk) {
+        const float tw = s_tw[mb * 16 + r16];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] *= tw;
+      }
+      store_row4<DT, MOE>(p, crow, ncol, v);
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -385,6 +483,11 @@ static fat_fn pick_fat2(bool zp, bool channel) {
   return channel ? fat_kernel<DT, false, true> : fat_kernel<DT, false, false>;
 }
 template <int DT>
+static fat_fn pick_fat_moe(bool zp, bool channel) {
+  if (zp) return channel ? fat_kernel<DT, true, true, 4, false, 0, false, true> : fat_kernel<DT, true, false, 4, false, 0, false, true>;
+  return channel ? fat_kernel<DT, false, true, 4, false, 0, false, true> : fat_kernel<DT, false, false, 4, false, 0, false, true>;
+}
+template <int DT>
 static fat_fn pick_fat8(bool fp8, bool channel) {
   if (fp8) return channel ? fat_kernel<DT, false, true, 8, true> : fat_kernel<DT, false, false, 8, true>;
   return channel ? fat_kernel<DT, false, true, 8, false> : fat_kernel<DT, false, false, 8, false>;
@@ -392,8 +495,13 @@ static fat_fn pick_fat8(bool fp8, bool channel) {
 
 int launch_fat(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
   const bool zp = a->b_zeros != nullptr, channel = pl.gm == GM_CHANNEL;
+  const bool moe = (a->flags & W4A16_F_MOE) != 0;
   fat_fn fn;
-  if (a->flags & W4A16_F_ZP_FLOAT) {
+  if (moe) {
+    if ((a->flags & W4A16_F_ZP_FLOAT) || (a->wtype != W4A16_WTYPE_U4B8 && a->wtype != W4A16_WTYPE_U4) || pl.dyn_slots <= 0)
+      return fail(W4A16_EINVAL, "unsupported kernel variant");
+    fn = a->dtype == DT_F16 ? pick_fat_moe<DT_F16>(zp, channel) : pick_fat_moe<DT_BF16>(zp, channel);
+  } else if (a->flags & W4A16_F_ZP_FLOAT) {
     if (a->dtype != DT_F16 || channel) return fail(W4A16_EINVAL, "unsupported kernel variant");
     fn = fat_kernel<DT_F16, false, false, 4, false, 0, true>;
   } else if (a->wtype == W4A16_WTYPE_FE2M1) {
@@ -409,10 +517,12 @@ int launch_fat(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
     fn = a->dtype == DT_F16 ? pick_fat2<DT_F16>(zp, channel) : pick_fat2<DT_BF16>(zp, channel);
   }
   KParams p = make_kparams(a, pl);
-  const int64_t grid = (int64_t)pl.tiles;
-  if (grid <= 0) return 0;
+  if (pl.tiles <= 0) return 0;
+  // MoE: at most dyn_slots pieces behind the whole tiles (the device knows how many), and the pass that adds them
+  const int64_t grid = pl.tiles + (moe ? mid_tail_pieces(pl.tiles, pl.dyn_slots) : 0);
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), FB_SMEM, stream, p);
   W4A16_HIP(hipGetLastError());
+  if (moe) return launch_tail_reduce(a, pl, p, FB_BM, FB_MIN_SPLIT, stream);
   return 0;
 }
 

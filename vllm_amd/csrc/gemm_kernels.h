@@ -48,18 +48,18 @@ struct KParams {
   int64_t zero_n16;
 };
 
-// 64-row kernel on MoE problems.  The number of live tiles L (blocks that hold tokens x column strips) is only known on
+// 64-row and prefill kernel on MoE problems.  The number of live tiles L (blocks that hold tokens x column strips) is only known on
 // the device, and whole tiles run in rounds of `slots` resident workgroups.  The tiles of the last, partly filled round
 // (all tiles, when there are fewer than `slots`) are therefore cut along K into S pieces each, as many as still fit that
 // round, and a second pass adds the pieces: F tiles run whole, the R = L - F tail tiles as R * S pieces of kps k-steps
-// (a multiple of 4, at least 32).  Only from S = 3 on: a tail of more than slots / 3 tiles already runs with fewer
-// workgroups per compute unit, hence faster, and halving it gains less than the partial tiles cost.  Both passes derive
-// the same numbers from L.
+// (a multiple of 4, at least 32).  The 64-row kernel only from S = min_split = 3 on: a tail of more than slots / 3 tiles already
+// runs with fewer workgroups per compute unit, hence faster, and halving it gains less than the partial tiles cost; the
+// prefill kernel (blocks of 128 slots, one workgroup per compute unit) from 2 on.  Both passes derive the same numbers from L.
 constexpr int TAIL_MIN_KSTEPS = 32;
 struct TailSplit {
   int F, R, S, kps;
 };
-__host__ __device__ inline TailSplit tail_split(int live_tiles, int slots, int total_ksteps) {
+__host__ __device__ inline TailSplit tail_split(int live_tiles, int slots, int total_ksteps, int min_split) {
   TailSplit d;
   d.F = (live_tiles / slots) * slots;
   d.R = live_tiles - d.F;
@@ -69,7 +69,7 @@ __host__ __device__ inline TailSplit tail_split(int live_tiles, int slots, int t
     int s = slots / d.R;
     if (s > 8) s = 8;
     if (s > total_ksteps / TAIL_MIN_KSTEPS) s = total_ksteps / TAIL_MIN_KSTEPS;
-    if (s >= 3) {
+    if (s >= min_split) {
       d.kps = ((total_ksteps + s - 1) / s + 3) / 4 * 4;
       d.S = (total_ksteps + d.kps - 1) / d.kps;
     }
@@ -208,6 +208,9 @@ inline hipError_t allow_dynamic_lds(const void* fn, int bytes) {
   if (n_seen < 256) seen[n_seen++] = Key{fn, dev};
   return hipSuccess;
 }
+
+// Second pass of a MoE launch whose tail tiles (bm rows) were cut along K on the device (gemm_mid.hip).
+int launch_tail_reduce(const w4a16_gemm_args* a, const Plan& pl, const KParams& p, int bm, int min_split, hipStream_t stream);
 
 // Host: translate the C-ABI arguments and the launch plan into the kernel parameter block.
 inline KParams make_kparams(const w4a16_gemm_args* a, const Plan& pl) {

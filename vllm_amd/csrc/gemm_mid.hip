@@ -27,6 +27,7 @@ namespace w4a16 {
 
 constexpr int MD_MB = 4;     // m-blocks per tile
 constexpr int MD_BM = 64;    // rows per tile
+constexpr int MD_MIN_SPLIT = 3;  // see tail_split
 constexpr int MD_D = 4;      // weight k-steps in flight per wavefront
 constexpr int MD_ABUF = 2 * MD_MB * 64 * 16;            // one A buffer: 2 k-steps x 4 m-blocks x 64 lanes x 16 B
 constexpr int MD_SLABS = 4 * 16 * RED_RS * 4;           // four wavefront slabs of the epilogue
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
     // live tiles in M-first order; the tail tiles' pieces walk the tiles first, then K (see tail_split)
     const int live = min((moe_ntp + MD_BM - 1) / MD_BM, mtiles);
     if (live == 0) return;
-    const TailSplit d = tail_split(live * p.ncp, p.dyn_slots, p.total_ksteps);
+    const TailSplit d = tail_split(live * p.ncp, p.dyn_slots, p.total_ksteps, MD_MIN_SPLIT);
     int j = blockIdx.x;
     if (j < d.F) {
       split = 0, nsplit = 1, kps = p.total_ksteps, tile = 0;
@@ -438,24 +439,24 @@ __global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
   }
 }
 
-// Second pass of a split-K launch of mid_kernel: out tile = sum over splits of the fp32 partial tiles (in split order,
+// Second pass of a split-K launch of mid_kernel (BM = 64) or of the prefill kernel on MoE blocks (BM = 128): out tile = sum over splits of the fp32 partial tiles (in split order,
 // so the result does not depend on timing), then channel scale, bias, routing weight, conversion and the row scatter
 // exactly as mid_kernel's own epilogue does.  One workgroup per (tile, 16-row block); thread -> 4 columns of 2 rows per pass.
-template <int DT, bool CHANNEL, bool MOE>
+template <int DT, bool CHANNEL, bool MOE, int BM, int MIN_SPLIT>
 __global__ __launch_bounds__(256) void mid_reduce_kernel(const KParams p) {
   const int t = threadIdx.x;
-  const int mtiles = MOE ? (p.n_sorted + MD_BM - 1) / MD_BM : (p.M + MD_BM - 1) / MD_BM;
-  const int tile = blockIdx.x >> 2, rb = blockIdx.x & 3;
+  const int mtiles = MOE ? (p.n_sorted + BM - 1) / BM : (p.M + BM - 1) / BM;
+  const int tile = blockIdx.x / (BM / 16), rb = blockIdx.x % (BM / 16);
   int mt = tile % mtiles, nt4 = p.strip0 + tile / mtiles, nsplit = p.splits;
   if (MOE && p.dyn_slots > 0) {  // tile: index among the tail tiles (see tail_split)
-    const int live = min((*p.ntpp + MD_BM - 1) / MD_BM, mtiles);
+    const int live = min((*p.ntpp + BM - 1) / BM, mtiles);
     if (live == 0) return;
-    const TailSplit d = tail_split(live * p.ncp, p.dyn_slots, p.total_ksteps);
+    const TailSplit d = tail_split(live * p.ncp, p.dyn_slots, p.total_ksteps, MIN_SPLIT);
     if (d.S == 1 || tile >= d.R) return;
     const int j = d.F + tile;
     mt = j % live, nt4 = p.strip0 + j / live, nsplit = d.S;
   }
-  const int row0 = mt * MD_BM;
+  const int row0 = mt * BM;
   const uint16_t* Sc = (const uint16_t*)p.S;
   const uint16_t* bias = (const uint16_t*)p.bias;
   const uint16_t* gscale = (const uint16_t*)p.gscale;  // NVFP4 only, else null
@@ -497,7 +498,7 @@ __global__ __launch_bounds__(256) void mid_reduce_kernel(const KParams p) {
   };
   col_consts(ncol, cs, bs);
   if (act) col_consts((p.N >> 1) + ncol, cu, bu);
-  const float* parts = p.ctmp + (int64_t)tile * nsplit * (MD_BM * 512) + fc4;
+  const float* parts = p.ctmp + (int64_t)tile * nsplit * (BM * 512) + fc4;
   // (the rows' slot ids, then per row the partial tiles of four splits at a time, are loaded together: the pass is bound
   //  by round trips, not by bytes)
   int crows[8];
@@ -520,7 +521,7 @@ __global__ __launch_bounds__(256) void mid_reduce_kernel(const KParams p) {
     for (int s0 = 0; s0 < nsplit; s0 += 4) {
       f32x4 a[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) a[q] = *(const f32x4*)(src + (int64_t)min(s0 + q, nsplit - 1) * (MD_BM * 512));
+      for (int q = 0; q < 4; ++q) a[q] = *(const f32x4*)(src + (int64_t)min(s0 + q, nsplit - 1) * (BM * 512));
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         if (s0 + q < nsplit) acc += a[q];
@@ -568,7 +569,18 @@ static mid_fn pick_mid8(bool fp8, bool channel) {
 }
 template <int DT, bool MOE>
 static mid_fn pick_reduce(bool channel) {
-  return channel ? mid_reduce_kernel<DT, true, MOE> : mid_reduce_kernel<DT, false, MOE>;
+  return channel ? mid_reduce_kernel<DT, true, MOE, MD_BM, MD_MIN_SPLIT> : mid_reduce_kernel<DT, false, MOE, MD_BM, MD_MIN_SPLIT>;
+}
+
+int launch_tail_reduce(const w4a16_gemm_args* a, const Plan& pl, const KParams& p, int bm, int min_split, hipStream_t stream) {
+  if (bm != 128 || min_split != 2) return fail(W4A16_EINVAL, "unsupported kernel variant");
+  const bool channel = pl.gm == GM_CHANNEL;
+  const mid_fn red = a->dtype == DT_F16 ? (channel ? mid_reduce_kernel<DT_F16, true, true, 128, 2> : mid_reduce_kernel<DT_F16, false, true, 128, 2>)
+                                        : (channel ? mid_reduce_kernel<DT_BF16, true, true, 128, 2> : mid_reduce_kernel<DT_BF16, false, true, 128, 2>);
+  const int64_t tail = pl.tiles < pl.dyn_slots ? pl.tiles : pl.dyn_slots;
+  hipLaunchKernelGGL(red, dim3((unsigned)(tail * (bm / 16))), dim3(256), 0, stream, p);
+  W4A16_HIP(hipGetLastError());
+  return 0;
 }
 
 int launch_mid(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {

@@ -307,7 +307,7 @@ Tensor moe_gemm(const Tensor& a, const OptTensor& c_or_none, const Tensor& w, co
   TORCH_CHECK(a.is_cuda() && a.is_contiguous() && a.dim() == 2, "A is not a contiguous 2-D GPU tensor");
   TORCH_CHECK(a.size(0) == size_m, "Shape mismatch: a.size(0) = ", a.size(0), ", size_m = ", size_m);
   TORCH_CHECK(a.size(1) == size_k, "Shape mismatch: a.size(1) = ", a.size(1), ", size_k = ", size_k);
-  TORCH_CHECK(block == 8 || (block % 16 == 0 && block >= 16 && block <= 64), "unsupported moe_block_size=", block);
+  TORCH_CHECK(block == 8 || (block % 16 == 0 && block >= 16 && block <= 64) || block == 128, "unsupported moe_block_size=", block);
   TORCH_CHECK(w.is_cuda() && w.is_contiguous() && w.dim() == 3 && w.scalar_type() == at::kInt,
               "b_q_weight is not a contiguous 3-D int32 GPU tensor");
   const int64_t experts = w.size(0);

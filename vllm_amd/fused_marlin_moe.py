@@ -29,7 +29,7 @@ from .scalar_type import ScalarType, scalar_types
 
 _MOE_WEIGHT_TYPES = (scalar_types.uint4, scalar_types.uint4b8, scalar_types.uint8b128, scalar_types.float8_e4m3fn,
                      scalar_types.float4_e2m1f)
-_BLOCK_SIZES = (8, 16, 32, 48, 64)  # token slots per expert block the MoE GEMM accepts
+_BLOCK_SIZES = (8, 16, 32, 48, 64)  # token slots per expert block the MoE GEMM accepts for every weight type; 128: see _tall_blocks
 
 
 def default_activation_func(activation: str, output: torch.Tensor, input: torch.Tensor) -> None:
@@ -38,14 +38,30 @@ def default_activation_func(activation: str, output: torch.Tensor, input: torch.
     ops.silu_and_mul(output, input)
 
 
-def pick_block_size(tokens: int, topk: int, num_experts: int, expert_bytes: int = 1 << 30) -> int:
+def _tall_blocks(quant_type: ScalarType, k: int, n: int, w1_scale, w2_scale, is_k_full: bool) -> bool:
+    """Whether blocks of 128 slots (the prefill kernel) can and should run both GEMMs [., k] x [k, 2n] and [., n] x [n, k].
+    Integer 4-bit weights, whole power-of-two groups, K a multiple of 128; and both K of 4096 or more: the kernel keeps one
+    workgroup per compute unit, so every tile pays for its start and its epilogue (64 experts of 2048 x 1408 at 384 rows each:
+    663 us against 569 with blocks of 64, whose two workgroups per compute unit hide them)."""
+    if quant_type not in (scalar_types.uint4, scalar_types.uint4b8) or not is_k_full or min(k, n) < 4096 or k % 128 or n % 128:
+        return False
+    groups = ((k, w1_scale.size(1)), (n, w2_scale.size(1)))
+    return all(g == 1 or (kk % g == 0 and (kk // g) % 32 == 0 and (kk // g) & (kk // g - 1) == 0) for kk, g in groups)
+
+
+def pick_block_size(tokens: int, topk: int, num_experts: int, expert_bytes: int = 1 << 30, tall: bool = False) -> int:
     """Token slots per expert block, from the average expert's share of the slots (the quantity the reference's rule
     uses, fused_marlin_moe.py:279-282), fitted to the kernels behind each size on MI355X: blocks of 16 slots run on the
     weight-streaming kernel, whose cost is one pass over the expert's weights per block; blocks of 64 on the 64-row
     kernel, which costs about two such passes per block, so it wins once an expert fills more than one and a quarter
     blocks of 16 (sooner for experts of a few MB, where the per-block fixed costs count).  Blocks of 8 never beat 16,
-    and 32 / 48 lost their niche (few, large experts) when the 64-row kernel began to split K for a thin last round."""
+    and 32 / 48 lost their niche (few, large experts) when the 64-row kernel began to split K for a thin last round.
+    tall (see _tall_blocks): blocks of 128 from 192 slots per expert; every weight is then dequantised once per 128 rows
+    (8 experts of 4096 x 14336, bf16: 1024 / 512 / 256 slots each 3159 / 1700 / 1004 -> 2702 / 1427 / 931 us; at 128 slots
+    the half-empty last blocks cost as much: 565 / 583)."""
     per_expert = tokens * topk / num_experts
+    if tall and per_expert >= 192:
+        return 128
     return 16 if per_expert < (20 if expert_bytes >= (12 << 20) else 14) else 64
 
 
@@ -180,7 +196,8 @@ def fused_marlin_moe(hidden_states, w1, w2, bias1, bias2, w1_scale, w2_scale, ga
     _check_layer(k, w1, w2, quant_type, hidden_states.dtype)
     num_local = w1.size(0)
     topk = topk_ids.size(1)
-    bs = pick_block_size(m, topk, num_local, (w1[0].numel() + w2[0].numel()) * 4)
+    bs = pick_block_size(m, topk, num_local, (w1[0].numel() + w2[0].numel()) * 4,
+                         _tall_blocks(quant_type, k, marlin_moe_intermediate_size(w1, w2), w1_scale, w2_scale, is_k_full))
     sorted_ids, expert_ids, post_pad = moe_align_block_size(
         topk_ids, bs, num_local if global_num_experts == -1 else global_num_experts, expert_map)
     ex = _Experts(quant_type, (w1, w2), (w1_scale, w2_scale), (bias1, bias2), (global_scale1, global_scale2),
