@@ -174,3 +174,19 @@ def test_moe_gemm_w8_act_order(ops, dev, dtype, k_full, m, topk, e, bs):
         for j in range(topk):
             assert torch.equal(out[i * topk + j], layers[int(ids[i, j])].w_ref[ks[i]])
     assert int(ws.abs().sum()) == 0
+
+
+# 16-row tiles: rows 1..16 and two tiles, K cut across wavefronts and workgroups or in one piece, an odd number of 64-column
+# tiles, more tiles than compute units; one-hot rows are exact, activations with a mean do not drown in the byte offset
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,k,n,group", [(1, 64, 64, 64), (8, 2048, 192, 128), (9, 4096, 320, -1), (16, 4096, 1024, 64),
+                                         (16, 256, 64 * 259, 128), (24, 8192, 256, 128)])
+def test_decode_tiles_w8(ops, dev, workspace, dtype, m, k, n, group):
+    layer = make_layer(k, n, group, dtype, seed=m + n, bits=8)
+    ks = torch.randperm(k, generator=torch.Generator().manual_seed(1))[:m]
+    a = torch.zeros(m, k, dtype=dtype)
+    a[torch.arange(m), ks] = 1.0
+    assert torch.equal(run_gemm(ops, layer, a.to(dev), dev, workspace).cpu(), layer.w_ref[ks])
+    a = (torch.randn(m, k, generator=torch.Generator().manual_seed(2)) + 1.0).to(dtype).to(dev)
+    check_close(run_gemm(ops, layer, a, dev, workspace), a, layer)
+    assert int(workspace.abs().sum()) == 0

@@ -134,7 +134,7 @@ static int make_plan(const w4a16_gemm_args* a, Plan& pl) {
   }
 
   const bool moe = (a->flags & W4A16_F_MOE) != 0;
-  // 8-bit weights and float zero points run on the general (skinny) kernel only
+  // weight types of the general (skinny) kernel; the exceptions follow (and dense uint8b128 on the decode kernel)
   const bool general_only = a->wtype == W4A16_WTYPE_U8B128 || a->wtype == W4A16_WTYPE_FE4M3 ||
                             a->wtype == W4A16_WTYPE_FE2M1 ||
                             (a->flags & W4A16_F_ZP_FLOAT) != 0;
@@ -371,7 +371,8 @@ static int make_plan(const w4a16_gemm_args* a, Plan& pl) {
   }
 
   // The decode kernel handles 16-row tiles whose scale groups span whole stages of 64 K rows.
-  const bool decode_shape = !general_only && pl.gm != GM_GIDX && pl.total_ksteps % 2 == 0 &&
+  const bool u8_dense = a->wtype == W4A16_WTYPE_U8B128 && !moe;
+  const bool decode_shape = (!general_only || u8_dense) && pl.gm != GM_GIDX && pl.total_ksteps % 2 == 0 &&
                             (pl.gm == GM_CHANNEL || (pl.group_ksteps % 2 == 0 && pow2_group)) && forced_kind != 0;
 
   // Launch-shape choice by a small cost model (microseconds) fitted to MI355X measurements of these
@@ -395,13 +396,17 @@ static int make_plan(const w4a16_gemm_args* a, Plan& pl) {
     for (int ti = 0; ti < n_tn; ++ti) {
       const int tn = ti == 0 ? 128 : 64;
       if (forced_tn && tn != forced_tn && decode_ok) continue;
+      if (tn == 128 && decode_ok && u8_dense) continue;             // the decode kernel takes 8-bit weights in 64-column tiles
       if (tn == 64 && (a->flags & W4A16_F_SILU_AND_MUL)) continue;  // gate and up n-tiles are paired in 128-column tiles
       const int64_t ncol_tiles = ceil_div(a->size_n, tn);
       const int64_t tiles = mtiles * ncol_tiles;
       if (tiles <= 0 || tiles >= (1LL << 31) / 64) continue;
       const double bytes = (double)tiles * a->size_k * tn / 2.0;
-      const double wg_rate = mb == 1 ? (tn == 64 ? 20e3 : 33e3) : mb == 2 ? 12e3 : 9e3;  // bytes per us
-      const double chip_rate = 4.7e6;
+      // bytes per us, of a 4-bit copy of the weights; 8-bit weights carry twice as many (decode kernel: 23 GB/s per workgroup
+      // and 4.7 TB/s of the bytes they have, measured; general kernel 0.7 of its 4-bit rate)
+      const double wg_rate = u8_dense ? (decode_ok ? 11.5e3 : mb == 2 ? 8.3e3 : 6.2e3)
+                             : mb == 1 ? (tn == 64 ? 20e3 : 33e3) : mb == 2 ? 12e3 : 9e3;
+      const double chip_rate = u8_dense ? 2.35e6 : 4.7e6;
       const double t_xchg = 2.2;
       const int unit = decode_ok ? 16 : 8;  // k-steps per split needed to give every wavefront work
       const int max_splits = pl.total_ksteps / unit > 0 ? pl.total_ksteps / unit : 1;

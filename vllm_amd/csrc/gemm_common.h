@@ -536,6 +536,23 @@ __device__ __forceinline__ void raw_pair(uint32_t xa, uint32_t xb, u32x4& o0, u3
   }
 }
 
+// The same for 8-bit weights: fp16 1024 + b (the byte moved into the mantissa by one v_perm_b32 per register), bf16 b itself
+// (at most 8 bits, exact; 128 + b would need nine).  xa0 / xa1: the lane's words of column half 0 / 1 in k-tile a.
+template <int DT>
+__device__ __forceinline__ void raw_pair8(uint32_t xa0, uint32_t xa1, uint32_t xb0, uint32_t xb1, u32x4& o0, u32x4& o1) {
+  // bytes of a word: K rows (k0, k0+8, k0+1, k0+9)
+  auto even = [](uint32_t x) {
+    if constexpr (DT == DT_F16) return __builtin_amdgcn_perm(0x64646464u, x, 0x04020400u);
+    else return pack_bf16(ubyte_f32<0>(x), ubyte_f32<2>(x));
+  };
+  auto odd = [](uint32_t x) {
+    if constexpr (DT == DT_F16) return __builtin_amdgcn_perm(0x64646464u, x, 0x04030401u);
+    else return pack_bf16(ubyte_f32<1>(x), ubyte_f32<3>(x));
+  };
+  o0 = u32x4{even(xa0), odd(xa0), even(xb0), odd(xb0)};
+  o1 = u32x4{even(xa1), odd(xa1), even(xb1), odd(xb1)};
+}
+
 // SiLU in fp32 exactly as PyTorch's device kernel and the reference's act_and_mul_kernel evaluate it
 // (csrc/activation_kernels.cu:28-32): x / (1 + expf(-x)) with the correctly rounded quotient, so that results equal
 // torch.nn.functional.silu on the same device bit for bit (the reference tests this op for exact equality,

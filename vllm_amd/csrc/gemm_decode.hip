@@ -45,7 +45,11 @@ struct DecodeCfg {
 // registers alone, so a small layer's first loads do not wait for a fetch of the argument block from memory (a round
 // trip as long as the weight load itself when the launch comes from a graph and the block is cold).
 //   eNcpX: column tiles, bit 30 set for the XCD-aware grid; eKpsG: k-steps per split, (group_shift + 1) << 24
-template <int DT, bool ZP, bool CHANNEL, int TN, int DNW, bool MOE>
+// BITS = 8: uint8b128 weights (dense, 64-column tiles only: with 128 columns the two stages in flight take 64 registers and the
+// launch 10-25 % longer): twice the words, the same MFMAs and fold.  1-3 conversion instructions per operand register instead of
+// the general kernel's five (4096 x 6144 / 4096 / 28672 and 14336 x 4096 at 16 rows, bf16:
+// 15.5 / 12.9 / 35.2 / 26.4 -> 10.5 / 8.1 / 25.7 / 15.3 us; 117 MB in 25.7 us is 4.6 TB/s).
+template <int DT, bool ZP, bool CHANNEL, int TN, int DNW, bool MOE, int BITS = 4>
 __global__ __launch_bounds__(DNW * 64, 2) void decode_kernel(const uint32_t* eB, const void* eA, const void* eS,
                                                              int64_t eLda, int eN, int eKpsG, int eTotal, int eTiles,
                                                              int eNcpX, int eM, const KParams p) {
@@ -53,9 +57,13 @@ __global__ __launch_bounds__(DNW * 64, 2) void decode_kernel(const uint32_t* eB,
   const bool eXcd = (eNcpX >> 30) & 1;
   const int eKps = eKpsG & 0xffffff, eGroupShift = (eKpsG >> 24) - 1;
   constexpr int W = TN / 32;  // Marlin words per lane and k-tile: 4 (128-bit load) or 2 (64-bit load)
-  constexpr bool HI_TRICK = (DT == DT_F16) && !ZP;
+  constexpr bool HI_TRICK = (DT == DT_F16) && !ZP && BITS == 4;
+  static_assert(BITS == 4 || (BITS == 8 && !ZP), "8-bit weights have no zero points");
   constexpr int RS = DecodeCfg<TN>::RS;
   using bvec = uint32_t __attribute__((ext_vector_type(W)));
+  // weights of a lane and k-tile: W words, twice as many at 8 bits (the halves of word w are elements 2w, 2w + 1), in NB loads
+  constexpr int BV = W * BITS / 4 > 4 ? 4 : W * BITS / 4, NB = W * BITS / 4 / BV;
+  using lvec = uint32_t __attribute__((ext_vector_type(BV)));
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_crow[16];
   __shared__ float s_tw[16];  // MoE: routing weight of each tile row
@@ -165,9 +173,9 @@ __global__ __launch_bounds__(DNW * 64, 2) void decode_kernel(const uint32_t* eB,
     nt = (MOE && p.act) ? (h ? (eN >> 7) + ct : ct) : ((2 * ct + h) * 64 < eN ? 2 * ct + h : 0);
   else
     nt = ct;
-  const int64_t b_row = (int64_t)eN * 2;  // words per k-tile row
+  const int64_t b_row = (int64_t)eN * (BITS / 2);  // words per k-tile row
   // TN=128: words th*4 .. +4 of the n-tile, th = 4c+g.  TN=64: words th*4 + 2h .. +2.
-  const uint32_t* bnext = Bq + (int64_t)nt * 128 + (4 * c + g) * 4 + (TN == 64 ? 2 * h : 0) + (int64_t)(4 * w_b) * b_row;
+  const uint32_t* bnext = Bq + (int64_t)nt * (32 * BITS) + (4 * c + g) * BITS + (TN == 64 ? BITS / 2 * h : 0) + (int64_t)(4 * w_b) * b_row;
   // scales of the lane's columns: permuted position 8c + j, j = 2w + half; TN=64 covers w = 2h, 2h+1 only
   const uint16_t* sp = Sc + (int64_t)nt * 64 + 8 * c + (TN == 64 ? 4 * h : 0);
   const uint32_t* zp = ZP ? Zp + nt * 8 + c : nullptr;
@@ -187,7 +195,7 @@ __global__ __launch_bounds__(DNW * 64, 2) void decode_kernel(const uint32_t* eB,
   auto group_of = [&](int sidx) { return CHANNEL ? (sidx >> 1) : ((2 * sidx) >> eGroupShift); };
   const int gmask = CHANNEL ? 1 : (((1 << eGroupShift) - 1) >> 1);  // stage index bits inside a group
   struct Stage {
-    bvec b[4];   // k-tiles 4s .. 4s+3
+    lvec b[4][NB];  // k-tiles 4s .. 4s+3
     u32x4 a[2];  // rows ar, ar+8
     bvec sc;     // scales (pairs half0|half1 per word)
     uint32_t zq;
@@ -213,7 +221,9 @@ __global__ __launch_bounds__(DNW * 64, 2) void decode_kernel(const uint32_t* eB,
     const uint32_t* q = bnext;  // (stages are issued in order: a running pointer instead of a 64-bit product per stage)
     bnext += 4 * b_row;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) s.b[t] = __builtin_nontemporal_load((const bvec*)(q + t * b_row));
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < NB; ++i) s.b[t][i] = __builtin_nontemporal_load((const lvec*)(q + t * b_row + 4 * i));
   };
 
   f32x4 acc[W][2], tmp[W][2];
@@ -244,10 +254,11 @@ __global__ __launch_bounds__(DNW * 64, 2) void decode_kernel(const uint32_t* eB,
       }
       float e0 = 1.0f, e1 = 1.0f;
       if constexpr (!HI_TRICK) {
-        const float E = (DT == DT_F16) ? 1024.0f : 128.0f;
+        // (8 bits: 1024 + b in fp16, b itself in bf16, b = q + 128)
+        const float E = (DT == DT_F16) ? 1024.0f : BITS == 8 ? 0.0f : 128.0f;
         const int wa = (TN == 64) ? 2 * h + w : w;  // absolute word index of the n-tile
-        e0 = E + (ZP ? (float)((cur_zq >> (4 * wa)) & 0xf) : 8.0f);
-        e1 = E + (ZP ? (float)((cur_zq >> (4 * wa + 16)) & 0xf) : 8.0f);
+        e0 = E + (ZP ? (float)((cur_zq >> (4 * wa)) & 0xf) : BITS == 8 ? 128.0f : 8.0f);
+        e1 = E + (ZP ? (float)((cur_zq >> (4 * wa + 16)) & 0xf) : BITS == 8 ? 128.0f : 8.0f);
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -288,7 +299,15 @@ __global__ __launch_bounds__(DNW * 64, 2) void decode_kernel(const uint32_t* eB,
     for (int kk = 0; kk < 2; ++kk) {
       u32x4 o[W][2];
 #pragma unroll
-      for (int w = 0; w < W; ++w) raw_pair<DT, HI_TRICK>(s.b[2 * kk][w], s.b[2 * kk + 1][w], o[w][0], o[w][1]);
+      for (int w = 0; w < W; ++w) {
+        if constexpr (BITS == 8) {
+          constexpr int V = BV / 2;  // words in a load
+          const lvec &xa = s.b[2 * kk][w / V], &xb = s.b[2 * kk + 1][w / V];
+          raw_pair8<DT>(xa[2 * (w % V)], xa[2 * (w % V) + 1], xb[2 * (w % V)], xb[2 * (w % V) + 1], o[w][0], o[w][1]);
+        } else {
+          raw_pair<DT, HI_TRICK>(s.b[2 * kk][0][w], s.b[2 * kk + 1][0][w], o[w][0], o[w][1]);
+        }
+      }
       if (kk == 0 && fresh) {
         rs = mfma16x16x32<DT>(af[kk], vb, zero);
 #pragma unroll
@@ -528,33 +547,38 @@ __global__ __launch_bounds__(DNW * 64, 2) void decode_kernel(const uint32_t* eB,
 typedef void (*decode_fn)(const uint32_t*, const void*, const void*, int64_t, int, int, int, int, int, int, const KParams);
 
 template <int DT, int TN, int NW, bool MOE>
-static decode_fn pick5(bool zp, bool channel) {
+static decode_fn pick5(bool w8, bool zp, bool channel) {
+  if constexpr (!MOE && TN == 64) {
+    if (w8) return channel ? decode_kernel<DT, false, true, TN, NW, false, 8> : decode_kernel<DT, false, false, TN, NW, false, 8>;
+  }
   if (zp) return channel ? decode_kernel<DT, true, true, TN, NW, MOE> : decode_kernel<DT, true, false, TN, NW, MOE>;
   return channel ? decode_kernel<DT, false, true, TN, NW, MOE> : decode_kernel<DT, false, false, TN, NW, MOE>;
 }
 template <int DT, int TN, int NW>
-static decode_fn pick4(bool moe, bool zp, bool channel) {
-  return moe ? pick5<DT, TN, NW, true>(zp, channel) : pick5<DT, TN, NW, false>(zp, channel);
+static decode_fn pick4(bool moe, bool w8, bool zp, bool channel) {
+  return moe ? pick5<DT, TN, NW, true>(w8, zp, channel) : pick5<DT, TN, NW, false>(w8, zp, channel);
 }
 template <int DT, int TN>
-static decode_fn pick3(int nw, bool moe, bool zp, bool channel) {
-  return nw == 4 ? pick4<DT, TN, 4>(moe, zp, channel) : pick4<DT, TN, 8>(moe, zp, channel);
+static decode_fn pick3(int nw, bool moe, bool w8, bool zp, bool channel) {
+  return nw == 4 ? pick4<DT, TN, 4>(moe, w8, zp, channel) : pick4<DT, TN, 8>(moe, w8, zp, channel);
 }
 template <int DT>
-static decode_fn pick2(int tn, int nw, bool moe, bool zp, bool channel) {
-  return tn == 64 ? pick3<DT, 64>(nw, moe, zp, channel) : pick3<DT, 128>(nw, moe, zp, channel);
+static decode_fn pick2(int tn, int nw, bool moe, bool w8, bool zp, bool channel) {
+  return tn == 64 ? pick3<DT, 64>(nw, moe, w8, zp, channel) : pick3<DT, 128>(nw, moe, w8, zp, channel);
 }
 
 // (act-order never reaches the kernel as such: the host gathers A's columns in front of the launch, see gemm.hip)
-static decode_fn pick_decode(int dt, int tn, int nw, bool moe, bool zp, bool channel) {
-  return dt == DT_F16 ? pick2<DT_F16>(tn, nw, moe, zp, channel) : pick2<DT_BF16>(tn, nw, moe, zp, channel);
+static decode_fn pick_decode(int dt, int tn, int nw, bool moe, bool w8, bool zp, bool channel) {
+  return dt == DT_F16 ? pick2<DT_F16>(tn, nw, moe, w8, zp, channel) : pick2<DT_BF16>(tn, nw, moe, w8, zp, channel);
 }
 
 int launch_decode(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
   const bool zp = a->b_zeros != nullptr;
   if (pl.use_perm) return fail(W4A16_EINVAL, "unsupported kernel variant");
   const int nw = pl.nw == 4 ? 4 : 8;
-  decode_fn fn = pick_decode(a->dtype, pl.tn, nw, (a->flags & W4A16_F_MOE) != 0, zp, pl.gm == GM_CHANNEL);
+  const bool w8 = a->wtype == W4A16_WTYPE_U8B128, moe = (a->flags & W4A16_F_MOE) != 0;
+  if (w8 && (moe || pl.tn != 64)) return fail(W4A16_EINVAL, "unsupported kernel variant");
+  decode_fn fn = pick_decode(a->dtype, pl.tn, nw, moe, w8, zp, pl.gm == GM_CHANNEL);
   KParams p = make_kparams(a, pl);
   const int smem = pl.tn == 64 ? DecodeCfg<64>::smem(nw) : DecodeCfg<128>::smem(nw);
   W4A16_HIP(allow_dynamic_lds((const void*)fn, smem));
