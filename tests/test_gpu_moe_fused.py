@@ -220,3 +220,27 @@ def test_epilogues_on_blocks_of_128(dev, m, k, d, variant):
     got = torch.zeros(m, k, dtype=dtype, device=dev)
     _fused(ops, act, got, w, ws, align, tw, bs, 1, True, m * topk, k, act.size(1), sum_top_k=2)
     assert torch.equal(got, want)
+
+
+# the native call for a whole layer against the launches one by one (which a caller's own output buffer asks for): one, two and
+# three experts per token, bias, act-order, no workspace; a half-size tensor argument or an id type it does not take
+@pytest.mark.parametrize("topk", [1, 2, 3])
+@pytest.mark.parametrize("variant,act_order", [("gptq_f16_g128", False), ("awq_bf16_g128", False), ("gptq_f16_g128", True)])
+@pytest.mark.parametrize("ids64", [False, True])
+def test_layer_in_one_call_equals_launches(dev, topk, variant, act_order, ids64):
+    from vllm_amd.fused_marlin_moe import fused_marlin_moe
+    from vllm_amd.scalar_type import scalar_types
+    m, e, k, n = 21, 4, 256, 256
+    dtype = torch.bfloat16 if "bf16" in variant else torch.float16
+    zp = variant.startswith("awq")
+    ops_ = [make_experts(e, kk, nn, 128, dtype, zp, act_order, seed=s) for kk, nn, s in ((k, 2 * n, 1), (n, k, 2))]
+    (_, q1, s1, z1, g1, p1), (_, q2, s2, z2, g2, p2) = [tuple(t.to(dev) if torch.is_tensor(t) else t for t in o) for o in ops_]
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(4)).to(dtype).to(dev)
+    ids = rand_topk(m, topk, e, seed=6).to(dev)
+    tw = torch.rand(m, topk, generator=torch.Generator().manual_seed(7)).to(dev)
+    kw = dict(quant_type_id=(scalar_types.uint4 if zp else scalar_types.uint4b8).id, global_num_experts=e,
+              w1_zeros=z1 if zp else None, w2_zeros=z2 if zp else None, g_idx1=g1, g_idx2=g2, sort_indices1=p1, sort_indices2=p2)
+    args = (x, q1, q2, None, None, s1, s2, None, tw, ids.long() if ids64 else ids)
+    got = fused_marlin_moe(*args, **kw)
+    want = fused_marlin_moe(*args, output=torch.empty_like(x), **kw)
+    assert torch.equal(got, want) and float(got.float().abs().max()) > 0

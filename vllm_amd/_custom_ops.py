@@ -140,6 +140,11 @@ _register()
 # (x, qweight, scales, zeros, g_idx, sort_indices, workspace, type id, N, K, is_k_full, bias, use_fp32_reduce) -> output, or
 # None when the call has to go through the dispatcher
 eager_linear = _native.linear if "_C::gptq_marlin_gemm" in REGISTERED else lambda *args: None
+# the same for routing, (gating_output, topk, renormalize) -> (weights, ids, source rows), and for a whole MoE layer (arguments at
+# py_moe in torch_ops.cpp)
+eager_topk = _native.topk if "_moe_C::topk_softmax" in REGISTERED else lambda *args: None
+eager_moe = (_native.moe if {"_moe_C::moe_align_block_size", "_moe_C::moe_wna16_marlin_gemm", "_moe_C::moe_sum"} <= set(REGISTERED)
+             else lambda *args: None)
 
 
 # ----------------------------------------------------------------- wrappers (reference names)

@@ -5,8 +5,8 @@
 // Why native: the 16-row GEMM of a decode projection runs 5.6-10 us, its launch costs the host about 2 us, and the same
 // checks written in Python with a ctypes call cost 28 us per call, so every decode call was bound by the host.
 //
-// `linear` at the end is a direct entry for eager calls on plain GPU tensors; it skips the dispatcher
-// (boxing of 18 arguments: 7.1 -> 5.2 us per call) and returns None when anything may want to see the operator (a tensor subclass,
+// `linear`, `topk` and `moe` at the end are direct entries for eager calls on plain GPU tensors; they skip the dispatcher
+// (boxing of 18 arguments: 7.1 -> 5.2 us per linear) and return None when anything may want to see the operator (a tensor subclass,
 // a dispatch or trace mode, the profiler, autograd): the caller then goes through torch.ops.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -560,8 +560,92 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// The tensors at `at` (None -> null) unpacked, or false: something there is not for this path.
+bool plain_args(PyObject* const* args, std::initializer_list<int> at, const Tensor** out) {
+  for (const int i : at) {
+    PyObject* o = args[i];
+    if (o != Py_None) {
+      if (!THPVariable_Check(o)) return false;
+      out[i] = &THPVariable_Unpack(o);
+      if (!plain(*out[i])) return false;
+    }
+  }
+  return true;
+}
+
+// topk(gating_output, topk, renormalize) -> (weights fp32, ids int32, source rows int32), each [tokens, topk], or None: not a call
+// for this path.
+PyObject* py_topk(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(nargs == 3, "topk: 3 arguments");
+  const Tensor* t[1] = {};
+  if (!nobody_listens() || !plain_args(args, {0}, t) || !t[0] || t[0]->dim() != 2 || !t[0]->is_contiguous()) Py_RETURN_NONE;
+  const int64_t topk = PyLong_AsLongLong(args[1]);
+  if (PyErr_Occurred()) return nullptr;
+  const bool renormalize = args[2] == Py_True;
+  Tensor w, ids, rows;
+  {
+    pybind11::gil_scoped_release nogil;
+    const auto i32 = t[0]->options().dtype(at::kInt);
+    w = at::empty({t[0]->size(0), topk}, t[0]->options().dtype(at::kFloat));
+    ids = at::empty({t[0]->size(0), topk}, i32);
+    rows = at::empty({t[0]->size(0), topk}, i32);
+    topk_softmax(w, ids, rows, *t[0], renormalize);
+  }
+  PyObject* out = PyTuple_New(3);
+  if (!out) return nullptr;
+  PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(w)));
+  PyTuple_SET_ITEM(out, 1, THPVariable_Wrap(std::move(ids)));
+  PyTuple_SET_ITEM(out, 2, THPVariable_Wrap(std::move(rows)));
+  return out;
+  END_HANDLE_TH_ERRORS
+}
+
+// moe(x, w1, w2, bias1, bias2, scales1, scales2, zeros1, zeros2, gscale1, gscale2, g_idx1, g_idx2, sort1, sort2, topk_weights,
+//     topk_ids, workspace, type_id, block, num_experts, weight_on_input, is_k_full) -> [M, K], or None: not a call for this path.
+// The launches of fused_marlin_moe's Python (align, GEMM1 with SiLU-and-mul, GEMM2, the top-k sum) for its default arguments:
+// a layer of small experts takes the GPU 30-60 us at a few tokens, those calls took the host 52-71 us, with the routing, from here 28-30.
+PyObject* py_moe(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(nargs == 23, "moe: 23 arguments");
+  const Tensor* t[18] = {};
+  if (!nobody_listens() || !plain_args(args, {0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17}, t)) Py_RETURN_NONE;
+  for (const int i : {0, 1, 2, 5, 6, 15, 16, 17})
+    if (!t[i]) Py_RETURN_NONE;
+  const Tensor &x = *t[0], &w1 = *t[1], &w2 = *t[2], &tw = *t[15], &ids = *t[16];
+  const int64_t q_type = PyLong_AsLongLong(args[18]), block = PyLong_AsLongLong(args[19]), experts = PyLong_AsLongLong(args[20]);
+  if (PyErr_Occurred()) return nullptr;
+  const bool weight_on_input = args[21] == Py_True, k_full = args[22] == Py_True;
+  if (x.dim() != 2 || w2.dim() != 3 || ids.dim() != 2 || ids.scalar_type() != at::kInt || !ids.is_contiguous()) Py_RETURN_NONE;
+  const int64_t m = x.size(0), k = x.size(1), n = w2.size(1) * 16, topk = ids.size(1), slots = m * topk;
+  if (m == 0 || topk < 1 || n % 64 != 0) Py_RETURN_NONE;  // (the fused activation pairs n-tiles of 64 columns)
+  Tensor out;
+  {
+    pybind11::gil_scoped_release nogil;
+    const auto i32 = ids.options();
+    const auto opt = [&](int i) { return t[i] ? OptTensor(*t[i]) : OptTensor(); };
+    const int64_t sorted_len = slots + experts * (block - 1);
+    const Tensor sorted = at::empty({sorted_len}, i32), owners = at::empty({(sorted_len + block - 1) / block}, i32),
+                 padded = at::empty({1}, i32);
+    moe_align_block_size(ids, experts, block, sorted, owners, padded);
+    const Tensor act = at::empty({slots, n}, x.options());
+    out = at::empty({m, k}, x.options());
+    const bool sum2 = topk == 2;
+    moe_gemm(x, act, w1, opt(3), *t[5], opt(9), opt(7), opt(11), opt(13), *t[17], sorted, owners, padded, tw, block, topk,
+             weight_on_input, q_type, m, 2 * n, k, k_full, false, true, false, true, 0, sum2 ? OptTensor(out) : OptTensor());
+    const Tensor y = topk <= 2 ? out : at::empty({slots, k}, x.options());
+    moe_gemm(act, y, w2, opt(4), *t[6], opt(10), opt(8), opt(12), opt(14), *t[17], sorted, owners, padded, tw, block, 1,
+             !weight_on_input, q_type, slots, k, n, k_full, false, true, false, false, sum2 ? 2 : 0, std::nullopt);
+    if (topk > 2) moe_sum(y.view({m, topk, k}), out);
+  }
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef kMethods[] = {{"register_impl", py_register_impl, METH_VARARGS, "attach the native implementation of an operator"},
                           {"linear", (PyCFunction)(void*)py_linear, METH_FASTCALL, "direct eager W4A16 linear"},
+                          {"topk", (PyCFunction)(void*)py_topk, METH_FASTCALL, "direct eager routing"},
+                          {"moe", (PyCFunction)(void*)py_moe, METH_FASTCALL, "direct eager fused MoE layer"},
                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_torch_ops", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

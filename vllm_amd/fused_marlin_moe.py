@@ -196,13 +196,24 @@ def fused_marlin_moe(hidden_states, w1, w2, bias1, bias2, w1_scale, w2_scale, ga
     _check_layer(k, w1, w2, quant_type, hidden_states.dtype)
     num_local = w1.size(0)
     topk = topk_ids.size(1)
-    bs = pick_block_size(m, topk, num_local, (w1[0].numel() + w2[0].numel()) * 4,
+    bs = pick_block_size(m, topk, num_local, (w1.numel() + w2.numel()) // num_local * 4,
                          _tall_blocks(quant_type, k, marlin_moe_intermediate_size(w1, w2), w1_scale, w2_scale, is_k_full))
+    if workspace is None:
+        workspace = marlin_make_workspace_new(hidden_states.device, 4)
+    # (eager calls with the defaults: one native call for the whole layer, which declines when anything has to see the operators)
+    if (not torch.compiler.is_compiling() and activation == "silu" and activation_func is default_activation_func and
+            moe_sum is None and expert_map is None and output is None and not inplace and intermediate_cache13 is None and intermediate_cache2 is None):
+        out = ops.eager_moe(hidden_states, w1, w2, bias1, bias2, w1_scale, w2_scale, w1_zeros, w2_zeros, global_scale1,
+                            global_scale2, g_idx1, g_idx2, sort_indices1, sort_indices2, topk_weights, topk_ids, workspace,
+                            quant_type_id, bs, num_local if global_num_experts == -1 else global_num_experts,
+                            apply_router_weight_on_input, is_k_full)
+        if out is not None:
+            return out
     sorted_ids, expert_ids, post_pad = moe_align_block_size(
         topk_ids, bs, num_local if global_num_experts == -1 else global_num_experts, expert_map)
     ex = _Experts(quant_type, (w1, w2), (w1_scale, w2_scale), (bias1, bias2), (global_scale1, global_scale2),
                   (w1_zeros, w2_zeros), (g_idx1, g_idx2), (sort_indices1, sort_indices2), is_k_full,
-                  workspace if workspace is not None else marlin_make_workspace_new(hidden_states.device, 4))
+                  workspace)
     rt = _Routing(sorted_ids, expert_ids, post_pad, topk_weights, bs, topk, expert_map is not None)
     return _run_experts(hidden_states, ex, rt, apply_router_weight_on_input, activation, activation_func, moe_sum,
                         hidden_states if inplace else output, intermediate_cache2, intermediate_cache13, True)

@@ -9,6 +9,10 @@ def fused_topk(hidden_states: torch.Tensor, gating_output: torch.Tensor, topk: i
                indices_type: torch.dtype | None = None) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Returns (topk_weights fp32 [M, topk], topk_ids [M, topk], token_expert_indices int32 [M, topk])."""
     assert hidden_states.size(0) == gating_output.size(0), "Number of tokens mismatch"
+    if not torch.compiler.is_compiling() and (indices_type is None or indices_type == torch.int32):
+        out = ops.eager_topk(gating_output, topk, renormalize)
+        if out is not None:
+            return out
     m = hidden_states.size(0)
     topk_weights = torch.empty(m, topk, dtype=torch.float32, device=hidden_states.device)
     topk_ids = torch.empty(m, topk, dtype=torch.int32 if indices_type is None else indices_type,
