@@ -401,3 +401,18 @@ def test_decode_more_tiles_than_compute_units(ops, dev, workspace, dtype, has_zp
         a = _a(m, size_k, dtype, dev, seed=22 + m)
         check_close(run_gemm(ops, layer, a, dev, workspace), a, layer)
     assert int(workspace.abs().sum()) == 0
+
+
+# tiles of three m-blocks (33..48 rows): the whole range's edges, K split across workgroups, groups that end inside a
+# wavefront's range, a last column pair that is half empty
+@pytest.mark.parametrize("m", [33, 40, 48])
+@pytest.mark.parametrize("k,n,group,dtype,zp", [(512, 192, 32, torch.float16, False), (1024, 28672, 128, torch.bfloat16, True),
+                                                (14336, 256, 64, torch.bfloat16, False), (768, 320, -1, torch.float16, True)])
+def test_three_row_blocks(ops, dev, workspace, m, k, n, group, dtype, zp):
+    layer = make_layer(k, n, group, dtype, has_zp=zp, seed=m + n)
+    ks = torch.randperm(k, generator=torch.Generator().manual_seed(1))[:m]
+    a = torch.zeros(m, k, dtype=dtype)
+    a[torch.arange(m), ks] = 1.0
+    assert torch.equal(run_gemm(ops, layer, a.to(dev), dev, workspace).cpu(), layer.w_ref[ks])
+    a = torch.randn(m, k, generator=torch.Generator().manual_seed(2)).to(dtype).to(dev)
+    check_close(run_gemm(ops, layer, a, dev, workspace), a, layer)

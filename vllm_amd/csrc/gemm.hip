@@ -144,6 +144,8 @@ static int make_plan(const w4a16_gemm_args* a, Plan& pl) {
   // the 64-row kernel has instantiations for all of them
   const bool mid_ok = !general_only || a->wtype == W4A16_WTYPE_FE2M1 || w8 || ((a->flags & W4A16_F_ZP_FLOAT) && !moe);
   const bool pow2_group = (pl.group_ksteps & (pl.group_ksteps - 1)) == 0;  // prefill / 64-row kernels shift
+  // the general kernel has tiles of three m-blocks for integer weights without a per-row scale lookup
+  const bool three_blocks = (!general_only || a->wtype == W4A16_WTYPE_U8B128) && pl.gm != GM_GIDX;
   if (moe && a->moe_block_size == 128) {
     // blocks of 128 slots: the prefill kernel.  One workgroup per compute unit; the tiles of the last, partly filled round of
     // the live ones are cut along K on the device (tail_split), at most one piece per compute unit.
@@ -169,11 +171,11 @@ static int make_plan(const w4a16_gemm_args* a, Plan& pl) {
   }
   if (moe) {
     const int bs = a->moe_block_size;
-    pl.mb = bs <= 16 ? 1 : bs <= 32 ? 2 : 4;
+    pl.mb = bs <= 16 ? 1 : bs <= 32 ? 2 : bs <= 48 && three_blocks ? 3 : 4;
     pl.bm = 16 * pl.mb;
     pl.mtiles = (int)ceil_div(a->n_sorted, bs);
   } else {
-    pl.mb = a->size_m <= 16 ? 1 : a->size_m <= 32 ? 2 : 4;
+    pl.mb = a->size_m <= 16 ? 1 : a->size_m <= 32 ? 2 : a->size_m <= 48 && three_blocks ? 3 : 4;
     pl.bm = 16 * pl.mb;
     pl.mtiles = (int)ceil_div(a->size_m, pl.bm);
   }

@@ -29,6 +29,9 @@
 
 namespace w4a16 {
 
+// Tiles of two and more m-blocks are bound by the vector instructions of dequantisation: per 32 K rows and 128 columns about 136
+// of them, and, when a word's constants were rebuilt for every k-step, another 30-60.  33..48 rows have tiles of three m-blocks
+// (4096 x 28672 at 37 rows, bf16 with zero points: 29.8 -> 25.8 us with both; fp16 at 48 rows 28.7 -> 26.4).
 // Wavefronts per workgroup (template parameter NW): 8; one-m-block tiles also come with 4, for launches with more
 // workgroups than compute units, where two 4-wavefront workgroups share a compute unit and each one's prologue and
 // epilogue run under the other's weight stream.
@@ -36,7 +39,7 @@ namespace w4a16 {
 template <int MB>
 struct SkinnyCfg {
   // k-steps in flight per wavefront (measured: deeper rings on the taller tiles cost registers, hence spills, and time)
-  static constexpr int D = (MB >= 4) ? 2 : (MB == 2) ? 4 : 6;
+  static constexpr int D = (MB >= 3) ? 2 : (MB == 2) ? 4 : 6;
   static constexpr int smem(int nw) { return nw * 16 * RED_RS * 4; }  // reduction slab; its head doubles as the A bounce slabs
 };
 
@@ -53,7 +56,7 @@ __global__ __launch_bounds__(NW * 64, 2) void skinny_kernel(const KParams p) {
   constexpr int BM = 16 * MB;
   // 8-bit stages hold twice the weight registers: shorter ring
   // ... and so do the variants that keep extra per-stage state (per-row scale lookup, fp4 scale records)
-  constexpr int D = (BITS == 8) ? (MB >= 4 ? 2 : 3) : ((FP4 != 0 || GM == GM_GIDX) && MB >= 2) ? 2 : SkinnyCfg<MB>::D;
+  constexpr int D = (BITS == 8) ? (MB >= 3 ? 2 : 3) : ((FP4 != 0 || GM == GM_GIDX) && MB >= 2) ? 2 : SkinnyCfg<MB>::D;
   constexpr bool UNIT = (GM == GM_CHANNEL);
   // Decode tiles (one m-block) keep the weights as raw magic numbers E+q in the MFMA and apply
   // "-(E+z)" and the group scale to the fp32 accumulator once per group (see fold() below).
@@ -225,6 +228,11 @@ __global__ __launch_bounds__(NW * 64, 2) void skinny_kernel(const KParams p) {
       s.b1h = __builtin_nontemporal_load(bp + (int64_t)(2 * ks + 1) * b_row + 1);
     }
   };
+  // integer 4-bit weights on several m-blocks: the dequantisation constants of the four word positions are kept while the scale
+  // group stays the same (bf16 has 32 of them, which a tile of four m-blocks leaves no registers for)
+  constexpr bool HOIST = (BITS == 4 && FP4 == 0 && !ZPF && GM != GM_GIDX && MB >= 2 && (MB < 4 || DT == DT_F16));
+  ColConst<DT> ccs[4];
+  int ccs_gi = -1;
   // B operands (column half 0 / 1) of Marlin word position w of a stage; unit: leave the scale out
   auto dequant_word = [&](const Stage& s, auto w_tag, auto unit_tag, u32x4& o0, u32x4& o1) {
     constexpr int w = decltype(w_tag)::value;
@@ -246,6 +254,8 @@ __global__ __launch_bounds__(NW * 64, 2) void skinny_kernel(const KParams p) {
     } else if constexpr (ZPF) {
       const uint32_t zs = as_u32(as_h2(s.zf[w]) * as_h2(s.sc[w]));
       dequant_pair_zpf(s.b0[w], s.b1[w], s.sc[w], zs, o0, o1);
+    } else if constexpr (HOIST) {
+      dequant_pair<DT, unit>(s.b0[w], s.b1[w], ccs[w], o0, o1);
     } else if constexpr (BITS == 4) {
       uint32_t z0 = 8, z1 = 8;
       if (ZP) {
@@ -411,6 +421,14 @@ __global__ __launch_bounds__(NW * 64, 2) void skinny_kernel(const KParams p) {
       gidx_word(std::integral_constant<int, 2>{});
       gidx_word(std::integral_constant<int, 3>{});
       return;
+    }
+    if constexpr (HOIST) {
+      if (s.gi != ccs_gi) {
+        ccs_gi = s.gi;
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+          ccs[w] = make_col_const<DT, UNIT>(UNIT ? 0u : s.sc[w], ZP ? (s.zq >> (4 * w)) & 0xf : 8, ZP ? (s.zq >> (4 * w + 16)) & 0xf : 8);
+      }
     }
     auto plain_word = [&](auto w_tag) {
       constexpr int w = decltype(w_tag)::value;
@@ -640,6 +658,7 @@ static skinny_fn pick_mb(int mb, int nw, bool zp, int gm) {
   switch (mb) {
     case 1: return nw == 4 ? pick_zp_gm<DT, 1, 4>(zp, gm) : pick_zp_gm<DT, 1>(zp, gm);
     case 2: return pick_zp_gm<DT, 2>(zp, gm);
+    case 3: return gm == GM_GIDX ? nullptr : pick_zp_gm<DT, 3>(zp, gm);
     default: return pick_zp_gm<DT, 4>(zp, gm);
   }
 }
@@ -654,7 +673,7 @@ static skinny_fn pick_w8_gm(int gm) {  // uint8b128: no zero points
 template <int DT>
 static skinny_fn pick_w8(int mb, int nw, int gm) {
   return mb == 1 ? (nw == 4 ? pick_w8_gm<DT, 1, 4>(gm) : pick_w8_gm<DT, 1>(gm))
-         : mb == 2 ? pick_w8_gm<DT, 2>(gm) : pick_w8_gm<DT, 4>(gm);
+         : mb == 2 ? pick_w8_gm<DT, 2>(gm) : mb == 3 ? (gm == GM_GIDX ? nullptr : pick_w8_gm<DT, 3>(gm)) : pick_w8_gm<DT, 4>(gm);
 }
 
 // (act-order never reaches a kernel as such: the host gathers A's columns in front of the launch, see gemm.hip)
