@@ -522,6 +522,18 @@ bool plain(const Tensor& t) {
   return (t.key_set().raw_repr() & ~keys) == 0 && t.is_cuda() && !(t.requires_grad() && at::GradMode::is_enabled());
 }
 
+// Flags and counts as Python's own bool and int.  The dispatcher also takes whatever has a truth value or an index (ints, numpy
+// scalars, tensors); false leaves such a call to it, so that it means the same here as there.
+bool read_flag(PyObject* o, bool* out) {
+  *out = o == Py_True;
+  return PyBool_Check(o);
+}
+bool read_int(PyObject* o, int64_t* out) {
+  int overflow = 0;
+  *out = PyLong_CheckExact(o) ? PyLong_AsLongLongAndOverflow(o, &overflow) : 0;
+  return PyLong_CheckExact(o) && !overflow;
+}
+
 // linear(x, qweight, scales, zeros, g_idx, sort_indices, workspace, type_id, size_n, size_k, is_k_full, bias, use_fp32_reduce)
 // -> [..., size_n], or None: not a call for this path.  zeros, g_idx, sort_indices and bias may be None or empty.
 PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -539,9 +551,11 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   }
   if (!t[0] || !t[1] || !t[2] || !t[6] || t[0]->dim() < 1) Py_RETURN_NONE;
   const auto some = [](const Tensor* x) { return x && x->numel() > 0 ? x : nullptr; };
-  const int64_t q_type = PyLong_AsLongLong(args[7]), n = PyLong_AsLongLong(args[8]), k = PyLong_AsLongLong(args[9]);
-  if (PyErr_Occurred()) return nullptr;
-  const bool k_full = args[10] == Py_True, fp32_reduce = args[12] == Py_True;
+  int64_t q_type, n, k;
+  bool k_full, fp32_reduce;
+  if (!read_int(args[7], &q_type) || !read_int(args[8], &n) || !read_int(args[9], &k) || !read_flag(args[10], &k_full) ||
+      !read_flag(args[12], &fp32_reduce))
+    Py_RETURN_NONE;
   const Tensor& x = *t[0];
   const Tensor* zeros = t[3] && t[3]->size(-1) > 0 ? t[3] : nullptr;
   Tensor y;
@@ -580,9 +594,9 @@ PyObject* py_topk(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   TORCH_CHECK(nargs == 3, "topk: 3 arguments");
   const Tensor* t[1] = {};
   if (!nobody_listens() || !plain_args(args, {0}, t) || !t[0] || t[0]->dim() != 2 || !t[0]->is_contiguous()) Py_RETURN_NONE;
-  const int64_t topk = PyLong_AsLongLong(args[1]);
-  if (PyErr_Occurred()) return nullptr;
-  const bool renormalize = args[2] == Py_True;
+  int64_t topk;
+  bool renormalize;
+  if (!read_int(args[1], &topk) || !read_flag(args[2], &renormalize)) Py_RETURN_NONE;
   Tensor w, ids, rows;
   {
     pybind11::gil_scoped_release nogil;
@@ -613,9 +627,11 @@ PyObject* py_moe(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   for (const int i : {0, 1, 2, 5, 6, 15, 16, 17})
     if (!t[i]) Py_RETURN_NONE;
   const Tensor &x = *t[0], &w1 = *t[1], &w2 = *t[2], &tw = *t[15], &ids = *t[16];
-  const int64_t q_type = PyLong_AsLongLong(args[18]), block = PyLong_AsLongLong(args[19]), experts = PyLong_AsLongLong(args[20]);
-  if (PyErr_Occurred()) return nullptr;
-  const bool weight_on_input = args[21] == Py_True, k_full = args[22] == Py_True;
+  int64_t q_type, block, experts;
+  bool weight_on_input, k_full;
+  if (!read_int(args[18], &q_type) || !read_int(args[19], &block) || !read_int(args[20], &experts) ||
+      !read_flag(args[21], &weight_on_input) || !read_flag(args[22], &k_full))
+    Py_RETURN_NONE;
   if (x.dim() != 2 || w2.dim() != 3 || ids.dim() != 2 || ids.scalar_type() != at::kInt || !ids.is_contiguous()) Py_RETURN_NONE;
   const int64_t m = x.size(0), k = x.size(1), n = w2.size(1) * 16, topk = ids.size(1), slots = m * topk;
   if (m == 0 || topk < 1 || n % 64 != 0) Py_RETURN_NONE;  // (the fused activation pairs n-tiles of 64 columns)
