@@ -1,5 +1,5 @@
 """The direct eager entries (`linear`, `topk`, `moe` of csrc/torch_ops.cpp) against the operators they stand in for: they take
-plain calls and leave to the dispatcher every call whose arguments it would convert."""
+plain calls and leave to the dispatcher every call that something else has to see, or whose arguments it would convert."""
 import numpy as np
 import pytest
 import torch
@@ -72,6 +72,7 @@ def same(a, b):
 
 
 NAMES = ["linear", "topk", "moe"]
+OPERATOR = {"linear": "gptq_marlin_gemm", "topk": "topk_softmax", "moe": "moe_sum"}
 
 
 @pytest.mark.parametrize("name", NAMES)
@@ -101,3 +102,67 @@ def test_counts_that_are_not_ints(calls):
     assert same(calls.topk(topk=np.int64(TOPK)), calls.topk())
     with pytest.raises((TypeError, RuntimeError)):
         calls.topk(topk=2.0)
+
+
+class Tagged(torch.Tensor):
+    seen: list = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.seen.append(str(func))
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_tensor_subclass_sees_the_operator(calls, name):
+    want = getattr(calls, name)()
+    Tagged.seen = []
+    got = getattr(calls, name)(calls.input(name).as_subclass(Tagged))
+    assert not calls.taken[name] and any(OPERATOR[name] in s or "moe_marlin_gemm_fused" in s for s in Tagged.seen)
+    assert same(got, want)
+    if name == "linear":
+        assert type(got) is Tagged
+
+
+@pytest.mark.parametrize("name", NAMES)
+@pytest.mark.parametrize("kind", ["function", "dispatch", "profiler"])
+def test_modes_see_the_operator(calls, name, kind):
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    want, seen = getattr(calls, name)(), []
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    if kind == "profiler":
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+            got = getattr(calls, name)()
+        seen += [e.key for e in prof.key_averages()]
+    else:
+        with (Function if kind == "function" else Dispatch)():
+            got = getattr(calls, name)()
+    assert not calls.taken[name] and any(OPERATOR[name] in s or "moe_marlin_gemm_fused" in s for s in seen), seen
+    assert same(got, want)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_autograd_goes_through_the_dispatcher(calls, name):
+    want = getattr(calls, name)()
+    got = getattr(calls, name)(calls.input(name).clone().requires_grad_())
+    assert not calls.taken[name]
+    assert same([t.detach() for t in got] if name == "topk" else got.detach(), list(want) if name == "topk" else want)
+
+
+def test_vmap_goes_through_the_dispatcher(calls):
+    x = torch.stack([calls.x, calls.x + 1, calls.x * 2])
+    want = torch.stack([calls.linear(r) for r in x])
+    got = torch.vmap(calls.linear)(x)
+    assert not calls.taken["linear"]
+    assert torch.equal(got, want)

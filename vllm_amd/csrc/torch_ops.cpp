@@ -7,11 +7,13 @@
 //
 // `linear`, `topk` and `moe` at the end are direct entries for eager calls on plain GPU tensors; they skip the dispatcher
 // (boxing of 18 arguments: 7.1 -> 5.2 us per linear) and return None when anything may want to see the operator (a tensor subclass,
-// a dispatch or trace mode, the profiler, autograd): the caller then goes through torch.ops.
+// a function, dispatch or trace mode, the profiler, autograd) or an argument is one the dispatcher would convert: the caller then
+// goes through torch.ops.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/grad_mode.h>
 #include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
@@ -510,11 +512,12 @@ PyObject* py_register_impl(PyObject*, PyObject* args) {
 }
 
 // ------------------------------------------------------------------------------------------ direct eager entry
-// Nothing but the CUDA kernel wants to see the call: no dispatch mode, tracer or profiler is on, and the tensor carries
-// no key beyond an ordinary GPU tensor's and needs no gradient.
+// Nothing but the CUDA kernel wants to see the call: no function or dispatch mode, tracer or profiler is on; the tensor is a
+// Tensor or Parameter itself (a subclass with only __torch_function__ has the keys of a plain tensor, so its type is looked at),
+// carries no key beyond an ordinary GPU tensor's and needs no gradient.
 bool nobody_listens() {
   const uint64_t on = c10::impl::tls_local_dispatch_key_set().included_.raw_repr();
-  return (on & ~c10::default_included_set.raw_repr()) == 0 && !at::hasCallbacks();
+  return (on & ~c10::default_included_set.raw_repr()) == 0 && !at::hasCallbacks() && !at::impl::torch_function_mode_enabled();
 }
 bool plain(const Tensor& t) {
   static const uint64_t keys = (c10::DispatchKeySet(c10::DispatchKey::CUDA) | c10::autocast_dispatch_keyset |
@@ -545,7 +548,7 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   for (int i = 0; i < 8; ++i) {
     PyObject* o = args[at_arg[i]];
     if (o == Py_None) continue;
-    if (!THPVariable_Check(o)) Py_RETURN_NONE;
+    if (!THPVariable_CheckExact(o)) Py_RETURN_NONE;
     t[i] = &THPVariable_Unpack(o);
     if (!plain(*t[i])) Py_RETURN_NONE;
   }
@@ -579,7 +582,7 @@ bool plain_args(PyObject* const* args, std::initializer_list<int> at, const Tens
   for (const int i : at) {
     PyObject* o = args[i];
     if (o != Py_None) {
-      if (!THPVariable_Check(o)) return false;
+      if (!THPVariable_CheckExact(o)) return false;
       out[i] = &THPVariable_Unpack(o);
       if (!plain(*out[i])) return false;
     }
