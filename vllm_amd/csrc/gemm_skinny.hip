@@ -30,8 +30,9 @@
 namespace w4a16 {
 
 // Tiles of two and more m-blocks are bound by the vector instructions of dequantisation: per 32 K rows and 128 columns about 136
-// of them, and, when a word's constants were rebuilt for every k-step, another 30-60.  33..48 rows have tiles of three m-blocks
-// (4096 x 28672 at 37 rows, bf16 with zero points: 29.8 -> 25.8 us with both; fp16 at 48 rows 28.7 -> 26.4).
+// of them, and, where a word's constants are rebuilt for every k-step, another 30-60 (see HOIST).  33..48 rows have tiles of three
+// m-blocks (4096 x 28672, bf16 with zero points: 49 rows on tiles of four 28.7 us, 37 rows on tiles of three 25.4, 24.9 with kept
+// constants).
 // Wavefronts per workgroup (template parameter NW): 8; one-m-block tiles also come with 4, for launches with more
 // workgroups than compute units, where two 4-wavefront workgroups share a compute unit and each one's prologue and
 // epilogue run under the other's weight stream.
@@ -228,9 +229,14 @@ __global__ __launch_bounds__(NW * 64, 2) void skinny_kernel(const KParams p) {
       s.b1h = __builtin_nontemporal_load(bp + (int64_t)(2 * ks + 1) * b_row + 1);
     }
   };
-  // integer 4-bit weights on several m-blocks: the dequantisation constants of the four word positions are kept while the scale
-  // group stays the same (bf16 has 32 of them, which a tile of four m-blocks leaves no registers for)
-  constexpr bool HOIST = (BITS == 4 && FP4 == 0 && !ZPF && GM != GM_GIDX && MB >= 2 && (MB < 4 || DT == DT_F16));
+  // Integer 4-bit weights on several m-blocks: the dequantisation constants of the four word positions are kept while the scale
+  // group stays the same.  Tiles of two and three m-blocks have the registers (4096 x 28672, bf16 with zero points, 37 / 48
+  // rows: 25.4 / 26.7 -> 24.9 / 25.9 us; fp16 within 1 %).  Tiles of four keep them in fp16 with channel-wise scales only, where
+  // nothing is reloaded (49 / 64 rows, zero points: 26.8 / 28.8 -> 26.0 / 27.9 us).  With grouped scales they lose there: bf16
+  // would hold 32 registers of constants; fp16 with zero points spills 19 (49 / 64 rows: 28.0 / 30.0 us without, 29.7 / 31.7
+  // with; 4096 x 4096 at 160 rows 19.7 / 21.4); fp16 without zero points neither spills nor gains (4096 x 6144 at 160 / 256
+  // rows: 23.1 / 24.9 us without, 23.4 / 25.0 with).
+  constexpr bool HOIST = (BITS == 4 && FP4 == 0 && !ZPF && GM != GM_GIDX && MB >= 2 && (MB < 4 || (DT == DT_F16 && UNIT)));
   ColConst<DT> ccs[4];
   int ccs_gi = -1;
   // B operands (column half 0 / 1) of Marlin word position w of a stage; unit: leave the scale out
