@@ -187,3 +187,30 @@ def test_moe_block_size_rule():
     assert pick_block_size(100, 2, 8) == 64               # default: large experts
     assert all(pick_block_size(t, k, e, b) in (16, 64) for t in (1, 7, 300, 5000) for k in (1, 2, 8) for e in (4, 64, 256)
                for b in (small, big))
+
+
+def test_moe_blocks_of_128_by_weight_type():
+    """From how many slots per expert blocks of 128 are taken: where the dequantisation they save is dear."""
+    import torch
+    from vllm_amd.fused_marlin_moe import _tall_from, pick_block_size
+    from vllm_amd.scalar_type import scalar_types as st
+
+    def tall_from(wtype, dtype, group, k=4096, n=14336, k_full=True):
+        scale = lambda kk: torch.empty(1, 1 if group == -1 else kk // group, 1, dtype=dtype)  # noqa: E731
+        return _tall_from(wtype, k, n, scale(k), scale(n), k_full)
+
+    fp16, bf16 = torch.float16, torch.bfloat16
+    for group in (128, 256, -1):
+        assert tall_from(st.uint4b8, bf16, group) == tall_from(st.uint4, bf16, group) == 192
+    assert tall_from(st.uint4, fp16, 128) == 192 and tall_from(st.uint4, fp16, -1) == 384
+    assert tall_from(st.uint4b8, fp16, 128) == 192 and tall_from(st.uint4b8, fp16, 128, n=8192) == 192
+    assert tall_from(st.uint4b8, fp16, 128, n=4096) == 384 and tall_from(st.uint4b8, fp16, -1) == 0
+    for group in (32, 64):
+        assert tall_from(st.uint4b8, bf16, group) == tall_from(st.uint4, fp16, group) == 384
+        assert tall_from(st.uint4b8, fp16, group) == 0
+    # what the kernel does not take: other types, partial K, other K, groups that are not powers of two
+    assert tall_from(st.uint8b128, bf16, 128) == 0 and tall_from(st.uint4b8, bf16, 128, k_full=False) == 0
+    assert tall_from(st.uint4b8, bf16, 128, k=2048) == 0 and tall_from(st.uint4b8, bf16, 32, k=4128) == 0
+    assert tall_from(st.uint4b8, bf16, 96, k=4608, n=4608) == 0
+    assert pick_block_size(768, 2, 8, tall_from=192) == 128 and pick_block_size(767, 2, 8, tall_from=192) == 64
+    assert pick_block_size(4096, 2, 8, tall_from=0) == 64

@@ -29,7 +29,7 @@ from .scalar_type import ScalarType, scalar_types
 
 _MOE_WEIGHT_TYPES = (scalar_types.uint4, scalar_types.uint4b8, scalar_types.uint8b128, scalar_types.float8_e4m3fn,
                      scalar_types.float4_e2m1f)
-_BLOCK_SIZES = (8, 16, 32, 48, 64)  # token slots per expert block the MoE GEMM accepts for every weight type; 128: see _tall_blocks
+_BLOCK_SIZES = (8, 16, 32, 48, 64)  # token slots per expert block the MoE GEMM accepts for every weight type; 128: see _tall_from
 
 
 def default_activation_func(activation: str, output: torch.Tensor, input: torch.Tensor) -> None:
@@ -38,29 +38,47 @@ def default_activation_func(activation: str, output: torch.Tensor, input: torch.
     ops.silu_and_mul(output, input)
 
 
-def _tall_blocks(quant_type: ScalarType, k: int, n: int, w1_scale, w2_scale, is_k_full: bool) -> bool:
-    """Whether blocks of 128 slots (the prefill kernel) can and should run both GEMMs [., k] x [k, 2n] and [., n] x [n, k].
-    Integer 4-bit weights, whole power-of-two groups, K a multiple of 128; and both K of 4096 or more: the kernel keeps one
-    workgroup per compute unit, so every tile pays for its start and its epilogue (64 experts of 2048 x 1408 at 384 rows each:
-    663 us against 569 with blocks of 64, whose two workgroups per compute unit hide them)."""
+def _tall_from(quant_type: ScalarType, k: int, n: int, w1_scale, w2_scale, is_k_full: bool) -> int:
+    """Slots per expert from which blocks of 128 slots (the prefill kernel) should run both GEMMs [., k] x [k, 2n] and
+    [., n] x [n, k]; 0: never.  The kernel takes integer 4-bit weights, whole power-of-two groups, K a multiple of 128.  It
+    dequantises every weight once per 128 rows instead of once per 64, but keeps one workgroup per compute unit, so every tile
+    pays for its start and its epilogue.  Time over that with blocks of 64, 8-32 experts of 4096 x 4096 to 6144 x 10752:
+
+                                      192-256 slots  384-1024 slots
+      bf16 or zero points, group 128    0.84 - 1.03    0.83 - 1.02    from 192
+      bf16, channel-wise                0.88 - 0.99    0.84 - 0.96    from 192
+      fp16 zero points, channel-wise    0.96 - 1.02    0.92 - 1.05    from 384 (mean 0.99 / 0.97)
+      bf16 or zero points, group 32/64  0.95 - 1.07    0.90 - 1.07    from 384 (mean 1.02 / 0.97)
+      fp16 uint4b8, group 128           0.95 - 1.07    0.95 - 1.07    from 384 (mean 1.02 / 0.99)
+        with k * n >= 4096 * 8192       0.95 - 1.02    0.93 - 0.98    from 192
+      fp16 uint4b8, others              1.02 - 1.11    0.93 - 1.12    never (mean 1.05 / 1.01): the cheapest dequantisation
+
+    The spread inside a row is how the tiles fill their last round.  With a K below 4096 the sides cross: 64 experts of 2048 x 1408
+    1.02 - 1.17, 32 of 4096 x 2048 0.94 - 1.05, while bf16 gains on 16 of 2048 x 8192 and 64 of 7168 x 2048 (0.89 - 0.94)."""
     if quant_type not in (scalar_types.uint4, scalar_types.uint4b8) or not is_k_full or min(k, n) < 4096 or k % 128 or n % 128:
-        return False
-    groups = ((k, w1_scale.size(1)), (n, w2_scale.size(1)))
-    return all(g == 1 or (kk % g == 0 and (kk // g) % 32 == 0 and (kk // g) & (kk // g - 1) == 0) for kk, g in groups)
+        return 0
+    rows = []  # K rows per scale row
+    for kk, g in ((k, w1_scale.size(1)), (n, w2_scale.size(1))):
+        if g > 1 and (kk % g or kk // g % 32 or kk // g & (kk // g - 1)):
+            return 0
+        rows.append(kk // g)
+    fp16, fine, channel = w1_scale.dtype == torch.float16, min(rows) < 128, rows[0] == k or rows[1] == n
+    if fp16 and quant_type == scalar_types.uint4b8:
+        return 0 if fine or channel else 192 if k * n >= 4096 * 8192 else 384
+    return 384 if fine or (fp16 and channel) else 192
 
 
-def pick_block_size(tokens: int, topk: int, num_experts: int, expert_bytes: int = 1 << 30, tall: bool = False) -> int:
+def pick_block_size(tokens: int, topk: int, num_experts: int, expert_bytes: int = 1 << 30, tall_from: int = 0) -> int:
     """Token slots per expert block, from the average expert's share of the slots (the quantity the reference's rule
     uses, fused_marlin_moe.py:279-282), fitted to the kernels behind each size on MI355X: blocks of 16 slots run on the
     weight-streaming kernel, whose cost is one pass over the expert's weights per block; blocks of 64 on the 64-row
     kernel, which costs about two such passes per block, so it wins once an expert fills more than one and a quarter
     blocks of 16 (sooner for experts of a few MB, where the per-block fixed costs count).  Blocks of 8 never beat 16,
-    and 32 / 48 lost their niche (few, large experts) when the 64-row kernel began to split K for a thin last round.
-    tall (see _tall_blocks): blocks of 128 from 192 slots per expert; every weight is then dequantised once per 128 rows
-    (8 experts of 4096 x 14336, bf16: 1024 / 512 / 256 slots each 3159 / 1700 / 1004 -> 2702 / 1427 / 931 us; at 128 slots
-    the half-empty last blocks cost as much: 565 / 583)."""
+    and 32 / 48 lost their niche (few, large experts) when the 64-row kernel began to split K for a thin last round (48 was timed
+    as four row blocks; on tiles of three it has not been).
+    tall_from: blocks of 128 from so many slots per expert (see _tall_from); 0: never."""
     per_expert = tokens * topk / num_experts
-    if tall and per_expert >= 192:
+    if tall_from and per_expert >= tall_from:
         return 128
     return 16 if per_expert < (20 if expert_bytes >= (12 << 20) else 14) else 64
 
@@ -197,7 +215,7 @@ def fused_marlin_moe(hidden_states, w1, w2, bias1, bias2, w1_scale, w2_scale, ga
     num_local = w1.size(0)
     topk = topk_ids.size(1)
     bs = pick_block_size(m, topk, num_local, (w1.numel() + w2.numel()) // num_local * 4,
-                         _tall_blocks(quant_type, k, marlin_moe_intermediate_size(w1, w2), w1_scale, w2_scale, is_k_full))
+                         _tall_from(quant_type, k, marlin_moe_intermediate_size(w1, w2), w1_scale, w2_scale, is_k_full))
     if workspace is None:
         workspace = marlin_make_workspace_new(hidden_states.device, 4)
     # (eager calls with the defaults: one native call for the whole layer, which declines when anything has to see the operators)
