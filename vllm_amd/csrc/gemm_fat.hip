@@ -14,7 +14,7 @@
 // of dequantisation (about 105 instructions per 64 MFMAs for fp16) is interleaved with them: the MFMAs run
 // word-major (16 per Marlin word), and as soon as a word's operands are dead the next k-step's word is
 // dequantised into the same registers.
-// MoE blocks of 128 sorted slots run here too when experts are large and full (pick_block_size): the 64-row kernel dequantises
+// MoE blocks of 128 sorted slots run here too when experts are large and full (_tall_from in fused_marlin_moe.py): the 64-row kernel dequantises
 // every weight once per 64 rows (8 experts of 4096 x 14336, top-2, 4096 tokens, bf16: GEMM1 2129 -> 1815 us, GEMM2 1011 -> 874).
 // Requirements (host-checked; otherwise the skinny kernel runs): K % 128 == 0, no per-row g_idx.
 #include <type_traits>
@@ -24,10 +24,8 @@
 namespace w4a16 {
 
 constexpr int FB_MB = 8;     // m-blocks per wavefront
-constexpr int FB_BM = 128;   // rows per workgroup tile
 constexpr int FB_D = 4;      // weight k-steps in flight per wavefront
 constexpr int FB_ABUF = 2 * FB_MB * 64 * 16;  // bytes of one A buffer: 2 k-steps x 8 m-blocks x 64 lanes x 16 B
-constexpr int FB_MIN_SPLIT = 2;  // tail tiles are cut in K pieces as soon as two of each fit the compute units
 constexpr int FB_SLABS = 4 * 16 * RED_RS * 4;                // four wavefront slabs of the epilogue
 constexpr int FB_SMEM = (2 * FB_ABUF > FB_SLABS ? 2 * FB_ABUF : FB_SLABS) + FB_BM * 8;  // + C row and routing weight of each tile row
 
@@ -522,7 +520,7 @@ int launch_fat(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
   const int64_t grid = pl.tiles + (moe ? mid_tail_pieces(pl.tiles, pl.dyn_slots) : 0);
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), FB_SMEM, stream, p);
   W4A16_HIP(hipGetLastError());
-  if (moe) return launch_tail_reduce(a, pl, p, FB_BM, FB_MIN_SPLIT, stream);
+  if (moe) return launch_fat_reduce(a, pl, p, stream);
   return 0;
 }
 

@@ -209,8 +209,12 @@ inline hipError_t allow_dynamic_lds(const void* fn, int bytes) {
   return hipSuccess;
 }
 
-// Second pass of a MoE launch whose tail tiles (bm rows) were cut along K on the device (gemm_mid.hip).
-int launch_tail_reduce(const w4a16_gemm_args* a, const Plan& pl, const KParams& p, int bm, int min_split, hipStream_t stream);
+// Prefill kernel: rows per workgroup tile; MoE: the tail tiles are cut in K pieces as soon as two of each fit the compute units
+constexpr int FB_BM = 128;
+constexpr int FB_MIN_SPLIT = 2;
+
+// Second pass of its MoE launches: adds the pieces of the tail tiles (gemm_mid.hip)
+int launch_fat_reduce(const w4a16_gemm_args* a, const Plan& pl, const KParams& p, hipStream_t stream);
 
 // Host: translate the C-ABI arguments and the launch plan into the kernel parameter block.
 inline KParams make_kparams(const w4a16_gemm_args* a, const Plan& pl) {

@@ -439,9 +439,9 @@ __global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
   }
 }
 
-// Second pass of a split-K launch of mid_kernel (BM = 64) or of the prefill kernel on MoE blocks (BM = 128): out tile = sum over splits of the fp32 partial tiles (in split order,
-// so the result does not depend on timing), then channel scale, bias, routing weight, conversion and the row scatter
-// exactly as mid_kernel's own epilogue does.  One workgroup per (tile, 16-row block); thread -> 4 columns of 2 rows per pass.
+// Second pass of a split-K launch of mid_kernel (BM = 64) or of the prefill kernel on MoE blocks (BM = 128): out tile = sum over
+// splits of the fp32 partial tiles (in split order, so the result does not depend on timing), then channel scale, bias, routing
+// weight, conversion and the row scatter exactly as mid_kernel's own epilogue does.  One workgroup per (tile, 16-row block); thread -> 4 columns of 2 rows per pass.
 template <int DT, bool CHANNEL, bool MOE, int BM, int MIN_SPLIT>
 __global__ __launch_bounds__(256) void mid_reduce_kernel(const KParams p) {
   const int t = threadIdx.x;
@@ -567,18 +567,17 @@ static mid_fn pick_mid8(bool fp8, bool channel) {
   if (fp8) return channel ? mid_kernel<DT, false, true, MOE, 0, 8, true> : mid_kernel<DT, false, false, MOE, 0, 8, true>;
   return channel ? mid_kernel<DT, false, true, MOE, 0, 8, false> : mid_kernel<DT, false, false, MOE, 0, 8, false>;
 }
-template <int DT, bool MOE>
+template <int DT, bool MOE, int BM = MD_BM, int MIN_SPLIT = MD_MIN_SPLIT>
 static mid_fn pick_reduce(bool channel) {
-  return channel ? mid_reduce_kernel<DT, true, MOE, MD_BM, MD_MIN_SPLIT> : mid_reduce_kernel<DT, false, MOE, MD_BM, MD_MIN_SPLIT>;
+  return channel ? mid_reduce_kernel<DT, true, MOE, BM, MIN_SPLIT> : mid_reduce_kernel<DT, false, MOE, BM, MIN_SPLIT>;
 }
 
-int launch_tail_reduce(const w4a16_gemm_args* a, const Plan& pl, const KParams& p, int bm, int min_split, hipStream_t stream) {
-  if (bm != 128 || min_split != 2) return fail(W4A16_EINVAL, "unsupported kernel variant");
+int launch_fat_reduce(const w4a16_gemm_args* a, const Plan& pl, const KParams& p, hipStream_t stream) {
   const bool channel = pl.gm == GM_CHANNEL;
-  const mid_fn red = a->dtype == DT_F16 ? (channel ? mid_reduce_kernel<DT_F16, true, true, 128, 2> : mid_reduce_kernel<DT_F16, false, true, 128, 2>)
-                                        : (channel ? mid_reduce_kernel<DT_BF16, true, true, 128, 2> : mid_reduce_kernel<DT_BF16, false, true, 128, 2>);
+  const mid_fn red = a->dtype == DT_F16 ? pick_reduce<DT_F16, true, FB_BM, FB_MIN_SPLIT>(channel)
+                                        : pick_reduce<DT_BF16, true, FB_BM, FB_MIN_SPLIT>(channel);
   const int64_t tail = pl.tiles < pl.dyn_slots ? pl.tiles : pl.dyn_slots;
-  hipLaunchKernelGGL(red, dim3((unsigned)(tail * (bm / 16))), dim3(256), 0, stream, p);
+  hipLaunchKernelGGL(red, dim3((unsigned)(tail * (FB_BM / 16))), dim3(256), 0, stream, p);
   W4A16_HIP(hipGetLastError());
   return 0;
 }

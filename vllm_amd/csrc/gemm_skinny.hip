@@ -646,6 +646,7 @@ __global__ __launch_bounds__(NW * 64, 2) void skinny_kernel(const KParams p) {
 // ------------------------------------------------------------------------------------ host side
 typedef void (*skinny_fn)(const KParams);
 
+// (tiles of three m-blocks have no per-row scale lookup; the planner asks for none)
 template <int DT, int MB, int NW = 8>
 static skinny_fn pick_zp_gm(bool zp, int gm) {
   if (zp) {
@@ -653,9 +654,10 @@ static skinny_fn pick_zp_gm(bool zp, int gm) {
     if (gm == GM_CHANNEL) return skinny_kernel<DT, MB, true, GM_CHANNEL, 4, false, false, 0, NW>;
     return nullptr;
   }
+  if constexpr (MB != 3)
+    if (gm == GM_GIDX) return skinny_kernel<DT, MB, false, GM_GIDX, 4, false, false, 0, NW>;
   if (gm == GM_GROUPED) return skinny_kernel<DT, MB, false, GM_GROUPED, 4, false, false, 0, NW>;
-  if (gm == GM_CHANNEL) return skinny_kernel<DT, MB, false, GM_CHANNEL, 4, false, false, 0, NW>;
-  return skinny_kernel<DT, MB, false, GM_GIDX, 4, false, false, 0, NW>;
+  return skinny_kernel<DT, MB, false, GM_CHANNEL, 4, false, false, 0, NW>;
 }
 
 // (nw = 4 exists for one-m-block tiles only; the planner asks for it nowhere else)
@@ -664,22 +666,23 @@ static skinny_fn pick_mb(int mb, int nw, bool zp, int gm) {
   switch (mb) {
     case 1: return nw == 4 ? pick_zp_gm<DT, 1, 4>(zp, gm) : pick_zp_gm<DT, 1>(zp, gm);
     case 2: return pick_zp_gm<DT, 2>(zp, gm);
-    case 3: return gm == GM_GIDX ? nullptr : pick_zp_gm<DT, 3>(zp, gm);
+    case 3: return pick_zp_gm<DT, 3>(zp, gm);
     default: return pick_zp_gm<DT, 4>(zp, gm);
   }
 }
 
 template <int DT, int MB, int NW = 8>
 static skinny_fn pick_w8_gm(int gm) {  // uint8b128: no zero points
+  if constexpr (MB != 3)
+    if (gm == GM_GIDX) return skinny_kernel<DT, MB, false, GM_GIDX, 8, false, false, 0, NW>;
   return gm == GM_GROUPED ? skinny_kernel<DT, MB, false, GM_GROUPED, 8, false, false, 0, NW>
-         : gm == GM_CHANNEL ? skinny_kernel<DT, MB, false, GM_CHANNEL, 8, false, false, 0, NW>
-                            : skinny_kernel<DT, MB, false, GM_GIDX, 8, false, false, 0, NW>;
+                          : skinny_kernel<DT, MB, false, GM_CHANNEL, 8, false, false, 0, NW>;
 }
 
 template <int DT>
 static skinny_fn pick_w8(int mb, int nw, int gm) {
   return mb == 1 ? (nw == 4 ? pick_w8_gm<DT, 1, 4>(gm) : pick_w8_gm<DT, 1>(gm))
-         : mb == 2 ? pick_w8_gm<DT, 2>(gm) : mb == 3 ? (gm == GM_GIDX ? nullptr : pick_w8_gm<DT, 3>(gm)) : pick_w8_gm<DT, 4>(gm);
+         : mb == 2 ? pick_w8_gm<DT, 2>(gm) : mb == 3 ? pick_w8_gm<DT, 3>(gm) : pick_w8_gm<DT, 4>(gm);
 }
 
 // (act-order never reaches a kernel as such: the host gathers A's columns in front of the launch, see gemm.hip)

@@ -321,7 +321,7 @@ __global__ __launch_bounds__(256) void silu_and_mul_kernel(const uint16_t* __res
 // index), as the reference's topk_softmax (csrc/moe/topk_softmax_kernels.cu:127-211, 676-705):
 // weights are the softmax probabilities of the chosen experts, optionally renormalised to sum to 1
 // (a zero sum divides by 1); token_expert_indices[t, k] = k * num_tokens + t.
-// One wavefront per token; lane l holds experts l, l + 64, ... (PL of them, the smallest power of two that covers the experts) in
+// One wavefront per token; lane l holds experts l, l + 64, ... (PL of them: 1, 2 or 4 up to 64, 128 or 256 experts, 16 above) in
 // registers.  A pick is a maximum over the wavefront by DPP moves (no LDS crossbar), then one ballot per register from the lowest
 // expert numbers up: the lowest index among equals.  Lane k keeps pick k; weights are rescaled and written once, at the end.
 // Bound by latency (a chain of topk maxima); with 16 registers per lane whatever the expert count, two-operand butterflies through
