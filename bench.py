@@ -12,8 +12,9 @@ Also printed in the same JSON line:
   roofline      algorithmic bytes per launch / average launch duration (HIP events on the launch
                 stream) against the 8 TB/s HBM peak, for the decode kernel
   cpu_baseline  the oracle's dequantize + torch.matmul path on the host cores, bounded sample
-  detail        per-shape µs / GB/s / TFLOP/s / roofline fractions (decode M in {1,4,16,64,256},
-                prefill M = 4096 bf16 AWQ; the latter against the 2.5 PFLOP/s dense MFMA peak)
+  summary       per-shape times (decode M in {1,4,16,64,256,1024}, prefill M = 4096 bf16 AWQ, act-order, MoE layers,
+                repack) and, for decode and prefill, the fraction of the HBM or dense MFMA peak
+The whole per-shape table goes to stderr row by row and, with --table FILE, to a JSON file.
 """
 import argparse
 import json
@@ -452,6 +453,18 @@ def cpu_baseline(m, budget_s=12.0, matmul_only_budget_s=4.0):
             "host_cpus": os.cpu_count(), "cpu_model": _cpu_model()}
 
 
+def result_line(result):
+    """The JSON line: all of `result` but the per-shape table, numbers to six digits.  A line with the table is 13 400
+    characters long, more than a reader that keeps the end of the output may hold."""
+    def rounded(v):
+        if isinstance(v, float):
+            return float(f"{v:.6g}")
+        if isinstance(v, dict):
+            return {k: rounded(x) for k, x in v.items()}
+        return [rounded(x) for x in v] if isinstance(v, (list, tuple)) else v
+    return json.dumps({k: rounded(v) for k, v in result.items() if k != "detail"})
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -599,7 +612,7 @@ def main():
         "metric": "W4A16 GEMM \u00b5s + %HBM roofline (M\u226416), %MFMA peak (M=4096), Llama-3-8B shapes",
         "metric_detail": "value = algorithmic HBM bytes per second over one decode step = the four Llama-3-8B linears "
                          "(qkv, o, gate_up, down) at M=16; per-shape microseconds and roofline fractions are in "
-                         "`detail` and `summary`",
+                         "`summary`",
         "value": value, "unit": "GB/s", "n_gpus": 1, "steps": timed_steps, "warmup": args.warmup,
         "ms_per_step": sec_per_step * 1e3, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f16", "data": "synthetic",
@@ -650,6 +663,10 @@ def main():
             "prefill_bf16_awq_us": {k: round(v["us"], 1) for k, v in detail["prefill_bf16_awq"].items()},
             "prefill_bf16_awq_mfma_frac": {k: round(v["mfma_frac"], 3) for k, v in detail["prefill_bf16_awq"].items()},
         }
+        for part in ("act_order_fp16_gptq", "mixtral_moe_fp16_gptq", "fine_grained_moe_fp16_gptq", "repack",
+                     "other_weight_types_gate_up_warm"):
+            result["summary"][part + "_us"] = {k: round(v["us"], 1) for k, v in detail[part].items()}
+        result["summary"]["load_path_us_per_decoder_layer"] = round(detail["load_path"]["us_per_decoder_layer"], 1)
         # the M = 4096 half of the metric: the prefill kernel on the four bf16 AWQ layers, against the dense MFMA peak
         pf = detail["prefill_bf16_awq"]
         pf_flops = sum(2.0 * v["m"] * v["n"] * v["k"] for v in pf.values())
@@ -658,7 +675,7 @@ def main():
             "bound": "mfma", "achieved": pf_flops / pf_sec / 1e12, "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": pf_flops / pf_sec / 1e12 / MFMA_PEAK_TFLOPS, "traffic": None,
             "kernel": "w4a16::fat_kernel<bf16, zero points, grouped> (qkv also runs its last 512-column strips on "
-                      "w4a16::mid_kernel)", "launches": sum(v["launches_timed"] for v in pf.values()),
+                      "w4a16::kq_kernel)", "launches": sum(v["launches_timed"] for v in pf.values()),
             "flops_per_launch_avg": pf_flops / 4, "avg_launch_us": pf_sec / 4 * 1e6,
             "workload": "llama3-8b linears at M=4096, bf16, AWQ uint4 + uint4 zero points g128 (qkv, o, gate_up, down), "
                         "time-weighted over the four layers",
@@ -678,7 +695,7 @@ def main():
 
     if not args.no_cpu:
         result["cpu_baseline"] = cpu_baseline(m)
-    print(json.dumps(result), flush=True)
+    print(result_line(result), flush=True)
 
 
 if __name__ == "__main__":

@@ -128,6 +128,20 @@ def test_kernel_selection_rejects_unsupported_configs():
         assert not ok and "ROCm device" in why
 
 
+def test_bench_line_is_short():
+    """The result line keeps every number of the contract and leaves the per-shape table out."""
+    import json
+    import bench
+    row = {"us": 12.345678901234, "GBps": 1234.5678901234, "TFLOPs": 1.23456789012e-07, "n": 4096}
+    result = {"metric": "m", "value": 2345.678901234, "ms_per_step": 0.0412345678, "n_gpus": 1, "vs_baseline": None,
+              "config": {"shapes_KN": [(4096, 6144)]}, "roofline": row, "detail": {str(i): row for i in range(200)}}
+    line = bench.result_line(result)
+    assert len(line) < 1000 and "\n" not in line
+    got = json.loads(line)
+    assert set(got) == set(result) - {"detail"} and got["value"] == 2345.68 and got["ms_per_step"] == 0.0412346
+    assert got["config"] == {"shapes_KN": [[4096, 6144]]} and got["roofline"]["n"] == 4096 and got["vs_baseline"] is None
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py measures one GPU; asking for more exits with a message instead of a JSON line."""
     import os
