@@ -541,3 +541,17 @@ def test_moe_gemm_blocks_of_128(dev, m, k, n, variant, foreign):
         ref = (a[rows // topk].float() @ layers[ex].w_ref.float()) * tw.flatten()[rows].unsqueeze(1)
         mtr = gr.error_metrics(out[rows], ref)
         assert mtr["max_rel"] <= tol_for(dtype) and mtr["mean_rel"] < 0.04, (ex, mtr)
+
+
+# rows whose softmax is not a number, beside one that is: experts that fill their registers and ones that do not
+@pytest.mark.parametrize("e,topk", [(8, 2), (64, 3), (128, 8), (129, 65)])
+@pytest.mark.parametrize("renormalize", [False, True])
+def test_topk_softmax_rows_without_probabilities(dev, e, topk, renormalize):
+    from vllm_amd.fused_moe import fused_topk
+    logits = torch.randn(5, e, generator=torch.Generator().manual_seed(e))
+    logits[1, 3], logits[2, 0], logits[3], logits[4, 1:] = float("nan"), float("inf"), float("-inf"), float("-inf")
+    w, ids, _ = fused_topk(torch.empty(5, 4, device=dev), logits.to(dev), topk, renormalize)
+    w, ids = w.cpu(), ids.cpu()
+    want = torch.arange(topk, dtype=torch.int32).expand(3, topk)
+    assert w[1:4].isnan().all() and torch.equal(ids[1:4], want)
+    assert w[0].isfinite().all() and w[4, 0] == 1 and torch.equal(ids[4], want[0])  # (-inf alone is a probability of 0)

@@ -379,10 +379,13 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
   }
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+  // A row with a NaN or +inf (or nothing but -inf) has no probabilities: every sum of exponentials but that is 1 or more.  It
+  // picks experts 0, 1, ... with NaN weights, so that its token's result is NaN and no id is out of range.
+  const bool bad = !(sum > 0.f);
 #pragma unroll
   for (int i = 0; i < PL; ++i) {
     const int e = lane + 64 * i;
-    v[i] = e < num_experts ? v[i] / sum : -1.f;  // probabilities are >= 0: -1 marks "not a candidate"
+    v[i] = e < num_experts ? fmaxf(v[i] / sum, 0.f) : -1.f;  // (0 for a NaN) probabilities are >= 0: -1 marks "not a candidate"
   }
   const int64_t base = (int64_t)tok * topk;
   float selected = 0.f, my_w = 0.f;
@@ -403,7 +406,7 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
       my_w = best;
       my_e = be;
       if (topk > 64) {  // more picks than lanes: kept in memory, each by the lane that rescales it
-        weights[base + k] = best;
+        weights[base + k] = bad ? __builtin_nanf("") : best;
         ids[base + k] = be;
         src_rows[base + k] = k * num_tokens + tok;
       }
@@ -412,6 +415,7 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
     for (int i = 0; i < PL; ++i)
       if (lane + 64 * i == be) v[i] = -1.f;
   }
+  if (bad) my_w = __builtin_nanf("");
   const float denom = renormalize && selected > 0.f ? selected : 1.f;
   if (topk <= 64) {
     if (lane < topk) {
