@@ -555,3 +555,35 @@ def test_topk_softmax_rows_without_probabilities(dev, e, topk, renormalize):
     want = torch.arange(topk, dtype=torch.int32).expand(3, topk)
     assert w[1:4].isnan().all() and torch.equal(ids[1:4], want)
     assert w[0].isfinite().all() and w[4, 0] == 1 and torch.equal(ids[4], want[0])  # (-inf alone is a probability of 0)
+
+
+# operands that a kernel would address as GPU memory, or past their end: refused on the host
+@pytest.mark.parametrize("what", ["perm", "sum", "silu", "weights", "ids", "rows", "workspace", "routing", "zeros"])
+def test_host_tensors_and_short_operands_are_refused(dev, what):
+    import vllm_amd.ops as ops
+    from vllm_amd.marlin_utils import marlin_make_workspace_new
+    from vllm_amd.moe_align_block_size import moe_align_block_size
+    from vllm_amd.scalar_type import scalar_types
+    m, e, topk, k, n, bs = 4, 4, 2, 256, 128, 16
+    x = torch.zeros(m, k, dtype=torch.float16, device=dev)
+
+    def route():
+        out = {"weights": torch.empty(m, topk, device=dev), "ids": torch.empty(m, topk, dtype=torch.int32, device=dev),
+               "rows": torch.empty(m, topk, dtype=torch.int32, device=dev)}
+        out[what] = out[what].cpu()
+        ops.topk_softmax(out["weights"], out["ids"], out["rows"], torch.zeros(m, e, device=dev), True)
+
+    def gemm():
+        _, q, s, z, _, _ = make_experts(e, k, n, 128, torch.float16, True, False, seed=1)
+        t = moe_align_block_size(rand_topk(m, topk, e, seed=2).to(dev), bs, e)
+        tw = torch.ones(m, topk, device=dev)
+        ws = marlin_make_workspace_new(dev, 4)
+        ops.moe_wna16_marlin_gemm(x, None, q.to(dev), None, s.to(dev), None, (z[:1] if what == "zeros" else z).to(dev), None, None,
+                                  ws.cpu() if what == "workspace" else ws, *t, tw[:-1] if what == "routing" else tw, bs, topk, True,
+                                  False, scalar_types.uint4, m, n, k, True, False, True, False)
+
+    call = {"perm": lambda: ops.permute_cols(x, torch.arange(k, dtype=torch.int32)),
+            "sum": lambda: ops.moe_sum(x.view(2, 2, k), torch.empty(2, k, dtype=x.dtype)),
+            "silu": lambda: ops.silu_and_mul(torch.empty(m, k // 2, dtype=x.dtype), x)}
+    with pytest.raises(RuntimeError):
+        call.get(what, route if what in ("weights", "ids", "rows") else gemm)()

@@ -148,7 +148,8 @@ Tensor awq_marlin_repack(const Tensor& b_q_weight, int64_t size_k, int64_t size_
 Tensor permute_cols(const Tensor& A, const Tensor& perm) {
   TORCH_CHECK(A.is_cuda() && A.dim() == 2 && A.stride(1) == 1, "A must be a 2-D GPU tensor with unit column stride");
   TORCH_CHECK(A.scalar_type() == at::kHalf || A.scalar_type() == at::kBFloat16, "A must be fp16 or bf16");
-  TORCH_CHECK(perm.scalar_type() == at::kInt && perm.is_contiguous() && perm.numel() == A.size(1), "bad perm");
+  TORCH_CHECK(perm.is_cuda() && perm.scalar_type() == at::kInt && perm.is_contiguous() && perm.numel() == A.size(1),
+              "perm must be a contiguous int32 GPU tensor with one entry per column");
   Tensor out = at::empty({A.size(0), A.size(1)}, A.options());
   if (out.numel()) {
     OnDevice on(A);
@@ -335,7 +336,7 @@ Tensor moe_gemm(const Tensor& a, const OptTensor& c_or_none, const Tensor& w, co
   if (zeros) {
     TORCH_CHECK(zeros->is_cuda() && zeros->is_contiguous() && zeros->scalar_type() == at::kInt && zeros->dim() == 3,
                 "b_zeros rank = ", zeros->dim(), " is not 3");
-    TORCH_CHECK(zeros->size(1) == groups && zeros->size(2) == size_n / 8, "b_zeros shape mismatch");
+    TORCH_CHECK(zeros->size(0) == experts && zeros->size(1) == groups && zeros->size(2) == size_n / 8, "b_zeros shape mismatch");
   }
   const int wtype = wtype_code(q_type, zeros != nullptr);
   const Tensor* bias = present(bias_or_none);
@@ -343,12 +344,15 @@ Tensor moe_gemm(const Tensor& a, const OptTensor& c_or_none, const Tensor& w, co
     TORCH_CHECK(bias->is_cuda() && bias->is_contiguous() && bias->dim() == 2 && bias->size(0) == experts && bias->size(1) == size_n &&
                     bias->scalar_type() == a.scalar_type(),
                 "b_bias must be [E, size_n]");
+  TORCH_CHECK(workspace.is_cuda() && workspace.scalar_type() == at::kInt, "workspace must be an int32 GPU tensor");
   check_gpu_i32(sorted_token_ids, "sorted_token_ids");
   check_gpu_i32(expert_ids, "expert_ids");
   check_gpu_i32(num_tokens_past_padded, "num_tokens_past_padded");
   TORCH_CHECK(expert_ids.numel() * block >= sorted_token_ids.numel() - block + 1, "expert_ids is too short for sorted_token_ids");
   TORCH_CHECK(topk_weights.is_cuda() && topk_weights.scalar_type() == at::kFloat && topk_weights.is_contiguous(),
               "topk_weights must be a contiguous fp32 GPU tensor");
+  TORCH_CHECK(!mul_topk_weights || topk_weights.numel() >= size_m * top_k, "topk_weights holds ", topk_weights.numel(),
+              " weights, the rows need ", size_m * top_k);
   const int64_t c_rows = size_m * top_k / (sum_top_k > 1 ? sum_top_k : 1), c_cols = silu_and_mul ? size_n / 2 : size_n;
   if (silu_and_mul)
     TORCH_CHECK(size_n % 128 == 0, "fused SiLU-and-mul: size_n = ", size_n, " must be 2 * d with d a multiple of 64");
@@ -446,9 +450,9 @@ void batched_moe_align_block_size(int64_t max_tokens_per_batch, int64_t block_si
 
 void moe_sum(const Tensor& input, const Tensor& output) {
   TORCH_CHECK(input.is_cuda() && input.is_contiguous() && input.dim() == 3, "input must be a contiguous [T, topk, d] GPU tensor");
-  TORCH_CHECK(output.is_contiguous() && output.scalar_type() == input.scalar_type() && output.dim() == 2 &&
+  TORCH_CHECK(output.is_cuda() && output.is_contiguous() && output.scalar_type() == input.scalar_type() && output.dim() == 2 &&
                   output.size(0) == input.size(0) && output.size(1) == input.size(2),
-              "output must be [T, d]");
+              "output must be a contiguous [T, d] GPU tensor");
   OnDevice on(input);
   check_rc(w4a16_moe_sum(input.const_data_ptr(), output.mutable_data_ptr(), input.size(0), (int32_t)input.size(1), input.size(2),
                          dtype_code(input.scalar_type()), stream_of(input)));
@@ -456,7 +460,8 @@ void moe_sum(const Tensor& input, const Tensor& output) {
 
 void silu_and_mul(const Tensor& result, const Tensor& input) {
   const int64_t d = input.size(-1) / 2;
-  TORCH_CHECK(input.is_cuda() && input.is_contiguous() && result.is_contiguous(), "tensors must be contiguous GPU tensors");
+  TORCH_CHECK(input.is_cuda() && result.is_cuda() && input.is_contiguous() && result.is_contiguous(),
+              "tensors must be contiguous GPU tensors");
   TORCH_CHECK(result.size(-1) == d && result.numel() * 2 == input.numel() && result.scalar_type() == input.scalar_type(), "shape mismatch");
   OnDevice on(input);
   check_rc(w4a16_silu_and_mul(input.const_data_ptr(), result.mutable_data_ptr(), d ? input.numel() / (2 * d) : 0, d,
@@ -468,7 +473,9 @@ void topk_softmax(const Tensor& topk_weights, const Tensor& topk_indices, const 
   TORCH_CHECK(gating_output.is_cuda() && gating_output.is_contiguous() && gating_output.dim() == 2,
               "gating_output must be a contiguous [num_tokens, num_experts] GPU tensor");
   const int64_t tokens = gating_output.size(0), experts = gating_output.size(1), topk = topk_weights.size(-1);
-  const auto shape_ok = [&](const Tensor& t) { return t.is_contiguous() && t.dim() == 2 && t.size(0) == tokens && t.size(1) == topk; };
+  const auto shape_ok = [&](const Tensor& t) {
+    return t.is_cuda() && t.is_contiguous() && t.dim() == 2 && t.size(0) == tokens && t.size(1) == topk;
+  };
   TORCH_CHECK(topk_weights.scalar_type() == at::kFloat && shape_ok(topk_weights), "topk_weights must be fp32 [num_tokens, topk]");
   TORCH_CHECK(token_expert_indices.scalar_type() == at::kInt && shape_ok(token_expert_indices),
               "token_expert_indices must be int32 [num_tokens, topk]");
