@@ -587,3 +587,8 @@ def test_host_tensors_and_short_operands_are_refused(dev, what):
             "silu": lambda: ops.silu_and_mul(torch.empty(m, k // 2, dtype=x.dtype), x)}
     with pytest.raises(RuntimeError):
         call.get(what, route if what in ("weights", "ids", "rows") else gemm)()
+
+
+@pytest.mark.parametrize("bs", [64, 128])
+def test_tall_blocks_never_use_memory_past_sorted_ids(dev, bs):
+    test_moe_gemm_never_uses_memory_past_sorted_ids(dev, bs)

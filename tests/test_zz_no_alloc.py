@@ -158,3 +158,8 @@ def test_static_scratch_moe_act_order_is_refused_when_it_does_not_fit(dev):
     assert rc == -1 and b"static buffer" in lib.w4a16_last_error()
     torch.cuda.synchronize()
     assert float(c.min()) == 7.0 and float(c.max()) == 7.0
+
+
+def test_static_scratch_moe_blocks_of_128(dev):
+    """Blocks of 128 slots (prefill kernel): the pieces of its tail tiles in the scratch."""
+    test_static_scratch_moe_gemm_matches(dev, 128, (1200, 300))
