@@ -420,8 +420,12 @@ static int make_plan(const w4a16_gemm_args* a, Plan& pl) {
         if (sp > 1 && wgs > cus) break;
         const int64_t rounds = ceil_div(wgs, cus);
         const double rate = (double)wgs / (double)rounds * wg_rate;  // workgroups resident at a time
-        // the last workgroup of a tile re-reads every split's partial tile at about one workgroup's stream rate
-        const double t_fix = sp > 1 ? t_xchg + sp * (double)(16 * mb * tn * 4) / 20e3 : 0.0;
+        // the last workgroup of a tile re-reads every split's partial tile at about one workgroup's stream rate, in rounds of four: a
+        // fifth or ninth split has a round to itself and counts twice on the general kernel's taller tiles (4 / 5 splits: 4096 x 6144,
+        // uint8b128, 64 rows 20.1 / 21.2 us; uint4b8, group 32, 48 rows 13.8 / 15.3; 8 / 9: 13440 x 1216, uint8b128, 100 rows 24.9 /
+        // 28.7.  Where K is long enough it still pays: 13568 x 1536, bf16 AWQ, 200 rows, 4 / 5 splits 30.7 / 29.3)
+        const int pieces = sp + (mb > 1 && sp % 4 == 1 ? 1 : 0);
+        const double t_fix = sp > 1 ? t_xchg + pieces * (double)(16 * mb * tn * 4) / 20e3 : 0.0;
         // HBM sees every weight byte once; further row tiles re-read the strips, from L2 at about twice that rate when
         // the whole weight fits the eight 4 MB L2s (down_proj at 64 rows: 128-column tiles with two splits take 22 us,
         // 64-column tiles without 27), else at the same rate again (gate_up: 2 row tiles cost 28 us, not 19)
