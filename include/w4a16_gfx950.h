@@ -119,7 +119,8 @@ typedef struct w4a16_gemm_args {
   const int32_t* num_tokens_past_padded; /* [1] device scalar                             */
   const float* topk_weights;             /* flat, indexed by sorted token id              */
   int64_t n_sorted;
-  int32_t moe_block_size;     /* 8 or a multiple of 16 in [16, 64]                        */
+  int32_t moe_block_size;     /* 8, a multiple of 16 in [16, 64], or 128 (integer 4-bit
+                                 weights, power-of-two groups, size_k a multiple of 128)  */
   int32_t top_k;
   int32_t num_experts;
   int32_t reserved;
