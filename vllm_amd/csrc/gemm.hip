@@ -1,6 +1,7 @@
 // Host side of the W4A16 GEMM entry points: argument checks in the spirit of the reference's
 // gptq_marlin_gemm / moe_wna16_marlin_gemm hosts (csrc/quantization/gptq_marlin/gptq_marlin.cu:674-959,
 // csrc/moe/marlin_moe_wna16/ops.cu:691-993), launch planning, kernel dispatch.
+#include <math.h>
 #include <stdlib.h>
 
 #include "gemm_kernels.h"
@@ -109,7 +110,13 @@ static int validate(const w4a16_gemm_args* a) {
   return 0;
 }
 
-static int make_plan(const w4a16_gemm_args* a, Plan& pl) {
+// Scratch of a plan: split-K partials, then the gathered copy of A (act-order), then A in two 8-bit terms
+static int64_t plan_scratch(const Plan& pl) {
+  const int64_t parts = ((pl.ctmp_bytes + 255) & ~255LL) + pl.atmp_bytes;
+  return pl.x8_bytes ? ((parts + 255) & ~255LL) + pl.x8_bytes : parts;
+}
+
+static int make_plan_16bit(const w4a16_gemm_args* a, Plan& pl) {
   const bool act_order = a->g_idx != nullptr;
   const bool k_full = (a->flags & W4A16_F_IS_K_FULL) != 0;
   pl.use_perm = act_order;
@@ -469,6 +476,107 @@ static int make_plan(const w4a16_gemm_args* a, Plan& pl) {
   return 0;
 }
 
+// ---- the 8-bit matrix unit (gemm_x8.hip): dense bf16 problems with integer 4-bit weights and scale groups of whole 128 rows (or one
+// scale per column).  Its buffer resources address a weight with 31 bits.
+static bool x8_types(const w4a16_gemm_args* a, const Plan& pl) {
+  return a->dtype == W4A16_DTYPE_BF16 && (a->wtype == W4A16_WTYPE_U4B8 || a->wtype == W4A16_WTYPE_U4) &&
+         !(a->flags & (W4A16_F_MOE | W4A16_F_ZP_FLOAT)) && pl.gm != GM_GIDX && a->size_k % 128 == 0 &&
+         (pl.gm == GM_CHANNEL || (pl.group_ksteps % 4 == 0 && (pl.group_ksteps & (pl.group_ksteps - 1)) == 0)) &&
+         a->size_k * a->size_n / 2 < (1LL << 31) && a->size_m < (1 << 24);
+}
+
+static void x8_plan(const w4a16_gemm_args* a, int mb, int ks, int tn, int sp, Plan& pl) {
+  pl.kind = 6;
+  pl.mb = mb;
+  pl.ks = ks;
+  pl.tn = tn;
+  pl.bm = 16 * mb;
+  pl.mtiles = (int)ceil_div(a->size_m, pl.bm);
+  pl.ncp = (int)ceil_div(a->size_n, tn);
+  pl.tiles = pl.mtiles * pl.ncp;
+  const int steps = (int)(a->size_k / 128), per = (int)ceil_div(steps, sp);
+  pl.splits = (int)ceil_div(steps, per);
+  pl.kps = per * 4;
+  pl.xcd_map = 0;
+  pl.tail_strips = 0;
+  pl.ctmp_bytes = pl.splits > 1 ? (int64_t)pl.tiles * pl.splits * pl.bm * tn * 4 : 0;
+  pl.x8_bytes = x8_scratch_bytes(a->size_m, a->size_k);
+}
+
+// Microseconds of a 16-bit plan for more than 128 rows of a 4-bit bf16 weight: a round of workgroups costs a fixed part and one per k-step.
+// Fitted to 384 launches (12 layer shapes x 16 row counts x uint4b8 / zero points, group 128): rms 3 (prefill, 128 x 256 tiles) to 8 %.
+static double plan16_us(const w4a16_gemm_args* a, const Plan& pl) {
+  const double cus = num_cus(), ks = (double)a->size_k / 32;
+  if (pl.kind == 2) {
+    double t = 5.1 + ceil((double)(pl.ncp - pl.tail_strips) * pl.mtiles / cus) * (9.6 + 0.793 * ks);
+    if (pl.tail_strips) t += pl.tail_kind == 5 ? 27 + 0.328 * ks : ks;
+    return t;
+  }
+  const double rounds = ceil((double)pl.tiles * pl.splits / cus), per = ks / pl.splits;
+  if (pl.kind == 5) return pl.mb == 8 ? 6.5 + rounds * (6.5 + 0.457 * per) : 5.2 + rounds * (5.2 + 0.281 * per);
+  if (pl.kind == 3) return 4.0 + rounds * (6.8 + 0.577 * per) + (pl.splits > 1 ? 2.8 : 0);
+  if (pl.kind == 0 && pl.mb == 4) return 2.0 + rounds * (6.6 + 0.156 * per) + (pl.splits > 1 ? 4.6 : 0);
+  return 0;  // 16-row tiles: not compared
+}
+
+// The same for a launch on the 8-bit unit, the pass that splits the activations included (3684 launches: 9 shapes x 15 row counts x
+// both types x every tile and split below; rms 5 %, the shape it picks within 1.3 % of the best on average).
+static double x8_us(const w4a16_gemm_args* a, int ks, int mb, int tn, int sp) {
+  const double cus = num_cus(), steps = (double)(a->size_k / 128), per = ceil(steps / sp), splits = ceil(steps / per);
+  const double wgs = (double)ceil_div(a->size_m, 16 * mb) * (double)ceil_div(a->size_n, tn) * splits;
+  double rounds = ceil(wgs / cus);
+  if (ks == 1 && tn == 256) {  // four wavefronts: two workgroups to a compute unit, one alone takes 0.62 of their time
+    const double full = floor(wgs / (2 * cus)), rest = wgs - full * 2 * cus;
+    rounds = full + (rest == 0 ? 0 : rest <= cus ? 0.62 : 1);
+  }
+  const double fixed = (ks == 1 && tn == 512 ? 11.2 : 11.0) + (a->b_zeros ? 4.4 : 0);
+  const double step = ks == 2 ? 1.01 + 0.167 * mb : tn == 512 ? 2.25 : 2.61;
+  const double fix_up = splits > 1 ? 2.9 + 0.82e-6 * splits * (double)a->size_m * (double)a->size_n : 0;
+  return 1.4 + 1.63e-6 * (double)a->size_m * (double)a->size_k + rounds * (fixed + ceil(per / ks) * step) + fix_up;
+}
+
+// Takes a 16-bit plan to the 8-bit unit where that is predicted to be 5 % and 1.5 us faster: over 270 problems (those of the fit) 11 % in
+// the mean, over 59 random ones 17 %, worst 3 % slower.  Up to 128 rows the split pass costs more than it brings.
+static void try_x8(const w4a16_gemm_args* a, Plan& pl) {
+  if (a->size_m <= 128 || !x8_types(a, pl)) return;
+  static const struct { int ks, mb, tn; } shapes[] = {{1, 8, 512}, {1, 8, 256}, {2, 8, 256}, {2, 7, 256}, {2, 6, 256}, {2, 5, 256}};
+  double best = 0.95 * plan16_us(a, pl) - 1.5;
+  const int steps = (int)(a->size_k / 128), cus = num_cus();
+  int mb = 0, ks = 0, tn = 0, sp = 0;
+  for (const auto& s : shapes) {
+    const int64_t tiles = ceil_div(a->size_m, 16 * s.mb) * ceil_div(a->size_n, s.tn);
+    for (int q : {1, 2, 3, 4, 6, 8, 12}) {
+      if (q > 1 && (tiles * q > (s.ks == 1 && s.tn == 256 ? 2 : 1) * cus || steps / q < 2 * s.ks)) break;
+      const double t = x8_us(a, s.ks, s.mb, s.tn, q);
+      if (t < best) best = t, mb = s.mb, ks = s.ks, tn = s.tn, sp = q;
+    }
+  }
+  if (mb && ceil_div(a->size_m, 16 * mb) * ceil_div(a->size_n, tn) * sp < (1LL << 31) / 64) x8_plan(a, mb, ks, tn, sp, pl);
+}
+
+static int make_plan(const w4a16_gemm_args* a, Plan& pl, bool allow_x8) {
+  if (int rc = make_plan_16bit(a, pl)) return rc;
+#ifdef W4A16_TUNING
+  static const int forced_kind = env_int("W4A16_KIND", -1);
+  if (env_int("W4A16_X8", 1) == 0) allow_x8 = false;
+  if (env_int("W4A16_DEBUG", 0) > 0)
+    fprintf(stderr, "[plan] %lld %lld %lld kind %d mb %d tn %d tiles %d mtiles %d ncp %d splits %d kps %d tail %d %d\n", (long long)a->size_k,
+            (long long)a->size_n, (long long)a->size_m, pl.kind, pl.mb, pl.tn, pl.tiles, pl.mtiles, pl.ncp, pl.splits, pl.kps, pl.tail_strips,
+            pl.tail_kind);
+  if (env_int("W4A16_X8MB", 0) > 0 && x8_types(a, pl)) {
+    const int ks = env_int("W4A16_X8KS", 1);
+    x8_plan(a, env_int("W4A16_X8MB", 8), ks, env_int("W4A16_X8TN", 512 / ks), env_int("W4A16_X8SP", 1), pl);
+    return 0;
+  }
+  if (forced_kind >= 0) allow_x8 = false;
+#endif
+  if (allow_x8) try_x8(a, pl);
+#ifdef W4A16_TUNING
+  if (env_int("W4A16_DEBUG", 0) > 0 && pl.kind == 6) fprintf(stderr, "[x8] mb %d ks %d tn %d splits %d\n", pl.mb, pl.ks, pl.tn, pl.splits);
+#endif
+  return 0;
+}
+
 }  // namespace w4a16
 
 using namespace w4a16;
@@ -477,8 +585,8 @@ extern "C" int64_t w4a16_gemm_scratch_bytes(const w4a16_gemm_args* args) {
   if (int rc = validate(args)) return rc;
   if (args->size_m == 0) return 0;
   Plan pl;
-  if (int rc = make_plan(args, pl)) return rc;
-  return ((pl.ctmp_bytes + 255) & ~255LL) + pl.atmp_bytes;
+  if (int rc = make_plan(args, pl, true)) return rc;
+  return plan_scratch(pl);
 }
 
 // Launches the planned kernels; `args` already carries the scratch (c_tmp) and counter (workspace) pointers to use.
@@ -521,6 +629,7 @@ static int run_planned(const w4a16_gemm_args* args, Plan& pl, void* stream) {
   }
   if (pl.kind == 3) return launch_mid(&b, pl, (hipStream_t)stream);
   if (pl.kind == 5) return launch_kq(&b, pl, (hipStream_t)stream);
+  if (pl.kind == 6) return launch_x8(&b, pl, (char*)args->c_tmp + plan_scratch(pl) - pl.x8_bytes, (hipStream_t)stream);
   return pl.kind == 1 ? launch_decode(&b, pl, (hipStream_t)stream) : launch_skinny(&b, pl, (hipStream_t)stream);
 }
 
@@ -528,11 +637,11 @@ extern "C" int w4a16_marlin_gemm(const w4a16_gemm_args* args, void* stream) {
   if (int rc = validate(args)) return rc;
   if (args->size_m == 0) return 0;
   Plan pl;
-  if (int rc = make_plan(args, pl)) return rc;
+  // (a caller without scratch gets a plan that may need none)
+  if (int rc = make_plan(args, pl, args->c_tmp != nullptr)) return rc;
   if (pl.mtiles == 0) return 0;
-  if (pl.ctmp_bytes + pl.atmp_bytes > 0)
-    W4A16_CHECK(args->c_tmp != nullptr, "c_tmp is null but %lld bytes are needed",
-                (long long)(pl.ctmp_bytes + pl.atmp_bytes));
+  if (plan_scratch(pl) > 0)
+    W4A16_CHECK(args->c_tmp != nullptr, "c_tmp is null but %lld bytes are needed", (long long)plan_scratch(pl));
   return run_planned(args, pl, stream);
 }
 
@@ -578,9 +687,13 @@ extern "C" int w4a16_marlin_gemm_static(const w4a16_gemm_args* args, void* strea
   b.workspace = (int32_t*)(base + W4A16_STATIC_SCRATCH_BYTES);
   b.workspace_len = STATIC_COUNTERS;
   Plan pl;
-  if (int rc = make_plan(&b, pl)) return rc;
+  if (int rc = make_plan(&b, pl, true)) return rc;
+  if (plan_scratch(pl) > (int64_t)W4A16_STATIC_SCRATCH_BYTES) {  // (activations split for the 8-bit unit do not fit: the 16-bit plan)
+    pl = Plan{};
+    if (int rc = make_plan(&b, pl, false)) return rc;
+  }
   if (pl.mtiles == 0) return 0;
-  const int64_t need = ((pl.ctmp_bytes + 255) & ~255LL) + pl.atmp_bytes;
+  const int64_t need = plan_scratch(pl);
   W4A16_CHECK(need <= (int64_t)W4A16_STATIC_SCRATCH_BYTES,
               "w4a16_marlin_gemm_static: this problem needs %lld bytes of scratch, the library's static buffer holds "
               "%lld; use w4a16_marlin_gemm with a caller-owned c_tmp",

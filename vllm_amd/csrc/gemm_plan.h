@@ -21,6 +21,8 @@ struct Plan {
   int dyn_slots = 0;   // 64-row kernel, MoE: resident workgroups that the device-side K split of the tail tiles fills
   int tail_strips = 0; // prefill plan: trailing 512-column strips handed to another kernel (0 = none)
   int tail_kind = 3;   // ... which one: 3 = 64-row kernel, 5 = 128 x 256 tiles with the K halves inside the workgroup
+  int ks = 1;          // 8-bit-unit kernel (kind 6): K parts inside a workgroup
+  int64_t x8_bytes = 0;  // 8-bit-unit kernel: the activations split in two 8-bit terms, behind the other scratch
   int64_t ctmp_bytes;  // fp32 split-K partials
   int64_t atmp_bytes;  // column-permuted copy of A (act-order), after the partials; MoE: one row per sorted slot
 };
@@ -36,6 +38,8 @@ int launch_skinny(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_decode(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_fat(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_mid(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
+int64_t x8_scratch_bytes(int64_t rows, int64_t k);
+int launch_x8(const w4a16_gemm_args* a, const Plan& pl, void* scratch, hipStream_t stream);
 int launch_kq(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 
 }  // namespace w4a16

@@ -1,0 +1,719 @@
+// W4A16 GEMM for gfx950 on the 8-bit matrix unit: C[M,N] = A[M,K] * dequant(Bq)[K,N] (+bias), bf16 activations, integer 4-bit
+// weights, scale groups of whole 128 K rows (or one scale per column), more than 128 rows.
+//
+// The 16-bit kernels spend their time on making weights: 4.25 VALU instructions per pair of bf16((q - z) * s), which a SIMD barely
+// overlaps with its MFMAs (prefill kernel, 4096^3: matrix pipe 52 % busy).  The 8-bit unit does twice the products per cycle and
+// takes the weight as it is: a byte 0 .. 15 is the e4m3 number q * 2^-9 (0 .. 7 subnormal, 8 .. 15 the first binade), so a word of
+// eight weights costs one shift, two ANDs and two byte permutes.  The activation becomes two e4m3 terms under one power of two per
+// row and 128 K rows ("step"): hi = e4m3(a * 2^-e), lo = e4m3(16 * (a * 2^-e - hi)).  bf16 has eight significant bits, the terms four
+// each: the pair is the activation, exactly, down to 2^-14 of the step's largest value, and has an absolute error of 2^-22 of that
+// below.  Two v_mfma_scale_f32_16x16x128_f8f6f4 (hi, lo; same weights) do what four bf16 MFMAs did, in the same 64 cycles; the step's
+// sums are then scaled in fp32, acc = fma(s, sum, acc), so no weight is rounded.  Zero points: see the end of the loop.
+//   Measured on the unit: subnormals are kept; lane l holds row / column l & 15 and the 32 bytes of K block l >> 4, one scale byte
+// per row serves the whole step when all four lanes of the row carry it; products of eight neighbouring bytes are added with the bits
+// below 2^-14 of the largest cut off, these sums then in fp32.  Against float64, normal activations: 1.7e-5 of a step's sum (a step of
+// bf16-rounded weights: 1.8e-3), one activation 300 times the others 2.8e-4; whole layers 1.66e-3, the rounding of the bf16 result
+// (16-bit kernels 2.12e-3 uint4b8, 2.18e-3 zero points).
+//
+//   split    x8_split_kernel writes the two terms of A in the order in which MFMA fragments are read (a fragment of 16 rows is one
+//            contiguous KB) with the scale byte and the sum of every row and step: 16 us at 4096 x 4096, 44 at 4096 x 14336 (5 TB/s).
+//   tile     a wavefront owns 16 MB rows x 64 columns (half of the words of a column pair): 128 accumulators at MB = 8, two
+//            wavefronts per SIMD, every register used.  The accumulators must be VGPRs (the VALU cannot add to AGPRs).
+//   shapes   <8, KS 1, WN 8>: 128 x 512, one workgroup per compute unit; <8, 1, 4>: 128 x 256, two; <5 .. 8, 2, 4>: 80 .. 128 rows x 256
+//            columns, K in two halves inside the workgroup, for problems that leave compute units idle otherwise.  gemm.hip picks by
+//            a fitted cost.
+//   staging  activations global -> LDS without registers, double buffered, one barrier per step, placed where a wavefront has read
+//            the last fragment of its step.  Addresses decide the rate: one KB costs the compute unit's memory pipe 17 cycles read
+//            contiguously, 64 in rows of 64 bytes (the first layout tried: 128 x 256 tiles with K halves 937 us, 815 with this one).
+//            Weights global -> registers, one step ahead, spread over the step (a wavefront whose load finds the queue full stands
+//            still).  Through LDS they cost more there than they save in the memory pipe (128 rows: 108 -> 114 us).
+//   bound    4096 x 28672 x 4096, uint4b8: 782 us before, 692 now; zero points 771 -> 725.  Matrix pipe 65 % busy at 2.03 GHz (16-bit
+//            kernel 52 % at 2.13); the same loop without memory accesses runs at 72 %, and the MFMAs with their FMAs alone are held to
+//            1.54 GHz by the power limit, 1.65 PFLOP/s.  At 203 rows 70 -> 54 (MFMA, start and end of the workgroups, the split 5).
+#include <type_traits>
+
+#include "gemm_kernels.h"
+
+namespace w4a16 {
+
+using i32x8 = int32_t __attribute__((ext_vector_type(8)));
+using u16x2 = uint16_t __attribute__((ext_vector_type(2)));
+
+constexpr int X8_G = 128;                       // K rows of one step
+constexpr int X8_RS = 76;                       // floats per row of an epilogue slab (40 per n-tile half: conflict-free, 16-byte aligned)
+constexpr int X8_SLAB = 2 * 16 * X8_RS * 4;     // a wavefront's two slabs of 16 rows
+
+__host__ __device__ constexpr int x8_buf(int mb, int wn) { return mb * 4096 + wn * 256; }  // one K part, one step: fragments, sums, scales
+__host__ __device__ constexpr int x8_smem(int mb, int ks, int wn) {
+  const int bufs = 2 * ks * x8_buf(mb, wn), comb = (ks - 1) * ks * wn * ((mb + ks - 1) / ks) * 4096, slabs = ks * wn * X8_SLAB;
+  return bufs > comb ? (bufs > slabs ? bufs : slabs) : (comb > slabs ? comb : slabs);
+}
+
+struct X8Params {
+  KParams k;
+  const unsigned char* rec;  // [K / 128][rows / 16][fragment 4][K group 4][row 16][16 bytes]: a fragment is one contiguous KB
+  const float* sum;          // [K / 128][rows]
+  const uint32_t* scl;       // [K / 128][rows]
+  int rows;                  // see x8_rows
+};
+// rows the split activations have: whole blocks of 16, and seven blocks more (a tile starts inside the matrix, and has up to eight)
+__host__ __device__ constexpr int64_t x8_rows(int64_t m) { return (m + 15) / 16 * 16 + 112; }
+
+// ------------------------------------------------------------------------------------------------ activations
+// A workgroup: 16 rows, wavefront w rows 4 w .. 4 w + 3, X8_SG steps one after the other (their loads are issued together).
+// Lane bits: 0 odd half of a k-tile, 1 which four k-tiles, 2-3 row, 4-5 k-tile.
+template <int X8_SG>
+__global__ __launch_bounds__(256) void x8_split_kernel(const uint16_t* a, int64_t lda, int rows, int stride, int groups, unsigned char* rec,
+                                                       float* sum, uint32_t* scl) {
+  const int lane = threadIdx.x & 63;
+  const int odd = lane & 1, j = (lane >> 1) & 1, rr = lane >> 4;
+  const int row = blockIdx.x * 16 + (threadIdx.x >> 6) * 4 + ((lane >> 2) & 3);
+  const int group0 = blockIdx.y * X8_SG;
+  __shared__ __align__(16) unsigned char sh[X8_SG * 4096];
+  u32x4 xs[X8_SG];
+#pragma unroll
+  for (int q = 0; q < X8_SG; ++q) {
+    xs[q] = u32x4{0, 0, 0, 0};
+    if (group0 + q < groups && row < rows) xs[q] = *(const u32x4*)(a + row * lda + (group0 + q) * X8_G + (4 * j + rr) * 16 + odd * 8);
+  }
+#pragma unroll
+  for (int q = 0; q < X8_SG; ++q) {
+    const int group = group0 + q;
+    if (group >= groups) break;  // (uniform)
+    u32x4 x = xs[q];
+    // maximum (as 15-bit integers: the order of the magnitudes) and sum over the step's 16 lanes: bits 0, 1, 4, 5
+    auto max_abs = [&](const u32x4& v) {
+      u16x2 t = __builtin_bit_cast(u16x2, v[0] & 0x7fff7fffu);
+#pragma unroll
+      for (int i = 1; i < 4; ++i) t = __builtin_elementwise_max(t, __builtin_bit_cast(u16x2, v[i] & 0x7fff7fffu));
+      uint32_t m = max((uint32_t)t.x, (uint32_t)t.y);
+      m = max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xb1, 0xf, 0xf, true));
+      m = max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x4e, 0xf, 0xf, true));
+      const auto p = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+      m = max(p[0], p[1]);
+      const auto r = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+      return max(r[0], r[1]);
+    };
+    uint32_t m = max_abs(x), flags = 0;
+    if (__any(m >= 0x7f80u)) {
+      // infinities and NaNs leave the operand; the GEMM's epilogue puts them back (x8_special)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t lo = x[i] & 0x7fffu, hi = (x[i] >> 16) & 0x7fffu;
+        if (lo >= 0x7f80u) flags |= lo == 0x7f80u ? 1u : 2u, x[i] &= 0xffff0000u;
+        if (hi >= 0x7f80u) flags |= hi == 0x7f80u ? 1u : 2u, x[i] &= 0x0000ffffu;
+      }
+      flags |= (uint32_t)__shfl_xor((int)flags, 1);
+      flags |= (uint32_t)__shfl_xor((int)flags, 2);
+      flags |= (uint32_t)__shfl_xor((int)flags, 16);
+      flags |= (uint32_t)__shfl_xor((int)flags, 32);
+      m = max_abs(x);
+    }
+    const int e = max((int)(m >> 7) - 134, -123);  // |a| * 2^-e < 256
+    const float inv = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);
+    float s = 0.f;
+    uint32_t hi01 = 0, hi23 = 0, lo01 = 0, lo23 = 0;
+    // element pair g of the lane: K rows 2g, 2g + 1 (+ 8 for odd lanes) of its k-tile; two bytes per pair
+    auto enc = [&](uint32_t pair, uint32_t& h, uint32_t& l, auto upper_tag) {
+      constexpr bool UPPER = decltype(upper_tag)::value;
+      const float x0 = bf16_lo_f32(pair), x1 = bf16_hi_f32(pair);
+      s = __builtin_fmaf(x0, 0x1.0p-9f, s);
+      s = __builtin_fmaf(x1, 0x1.0p-9f, s);
+      const float y0 = x0 * inv, y1 = x1 * inv;
+      h = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(y0, y1, (int)h, UPPER);
+      const auto b = __builtin_amdgcn_cvt_pk_f32_fp8((int)h, UPPER);
+      l = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32((y0 - b[0]) * 16.f, (y1 - b[1]) * 16.f, (int)l, UPPER);
+    };
+    enc(x[0], hi01, lo01, std::false_type{});
+    enc(x[1], hi01, lo01, std::true_type{});
+    enc(x[2], hi23, lo23, std::false_type{});
+    enc(x[3], hi23, lo23, std::true_type{});
+    s += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, s), 0xb1, 0xf, 0xf, true));
+    s += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, s), 0x4e, 0xf, 0xf, true));
+    {
+      const uint32_t si = __builtin_bit_cast(uint32_t, s);
+      const auto p = __builtin_amdgcn_permlane16_swap(si, si, false, false);
+      const uint32_t p0 = p[0], p1 = p[1];  // (bit casts take element 0 of a vector whatever the index)
+      s = __builtin_bit_cast(float, p0) + __builtin_bit_cast(float, p1);
+      const uint32_t sj = __builtin_bit_cast(uint32_t, s);
+      const auto r = __builtin_amdgcn_permlane32_swap(sj, sj, false, false);
+      const uint32_t r0 = r[0], r1 = r[1];
+      s = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+    }
+    // even lanes collect pairs 0, 1 of both halves, odd lanes pairs 2, 3: bytes [k, k + 1, k + 8, k + 9]
+    auto join = [&](uint32_t p01, uint32_t p23, uint32_t& d0, uint32_t& d1) {
+      const uint32_t got = (uint32_t)__builtin_amdgcn_mov_dpp((int)(odd ? p01 : p23), 0xb1, 0xf, 0xf, true);
+      const uint32_t first = odd ? got : p01, second = odd ? p23 : got;
+      d0 = __builtin_amdgcn_perm(second, first, 0x05040100u);
+      d1 = __builtin_amdgcn_perm(second, first, 0x07060302u);
+    };
+    uint32_t d[4];
+    join(hi01, hi23, d[0], d[1]);
+    join(lo01, lo23, d[2], d[3]);
+    // transpose over lane bits 4-5: lane rr gets dword rr of the four k-tiles
+    auto swap32 = [](uint32_t& p, uint32_t& q) {
+      const auto r = __builtin_amdgcn_permlane32_swap(p, q, false, false);
+      p = r[0], q = r[1];
+    };
+    auto swap16 = [](uint32_t& p, uint32_t& q) {
+      const auto r = __builtin_amdgcn_permlane16_swap(p, q, false, false);
+      p = r[0], q = r[1];
+    };
+    swap32(d[0], d[2]);
+    swap32(d[1], d[3]);
+    swap16(d[0], d[1]);
+    swap16(d[2], d[3]);
+    // (fragment, K group, row) of the lane's 16 bytes; stored below, a fragment per wavefront
+    *(u32x4*)(sh + q * 4096 + ((rr >> 1) * 2 + j) * 1024 + (2 * odd + (rr & 1)) * 256 + (row & 15) * 16) = u32x4{d[0], d[1], d[2], d[3]};
+    if ((lane & 0x33) == 0) {
+      sum[(int64_t)group * stride + row] = s;
+      scl[(int64_t)group * stride + row] = (uint32_t)(127 + e) | (uint32_t)(127 + e - 4) << 8 | flags << 16;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < X8_SG; ++q)
+    if (group0 + q < groups)
+      *(u32x4*)(rec + ((int64_t)(group0 + q) * stride + blockIdx.x * 16) * 256 + threadIdx.x * 16) = *(const u32x4*)(sh + q * 4096 + threadIdx.x * 16);
+}
+
+// ------------------------------------------------------------------------------------------------ GEMM
+// Contribution of the infinities and NaNs of A row `arow` in K columns [k0, k1) to columns n .. n + 3 (before scales of a
+// channel-wise weight): what inf * w adds up to.
+template <bool ZP, bool CHANNEL>
+__device__ __forceinline__ f32x4 x8_special(const uint16_t* arow, int k0, int k1, const uint32_t* Bq, const uint16_t* Sc, const uint32_t* Zp,
+                                            int N, int group_shift, int n) {
+  f32x4 v = {0, 0, 0, 0};
+#pragma unroll 1
+  for (int k = k0; k < k1; ++k) {
+    const uint32_t b = arow[k];
+    if ((b & 0x7fffu) < 0x7f80u) continue;
+    const float av = __builtin_bit_cast(float, b << 16);
+    const int grp = CHANNEL ? 0 : (k >> 5) >> group_shift;
+    const int r = k & 15, g = (r & 7) >> 1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int col = n + i, cc = col & 63, w = cc >> 4, half = (cc >> 3) & 1, c = cc & 7;
+      const uint32_t word = Bq[(int64_t)(k >> 4) * (2 * N) + (col >> 6) * 128 + (4 * c + g) * 4 + w];
+      const int q = (int)((word >> (4 * ((r & 1) * 4 + half * 2 + (r >> 3)))) & 15u);
+      int z = 8;
+      if (ZP) z = (int)((Zp[(int64_t)grp * (N >> 3) + (col >> 6) * 8 + c] >> (4 * w + 16 * half)) & 15u);
+      float s = 1.f;
+      if (!CHANNEL) s = bf16_lo_f32(Sc[(int64_t)grp * N + (col & ~63) + 8 * c + 2 * w + half]);
+      v[i] += av * ((float)(q - z) * s);
+    }
+  }
+  return v;
+}
+
+// One 16- or 4-byte piece per lane, global memory -> LDS (lane l's piece at lds + 16 l or 4 l) without passing through registers.
+// The statements are opaque to the compiler: whoever reads the data waits for vmcnt(0) and then at a workgroup barrier.
+__device__ __forceinline__ void x8_load_lds16(uint32_t lds, uint32_t off, const void* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ void x8_load_lds4(uint32_t lds, uint32_t off, const void* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
+
+// Eight fp32 values as two bf16 terms each (an MFMA operand per term), and what those leave
+__device__ __forceinline__ void x8_bf16_terms(const float (&v)[8], u32x4& t1, u32x4& t2, float (&rest)[8]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    t1[q] = pack_bf16(v[2 * q], v[2 * q + 1]);
+    const float r0 = v[2 * q] - bf16_lo_f32(t1[q]), r1 = v[2 * q + 1] - bf16_hi_f32(t1[q]);
+    t2[q] = pack_bf16(r0, r1);
+    rest[2 * q] = r0 - bf16_lo_f32(t2[q]), rest[2 * q + 1] = r1 - bf16_hi_f32(t2[q]);
+  }
+}
+__device__ __forceinline__ void x8_bf16_terms(const float (&v)[8], u32x4& t1, u32x4& t2) {
+  float rest[8];
+  x8_bf16_terms(v, t1, t2, rest);
+}
+
+template <bool ZP, bool CHANNEL, int MB, int KS, int WN>
+__global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) {
+  const KParams& p = xp.k;
+  constexpr int BM = 16 * MB, BN = WN * 64;
+  constexpr int NL = MB * 4 / WN;  // 1 KB fragments staged per wavefront and step
+  constexpr int NM = (BM + 63) / 64;          // 64-row pieces of the step's sums (and of its scales)
+  static_assert(2 * NM <= WN && MB * 4 % WN == 0, "one piece of sums or scales and as many fragments for every wavefront");
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int part = wv / WN, wn = wv % WN;
+  const int c = lane & 7, h = (lane >> 3) & 1, g = lane >> 4;
+  const int G = p.K / X8_G;
+
+  const int mtiles = (p.M + BM - 1) / BM, nsplit = p.splits;
+  int j = blockIdx.x, split = 0, slot = 0;
+  int gb = 0, ge = G;
+  if (nsplit > 1) {
+    const int tiles = mtiles * p.ncp, per = p.ksteps_per_split / 4;
+    split = j / tiles;
+    j -= split * tiles;
+    slot = j;
+    gb = split * per, ge = min(gb + per, G);
+  }
+  const int gb0 = gb, ge0 = ge;
+  const int max_steps = (ge - gb + KS - 1) / KS;  // of a K part
+  gb += part * max_steps;
+  ge = min(gb + max_steps, ge);
+  const int steps = ge - gb;  // the last part may have fewer (or none)
+  const int mt = j % mtiles, strip = p.strip0 + j / mtiles;
+  const int row0 = mt * BM;
+  const int u = strip * WN + wn, cp = u >> 1, wsel = (u & 1) * 2;
+  const bool wave_on = cp * 128 < p.N;
+
+  const uint16_t* Sc = (const uint16_t*)p.S;
+  const uint16_t* bias = (const uint16_t*)p.bias;
+  const int nt = !wave_on ? 0 : ((2 * cp + h) * 64 < p.N ? 2 * cp + h : 0);
+  // byte offsets of the lane; everything else in an address is uniform
+  const uint32_t b_off = (uint32_t)(nt * 128 + (4 * c + g) * 4 + wsel) * 4;
+  // (nt * 64 + 8 c + 2 wsel) * 2 of the scales; two instructions per step for a register of the loop's 256
+  auto s_off = [&]() {
+    uint32_t v;
+    asm volatile("v_lshrrev_b32 %0, 2, %1" : "=v"(v) : "v"(b_off));
+    return (v & ~15u) + 4 * wsel;
+  };
+  const uint32_t b_row = (uint32_t)p.N * 8;  // bytes of one k-tile
+  // buffer resources: 32-bit offsets, nothing per lane but the lane's own (the host checks the sizes)
+  const int b_bytes = (int)((uint32_t)(p.K / 16) * b_row), sg = CHANNEL ? 1 : (4 * G) >> p.group_shift;
+  const auto b_res = __builtin_amdgcn_make_buffer_rsrc((void*)p.B, 0, b_bytes, 0x00020000);
+  const auto s_res = __builtin_amdgcn_make_buffer_rsrc((void*)Sc, 0, sg * p.N * 2, 0x00020000);
+  const auto z_res = __builtin_amdgcn_make_buffer_rsrc((void*)p.Z, 0, sg * (p.N / 2), 0x00020000);
+
+  // activations: fragment f = 4 mb + piece, one KB each; f = wn + WN i for this wavefront
+  const int64_t a_step = (int64_t)xp.rows * 256;
+  const unsigned char* a_ptr = xp.rec + gb * a_step + (int64_t)row0 * 256;
+  const uint32_t* m_ptr = (wn < NM ? (const uint32_t*)xp.sum : xp.scl) + (int64_t)gb * xp.rows + row0 + wn % NM * 64;
+  unsigned char* pbuf = smem + part * 2 * x8_buf(MB, WN);
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)pbuf);
+  // step i of the part -> LDS; complete after sync_stage
+  auto stage_frag = [&](int i, int buf, int q) {
+    const int f = wn + WN * q;
+    x8_load_lds16(lds0 + buf * x8_buf(MB, WN) + f * 1024, lane * 16, a_ptr + i * a_step + f * 1024);
+  };
+  auto stage_meta = [&](int i, int buf) {  // (wavefronts from 2 NM on: a copy nobody reads)
+    uint32_t off;  // (lane * 4, not kept either)
+    asm volatile("v_lshrrev_b32 %0, 2, %1" : "=v"(off) : "v"(lane * 16));
+    x8_load_lds4(lds0 + buf * x8_buf(MB, WN) + MB * 4096 + wn * 256, off, m_ptr + (int64_t)i * xp.rows);
+  };
+
+  u32x2 raw[8], sraw = {0, 0};
+  auto load_b = [&](int i, int kt) {
+    raw[kt] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(b_res, b_off, (uint32_t)((gb + i) * 8 + kt) * b_row, 0));
+  };
+  auto load_s = [&](int i) {
+    const uint32_t grp = CHANNEL ? 0 : (uint32_t)(4 * (gb + i)) >> p.group_shift;
+    if (!CHANNEL) sraw = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(s_res, s_off(), grp * p.N * 2, 0));
+  };
+  // k-tile kt of word w (0 or 1 of the wavefront's two) -> its dword of the two operands
+  auto dequant = [&](int w, int kt, i32x8 (&o)[2]) {
+    const uint32_t x = raw[kt][w], lo = x & 0x0f0f0f0fu, hi = (x >> 4) & 0x0f0f0f0fu;
+    o[0][kt] = (int)__builtin_amdgcn_perm(hi, lo, 0x06040200u);
+    o[1][kt] = (int)__builtin_amdgcn_perm(hi, lo, 0x07050301u);
+  };
+
+  f32x4 acc[MB][4];
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[m][i] = f32x4{0, 0, 0, 0};
+  i32x8 bx[2], by[2], b23[2], ah, al;
+  f32x4 T[2][2] = {}, sm = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
+  float sc[4] = {512.f, 512.f, 512.f, 512.f};
+  uint32_t any = 0, sl = 0, sl_n = 0;
+  auto frag = [&](int buf, int m, int half, i32x8& o) {
+    const u32x4* f = (const u32x4*)(pbuf + buf * x8_buf(MB, WN) + m * 4096 + half * 2048) + lane;
+    const u32x4 f0 = f[0], f1 = f[64];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] = (int)f0[q], o[4 + q] = (int)f1[q];
+  };
+  auto meta = [&](int buf, int m) {
+    const unsigned char* d = pbuf + buf * x8_buf(MB, WN) + MB * 4096;
+    sm = *(const f32x4*)(d + (m * 16 + 4 * g) * 4);
+    sl_n = *(const uint32_t*)(d + NM * 256 + (m * 16 + (lane & 15)) * 4);
+  };
+  // word w's two operands: factors of the step's product sums, from the loaded words
+  auto scales = [&](int w) {
+    if (!CHANNEL) {
+      sc[2 * w] = bf16_lo_f32(sraw[w]) * 512.f;
+      sc[2 * w + 1] = bf16_hi_f32(sraw[w]) * 512.f;
+    }
+  };
+  auto fold = [&](int m, int pr, int i) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[m][2 * pr + i][r] = __builtin_fmaf(sc[2 * pr + i], T[pr][i][r], acc[m][2 * pr + i][r]);
+  };
+  auto init = [&]() {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ci[r] = -8.f * sm[r];
+  };
+  auto mfma_lo = [&](int pr, int i, const i32x8& b) {
+    T[pr][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(al, b, ci, 0, 0, 1, (int)sl, 0, 127);
+  };
+  auto mfma_hi = [&](int pr, int i, const i32x8& b) {
+    T[pr][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ah, b, T[pr][i], 0, 0, 0, (int)sl, 0, 127);
+  };
+  auto sync_stage = [&]() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+#define X8_SB __builtin_amdgcn_sched_barrier(0)
+  auto step = [&](int i, int buf, i32x8 (&b01)[2], i32x8 (&n01)[2]) {
+    constexpr int FROM = MB > 3 ? MB - 3 : 1, PER = (8 + MB - FROM - 1) / (MB - FROM);  // next step's word 0: spread over the last row blocks
+    // The next step's loads, spread over the step: a wavefront whose load finds the memory pipeline's queue full stands still with
+    // its MFMAs.  u: 2 m + word; the weight registers are free from u = 1 on and wanted from m = FROM on.
+    const int nx = min(i + 1, steps - 1);
+    auto loads = [&](int u) {
+      constexpr int LAST = 2 * FROM - 1, WPER = (8 + LAST - 1) / LAST, SPER = (NL + LAST - 1) / LAST;
+      if (u == 1) load_s(nx), stage_meta(nx, buf ^ 1);
+#pragma unroll
+      for (int q = 0; q < WPER; ++q)
+        if ((u - 1) * WPER + q < 8) load_b(nx, (u - 1) * WPER + q);
+#pragma unroll
+      for (int q = 0; q < SPER; ++q)
+        if ((u - 1) * SPER + q < NL) stage_frag(nx, buf ^ 1, (u - 1) * SPER + q);
+    };
+    scales(0);
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      // columns of word 0; the product sums of word 1 of the row block before are folded meanwhile
+      X8_SB;
+      mfma_lo(0, 0, b01[0]);
+      fold(m > 0 ? m - 1 : MB - 1, 1, 0);  // (zeros in front of the first step)
+      if (m == 0) dequant(1, 0, b23), dequant(1, 1, b23);
+      X8_SB;
+      mfma_lo(0, 1, b01[1]);
+      fold(m > 0 ? m - 1 : MB - 1, 1, 1);
+      if (m == 0) dequant(1, 2, b23), dequant(1, 3, b23);
+      X8_SB;
+      mfma_hi(0, 0, b01[0]);
+      if (m == 0) scales(1), dequant(1, 4, b23), dequant(1, 5, b23);
+      X8_SB;
+      mfma_hi(0, 1, b01[1]);
+      if (m + 1 < MB) meta(buf, m + 1);
+      if (m == 0) {
+        dequant(1, 6, b23), dequant(1, 7, b23);
+        X8_SB;
+      }
+      if (m > 0) loads(2 * m);
+#pragma unroll
+      for (int q = 0; q < PER; ++q)
+        if (m >= FROM && (m - FROM) * PER + q < 8) dequant(0, (m - FROM) * PER + q, n01);
+      X8_SB;
+      // columns of word 1
+      loads(2 * m + 1);
+      X8_SB;
+      if (m == MB - 1) {
+        sync_stage();
+        meta(buf ^ 1, 0);
+        X8_SB;
+      }
+      mfma_lo(1, 0, b23[0]);
+      fold(m, 0, 0);
+      X8_SB;
+      mfma_lo(1, 1, b23[1]);
+      fold(m, 0, 1);
+      X8_SB;
+      frag(m + 1 < MB ? buf : buf ^ 1, m + 1 < MB ? m + 1 : 0, 1, al);
+      mfma_hi(1, 0, b23[0]);
+      X8_SB;
+      mfma_hi(1, 1, b23[1]);
+      init();
+      any |= sl;
+      sl = sl_n;
+      X8_SB;
+      frag(m + 1 < MB ? buf : buf ^ 1, m + 1 < MB ? m + 1 : 0, 0, ah);
+    }
+  };
+
+  // ---- prologue and main loop: one step (128 K rows) per barrier
+  if (steps > 0) {
+#pragma unroll
+    for (int q = 0; q < NL; ++q) stage_frag(0, 0, q);
+    stage_meta(0, 0);
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt) load_b(0, kt);
+    load_s(0);
+  }
+  sync_stage();
+  if (steps > 0) {
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt) dequant(0, kt, bx);
+    meta(0, 0);
+    init();
+    sl = sl_n;
+    frag(0, 0, 1, al);
+    frag(0, 0, 0, ah);
+  }
+#pragma unroll 1
+  for (int i = 0; i < max_steps; i += 2) {
+    if (i < steps)
+      step(i, 0, bx, by);
+    else
+      sync_stage();
+    if (i + 1 >= max_steps) break;
+    if (i + 1 < steps)
+      step(i + 1, 1, by, bx);
+    else
+      sync_stage();
+  }
+  if (steps > 0) {
+    fold(MB - 1, 1, 0);
+    fold(MB - 1, 1, 1);
+  }
+  __syncthreads();
+
+  // ---- zero points: a product sum started at -8 * (sum of the row's activations in the step), which is all there is to uint4b8.
+  // What (8 - z) * s of those sums adds is a product of its own, [rows, steps] x [steps, columns], 32 steps to an MFMA: the sums in
+  // three bf16 terms (their 24 bits), (8 - z) * s in two (8 + 5 bits), the product of the two smallest left out (2^-24 of the sum).
+  // As two more FMAs per accumulator and step in the loop it took 12 % of the kernel (4096 x 4096 x 4096: 120 -> 108 us).
+  if constexpr (ZP) {
+#pragma unroll 1
+    for (int g0 = gb; g0 < ge; g0 += 32) {
+      u32x4 zh[4], zl[4];
+      {
+        u32x2 sv[8];
+        uint32_t zv[8];
+        const uint32_t so = s_off(), z_off = (uint32_t)(nt * 8 + c) * 4;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const int gi = min(g0 + 8 * g + q, ge - 1);
+          const uint32_t grp = CHANNEL ? 0 : (uint32_t)(4 * gi) >> p.group_shift;
+          if (!CHANNEL) sv[q] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(s_res, so + grp * p.N * 2, 0, 0));
+          zv[q] = __builtin_amdgcn_raw_buffer_load_b32(z_res, z_off + grp * (p.N / 2), 0, 0) >> (4 * wsel);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float v[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            const float sc1 = CHANNEL ? 1.f : (i & 1) ? bf16_hi_f32(sv[q][i >> 1]) : bf16_lo_f32(sv[q][i >> 1]);
+            v[q] = g0 + 8 * g + q < ge ? (8.f - (float)((zv[q] >> (4 * (i >> 1) + 16 * (i & 1))) & 15u)) * sc1 * 512.f : 0.f;
+          }
+          x8_bf16_terms(v, zh[i], zl[i]);
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        float v[8], rest[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = xp.sum[(int64_t)min(g0 + 8 * g + q, ge - 1) * xp.rows + row0 + m * 16 + (lane & 15)];
+        u32x4 a1, a2, a3, a4;
+        x8_bf16_terms(v, a1, a2, rest);
+        x8_bf16_terms(rest, a3, a4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          acc[m][i] = mfma16x16x32<DT_BF16>(a3, zh[i], acc[m][i]);
+          acc[m][i] = mfma16x16x32<DT_BF16>(a2, zl[i], acc[m][i]);
+          acc[m][i] = mfma16x16x32<DT_BF16>(a2, zh[i], acc[m][i]);
+          acc[m][i] = mfma16x16x32<DT_BF16>(a1, zl[i], acc[m][i]);
+          acc[m][i] = mfma16x16x32<DT_BF16>(a1, zh[i], acc[m][i]);
+        }
+        X8_SB;  // (one row block's operands at a time)
+      }
+    }
+  }
+
+  // ---- K parts: every part finishes its share of the row blocks and collects the others' accumulators of it through LDS
+  constexpr int MS = (MB + KS - 1) / KS;  // row blocks of a part
+  const int m0 = part * MS;
+  if constexpr (KS > 1) {
+    // piece of row blocks MS * owner .. that part `from` hands over
+    auto piece = [&](int owner, int from, int mm, int i) {
+      return (f32x4*)smem + (((owner * (KS - 1) + (from - owner - 1 + KS) % KS) * WN + wn) * MS * 4 + mm * 4 + i) * 64 + lane;
+    };
+    auto hand_over = [&](auto part_tag) {  // (the part as a constant: accumulators are registers)
+      constexpr int P = decltype(part_tag)::value;
+#pragma unroll
+      for (int m = 0; m < MB; ++m)
+        if (m / MS != P) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) *piece(m / MS, P, m % MS, i) = acc[m][i];
+        }
+    };
+    auto collect = [&](auto part_tag) {
+      constexpr int P = decltype(part_tag)::value;
+#pragma unroll
+      for (int mm = 0; mm < MS; ++mm)
+        if (P * MS + mm < MB) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            f32x4 v = acc[P * MS + mm][i];
+#pragma unroll
+            for (int q = 0; q < KS; ++q)
+              if (q != P) v += *piece(P, q, mm, i);
+            acc[mm][i] = v;
+          }
+        }
+    };
+#define X8_FOR_PART(f)                              \
+  if (part == 0)                                    \
+    f(std::integral_constant<int, 0>{});            \
+  else if (part == 1)                               \
+    f(std::integral_constant<int, 1>{});            \
+  else if constexpr (KS > 2) {                      \
+    if (part == 2)                                  \
+      f(std::integral_constant<int, 2>{});          \
+    else                                            \
+      f(std::integral_constant<int, 3>{});          \
+  }
+    X8_FOR_PART(hand_over)
+    any = __syncthreads_or((any >> 16) != 0) ? 1u << 16 : 0u;
+    X8_FOR_PART(collect)
+    __syncthreads();
+  }
+
+  // ---- epilogue: two row blocks at a time, accumulators -> slabs of the wavefront -> rows of 2 x 32 columns, 8-byte stores
+  float* slab = (float*)(smem + wv * X8_SLAB);
+  const int lc = (lane & 15) * 4, lh = lc >> 5, lpos = lh * 40 + (lc & 31);
+  const int ncol = 64 * (2 * cp + lh) + 16 * wsel + (lc & 31);
+  const bool col_ok = wave_on && ncol < p.N;
+  float cs[4] = {1.f, 1.f, 1.f, 1.f}, bs[4] = {0.f, 0.f, 0.f, 0.f};
+  if (col_ok) {
+    const int base = ncol & ~31, cl = ncol & 31;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (CHANNEL) cs[i] = bf16_lo_f32(Sc[base + single_perm_pos(cl + i)]);
+      if (bias) bs[i] = bf16_lo_f32(bias[base + single_perm_pos(cl + i)]);
+    }
+  }
+  auto finish = [&](int r, f32x4 v) {  // r: row of the tile
+    if (nsplit > 1) {
+      *(f32x4*)(p.ctmp + (((int64_t)slot * nsplit + split) * BM + r) * BN + (ncol - strip * BN)) = v;
+      return;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = v[q] * cs[q] + bs[q];
+    store_row4<DT_BF16, false>(p, row0 + r, ncol, v);
+  };
+#pragma unroll
+  for (int m = 0; m < MS; m += 2) {
+#pragma unroll
+    for (int e = 0; e < 2 && m + e < MS; ++e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) slab[(16 * e + 4 * g + r) * X8_RS + 40 * h + 8 * i + c] = acc[m + e][i][r];
+    __builtin_amdgcn_wave_barrier();
+    f32x4 v[2 * 4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < 4 || m + 1 < MS) v[i] = *(const f32x4*)(slab + ((lane >> 4) + 4 * i) * X8_RS + lpos);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = (m0 + m) * 16 + (lane >> 4) + 4 * i;
+      if ((i < 4 || m + 1 < MS) && r < BM && col_ok && row0 + r < p.M) finish(r, v[i]);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (__any((any >> 16) != 0)) {
+    // rows with infinities or NaNs: whatever else they hold, their results are what inf * w adds up to
+#pragma unroll 1
+    for (int r = m0 * 16 + (lane >> 4); r < min(BM, (m0 + MS) * 16); r += 4) {
+      if (!col_ok || row0 + r >= p.M) continue;
+      uint32_t f = 0;
+#pragma unroll 1
+      for (int gi = gb0; gi < ge0; ++gi) f |= xp.scl[(int64_t)gi * xp.rows + row0 + r];
+      if (f >> 16)
+        finish(r, x8_special<ZP, CHANNEL>((const uint16_t*)p.A + (int64_t)(row0 + r) * p.lda, gb0 * X8_G, ge0 * X8_G, p.B, Sc, p.Z, p.N,
+                                          p.group_shift, ncol));
+    }
+  }
+}
+
+// Second pass of a launch with K also split across workgroups: adds the fp32 partial tiles in split order.
+template <bool CHANNEL>
+__global__ __launch_bounds__(256) void x8_reduce_kernel(const KParams p, int bm, int bn) {
+  const int mtiles = (p.M + bm - 1) / bm;
+  const int64_t piece = (int64_t)blockIdx.x * 256 + threadIdx.x;  // four columns of a row
+  const int per_row = p.N >> 2;
+  const int row = (int)(piece / per_row), n = (int)(piece - (int64_t)row * per_row) * 4;
+  if (row >= p.M) return;
+  const int mt = row / bm, strip = n / bn;
+  const float* src = p.ctmp + (((int64_t)(strip * mtiles + mt) * p.splits) * bm + (row - mt * bm)) * bn + (n - strip * bn);
+  f32x4 v = {0, 0, 0, 0};
+  for (int s0 = 0; s0 < p.splits; s0 += 4) {
+    f32x4 a[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a[q] = *(const f32x4*)(src + (int64_t)min(s0 + q, p.splits - 1) * bm * bn);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (s0 + q < p.splits) v += a[q];
+  }
+  const int base = n & ~31, cl = n & 31;
+  const uint16_t* Sc = (const uint16_t*)p.S;
+  const uint16_t* bias = (const uint16_t*)p.bias;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (CHANNEL) v[q] *= bf16_lo_f32(Sc[base + single_perm_pos(cl + q)]);
+    if (bias) v[q] += bf16_lo_f32(bias[base + single_perm_pos(cl + q)]);
+  }
+  store_row4<DT_BF16, false>(p, row, n, v);
+}
+
+typedef void (*x8_fn)(const X8Params);
+template <int MB, int KS, int WN>
+static x8_fn pick_x8(bool zp, bool channel) {
+  if (zp) return channel ? x8_kernel<true, true, MB, KS, WN> : x8_kernel<true, false, MB, KS, WN>;
+  return channel ? x8_kernel<false, true, MB, KS, WN> : x8_kernel<false, false, MB, KS, WN>;
+}
+
+int64_t x8_scratch_bytes(int64_t rows, int64_t k) {
+  const int64_t r = x8_rows(rows), g = k / X8_G;
+  return r * g * 256 + 2 * ((r * g * 4 + 255) / 256 * 256);
+}
+
+static x8_fn pick_x8_shape(int mb, int ks, int tn, bool zp, bool channel) {
+  if (ks == 1 && mb == 8) return tn == 512 ? pick_x8<8, 1, 8>(zp, channel) : tn == 256 ? pick_x8<8, 1, 4>(zp, channel) : nullptr;
+  if (ks != 2 || tn != 256) return nullptr;
+  switch (mb) {
+    case 8: return pick_x8<8, 2, 4>(zp, channel);
+    case 7: return pick_x8<7, 2, 4>(zp, channel);
+    case 6: return pick_x8<6, 2, 4>(zp, channel);
+    case 5: return pick_x8<5, 2, 4>(zp, channel);
+    default: return nullptr;
+  }
+}
+
+int launch_x8(const w4a16_gemm_args* a, const Plan& pl, void* scratch, hipStream_t stream) {
+  const bool zp = a->b_zeros != nullptr, channel = pl.gm == GM_CHANNEL;
+  const x8_fn fn = pick_x8_shape(pl.mb, pl.ks, pl.tn, zp, channel);
+  if (!fn || a->dtype != DT_BF16 || (a->wtype != W4A16_WTYPE_U4B8 && a->wtype != W4A16_WTYPE_U4) ||
+      (a->flags & (W4A16_F_ZP_FLOAT | W4A16_F_MOE)) || pl.gm == GM_GIDX || pl.use_perm || pl.splits < 1 || pl.kps % 4 != 0)
+    return fail(W4A16_EINVAL, "unsupported kernel variant");
+  if (pl.tiles <= 0) return 0;
+  X8Params xp;
+  xp.k = make_kparams(a, pl);
+  const int groups = (int)(a->size_k / X8_G);
+  const int64_t r = x8_rows(a->size_m), meta = (r * groups * 4 + 255) / 256 * 256;
+  unsigned char* base = (unsigned char*)scratch;
+  xp.rec = base;
+  xp.sum = (const float*)(base + r * groups * 256);
+  xp.scl = (const uint32_t*)(base + r * groups * 256 + meta);
+  xp.rows = (int)r;
+  // (steps per workgroup: few rows fill the chip only with one)
+  const int sg = (r / 16) * groups >= 16 * num_cus() ? 4 : 1;
+  hipLaunchKernelGGL((sg == 4 ? x8_split_kernel<4> : x8_split_kernel<1>), dim3((unsigned)(r / 16), (unsigned)ceil_div(groups, sg)), dim3(256), 0,
+                     stream, (const uint16_t*)a->a, a->lda, (int)a->size_m, (int)r, groups, (unsigned char*)xp.rec, (float*)xp.sum,
+                     (uint32_t*)xp.scl);
+  W4A16_HIP(hipGetLastError());
+  const int smem = x8_smem(pl.mb, pl.ks, pl.tn / 64);
+  W4A16_HIP(allow_dynamic_lds((const void*)fn, smem));
+  hipLaunchKernelGGL(fn, dim3((unsigned)((int64_t)pl.tiles * pl.splits)), dim3((unsigned)(pl.ks * pl.tn)), smem, stream, xp);
+  W4A16_HIP(hipGetLastError());
+  if (pl.splits > 1) {
+    const dim3 n((unsigned)ceil_div(a->size_m * (a->size_n / 4), 256));
+    if (channel)
+      hipLaunchKernelGGL(x8_reduce_kernel<true>, n, dim3(256), 0, stream, xp.k, pl.bm, pl.tn);
+    else
+      hipLaunchKernelGGL(x8_reduce_kernel<false>, n, dim3(256), 0, stream, xp.k, pl.bm, pl.tn);
+    W4A16_HIP(hipGetLastError());
+  }
+  return 0;
+}
+
+}  // namespace w4a16
