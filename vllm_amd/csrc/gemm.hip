@@ -503,20 +503,59 @@ static void x8_plan(const w4a16_gemm_args* a, int mb, int ks, int tn, int sp, Pl
   pl.x8_bytes = x8_scratch_bytes(a->size_m, a->size_k);
 }
 
-// Microseconds of a 16-bit plan for more than 128 rows of a 4-bit bf16 weight: a round of workgroups costs a fixed part and one per k-step.
-// Fitted to 384 launches (12 layer shapes x 16 row counts x uint4b8 / zero points, group 128): rms 3 (prefill, 128 x 256 tiles) to 8 %.
+// ---- predicted times, integer 4-bit weights, more than 64 rows, microseconds: a round of workgroups costs a fixed part and one per
+// k-step.  Fitted to 1120 problems (10 layer shapes x 16 row counts from 80 to 3000; fp16 and bf16, with and without zero points, groups
+// of 128, 64, 32 and one per column): rms 5 (general kernel), 4 (64-row kernels), 3 % (prefill kernel); 16177 launches of the tall K-split
+// tiles (all of them in every problem): 4 %.
+struct CostClass {
+  bool bf16, zp, channel, short_groups;  // short: below 128 rows of K, dequantisation constants made for every k-step
+};
+static CostClass cost_class(const w4a16_gemm_args* a, const Plan& pl) {
+  return {a->dtype == W4A16_DTYPE_BF16, a->b_zeros != nullptr, pl.gm == GM_CHANNEL, pl.gm != GM_CHANNEL && pl.group_ksteps < 4};
+}
+
+// tall K-split tiles (gemm_kq.hip, 16 mb x 256): `cols` columns, K in `splits` of `kps` k-steps
+static double kq_us(const CostClass& c, int64_t m, int64_t cols, int mb, int splits, int kps) {
+  const double rounds = (double)ceil_div(ceil_div(m, 16 * mb) * ceil_div(cols, 256) * splits, num_cus());
+  const double other = c.bf16 ? (c.short_groups ? 0.085 : 0.065) : c.channel ? -0.03 : c.short_groups ? 0.03 : 0.003;
+  const double t = 5.2 + rounds * (5.6 + kps * (other + 0.049 * mb));
+  // (a second and third round of whole tiles cost more than the first)
+  return splits > 1 ? t + 3.9 + 0.9e-6 * splits * (double)m * (double)cols : t * (0.965 + 0.035 * (rounds < 4 ? rounds : 4));
+}
+
+static double fat_us(const CostClass& c, double rounds, int ksteps) {
+  if (c.bf16) return 5.1 + rounds * (9.5 + (!c.short_groups ? 0.793 : c.zp ? 0.885 : 0.85) * ksteps);
+  const double step = c.channel ? 0.63 : c.short_groups ? (c.zp ? 0.775 : 0.73) : (c.zp ? 0.715 : 0.695);
+  return 1.5 + rounds * (11.8 + step * ksteps);
+}
+
+// a plan of make_plan_16bit or try_kq; 0: a kernel that is not compared (16-row tiles)
 static double plan16_us(const w4a16_gemm_args* a, const Plan& pl) {
-  const double cus = num_cus(), ks = (double)a->size_k / 32;
+  const CostClass c = cost_class(a, pl);
+  const int cus = num_cus();
   if (pl.kind == 2) {
-    double t = 5.1 + ceil((double)(pl.ncp - pl.tail_strips) * pl.mtiles / cus) * (9.6 + 0.793 * ks);
-    if (pl.tail_strips) t += pl.tail_kind == 5 ? 27 + 0.328 * ks : ks;
+    const int head = pl.ncp - pl.tail_strips;
+    double t = fat_us(c, (double)ceil_div((int64_t)head * pl.mtiles, cus), pl.total_ksteps);
+    if (pl.tail_strips)
+      t += pl.tail_kind == 5 ? kq_us(c, a->size_m, a->size_n - head * 512LL, pl.tail_mb, 1, pl.total_ksteps) : (double)pl.total_ksteps;
     return t;
   }
-  const double rounds = ceil((double)pl.tiles * pl.splits / cus), per = ks / pl.splits;
-  if (pl.kind == 5) return pl.mb == 8 ? 6.5 + rounds * (6.5 + 0.457 * per) : 5.2 + rounds * (5.2 + 0.281 * per);
-  if (pl.kind == 3) return 4.0 + rounds * (6.8 + 0.577 * per) + (pl.splits > 1 ? 2.8 : 0);
-  if (pl.kind == 0 && pl.mb == 4) return 2.0 + rounds * (6.6 + 0.156 * per) + (pl.splits > 1 ? 4.6 : 0);
-  return 0;  // 16-row tiles: not compared
+  if (pl.kind == 5 && pl.mb > 4) return kq_us(c, a->size_m, a->size_n, pl.mb, pl.splits, pl.kps);
+  const double rounds = (double)ceil_div((int64_t)pl.tiles * pl.splits, cus), per = pl.kps;
+  const bool split = pl.splits > 1;
+  if (pl.kind == 5) {
+    const double step = c.bf16 ? (c.zp ? 0.28 : 0.27) : c.channel ? 0.17 : c.zp ? 0.23 : 0.205;
+    return 5.1 + rounds * (5.1 + step * per) + (split ? 6.9 : 0);
+  }
+  if (pl.kind == 3) {
+    const double step = c.bf16 ? 0.575 : c.channel ? 0.385 : c.zp ? 0.506 : 0.466;
+    return 2.9 + rounds * (6.4 + step * per) + (split ? 3.6 : 0);
+  }
+  if (pl.kind == 0 && pl.mb == 4) {
+    if (c.bf16) return 2.0 + rounds * (6.6 + 0.156 * per) + (split ? 4.6 : 0);
+    return 3.5 + rounds * (4.9 + (c.channel ? 0.141 : 0.152) * per) + (split ? 4.0 : 0);
+  }
+  return 0;
 }
 
 // The same for a launch on the 8-bit unit, the pass that splits the activations included (3684 launches: 9 shapes x 15 row counts x
@@ -554,11 +593,65 @@ static void try_x8(const w4a16_gemm_args* a, Plan& pl) {
   if (mb && ceil_div(a->size_m, 16 * mb) * ceil_div(a->size_n, tn) * sp < (1LL << 31) / 64) x8_plan(a, mb, ks, tn, sp, pl);
 }
 
-static int make_plan(const w4a16_gemm_args* a, Plan& pl, bool allow_x8) {
+// Tall K-split tiles for a whole problem, or for the trailing strips of a prefill launch, where they are predicted to be 5 % and 1 us
+// faster than the plan made above: that has 64- and 128-row tiles, one split count and one way to end a partly filled round; here the tile's
+// height and the splits follow the number of rows, the layer and the compute units.  Over the 1120 problems 384 change, to 0.57 .. 1.07
+// of their time, 0.85 in the mean (all problems 0.943; the best choice for each would give 0.936); over 72 random ones 0.84, worst 1.00.  Without `more_scratch` only unsplit
+// ones, which need none.
+static void try_kq(const w4a16_gemm_args* a, Plan& pl, bool more_scratch) {
+  if ((a->flags & (W4A16_F_MOE | W4A16_F_ZP_FLOAT)) || (a->wtype != W4A16_WTYPE_U4B8 && a->wtype != W4A16_WTYPE_U4) || pl.gm == GM_GIDX ||
+      (pl.group_ksteps & (pl.group_ksteps - 1)) != 0 || a->size_k % 256 != 0 || a->size_m <= 64)
+    return;
+  const CostClass c = cost_class(a, pl);
+  const int cus = num_cus(), octets = (int)(a->size_k / 256);
+  double best = 0.95 * plan16_us(a, pl) - 1.0;
+  int mb = 0, sp = 0, tail = 0;
+  for (int q = 8; q >= 5; --q) {
+    const int64_t tiles = ceil_div(a->size_m, 16 * q) * ceil_div(a->size_n, 256);
+    if (tiles >= (1LL << 31) / 64) return;
+    for (int s = 1; s <= 16 && (s == 1 || (more_scratch && tiles * s <= 2 * cus && octets >= 2 * s)); ++s) {
+      const int kps = (int)ceil_div(octets, s) * 8;
+      if ((s - 1) * kps >= pl.total_ksteps) continue;  // (fewer splits of that length)
+      const double t = kq_us(c, a->size_m, a->size_n, q, s, kps);
+      if (t < best) best = t, mb = q, sp = s, tail = 0;
+    }
+    // (head: whole rounds, all there are or one fewer)
+    if (pl.kind == 2)
+      for (int64_t rounds = (int64_t)pl.tiles / cus; rounds > 0 && rounds >= (int64_t)pl.tiles / cus - 1; --rounds) {
+        const int head = (int)(rounds * cus / pl.mtiles);
+        if (head < 1 || head >= pl.ncp) continue;
+        const double t = fat_us(c, (double)ceil_div((int64_t)head * pl.mtiles, cus), pl.total_ksteps) +
+                         kq_us(c, a->size_m, a->size_n - head * 512LL, q, 1, pl.total_ksteps);
+        if (t < best) best = t, mb = q, sp = 1, tail = pl.ncp - head;
+      }
+  }
+  if (!mb) return;
+  if (tail) {
+    pl.tail_strips = tail;
+    pl.tail_kind = 5;
+    pl.tail_mb = mb;
+    return;
+  }
+  pl.kind = 5;
+  pl.tn = 256;
+  pl.mb = mb;
+  pl.bm = 16 * mb;
+  pl.mtiles = (int)ceil_div(a->size_m, pl.bm);
+  pl.ncp = (int)ceil_div(a->size_n, 256);
+  pl.tiles = pl.mtiles * pl.ncp;
+  pl.kps = (int)ceil_div(octets, sp) * 8;
+  pl.splits = (int)ceil_div(pl.total_ksteps, pl.kps);
+  pl.xcd_map = 0;
+  pl.tail_strips = 0;
+  pl.ctmp_bytes = pl.splits > 1 ? (int64_t)pl.tiles * pl.splits * pl.bm * 256 * 4 : 0;
+}
+
+// more_scratch: plans may need more scratch than make_plan_16bit's
+static int make_plan(const w4a16_gemm_args* a, Plan& pl, bool more_scratch) {
   if (int rc = make_plan_16bit(a, pl)) return rc;
 #ifdef W4A16_TUNING
   static const int forced_kind = env_int("W4A16_KIND", -1);
-  if (env_int("W4A16_X8", 1) == 0) allow_x8 = false;
+  bool kq = env_int("W4A16_KQ", 1) != 0, x8 = env_int("W4A16_X8", 1) != 0;
   if (env_int("W4A16_DEBUG", 0) > 0)
     fprintf(stderr, "[plan] %lld %lld %lld kind %d mb %d tn %d tiles %d mtiles %d ncp %d splits %d kps %d tail %d %d\n", (long long)a->size_k,
             (long long)a->size_n, (long long)a->size_m, pl.kind, pl.mb, pl.tn, pl.tiles, pl.mtiles, pl.ncp, pl.splits, pl.kps, pl.tail_strips,
@@ -568,10 +661,16 @@ static int make_plan(const w4a16_gemm_args* a, Plan& pl, bool allow_x8) {
     x8_plan(a, env_int("W4A16_X8MB", 8), ks, env_int("W4A16_X8TN", 512 / ks), env_int("W4A16_X8SP", 1), pl);
     return 0;
   }
-  if (forced_kind >= 0) allow_x8 = false;
+  if (forced_kind >= 0) kq = x8 = false;
+#else
+  constexpr bool kq = true, x8 = true;
 #endif
-  if (allow_x8) try_x8(a, pl);
+  // (the 8-bit unit first: its results are the closer ones)
+  if (x8 && more_scratch) try_x8(a, pl);
+  if (kq && pl.kind != 6) try_kq(a, pl, more_scratch);
 #ifdef W4A16_TUNING
+  if (env_int("W4A16_DEBUG", 0) > 0)
+    fprintf(stderr, "[kq] kind %d mb %d splits %d kps %d tail %d %d\n", pl.kind, pl.mb, pl.splits, pl.kps, pl.tail_strips, pl.tail_mb);
   if (env_int("W4A16_DEBUG", 0) > 0 && pl.kind == 6) fprintf(stderr, "[x8] mb %d ks %d tn %d splits %d\n", pl.mb, pl.ks, pl.tn, pl.splits);
 #endif
   return 0;
@@ -610,10 +709,13 @@ static int run_planned(const w4a16_gemm_args* args, Plan& pl, void* stream) {
     head.ncp = pl.ncp - pl.tail_strips;
     head.tiles = head.ncp * pl.mtiles;
     if (int rc = launch_fat(&b, head, (hipStream_t)stream)) return rc;
-    if (pl.tail_kind == 5) {  // 128 x 256 tiles, K halves inside the workgroup
+    if (pl.tail_kind == 5) {  // tall tiles, K halves inside the workgroup
       tail.kind = 5;
       tail.tn = 256;
-      tail.ncp = 2 * pl.tail_strips;
+      tail.mb = pl.tail_mb;
+      tail.bm = 16 * tail.mb;
+      tail.mtiles = (int)ceil_div(args->size_m, tail.bm);
+      tail.ncp = (int)ceil_div(args->size_n - head.ncp * 512LL, 256);
       tail.tiles = tail.mtiles * tail.ncp;
       tail.strip0 = 2 * head.ncp;
       return launch_kq(&b, tail, (hipStream_t)stream);

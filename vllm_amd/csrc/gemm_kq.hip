@@ -17,13 +17,17 @@
 //                kernel's partial bytes for the same number of wavefronts on the problem.
 // Compared with 16-row tiles (which re-read and re-convert the weight strip once per 16 rows) every weight is fetched
 // and dequantised once per 64 rows; compared with the 64 x 512 tile there are 2 x 4 times as many independent streams.
-// A second shape of the same kernel (MB = 8, Q = 2: 4 wavefronts, one per SIMD, 128 rows x 256 columns, K in halves, 256
-// accumulators per lane) serves problems with 128-row tiles that are too few for the prefill kernel's 128 x 512 tiles:
-// every dequantised operand register feeds eight row blocks as in the prefill kernel, and the two K halves are added
-// through LDS instead of through memory.  The host uses it for more than 128 rows when these tiles fill 3/4 to all of the
-// compute units in one round, and for the trailing strips of a prefill launch whose last round is at most half full
-// (KParams.strip0: first 256-column strip of the launch).
-// Requirements (host-checked): K % 512 == 0 (second shape: K % 256 == 0), so that every K part runs whole ring periods of
+// The taller shapes of the same kernel (MB = 5 .. 8, Q = 2: 4 wavefronts, one per SIMD, 80 .. 128 rows x 256 columns, K in halves, up to
+// 256 accumulators per lane) serve problems that 128 x 512 tiles of the prefill kernel cut badly: every dequantised operand register feeds
+// MB row blocks, and the two K halves are added through LDS instead of through memory.  What bounds such a problem is how its tiles fill the
+// rounds of 256 workgroups, so the tile's height and the number of K splits across workgroups (of whole multiples of 256 K rows, the last
+// may be shorter) follow from the problem, by the times fitted in gemm.hip; a step of 32 K rows costs 0.25 us at 80 rows, 0.40 at 128.
+//   fp16, uint4b8, group 128, before (64- and 128-row tiles, unsplit ones only where they fill 3/4 of a round) and now: 4096 x 28672 at 160
+// rows 64 -> 44 us (80-row tiles), 14336 x 4096 at 300 rows 60 -> 49 (80 rows, four splits) and at 1501 rows 188 -> 160 (96 rows: 16 x 16
+// tiles instead of 12 x 16), 4096 x 6144 at 768 rows 60 -> 45, 2048 x 3072 at 1501 rows 44 -> 28.
+// They also finish the trailing strips of a prefill launch whose last round would be partly filled (KParams.strip0: first 256-column strip
+// of the launch).
+// Requirements (host-checked): K % 512 == 0 (taller shapes: K % 256 == 0), so that every K part runs whole ring periods of
 // 4 k-steps; scales grouped (a power-of-two number of k-steps) or channelwise, no per-row g_idx, A's columns already in
 // weight order.
 #include <type_traits>
@@ -43,7 +47,7 @@ constexpr int kq_smem(int MB, int Q) {
 
 template <int DT, bool ZP, bool CHANNEL, int MB = 4, int Q = 4>
 __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
-  static_assert((MB == 4 && Q == 4) || (MB == 8 && Q == 2), "64 x 256 in K quarters or 128 x 256 in K halves");
+  static_assert((MB == 4 && Q == 4) || (MB > 4 && MB <= 8 && Q == 2), "64 x 256 in K quarters or 80 .. 128 x 256 in K halves");
   constexpr int KQ_MB = MB, KQ_BM = 16 * MB, KQ_Q = Q, KQ_ABUF = kq_abuf(MB), KQ_SMEM = kq_smem(MB, Q);
   constexpr bool UNIT = CHANNEL;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -86,7 +90,8 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
   const uint32_t* zp = ZP ? Zp + nt * 8 + c : nullptr;
 
   // ---- this quarter's k-steps: [ks_b, ks_e), a multiple of 4 long
-  const int per_q = p.ksteps_per_split / KQ_Q;  // host: a multiple of 4, and the splits are equally long
+  // (host: whole splits and the rest behind them are multiples of 4 Q k-steps, so the parts of a workgroup are equally long)
+  const int per_q = min(p.ksteps_per_split, p.total_ksteps - split * p.ksteps_per_split) / KQ_Q;
   const int ks_b = split * p.ksteps_per_split + q * per_q, ks_e = ks_b + per_q;
 
   // ---- activation staging: the K part's 128 threads; thread tq loads piece (tq & 7) of tile rows (tq >> 3) + 16 i
@@ -171,7 +176,7 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
   // covers four k-steps (128 rows of K, aligned: every K part starts at a multiple of four k-steps), so with groups of
   // 128 rows or more, or one scale per column, they are rebuilt once per iteration instead of once per k-step.
   // (128-row tiles only: with two wavefronts per SIMD the 64-row tiles have no registers to spare for them.)
-  constexpr bool HOIST = (KQ_MB == 8);
+  constexpr bool HOIST = (KQ_MB > 4);
   ColConst<DT> ccs[4];
 #pragma unroll
   for (int w = 0; w < 4; ++w) ccs[w] = col_const(st[0], w);
@@ -201,12 +206,8 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
       const uint32_t xa = src.b0[wn2], xb = src.b1[wn2];
       auto step = [&](auto j_tag) {
         constexpr int J = decltype(j_tag)::value;
-        if constexpr (KQ_MB == 4) {
-          mfma_inplace<DT>(acc[J >> 1][w][J & 1], af[J >> 1], ob[w & 1][J & 1]);
-        } else {
-          mfma_inplace<DT>(acc[J][w][0], af[J], ob[w & 1][0]);
-          mfma_inplace<DT>(acc[J][w][1], af[J], ob[w & 1][1]);
-        }
+#pragma unroll
+        for (int i = J * KQ_MB / 4; i < (J + 1) * KQ_MB / 4; ++i) mfma_inplace<DT>(acc[i >> 1][w][i & 1], af[i >> 1], ob[w & 1][i & 1]);
         const uint32_t r = dequant_piece<DT, UNIT, J>(xa, xb, cc);
         if constexpr (J < 4)
           ob[wn2 & 1][0][J] = r;
@@ -327,12 +328,12 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
 
 // Second pass of a split-K launch: adds the splits' partial tiles in split order, then channel scale, bias and
 // conversion as kq_kernel's own epilogue.  One workgroup per (tile, 16-row block); thread -> 4 columns of 4 rows.
-template <int DT, bool CHANNEL, int MB = 4>
-__global__ __launch_bounds__(256) void kq_reduce_kernel(const KParams p) {
-  constexpr int KQ_BM = 16 * MB;
+template <int DT, bool CHANNEL>
+__global__ __launch_bounds__(256) void kq_reduce_kernel(const KParams p, int mb) {
+  const int KQ_BM = 16 * mb;
   const int t = threadIdx.x;
   const int mtiles = (p.M + KQ_BM - 1) / KQ_BM;
-  const int tile = blockIdx.x / MB, rb = blockIdx.x % MB;
+  const int tile = blockIdx.x / mb, rb = blockIdx.x % mb;
   const int mt = tile % mtiles, strip = tile / mtiles;
   const int fc4 = (t & 63) * 4;
   const int ncol = (p.strip0 + strip) * KQ_TN + fc4;
@@ -361,7 +362,14 @@ __global__ __launch_bounds__(256) void kq_reduce_kernel(const KParams p) {
     const int crow = mt * KQ_BM + r;
     if (crow >= p.M) continue;
     f32x4 v = {0, 0, 0, 0};
-    for (int sidx = 0; sidx < p.splits; ++sidx) v += *(const f32x4*)(parts + ((int64_t)sidx * KQ_BM + r) * KQ_TN);
+    for (int s0 = 0; s0 < p.splits; s0 += 4) {  // (four splits' loads are in flight together)
+      f32x4 a[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a[j] = *(const f32x4*)(parts + ((int64_t)min(s0 + j, p.splits - 1) * KQ_BM + r) * KQ_TN);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (s0 + j < p.splits) v += a[j];
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = v[j] * cs[j] + bs[j];
     u32x2 o;
@@ -374,38 +382,44 @@ __global__ __launch_bounds__(256) void kq_reduce_kernel(const KParams p) {
 }
 
 typedef void (*kq_fn)(const KParams);
+typedef void (*kq_reduce_fn)(const KParams, int);
 
 template <int DT, int MB, int Q>
 static kq_fn pick_kq(bool zp, bool channel) {
   if (zp) return channel ? kq_kernel<DT, true, true, MB, Q> : kq_kernel<DT, true, false, MB, Q>;
   return channel ? kq_kernel<DT, false, true, MB, Q> : kq_kernel<DT, false, false, MB, Q>;
 }
-template <int DT, int MB>
-static kq_fn pick_kq_reduce(bool channel) {
-  return channel ? kq_reduce_kernel<DT, true, MB> : kq_reduce_kernel<DT, false, MB>;
+template <int DT>
+static kq_fn pick_kq(int mb, bool zp, bool channel) {
+  switch (mb) {
+    case 4: return pick_kq<DT, 4, 4>(zp, channel);
+    case 5: return pick_kq<DT, 5, 2>(zp, channel);
+    case 6: return pick_kq<DT, 6, 2>(zp, channel);
+    case 7: return pick_kq<DT, 7, 2>(zp, channel);
+    case 8: return pick_kq<DT, 8, 2>(zp, channel);
+    default: return nullptr;
+  }
 }
 
 int launch_kq(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
   const bool zp = a->b_zeros != nullptr, channel = pl.gm == GM_CHANNEL;
-  const bool tall = pl.mb == 8;  // 128 x 256 tiles with K in halves; otherwise 64 x 256 with K in quarters
-  const int parts = tall ? 2 : 4;
-  if ((a->wtype != W4A16_WTYPE_U4B8 && a->wtype != W4A16_WTYPE_U4) || (a->flags & (W4A16_F_ZP_FLOAT | W4A16_F_MOE)) ||
-      pl.gm == GM_GIDX || pl.use_perm || pl.splits < 1 || pl.kps * pl.splits != pl.total_ksteps ||
-      pl.kps % (4 * parts) != 0 || pl.tn != KQ_TN || (pl.mb != 4 && pl.mb != 8))
-    return fail(W4A16_EINVAL, "unsupported kernel variant");
+  const int parts = pl.mb == 4 ? 4 : 2;  // 64 x 256 tiles with K in quarters, taller ones with K in halves
   const bool f16 = a->dtype == DT_F16;
-  const kq_fn fn = tall ? (f16 ? pick_kq<DT_F16, 8, 2>(zp, channel) : pick_kq<DT_BF16, 8, 2>(zp, channel))
-                        : (f16 ? pick_kq<DT_F16, 4, 4>(zp, channel) : pick_kq<DT_BF16, 4, 4>(zp, channel));
-  const int smem = tall ? kq_smem(8, 2) : kq_smem(4, 4);
+  const kq_fn fn = f16 ? pick_kq<DT_F16>(pl.mb, zp, channel) : pick_kq<DT_BF16>(pl.mb, zp, channel);
+  if ((a->wtype != W4A16_WTYPE_U4B8 && a->wtype != W4A16_WTYPE_U4) || (a->flags & (W4A16_F_ZP_FLOAT | W4A16_F_MOE)) ||
+      pl.gm == GM_GIDX || pl.use_perm || pl.splits < 1 || (int64_t)pl.kps * pl.splits < pl.total_ksteps ||
+      pl.kps * (pl.splits - 1) >= pl.total_ksteps || pl.kps % (4 * parts) != 0 || pl.total_ksteps % (4 * parts) != 0 || pl.tn != KQ_TN || !fn)
+    return fail(W4A16_EINVAL, "unsupported kernel variant");
+  const int smem = kq_smem(pl.mb, parts);
   KParams p = make_kparams(a, pl);
   if (pl.tiles <= 0) return 0;
   W4A16_HIP(allow_dynamic_lds((const void*)fn, smem));
   hipLaunchKernelGGL(fn, dim3((unsigned)((int64_t)pl.tiles * pl.splits)), dim3(128 * parts), smem, stream, p);
   W4A16_HIP(hipGetLastError());
   if (pl.splits > 1) {
-    const kq_fn red = tall ? (f16 ? pick_kq_reduce<DT_F16, 8>(channel) : pick_kq_reduce<DT_BF16, 8>(channel))
-                           : (f16 ? pick_kq_reduce<DT_F16, 4>(channel) : pick_kq_reduce<DT_BF16, 4>(channel));
-    hipLaunchKernelGGL(red, dim3((unsigned)pl.tiles * pl.mb), dim3(256), 0, stream, p);
+    const kq_reduce_fn red = f16 ? (channel ? kq_reduce_kernel<DT_F16, true> : kq_reduce_kernel<DT_F16, false>)
+                                 : (channel ? kq_reduce_kernel<DT_BF16, true> : kq_reduce_kernel<DT_BF16, false>);
+    hipLaunchKernelGGL(red, dim3((unsigned)pl.tiles * pl.mb), dim3(256), 0, stream, p, pl.mb);
     W4A16_HIP(hipGetLastError());
   }
   return 0;
