@@ -1,5 +1,6 @@
 """Tall K-split tiles (gemm_kq.hip) of 80, 96, 112 and 128 rows x 256 columns: whole problems unsplit and with K in two or three equal or
-unequal splits across workgroups, and the trailing strips of a prefill launch.
+unequal splits across workgroups, and the trailing strips of a prefill launch.  And tiles of 32, 48 and 64 rows x 128 columns whose K parts
+are single wavefronts.
 
 Operands are the 16-bit rounded weights (with one scale per column: the integers, the scale applied to the fp32 sum), so results are held
 to the float64 product with those.  What is left is the rounding of the result: 2^-11 / sqrt(12) of a value at the bottom of a binade of
@@ -31,6 +32,25 @@ MODES = [
     (torch.float16, "uint4", 32, False),
     (torch.bfloat16, "uint4b8", 64, False),
     (torch.float16, "uint4", -1, False),
+    (torch.float16, "uint4b8", 128, True),
+]
+
+# tiles whose eight K parts are single wavefronts
+PRIVATE_SHAPES = [
+    (29, 4096, 28672),    # 32 rows
+    (37, 4096, 28672),    # 48 rows
+    (135, 1024, 10816),   # ... one iteration per part, last tile one n-tile
+    (162, 2560, 1344),    # ... K in 28 + 28 + 24 k-steps: parts of 0, 4 and 8
+    (149, 4096, 3968),    # ... two splits
+    (60, 4096, 28672),    # 64 rows
+]
+PRIVATE_MODES = [
+    (torch.float16, "uint4b8", 128, False),
+    (torch.float16, "uint4", 128, False),
+    (torch.bfloat16, "uint4b8", 128, False),
+    (torch.bfloat16, "uint4", -1, False),
+    (torch.float16, "uint4b8", -1, False),
+    (torch.float16, "uint4b8", 256, False),
     (torch.float16, "uint4b8", 128, True),
 ]
 
@@ -79,8 +99,8 @@ def _rel(out, ref):
     return float((out.double() - ref).norm() / ref.norm())
 
 
-@pytest.mark.parametrize("m,k,n", SHAPES)
-@pytest.mark.parametrize("dtype,fmt,group,act_order", MODES)
+@pytest.mark.parametrize("m,k,n,dtype,fmt,group,act_order",
+                         [s + t for s in SHAPES for t in MODES] + [s + t for s in PRIVATE_SHAPES for t in PRIVATE_MODES])
 def test_against_float64(dev, workspace, m, k, n, dtype, fmt, group, act_order):
     print(f"kq heights m={m} k={k} n={n} {dtype} {fmt} group={group} act_order={act_order}", flush=True)
     from vllm_amd.marlin_utils import marlin_permute_bias
@@ -97,7 +117,7 @@ def test_against_float64(dev, workspace, m, k, n, dtype, fmt, group, act_order):
     assert int(workspace.abs().sum()) == 0
 
 
-@pytest.mark.parametrize("m,k,n", [(212, 2304, 9728), (161, 2816, 12352)])
+@pytest.mark.parametrize("m,k,n", [(508, 3840, 4224), (356, 3840, 6528)])
 def test_entry_point_without_scratch(dev, m, k, n):
     """A caller of the C entry point without scratch still gets a plan that needs none."""
     from vllm_amd import _lib

@@ -520,7 +520,21 @@ static double kq_us(const CostClass& c, int64_t m, int64_t cols, int mb, int spl
   const double other = c.bf16 ? (c.short_groups ? 0.085 : 0.065) : c.channel ? -0.03 : c.short_groups ? 0.03 : 0.003;
   const double t = 5.2 + rounds * (5.6 + kps * (other + 0.049 * mb));
   // (a second and third round of whole tiles cost more than the first)
-  return splits > 1 ? t + 3.9 + 0.9e-6 * splits * (double)m * (double)cols : t * (0.965 + 0.035 * (rounds < 4 ? rounds : 4));
+  return splits > 1 ? t + 3.9 + 0.9e-6 * splits * (double)m * (double)cols : t * (rounds < 2 ? 1 : rounds < 3 ? 1.045 : 1.15);
+}
+
+// private K parts (gemm_kq.hip, 16 mb x 128, groups of 128 rows or one scale per column): 3488 launches of 1116 problems of 17 to 512
+// rows, 5 %.  `steps`: of the longest part.
+static double priv_us(const CostClass& c, int64_t m, int64_t n, int mb, int splits, int steps) {
+  static const struct { double fixed, round, bf16, f16, channel, split, bytes; } by_mb[3] = {
+      {2.9, 4.6, 0.67, 0.545, 0.45, 3.4, 1.6e-6}, {3.1, 5.0, 0.785, 0.65, 0.58, 2.2, 2.3e-6}, {1.9, 7.4, 0.96, 0.77, 0.66, 1.9, 2.25e-6}};
+  const auto& s = by_mb[mb - 2];
+  const double zp = !c.zp ? 0 : c.bf16 ? (mb == 4 ? 0.09 : 0.04) : c.channel ? 0 : mb == 4 ? 0.11 : 0.045;
+  const double step = c.bf16 ? s.bf16 + (c.channel && mb < 4 ? 0.08 : 0) : c.channel ? s.channel : s.f16;
+  const double rounds = (double)ceil_div(ceil_div(m, 16 * mb) * ceil_div(n, 128) * splits, num_cus());
+  const double t = s.fixed + rounds * (s.round + (step + zp) * steps);
+  if (splits > 1) return t + s.split + s.bytes * splits * (double)m * (double)n;
+  return rounds > 1 ? t * (mb == 4 ? 1.06 : 1.10) : t;
 }
 
 static double fat_us(const CostClass& c, double rounds, int ksteps) {
@@ -540,6 +554,8 @@ static double plan16_us(const w4a16_gemm_args* a, const Plan& pl) {
       t += pl.tail_kind == 5 ? kq_us(c, a->size_m, a->size_n - head * 512LL, pl.tail_mb, 1, pl.total_ksteps) : (double)pl.total_ksteps;
     return t;
   }
+  if (pl.kind == 0 && (pl.mb == 2 || pl.mb == 3) && pl.splits == 1)
+    return (double)ceil_div(pl.tiles, cus) * (0.2 + (pl.mb == 2 ? (c.bf16 ? 0.174 : 0.162) : (c.bf16 ? 0.202 : 0.194)) * pl.kps);
   if (pl.kind == 5 && pl.mb > 4) return kq_us(c, a->size_m, a->size_n, pl.mb, pl.splits, pl.kps);
   const double rounds = (double)ceil_div((int64_t)pl.tiles * pl.splits, cus), per = pl.kps;
   const bool split = pl.splits > 1;
@@ -595,24 +611,30 @@ static void try_x8(const w4a16_gemm_args* a, Plan& pl) {
 
 // Tall K-split tiles for a whole problem, or for the trailing strips of a prefill launch, where they are predicted to be 5 % and 1 us
 // faster than the plan made above: that has 64- and 128-row tiles, one split count and one way to end a partly filled round; here the tile's
-// height and the splits follow the number of rows, the layer and the compute units.  Over the 1120 problems 384 change, to 0.57 .. 1.07
-// of their time, 0.85 in the mean (all problems 0.943; the best choice for each would give 0.936); over 72 random ones 0.84, worst 1.00.  Without `more_scratch` only unsplit
-// ones, which need none.
+// height and the splits follow the number of rows, the layer and the compute units.  In the same way 32 .. 64 x 128 tiles whose K parts are
+// single wavefronts take the place of the general kernel (groups of 128 rows at least: shorter ones need their constants more often than
+// once per loop iteration).  16-row tiles keep their problems: their sums are of unrounded weights.  2500 random problems (17 to 4096
+// rows, all types and groups): 423 change, to 0.8 of their time in the mean, eight of them to more than 1.00, at worst 1.07.
+// Without `more_scratch` only unsplit ones, which need none.
 static void try_kq(const w4a16_gemm_args* a, Plan& pl, bool more_scratch) {
   if ((a->flags & (W4A16_F_MOE | W4A16_F_ZP_FLOAT)) || (a->wtype != W4A16_WTYPE_U4B8 && a->wtype != W4A16_WTYPE_U4) || pl.gm == GM_GIDX ||
-      (pl.group_ksteps & (pl.group_ksteps - 1)) != 0 || a->size_k % 256 != 0 || a->size_m <= 64)
+      (pl.group_ksteps & (pl.group_ksteps - 1)) != 0 || a->size_k % 128 != 0 || a->size_m <= 16)
     return;
   const CostClass c = cost_class(a, pl);
-  const int cus = num_cus(), octets = (int)(a->size_k / 256);
-  double best = 0.95 * plan16_us(a, pl) - 1.0;
-  int mb = 0, sp = 0, tail = 0;
-  for (int q = 8; q >= 5; --q) {
+  const int cus = num_cus();
+  double best = plan16_us(a, pl);
+  if (best == 0) return;
+  const double third = pl.use_perm && best < 25 ? 4 : 0;  // a third launch behind the gather of act-order: small problems wait for the host
+  best = 0.95 * best - 1.0;
+  int mb = 0, sp = 0, tail = 0, tn = 256;
+  for (int q = 8; q >= 5 && a->size_m > 64 && a->size_k % 256 == 0; --q) {
     const int64_t tiles = ceil_div(a->size_m, 16 * q) * ceil_div(a->size_n, 256);
+    const int octets = (int)(a->size_k / 256);
     if (tiles >= (1LL << 31) / 64) return;
     for (int s = 1; s <= 16 && (s == 1 || (more_scratch && tiles * s <= 2 * cus && octets >= 2 * s)); ++s) {
       const int kps = (int)ceil_div(octets, s) * 8;
       if ((s - 1) * kps >= pl.total_ksteps) continue;  // (fewer splits of that length)
-      const double t = kq_us(c, a->size_m, a->size_n, q, s, kps);
+      const double t = kq_us(c, a->size_m, a->size_n, q, s, kps) + (s > 1 ? third : 0);
       if (t < best) best = t, mb = q, sp = s, tail = 0;
     }
     // (head: whole rounds, all there are or one fewer)
@@ -625,6 +647,17 @@ static void try_kq(const w4a16_gemm_args* a, Plan& pl, bool more_scratch) {
         if (t < best) best = t, mb = q, sp = 1, tail = pl.ncp - head;
       }
   }
+  const int64_t lda = pl.use_perm ? a->size_k : a->lda;
+  for (int q = 4; q >= 2 && (c.channel || pl.group_ksteps >= 4) && lda >= 0 && lda < (1 << 23); --q) {
+    const int64_t tiles = ceil_div(a->size_m, 16 * q) * ceil_div(a->size_n, 128);
+    if (a->size_m > (q < 4 ? 128 * q : 1024) || tiles > 2 * cus) continue;  // (the times are of one and two rounds)
+    for (int s = 1; s <= 8 && (s == 1 || (more_scratch && tiles * s <= cus && pl.total_ksteps >= 16 * s)); ++s) {
+      const int quads = (int)ceil_div(pl.total_ksteps / 4, s);
+      if ((s - 1) * quads * 4 >= pl.total_ksteps) continue;
+      const double t = priv_us(c, a->size_m, a->size_n, q, s, 4 * (int)ceil_div(quads, 8)) + (s > 1 ? third : 0);
+      if (t < (mb > 4 ? 0.94 * best : best)) best = t, mb = q, sp = s, tail = 0, tn = 128;  // (tall tiles read less: they win close calls)
+    }
+  }
   if (!mb) return;
   if (tail) {
     pl.tail_strips = tail;
@@ -632,18 +665,19 @@ static void try_kq(const w4a16_gemm_args* a, Plan& pl, bool more_scratch) {
     pl.tail_mb = mb;
     return;
   }
+  const int period = tn == 128 ? 4 : 8;  // k-steps
   pl.kind = 5;
-  pl.tn = 256;
+  pl.tn = tn;
   pl.mb = mb;
   pl.bm = 16 * mb;
   pl.mtiles = (int)ceil_div(a->size_m, pl.bm);
-  pl.ncp = (int)ceil_div(a->size_n, 256);
+  pl.ncp = (int)ceil_div(a->size_n, tn);
   pl.tiles = pl.mtiles * pl.ncp;
-  pl.kps = (int)ceil_div(octets, sp) * 8;
+  pl.kps = (int)ceil_div(pl.total_ksteps / period, sp) * period;
   pl.splits = (int)ceil_div(pl.total_ksteps, pl.kps);
   pl.xcd_map = 0;
   pl.tail_strips = 0;
-  pl.ctmp_bytes = pl.splits > 1 ? (int64_t)pl.tiles * pl.splits * pl.bm * 256 * 4 : 0;
+  pl.ctmp_bytes = pl.splits > 1 ? (int64_t)pl.tiles * pl.splits * pl.bm * tn * 4 : 0;
 }
 
 // more_scratch: plans may need more scratch than make_plan_16bit's

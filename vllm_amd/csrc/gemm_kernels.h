@@ -297,6 +297,15 @@ __device__ __forceinline__ void mfma_inplace(f32x4& acc, const u32x4& a, const u
     asm(W4A16_MFMA_PRE "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
+// ... accumulators in VGPRs: a kernel that uses no AGPRs has all 256 registers of a wavefront (two per SIMD) as VGPRs, otherwise 128
+template <int DT>
+__device__ __forceinline__ void mfma_inplace_v(f32x4& acc, const u32x4& a, const u32x4& b) {
+  if constexpr (DT == DT_F16)
+    asm(W4A16_MFMA_PRE "v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+  else
+    asm(W4A16_MFMA_PRE "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+}
+
 constexpr int RED_RS = 148;  // row stride (floats) of the 128-column reduction slab (4 mod 16: conflict-free)
 
 }  // namespace w4a16

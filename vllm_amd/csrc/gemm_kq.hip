@@ -27,43 +27,61 @@
 // tiles instead of 12 x 16), 4096 x 6144 at 768 rows 60 -> 45, 2048 x 3072 at 1501 rows 44 -> 28.
 // They also finish the trailing strips of a prefill launch whose last round would be partly filled (KParams.strip0: first 256-column strip
 // of the launch).
-// Requirements (host-checked): K % 512 == 0 (taller shapes: K % 256 == 0), so that every K part runs whole ring periods of
-// 4 k-steps; scales grouped (a power-of-two number of k-steps) or channelwise, no per-row g_idx, A's columns already in
-// weight order.
+//   A third shape (MB = 2 .. 4, Q = 8, one column pair: 32 .. 64 rows x 128 columns, 8 wavefronts, each a K eighth) is the general kernel's
+// tile with this kernel's loop.  There a wavefront loads, bounces and converts a k-step and then multiplies: VALU and MFMA add up (203 rows:
+// 1280 cycles of a SIMD per k-step of 64 x 128, 544 VALU + 512 MFMA).  Here the operands of the next word are made between the MFMAs,
+// activations arrive two k-steps at a time in rows of 128 bytes (17 cycles of the memory pipe per KB; rows of 64 bytes take 34) and are in
+// LDS one chunk ahead, scales come and constants are made once per 128 rows of K.  A K part is one wavefront, so nothing in the loop waits
+// for another and parts may differ in length.  Accumulators of 32- and 48-row tiles are VGPRs: without AGPRs all 256 registers can hold
+// operands.  fp16 uint4b8 / bf16 with zero points, before and now: 4096 x 28672 at 37 rows 23.4 -> 19.4 / 24.8 -> 22.6 us, at 64 rows 29.1 ->
+// 23.2 / 31.5 -> 28.2; 4096 x 6144 at 203 rows 26.1 -> 20.2 / 29.1 -> 23.9; 4096 x 4096 at 300 rows 25.7 -> 21.4 / 28.3 -> 26.0.
+// Requirements (host-checked): K % 512 == 0 (taller shapes: K % 256 == 0, third shape: K % 128 == 0), so that every K part runs whole ring
+// periods of 4 k-steps; scales grouped (a power-of-two number of k-steps; third shape: four at least) or channelwise, no per-row g_idx, A's
+// columns already in weight order.
 #include <type_traits>
 
 #include "gemm_kernels.h"
 
 namespace w4a16 {
 
-constexpr int KQ_TN = 256;   // columns per tile
 constexpr int KQ_D = 4;      // weight k-steps in flight per wavefront
 // MB m-blocks of 16 rows per tile, K cut into Q parts inside the workgroup (2 Q wavefronts)
 constexpr int kq_abuf(int MB) { return 2 * MB * 64 * 16; }  // one A buffer of one K part: 2 k-steps x MB m-blocks x 64 lanes x 16 B
-constexpr int kq_smem(int MB, int Q) {
-  const int stage = Q * 2 * kq_abuf(MB), slabs = 2 * Q * 16 * RED_RS * 4;  // staging rings | the wavefronts' epilogue slabs
+constexpr int kq_smem(int MB, int Q, int WN) {
+  const int stage = Q * 2 * kq_abuf(MB), slabs = WN * Q * 16 * RED_RS * 4;  // staging rings | the wavefronts' epilogue slabs
   return (stage > slabs ? stage : slabs) + 16 * MB * 4;                     // + C row of each tile row
 }
 
-template <int DT, bool ZP, bool CHANNEL, int MB = 4, int Q = 4>
-__global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
-  static_assert((MB == 4 && Q == 4) || (MB > 4 && MB <= 8 && Q == 2), "64 x 256 in K quarters or 80 .. 128 x 256 in K halves");
-  constexpr int KQ_MB = MB, KQ_BM = 16 * MB, KQ_Q = Q, KQ_ABUF = kq_abuf(MB), KQ_SMEM = kq_smem(MB, Q);
+template <int DT, bool ZP, bool CHANNEL, int MB = 4, int Q = 4, int WN = 2>
+__global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
+  static_assert((MB == 4 && Q == 4 && WN == 2) || (MB > 4 && MB <= 8 && Q == 2 && WN == 2) || (MB >= 2 && MB <= 4 && Q == 8 && WN == 1),
+                "64 x 256 in K quarters, 80 .. 128 x 256 in K halves or 32 .. 64 x 128 in K eighths");
+  constexpr int KQ_MB = MB, KQ_BM = 16 * MB, KQ_Q = Q, KQ_ABUF = kq_abuf(MB), KQ_SMEM = kq_smem(MB, Q, WN), KQ_TN = 128 * WN;
+  constexpr bool PRIV = (WN == 1);  // a K part is one wavefront: it stages its own activations, nothing in the loop waits for another
+  // HOIST: the dequantisation constants of the four word positions are kept for the k-step whose operands are being built.  A loop
+  // iteration covers four k-steps (128 rows of K, aligned: every K part starts at a multiple of four k-steps), so with groups of
+  // 128 rows or more, or one scale per column, they are rebuilt once per iteration instead of once per k-step.  (Not where the registers
+  // are short: 64-row tiles keep them in the 128-column form only, and there not in bf16 or with zero points: 12 to 38 would spill.)
+  constexpr bool HOIST = KQ_MB > 4 || (PRIV && (KQ_MB < 4 || CHANNEL || (DT == DT_F16 && !ZP)));
   constexpr bool UNIT = CHANNEL;
   extern __shared__ __align__(16) unsigned char smem[];
   int* s_crow = (int*)(smem + KQ_SMEM - KQ_BM * 4);
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int wn = wv & 1, q = wv >> 1;  // column pair inside the tile, K-quarter
+  const int wn = wv % WN, q = wv / WN;  // column pair inside the tile, K part
   const int c = lane & 7, h = (lane >> 3) & 1, g = lane >> 4;
 
   // tile order: consecutive workgroups walk M first, so workgroups resident together share weight strips
   const int mtiles = (p.M + KQ_BM - 1) / KQ_BM;
-  const int mt = blockIdx.x % mtiles;
-  const int split = (blockIdx.x / mtiles) % p.splits, strip = blockIdx.x / (mtiles * p.splits);
-  const int cp = (p.strip0 + strip) * 2 + wn;  // column pair of this wavefront (strip0: first 256-column strip of the launch)
-  const bool wave_on = cp * 128 < p.N;         // N not a multiple of 256: the trailing wavefronts only help staging
+  // and share them in one L2: workgroup ids rotate over the eight XCDs, each takes a contiguous run of the tiles (0 .. 4 %: 10496 x 26688,
+  // 555 rows 369 -> 354 us; 4096 x 6144, 203 rows 21.9 -> 21.2; 14336 x 4096, 300 rows 48.8 -> 47.8)
+  const int xcd = blockIdx.x & 7, rem = gridDim.x & 7;
+  const int wg = xcd * (int)(gridDim.x >> 3) + min(xcd, rem) + (int)(blockIdx.x >> 3);
+  const int mt = wg % mtiles;
+  const int split = (wg / mtiles) % p.splits, strip = wg / (mtiles * p.splits);
+  const int cp = (p.strip0 + strip) * WN + wn;  // column pair of this wavefront (strip0: first 256-column strip of the launch)
+  const bool wave_on = cp * 128 < p.N;          // N not a multiple of 256: the trailing wavefronts only help staging
   const int row0 = mt * KQ_BM;
 
   const uint32_t* Bq = p.B;
@@ -91,44 +109,60 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
 
   // ---- this quarter's k-steps: [ks_b, ks_e), a multiple of 4 long
   // (host: whole splits and the rest behind them are multiples of 4 Q k-steps, so the parts of a workgroup are equally long)
-  const int per_q = min(p.ksteps_per_split, p.total_ksteps - split * p.ksteps_per_split) / KQ_Q;
-  const int ks_b = split * p.ksteps_per_split + q * per_q, ks_e = ks_b + per_q;
+  // (private parts: as equally long as multiples of 4 k-steps go, some may be empty)
+  const int in_split = min(p.ksteps_per_split, p.total_ksteps - split * p.ksteps_per_split);
+  const int ks_b = split * p.ksteps_per_split + (PRIV ? in_split / 4 * q / KQ_Q * 4 : q * (in_split / KQ_Q));
+  const int per_q = PRIV ? in_split / 4 * (q + 1) / KQ_Q * 4 - in_split / 4 * q / KQ_Q * 4 : in_split / KQ_Q, ks_e = ks_b + per_q;
 
   // ---- activation staging: the K part's 128 threads; thread tq loads piece (tq & 7) of tile rows (tq >> 3) + 16 i
   // (rows without a source read row 0 of A; their results are never stored)
+  // (private parts: its 64 threads, rows (tq >> 3) + 8 i, MB / NH of them at a time, the last row of the problem in place of the rows
+  //  behind it)
+  constexpr int AR = PRIV ? 8 : 16, AN = KQ_BM / AR;           // rows per load instruction, loads per chunk
+  constexpr int NH = PRIV && KQ_MB == 4 ? 2 : 1, AH = AN / NH;  // (64 rows: the chunk in two halves, for its registers)
   const int tq = wn * 64 + lane;
   const int piece = tq & 7;
-  const uint16_t* arow[KQ_MB];
+  const uint16_t* arow[PRIV ? 1 : AN];
+  uint32_t aoff[PRIV ? AN : 1];
+  const char* abase = (const char*)p.A + (int64_t)row0 * p.lda * 2;
 #pragma unroll
-  for (int i = 0; i < KQ_MB; ++i) {
-    int src, dst;
-    tile_row_ids((tq >> 3) + 16 * i, src, dst);
-    arow[i] = (const uint16_t*)p.A + (int64_t)(src < 0 ? 0 : src) * p.lda + piece * 8;
+  for (int i = 0; i < AN; ++i) {
+    if constexpr (PRIV) {
+      aoff[i] = (uint32_t)min((tq >> 3) + AR * i, p.M - 1 - row0) * ((uint32_t)p.lda * 2) + piece * 16;  // (the host checks the size)
+    } else {
+      int src, dst;
+      tile_row_ids((tq >> 3) + AR * i, src, dst);
+      arow[i] = (const uint16_t*)p.A + (int64_t)(src < 0 ? 0 : src) * p.lda + piece * 8;
+    }
   }
-  // LDS A layout per quarter: [buffer][k-step 2][m-block 4][lane 64][4 dwords]; the 16 bytes of (row, piece) are the
+  // LDS A layout per part: [buffer][k-step 2][m-block][lane 64][4 dwords]; the 16 bytes of (row, piece) are the
   // K pairs 8*pp + 2j (pp = piece & 3), which belong to lane (j*16 + row%16), dword pp, of k-step piece >> 2.
   uint32_t* lds = (uint32_t*)smem + q * (2 * KQ_ABUF / 4);
-  int a_wr[KQ_MB];
-#pragma unroll
-  for (int i = 0; i < KQ_MB; ++i) {
-    const int r = (tq >> 3) + 16 * i;
-    a_wr[i] = (((piece >> 2) * KQ_MB + (r >> 4)) * 64 + (r & 15)) * 4 + (piece & 3);
-  }
-  u32x4 areg[KQ_MB];
+  const int a_wr0 = (((piece >> 2) * KQ_MB) * 64 + (tq >> 3)) * 4 + (piece & 3);
+  u32x4 areg[AH];
   // (chunk and k-step indices are clamped instead of guarded: the last iteration re-reads its own data, which
   //  keeps the main loop free of branches)
-  auto load_a = [&](int chunk) {  // chunk: relative to ks_b
+  auto load_a = [&](int chunk, int half) {  // chunk: relative to ks_b
     chunk = min(ks_b / 2 + chunk, ks_e / 2 - 1);
 #pragma unroll
-    for (int i = 0; i < KQ_MB; ++i) areg[i] = *(const u32x4*)(arow[i] + chunk * 64);
-  };
-  auto store_a = [&](int buf) {
-    uint32_t* dst = lds + buf * (KQ_ABUF / 4);
-#pragma unroll
-    for (int i = 0; i < KQ_MB; ++i) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) dst[a_wr[i] + j * 64] = areg[i][j];
+    for (int i = 0; i < AH; ++i) {
+      if constexpr (PRIV)
+        areg[i] = *(const u32x4*)(abase + (int64_t)chunk * 128 + aoff[half * AH + i]);
+      else
+        areg[i] = *(const u32x4*)(arow[i] + chunk * 64);
     }
+  };
+  auto store_a = [&](int buf, int half) {
+    uint32_t* dst = lds + buf * (KQ_ABUF / 4) + a_wr0;
+#pragma unroll
+    for (int i = 0; i < AH; ++i) {
+      const int r = AR * (half * AH + i);  // (row (tq >> 3) + r: m-block r / 16, AR = 8: upper half of it for odd loads)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dst[(r / 16) * 256 + (r % 16) * 4 + j * 64] = areg[i][j];
+    }
+  };
+  auto loop_barrier = [&]() {
+    if constexpr (!PRIV) __syncthreads();
   };
 
   struct Stage {
@@ -136,22 +170,32 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
     uint32_t zq;
   };
   Stage st[KQ_D];
+  // private parts have groups of 128 rows at least (host): scales and zero points once per loop iteration, loaded with its first k-step
+  u32x4 sc128 = {0, 0, 0, 0}, sc_now = {0, 0, 0, 0};
+  uint32_t zq128 = 0, zq_now = 0;
+  auto next_scales = [&]() { sc_now = sc128, zq_now = zq128; };
+  auto issue_scales = [&](int ks) {
+    const int gi = CHANNEL ? 0 : min(ks_b + ks, ks_e - 1) >> p.group_shift;
+    if (!CHANNEL) sc128 = sp[(int64_t)gi * s_row];
+    if (ZP) zq128 = zp[(int64_t)gi * s_row];
+  };
   auto issue = [&](Stage& s, int ks) {  // ks: relative to ks_b
     ks = min(ks_b + ks, ks_e - 1);
     int gi = 0;
     if (!CHANNEL) gi = ks >> p.group_shift;
-    if (!CHANNEL) s.sc = sp[(int64_t)gi * s_row];
-    if (ZP) s.zq = zp[(int64_t)gi * s_row];
+    if (!CHANNEL && !PRIV) s.sc = sp[(int64_t)gi * s_row];
+    if (ZP && !PRIV) s.zq = zp[(int64_t)gi * s_row];
     s.b0 = bp[(int64_t)(2 * ks) * b_row];
     s.b1 = bp[(int64_t)(2 * ks + 1) * b_row];
   };
   auto col_const = [&](const Stage& s, int w) {
     uint32_t z0 = 8, z1 = 8;
+    const uint32_t zq = PRIV ? zq_now : s.zq;
     if (ZP) {
-      z0 = (s.zq >> (4 * w)) & 0xf;
-      z1 = (s.zq >> (4 * w + 16)) & 0xf;
+      z0 = (zq >> (4 * w)) & 0xf;
+      z1 = (zq >> (4 * w + 16)) & 0xf;
     }
-    return make_col_const<DT, UNIT>(CHANNEL ? 0u : s.sc[w], z0, z1);
+    return make_col_const<DT, UNIT>(CHANNEL ? 0u : PRIV ? sc_now[w] : s.sc[w], z0, z1);
   };
 
   f32x4 acc[KQ_MB][4][2];
@@ -166,21 +210,28 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
   const int nchunks = per_q / 2;  // even
 
   // ---- prologue
-  load_a(0);
+  const bool any = !PRIV || nchunks > 0;
+  if (any) {
 #pragma unroll
-  for (int j = 0; j < KQ_D; ++j) issue(st[j], j);
-  store_a(0);
+    for (int hf = 0; hf < NH; ++hf) {
+      load_a(0, hf);
+      if (hf == 0) {
+        if constexpr (PRIV) issue_scales(0);
+#pragma unroll
+        for (int j = 0; j < KQ_D; ++j) issue(st[j], j);
+      }
+      store_a(0, hf);
+    }
+  }
   // B operands of two Marlin words: the one whose MFMAs are being issued and the one being dequantised
   u32x4 ob[2][2];
-  // dequantisation constants of the four word positions for the k-step whose operands are being built.  A loop iteration
-  // covers four k-steps (128 rows of K, aligned: every K part starts at a multiple of four k-steps), so with groups of
-  // 128 rows or more, or one scale per column, they are rebuilt once per iteration instead of once per k-step.
-  // (128-row tiles only: with two wavefronts per SIMD the 64-row tiles have no registers to spare for them.)
-  constexpr bool HOIST = (KQ_MB > 4);
   ColConst<DT> ccs[4];
+  if (any) {
+    next_scales();
 #pragma unroll
-  for (int w = 0; w < 4; ++w) ccs[w] = col_const(st[0], w);
-  dequant_pair<DT, UNIT>(st[0].b0[0], st[0].b1[0], ccs[0], ob[0][0], ob[0][1]);
+    for (int w = 0; w < 4; ++w) ccs[w] = col_const(st[0], w);
+    dequant_pair<DT, UNIT>(st[0].b0[0], st[0].b1[0], ccs[0], ob[0][0], ob[0][1]);
+  }
   __syncthreads();
 
   // One k-step: per Marlin word w, 2 MB MFMAs on ob[w & 1]; after each MFMA (MB = 8: pair of MFMAs) one register of the following word's
@@ -196,7 +247,9 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
       constexpr int wn2 = (w + 1) & 3;
       const Stage& src = w == 3 ? nxt : cur;
       ColConst<DT> cc_word;
+      if constexpr (PRIV && w == 3 && decltype(refresh_tag)::value) next_scales();
       if constexpr (!HOIST) {
+        if constexpr (PRIV) asm volatile("" : "+v"(sc_now), "+v"(zq_now));  // (or the compiler keeps all four words' constants)
         cc_word = col_const(src, wn2);
       } else if constexpr (w == 3 && decltype(refresh_tag)::value) {  // the words of `cur` are done: constants of `nxt`
 #pragma unroll
@@ -207,7 +260,12 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
       auto step = [&](auto j_tag) {
         constexpr int J = decltype(j_tag)::value;
 #pragma unroll
-        for (int i = J * KQ_MB / 4; i < (J + 1) * KQ_MB / 4; ++i) mfma_inplace<DT>(acc[i >> 1][w][i & 1], af[i >> 1], ob[w & 1][i & 1]);
+        for (int i = J * KQ_MB / 4; i < (J + 1) * KQ_MB / 4; ++i) {
+          if constexpr (KQ_MB < 4)
+            mfma_inplace_v<DT>(acc[i >> 1][w][i & 1], af[i >> 1], ob[w & 1][i & 1]);
+          else
+            mfma_inplace<DT>(acc[i >> 1][w][i & 1], af[i >> 1], ob[w & 1][i & 1]);
+        }
         const uint32_t r = dequant_piece<DT, UNIT, J>(xa, xb, cc);
         if constexpr (J < 4)
           ob[wn2 & 1][0][J] = r;
@@ -238,23 +296,26 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
 #pragma unroll 1
     for (int c0 = 0; c0 < nchunks; c0 += 2) {
       const int ks0 = 2 * c0;
-      load_a(c0 + 1);
+      load_a(c0 + 1, 0);
       kstep(0, 0, st[0], st[1], every_tag);
+      if constexpr (PRIV) issue_scales(ks0 + 4);
       issue(st[0], ks0 + 4);
+      if constexpr (NH == 2) store_a(1, 0), load_a(c0 + 1, 1);
       kstep(0, 1, st[1], st[2], every_tag);
       issue(st[1], ks0 + 5);
-      store_a(1);
-      __syncthreads();
-      load_a(c0 + 2);
+      store_a(1, NH - 1);
+      loop_barrier();
+      load_a(c0 + 2, 0);
       kstep(1, 0, st[2], st[3], every_tag);
       issue(st[2], ks0 + 6);
+      if constexpr (NH == 2) store_a(0, 0), load_a(c0 + 2, 1);
       kstep(1, 1, st[3], st[0], refresh);
       issue(st[3], ks0 + 7);
-      store_a(0);
-      __syncthreads();
+      store_a(0, NH - 1);
+      loop_barrier();
     }
   };
-  if constexpr (CHANNEL || !HOIST) {
+  if constexpr (CHANNEL || !HOIST || PRIV) {
     main_loop(std::false_type{});
   } else {
     if (p.group_shift < 2)
@@ -269,7 +330,8 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
   // per m-block: every wavefront writes its 16 x 128 partial to its slab [16 rows][RED_RS]; after a barrier the
   // wavefront of K part q adds the Q parts' slabs of its column pair for rows (16 / Q) q .. and finishes them.
-  // (the last barrier of the loop separates the slabs from the A buffers they overlay)
+  // (the last barrier of the loop, or this one, separates the slabs from the A buffers they overlay)
+  if constexpr (PRIV) __syncthreads();
   float* slabs = (float*)smem;
   float* mine = slabs + wv * (16 * RED_RS);
   const int fc4 = (lane & 31) * 4;
@@ -306,7 +368,7 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
       const int crow = s_crow[mb * 16 + r16];
       f32x4 v = {0, 0, 0, 0};
 #pragma unroll
-      for (int qq = 0; qq < KQ_Q; ++qq) v += *(const f32x4*)(slabs + (qq * 2 + wn) * (16 * RED_RS) + r16 * RED_RS + fpos);
+      for (int qq = 0; qq < KQ_Q; ++qq) v += *(const f32x4*)(slabs + (qq * WN + wn) * (16 * RED_RS) + r16 * RED_RS + fpos);
       if (p.splits > 1) {
         if (crow >= 0)
           *(f32x4*)(p.ctmp + (((int64_t)(strip * mtiles + mt) * p.splits + split) * KQ_BM + mb * 16 + r16) * KQ_TN +
@@ -328,14 +390,15 @@ __global__ __launch_bounds__(128 * Q) void kq_kernel(const KParams p) {
 
 // Second pass of a split-K launch: adds the splits' partial tiles in split order, then channel scale, bias and
 // conversion as kq_kernel's own epilogue.  One workgroup per (tile, 16-row block); thread -> 4 columns of 4 rows.
-template <int DT, bool CHANNEL>
+template <int DT, bool CHANNEL, int KQ_TN>
 __global__ __launch_bounds__(256) void kq_reduce_kernel(const KParams p, int mb) {
   const int KQ_BM = 16 * mb;
   const int t = threadIdx.x;
   const int mtiles = (p.M + KQ_BM - 1) / KQ_BM;
   const int tile = blockIdx.x / mb, rb = blockIdx.x % mb;
   const int mt = tile % mtiles, strip = tile / mtiles;
-  const int fc4 = (t & 63) * 4;
+  constexpr int TR = 1024 / KQ_TN;  // rows per pass
+  const int fc4 = (t % (KQ_TN / 4)) * 4;
   const int ncol = (p.strip0 + strip) * KQ_TN + fc4;
   if (ncol >= p.N) return;
   const uint16_t* Sc = (const uint16_t*)p.S;
@@ -357,8 +420,8 @@ __global__ __launch_bounds__(256) void kq_reduce_kernel(const KParams p, int mb)
   }
   const float* parts = p.ctmp + (int64_t)tile * p.splits * (KQ_BM * KQ_TN) + fc4;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = rb * 16 + (t >> 6) + 4 * i;
+  for (int i = 0; i < 16 / TR; ++i) {
+    const int r = rb * 16 + t / (KQ_TN / 4) + TR * i;
     const int crow = mt * KQ_BM + r;
     if (crow >= p.M) continue;
     f32x4 v = {0, 0, 0, 0};
@@ -384,41 +447,50 @@ __global__ __launch_bounds__(256) void kq_reduce_kernel(const KParams p, int mb)
 typedef void (*kq_fn)(const KParams);
 typedef void (*kq_reduce_fn)(const KParams, int);
 
-template <int DT, int MB, int Q>
+template <int DT, int MB, int Q, int WN>
 static kq_fn pick_kq(bool zp, bool channel) {
-  if (zp) return channel ? kq_kernel<DT, true, true, MB, Q> : kq_kernel<DT, true, false, MB, Q>;
-  return channel ? kq_kernel<DT, false, true, MB, Q> : kq_kernel<DT, false, false, MB, Q>;
+  if (zp) return channel ? kq_kernel<DT, true, true, MB, Q, WN> : kq_kernel<DT, true, false, MB, Q, WN>;
+  return channel ? kq_kernel<DT, false, true, MB, Q, WN> : kq_kernel<DT, false, false, MB, Q, WN>;
 }
 template <int DT>
-static kq_fn pick_kq(int mb, bool zp, bool channel) {
-  switch (mb) {
-    case 4: return pick_kq<DT, 4, 4>(zp, channel);
-    case 5: return pick_kq<DT, 5, 2>(zp, channel);
-    case 6: return pick_kq<DT, 6, 2>(zp, channel);
-    case 7: return pick_kq<DT, 7, 2>(zp, channel);
-    case 8: return pick_kq<DT, 8, 2>(zp, channel);
+static kq_fn pick_kq(int mb, int tn, bool zp, bool channel) {
+  switch (tn == 128 ? -mb : mb) {
+    case -2: return pick_kq<DT, 2, 8, 1>(zp, channel);
+    case -3: return pick_kq<DT, 3, 8, 1>(zp, channel);
+    case -4: return pick_kq<DT, 4, 8, 1>(zp, channel);
+    case 4: return pick_kq<DT, 4, 4, 2>(zp, channel);
+    case 5: return pick_kq<DT, 5, 2, 2>(zp, channel);
+    case 6: return pick_kq<DT, 6, 2, 2>(zp, channel);
+    case 7: return pick_kq<DT, 7, 2, 2>(zp, channel);
+    case 8: return pick_kq<DT, 8, 2, 2>(zp, channel);
     default: return nullptr;
   }
 }
+template <int DT>
+static kq_reduce_fn pick_kq_reduce(int tn, bool channel) {
+  if (tn == 128) return channel ? kq_reduce_kernel<DT, true, 128> : kq_reduce_kernel<DT, false, 128>;
+  return channel ? kq_reduce_kernel<DT, true, 256> : kq_reduce_kernel<DT, false, 256>;
+}
 
 int launch_kq(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
-  const bool zp = a->b_zeros != nullptr, channel = pl.gm == GM_CHANNEL;
-  const int parts = pl.mb == 4 ? 4 : 2;  // 64 x 256 tiles with K in quarters, taller ones with K in halves
+  const bool zp = a->b_zeros != nullptr, channel = pl.gm == GM_CHANNEL, priv = pl.tn == 128;
+  const int parts = priv ? 8 : pl.mb == 4 ? 4 : 2, wn = pl.tn / 128;
+  const int period = priv ? 4 : 4 * parts;  // splits are whole multiples of so many k-steps
   const bool f16 = a->dtype == DT_F16;
-  const kq_fn fn = f16 ? pick_kq<DT_F16>(pl.mb, zp, channel) : pick_kq<DT_BF16>(pl.mb, zp, channel);
+  const kq_fn fn = f16 ? pick_kq<DT_F16>(pl.mb, pl.tn, zp, channel) : pick_kq<DT_BF16>(pl.mb, pl.tn, zp, channel);
   if ((a->wtype != W4A16_WTYPE_U4B8 && a->wtype != W4A16_WTYPE_U4) || (a->flags & (W4A16_F_ZP_FLOAT | W4A16_F_MOE)) ||
       pl.gm == GM_GIDX || pl.use_perm || pl.splits < 1 || (int64_t)pl.kps * pl.splits < pl.total_ksteps ||
-      pl.kps * (pl.splits - 1) >= pl.total_ksteps || pl.kps % (4 * parts) != 0 || pl.total_ksteps % (4 * parts) != 0 || pl.tn != KQ_TN || !fn)
+      pl.kps * (pl.splits - 1) >= pl.total_ksteps || pl.kps % period != 0 || pl.total_ksteps % period != 0 ||
+      (pl.tn != 256 && !priv) || !fn || (priv && !channel && pl.group_ksteps < 4) || (priv && (a->lda < 0 || a->lda * 2 * pl.bm >= (1LL << 31))))
     return fail(W4A16_EINVAL, "unsupported kernel variant");
-  const int smem = kq_smem(pl.mb, parts);
+  const int smem = kq_smem(pl.mb, parts, wn);
   KParams p = make_kparams(a, pl);
   if (pl.tiles <= 0) return 0;
   W4A16_HIP(allow_dynamic_lds((const void*)fn, smem));
-  hipLaunchKernelGGL(fn, dim3((unsigned)((int64_t)pl.tiles * pl.splits)), dim3(128 * parts), smem, stream, p);
+  hipLaunchKernelGGL(fn, dim3((unsigned)((int64_t)pl.tiles * pl.splits)), dim3(64 * wn * parts), smem, stream, p);
   W4A16_HIP(hipGetLastError());
   if (pl.splits > 1) {
-    const kq_reduce_fn red = f16 ? (channel ? kq_reduce_kernel<DT_F16, true> : kq_reduce_kernel<DT_F16, false>)
-                                 : (channel ? kq_reduce_kernel<DT_BF16, true> : kq_reduce_kernel<DT_BF16, false>);
+    const kq_reduce_fn red = f16 ? pick_kq_reduce<DT_F16>(pl.tn, channel) : pick_kq_reduce<DT_BF16>(pl.tn, channel);
     hipLaunchKernelGGL(red, dim3((unsigned)pl.tiles * pl.mb), dim3(256), 0, stream, p, pl.mb);
     W4A16_HIP(hipGetLastError());
   }

@@ -14,7 +14,8 @@ struct Plan {
   int total_ksteps, splits, kps;  // k-steps of 32 rows; K splits; k-steps per split
   int xcd_map;
   int kind;  // 0: skinny kernel, 1: decode kernel, 2: prefill ("fat") kernel, 3: 64-row ("mid") kernel,
-             // 5: in-workgroup K split (gemm_kq.hip): 64 x 256 tiles in K quarters (mb = 4), 80 .. 128 x 256 in halves (mb = 5 .. 8)
+             // 5: in-workgroup K split (gemm_kq.hip): 64 x 256 tiles in K quarters (mb = 4), 80 .. 128 x 256 in halves (mb = 5 .. 8), 32 .. 64 x 128
+             // in eighths (mb = 2 .. 4, tn = 128)
   int tn;    // tile width in columns (128; the decode kernel also has 64)
   int nw = 8;  // 16-row tiles (decode kernel, general kernel with one m-block): wavefronts per workgroup (8 or 4)
   int strip0 = 0;      // 64-row kernel / K-split kernel: first 512- / 256-column strip handled by the launch
