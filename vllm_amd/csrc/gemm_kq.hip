@@ -46,7 +46,10 @@ namespace w4a16 {
 
 constexpr int KQ_D = 4;      // weight k-steps in flight per wavefront
 // MB m-blocks of 16 rows per tile, K cut into Q parts inside the workgroup (2 Q wavefronts)
-constexpr int kq_abuf(int MB) { return 2 * MB * 64 * 16; }  // one A buffer of one K part: 2 k-steps x MB m-blocks x 64 lanes x 16 B
+// dwords of one k-step of an A buffer: MB m-blocks x 64 lanes x 16 B, and half a row of the 64 banks: a wavefront's staging stores, 8 rows x
+// 2 k-steps x 4 dwords, then hit 64 different ones
+constexpr int kq_kstep(int MB) { return MB * 256 + 32; }
+constexpr int kq_abuf(int MB) { return 2 * kq_kstep(MB) * 4; }  // one A buffer of one K part: 2 k-steps
 constexpr int kq_smem(int MB, int Q, int WN) {
   const int stage = Q * 2 * kq_abuf(MB), slabs = WN * Q * 16 * RED_RS * 4;  // staging rings | the wavefronts' epilogue slabs
   return (stage > slabs ? stage : slabs) + 16 * MB * 4;                     // + C row of each tile row
@@ -138,7 +141,7 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   // LDS A layout per part: [buffer][k-step 2][m-block][lane 64][4 dwords]; the 16 bytes of (row, piece) are the
   // K pairs 8*pp + 2j (pp = piece & 3), which belong to lane (j*16 + row%16), dword pp, of k-step piece >> 2.
   uint32_t* lds = (uint32_t*)smem + q * (2 * KQ_ABUF / 4);
-  const int a_wr0 = (((piece >> 2) * KQ_MB) * 64 + (tq >> 3)) * 4 + (piece & 3);
+  const int a_wr0 = (piece >> 2) * kq_kstep(KQ_MB) + (tq >> 3) * 4 + (piece & 3);
   u32x4 areg[AH];
   // (chunk and k-step indices are clamped instead of guarded: the last iteration re-reads its own data, which
   //  keeps the main loop free of branches)
@@ -238,7 +241,7 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   // operands (word w + 1 of this k-step, or word 0 of the next k-step `nxt`) is dequantised into ob[(w + 1) & 1].
   // The scheduling barriers keep the compiler from regrouping this into MFMA-only and VALU-only blocks.
   auto kstep = [&](int buf, int kk, const Stage& cur, const Stage& nxt, auto refresh_tag) {
-    const u32x4* abase = (const u32x4*)(lds + buf * (KQ_ABUF / 4)) + (kk * KQ_MB) * 64 + lane;
+    const u32x4* abase = (const u32x4*)(lds + buf * (KQ_ABUF / 4) + kk * kq_kstep(KQ_MB)) + lane;
     u32x4 af[KQ_MB];
 #pragma unroll
     for (int mb = 0; mb < KQ_MB; ++mb) af[mb] = abase[mb * 64];
