@@ -47,8 +47,8 @@ namespace w4a16 {
 constexpr int KQ_D = 4;      // weight k-steps in flight per wavefront
 // MB m-blocks of 16 rows per tile, K cut into Q parts inside the workgroup (2 Q wavefronts)
 // dwords of one k-step of an A buffer: MB m-blocks x 64 lanes x 16 B, and half a row of the 64 banks: a wavefront's staging stores, 8 rows x
-// 2 k-steps x 4 dwords, then hit 64 different ones
-constexpr int kq_kstep(int MB) { return MB * 256 + 32; }
+// 2 k-steps x 4 dwords, then hit 64 different ones (128-row tiles without: 4096 x 4096 at 1024 rows 41.4 us, 41.6 with, and three spills)
+constexpr int kq_kstep(int MB) { return MB * 256 + (MB < 8 ? 32 : 0); }
 constexpr int kq_abuf(int MB) { return 2 * kq_kstep(MB) * 4; }  // one A buffer of one K part: 2 k-steps
 constexpr int kq_smem(int MB, int Q, int WN) {
   const int stage = Q * 2 * kq_abuf(MB), slabs = WN * Q * 16 * RED_RS * 4;  // staging rings | the wavefronts' epilogue slabs
