@@ -1,4 +1,4 @@
-// W4A16 GEMM for gfx950 with an in-workgroup K split: C[M,N] = A[M,K] * dequant(Bq)[K,N] (+bias), dense, in two shapes.
+// W4A16 GEMM for gfx950 with an in-workgroup K split: C[M,N] = A[M,K] * dequant(Bq)[K,N] (+bias), dense, in three shapes.
 // First shape, 64-row tiles: 33..128 rows and wide N, where the 64 x 512 tiles of the 64-row kernel are too few to fill
 // the chip (the reference's small-batch thread configurations, csrc/quantization/gptq_marlin/gptq_marlin.cu:120-170).
 //
