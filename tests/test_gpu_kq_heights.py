@@ -52,6 +52,11 @@ PRIVATE_MODES = [
     (torch.float16, "uint4b8", -1, False),
     (torch.float16, "uint4b8", 256, False),
     (torch.float16, "uint4b8", 128, True),
+    # scales with every k-step
+    (torch.float16, "uint4b8", 64, False),
+    (torch.float16, "uint4", 32, False),
+    (torch.bfloat16, "uint4b8", 32, False),
+    (torch.bfloat16, "uint4", 64, False),
 ]
 
 

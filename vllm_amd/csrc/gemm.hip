@@ -523,7 +523,7 @@ static double kq_us(const CostClass& c, int64_t m, int64_t cols, int mb, int spl
   return splits > 1 ? t + 3.9 + 0.9e-6 * splits * (double)m * (double)cols : t * (rounds < 2 ? 1 : rounds < 3 ? 1.045 : 1.15);
 }
 
-// private K parts (gemm_kq.hip, 16 mb x 128, groups of 128 rows or one scale per column): 3488 launches of 1116 problems of 17 to 512
+// private K parts (gemm_kq.hip, 16 mb x 128): 3488 launches of 1116 problems of 17 to 512
 // rows, 5 %.  `steps`: of the longest part.
 static double priv_us(const CostClass& c, int64_t m, int64_t n, int mb, int splits, int steps) {
   static const struct { double fixed, round, bf16, f16, channel, split, bytes; } by_mb[3] = {
@@ -531,8 +531,10 @@ static double priv_us(const CostClass& c, int64_t m, int64_t n, int mb, int spli
   const auto& s = by_mb[mb - 2];
   const double zp = !c.zp ? 0 : c.bf16 ? (mb == 4 ? 0.09 : 0.04) : c.channel ? 0 : mb == 4 ? 0.11 : 0.045;
   const double step = c.bf16 ? s.bf16 + (c.channel && mb < 4 ? 0.08 : 0) : c.channel ? s.channel : s.f16;
+  // (constants for every k-step: 1596 launches of 596 problems, groups of 32 and 64, 4 %)
+  const double often = !c.short_groups ? 0 : mb == 4 ? (c.bf16 ? 0.02 : 0) : c.bf16 ? (c.zp ? 0.17 : 0.115) : c.zp ? 0.1 : 0.035;
   const double rounds = (double)ceil_div(ceil_div(m, 16 * mb) * ceil_div(n, 128) * splits, num_cus());
-  const double t = s.fixed + rounds * (s.round + (step + zp) * steps);
+  const double t = s.fixed + rounds * (s.round + (step + zp + often) * steps);
   if (splits > 1) return t + s.split + s.bytes * splits * (double)m * (double)n;
   return rounds > 1 ? t * (mb == 4 ? 1.06 : 1.10) : t;
 }
@@ -609,13 +611,12 @@ static void try_x8(const w4a16_gemm_args* a, Plan& pl) {
   if (mb && ceil_div(a->size_m, 16 * mb) * ceil_div(a->size_n, tn) * sp < (1LL << 31) / 64) x8_plan(a, mb, ks, tn, sp, pl);
 }
 
-// Tall K-split tiles for a whole problem, or for the trailing strips of a prefill launch, where they are predicted to be 5 % and 1 us
-// faster than the plan made above: that has 64- and 128-row tiles, one split count and one way to end a partly filled round; here the tile's
-// height and the splits follow the number of rows, the layer and the compute units.  In the same way 32 .. 64 x 128 tiles whose K parts are
-// single wavefronts take the place of the general kernel (groups of 128 rows at least: shorter ones need their constants more often than
-// once per loop iteration).  16-row tiles keep their problems: their sums are of unrounded weights.  2500 random problems (17 to 4096
-// rows, all types and groups): 423 change, to 0.8 of their time in the mean, eight of them to more than 1.00, at worst 1.07.
-// Without `more_scratch` only unsplit ones, which need none.
+// Tall K-split tiles for a whole problem, or for the trailing strips of a prefill launch (in one round), where they are predicted to be
+// 5 % and 1 us faster than the plan made above: that has 64- and 128-row tiles, one split count and one way to end a partly filled round;
+// here the tile's height and the splits follow the number of rows, the layer and the compute units.  In the same way 32 .. 64 x 128 tiles
+// whose K parts are single wavefronts take the place of the general kernel.  16-row tiles keep their problems: their sums are of unrounded
+// weights.  Random problems of 17 to 4096 rows, all types and groups: of 4100 770 change, to 0.8 of their time in the mean, 2 % of those to
+// more than 1.00, at worst 1.1.  Without `more_scratch` only unsplit ones, which need none.
 static void try_kq(const w4a16_gemm_args* a, Plan& pl, bool more_scratch) {
   if ((a->flags & (W4A16_F_MOE | W4A16_F_ZP_FLOAT)) || (a->wtype != W4A16_WTYPE_U4B8 && a->wtype != W4A16_WTYPE_U4) || pl.gm == GM_GIDX ||
       (pl.group_ksteps & (pl.group_ksteps - 1)) != 0 || a->size_k % 128 != 0 || a->size_m <= 16)
@@ -624,7 +625,8 @@ static void try_kq(const w4a16_gemm_args* a, Plan& pl, bool more_scratch) {
   const int cus = num_cus();
   double best = plan16_us(a, pl);
   if (best == 0) return;
-  const double third = pl.use_perm && best < 25 ? 4 : 0;  // a third launch behind the gather of act-order: small problems wait for the host
+  // a second launch, or a third behind the gather of act-order: small problems wait for the host
+  const double launch = best < 25 && pl.use_perm ? 4 : best < 18 ? 1.5 : 0;
   best = 0.95 * best - 1.0;
   int mb = 0, sp = 0, tail = 0, tn = 256;
   for (int q = 8; q >= 5 && a->size_m > 64 && a->size_k % 256 == 0; --q) {
@@ -634,27 +636,28 @@ static void try_kq(const w4a16_gemm_args* a, Plan& pl, bool more_scratch) {
     for (int s = 1; s <= 16 && (s == 1 || (more_scratch && tiles * s <= 2 * cus && octets >= 2 * s)); ++s) {
       const int kps = (int)ceil_div(octets, s) * 8;
       if ((s - 1) * kps >= pl.total_ksteps) continue;  // (fewer splits of that length)
-      const double t = kq_us(c, a->size_m, a->size_n, q, s, kps) + (s > 1 ? third : 0);
+      const double t = kq_us(c, a->size_m, a->size_n, q, s, kps) + (s > 1 ? launch : 0);
       if (t < best) best = t, mb = q, sp = s, tail = 0;
     }
     // (head: whole rounds, all there are or one fewer)
     if (pl.kind == 2)
       for (int64_t rounds = (int64_t)pl.tiles / cus; rounds > 0 && rounds >= (int64_t)pl.tiles / cus - 1; --rounds) {
         const int head = (int)(rounds * cus / pl.mtiles);
-        if (head < 1 || head >= pl.ncp) continue;
+        if (head < 1 || head >= pl.ncp || ceil_div(a->size_m, 16 * q) * ceil_div(a->size_n - head * 512LL, 256) > cus) continue;
         const double t = fat_us(c, (double)ceil_div((int64_t)head * pl.mtiles, cus), pl.total_ksteps) +
                          kq_us(c, a->size_m, a->size_n - head * 512LL, q, 1, pl.total_ksteps);
         if (t < best) best = t, mb = q, sp = 1, tail = pl.ncp - head;
       }
   }
   const int64_t lda = pl.use_perm ? a->size_k : a->lda;
-  for (int q = 4; q >= 2 && (c.channel || pl.group_ksteps >= 4) && lda >= 0 && lda < (1 << 23); --q) {
+  for (int q = 4; q >= 2 && lda >= 0 && lda < (1 << 23); --q) {
+    if (q == 4 && c.short_groups && c.zp) continue;  // (no such kernel: it would spill)
     const int64_t tiles = ceil_div(a->size_m, 16 * q) * ceil_div(a->size_n, 128);
     if (a->size_m > (q < 4 ? 128 * q : 1024) || tiles > 2 * cus) continue;  // (the times are of one and two rounds)
     for (int s = 1; s <= 8 && (s == 1 || (more_scratch && tiles * s <= cus && pl.total_ksteps >= 16 * s)); ++s) {
       const int quads = (int)ceil_div(pl.total_ksteps / 4, s);
       if ((s - 1) * quads * 4 >= pl.total_ksteps) continue;
-      const double t = priv_us(c, a->size_m, a->size_n, q, s, 4 * (int)ceil_div(quads, 8)) + (s > 1 ? third : 0);
+      const double t = priv_us(c, a->size_m, a->size_n, q, s, 4 * (int)ceil_div(quads, 8)) + (s > 1 ? launch : 0);
       if (t < (mb > 4 ? 0.94 * best : best)) best = t, mb = q, sp = s, tail = 0, tn = 128;  // (tall tiles read less: they win close calls)
     }
   }

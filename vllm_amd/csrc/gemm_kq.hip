@@ -35,9 +35,12 @@
 // for another and parts may differ in length.  Accumulators of 32- and 48-row tiles are VGPRs: without AGPRs all 256 registers can hold
 // operands.  fp16 uint4b8 / bf16 with zero points, before and now: 4096 x 28672 at 37 rows 23.4 -> 19.4 / 24.8 -> 22.6 us, at 64 rows 29.1 ->
 // 23.2 / 31.5 -> 28.2; 4096 x 6144 at 203 rows 26.1 -> 20.2 / 29.1 -> 23.9; 4096 x 4096 at 300 rows 25.7 -> 21.4 / 28.3 -> 26.0.
+// Groups of 32 and 64 rows have a variant with scales in every k-step's stage and constants made for every word (SHORT; a k-step costs it
+// 6 % more in fp16, 15 to 25 % in bf16; 64-row tiles with zero points would spill 2 to 18 registers and do not exist): over 900 random
+// problems of 17 to 900 rows, mostly of such groups, 218 change, to 0.80 of their time in the mean, worst 1.02.
 // Requirements (host-checked): K % 512 == 0 (taller shapes: K % 256 == 0, third shape: K % 128 == 0), so that every K part runs whole ring
-// periods of 4 k-steps; scales grouped (a power-of-two number of k-steps; third shape: four at least) or channelwise, no per-row g_idx, A's
-// columns already in weight order.
+// periods of 4 k-steps; scales grouped (a power-of-two number of k-steps) or channelwise, no per-row g_idx, A's columns already in
+// weight order.
 #include <type_traits>
 
 #include "gemm_kernels.h"
@@ -55,7 +58,8 @@ constexpr int kq_smem(int MB, int Q, int WN) {
   return (stage > slabs ? stage : slabs) + 16 * MB * 4;                     // + C row of each tile row
 }
 
-template <int DT, bool ZP, bool CHANNEL, int MB = 4, int Q = 4, int WN = 2>
+// SHORT: private parts with groups below 128 rows, whose scales and constants come with every k-step
+template <int DT, bool ZP, bool CHANNEL, int MB = 4, int Q = 4, int WN = 2, bool SHORT = false>
 __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   static_assert((MB == 4 && Q == 4 && WN == 2) || (MB > 4 && MB <= 8 && Q == 2 && WN == 2) || (MB >= 2 && MB <= 4 && Q == 8 && WN == 1),
                 "64 x 256 in K quarters, 80 .. 128 x 256 in K halves or 32 .. 64 x 128 in K eighths");
@@ -65,7 +69,8 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   // iteration covers four k-steps (128 rows of K, aligned: every K part starts at a multiple of four k-steps), so with groups of
   // 128 rows or more, or one scale per column, they are rebuilt once per iteration instead of once per k-step.  (Not where the registers
   // are short: 64-row tiles keep them in the 128-column form only, and there not in bf16 or with zero points: 12 to 38 would spill.)
-  constexpr bool HOIST = KQ_MB > 4 || (PRIV && (KQ_MB < 4 || CHANNEL || (DT == DT_F16 && !ZP)));
+  constexpr bool ONCE = PRIV && !SHORT;
+  constexpr bool HOIST = KQ_MB > 4 || (ONCE && (KQ_MB < 4 || CHANNEL || (DT == DT_F16 && !ZP)));
   constexpr bool UNIT = CHANNEL;
   extern __shared__ __align__(16) unsigned char smem[];
   int* s_crow = (int*)(smem + KQ_SMEM - KQ_BM * 4);
@@ -173,7 +178,7 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
     uint32_t zq;
   };
   Stage st[KQ_D];
-  // private parts have groups of 128 rows at least (host): scales and zero points once per loop iteration, loaded with its first k-step
+  // groups of 128 rows at least (host): scales and zero points once per loop iteration, loaded with its first k-step
   u32x4 sc128 = {0, 0, 0, 0}, sc_now = {0, 0, 0, 0};
   uint32_t zq128 = 0, zq_now = 0;
   auto next_scales = [&]() { sc_now = sc128, zq_now = zq128; };
@@ -186,19 +191,19 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
     ks = min(ks_b + ks, ks_e - 1);
     int gi = 0;
     if (!CHANNEL) gi = ks >> p.group_shift;
-    if (!CHANNEL && !PRIV) s.sc = sp[(int64_t)gi * s_row];
-    if (ZP && !PRIV) s.zq = zp[(int64_t)gi * s_row];
+    if (!CHANNEL && !ONCE) s.sc = sp[(int64_t)gi * s_row];
+    if (ZP && !ONCE) s.zq = zp[(int64_t)gi * s_row];
     s.b0 = bp[(int64_t)(2 * ks) * b_row];
     s.b1 = bp[(int64_t)(2 * ks + 1) * b_row];
   };
   auto col_const = [&](const Stage& s, int w) {
     uint32_t z0 = 8, z1 = 8;
-    const uint32_t zq = PRIV ? zq_now : s.zq;
+    const uint32_t zq = ONCE ? zq_now : s.zq;
     if (ZP) {
       z0 = (zq >> (4 * w)) & 0xf;
       z1 = (zq >> (4 * w + 16)) & 0xf;
     }
-    return make_col_const<DT, UNIT>(CHANNEL ? 0u : PRIV ? sc_now[w] : s.sc[w], z0, z1);
+    return make_col_const<DT, UNIT>(CHANNEL ? 0u : ONCE ? sc_now[w] : s.sc[w], z0, z1);
   };
 
   f32x4 acc[KQ_MB][4][2];
@@ -219,7 +224,7 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
     for (int hf = 0; hf < NH; ++hf) {
       load_a(0, hf);
       if (hf == 0) {
-        if constexpr (PRIV) issue_scales(0);
+        if constexpr (ONCE) issue_scales(0);
 #pragma unroll
         for (int j = 0; j < KQ_D; ++j) issue(st[j], j);
       }
@@ -250,9 +255,9 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
       constexpr int wn2 = (w + 1) & 3;
       const Stage& src = w == 3 ? nxt : cur;
       ColConst<DT> cc_word;
-      if constexpr (PRIV && w == 3 && decltype(refresh_tag)::value) next_scales();
+      if constexpr (ONCE && w == 3 && decltype(refresh_tag)::value) next_scales();
       if constexpr (!HOIST) {
-        if constexpr (PRIV) asm volatile("" : "+v"(sc_now), "+v"(zq_now));  // (or the compiler keeps all four words' constants)
+        if constexpr (ONCE) asm volatile("" : "+v"(sc_now), "+v"(zq_now));  // (or the compiler keeps all four words' constants)
         cc_word = col_const(src, wn2);
       } else if constexpr (w == 3 && decltype(refresh_tag)::value) {  // the words of `cur` are done: constants of `nxt`
 #pragma unroll
@@ -301,7 +306,7 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
       const int ks0 = 2 * c0;
       load_a(c0 + 1, 0);
       kstep(0, 0, st[0], st[1], every_tag);
-      if constexpr (PRIV) issue_scales(ks0 + 4);
+      if constexpr (ONCE) issue_scales(ks0 + 4);
       issue(st[0], ks0 + 4);
       if constexpr (NH == 2) store_a(1, 0), load_a(c0 + 1, 1);
       kstep(0, 1, st[1], st[2], every_tag);
@@ -455,8 +460,18 @@ static kq_fn pick_kq(bool zp, bool channel) {
   if (zp) return channel ? kq_kernel<DT, true, true, MB, Q, WN> : kq_kernel<DT, true, false, MB, Q, WN>;
   return channel ? kq_kernel<DT, false, true, MB, Q, WN> : kq_kernel<DT, false, false, MB, Q, WN>;
 }
+// (64-row tiles with zero points would spill)
+template <int DT, int MB>
+static kq_fn pick_kq_short(bool zp) {
+  if (!zp) return kq_kernel<DT, false, false, MB, 8, 1, true>;
+  if constexpr (MB == 4)
+    return nullptr;
+  else
+    return kq_kernel<DT, true, false, MB, 8, 1, true>;
+}
 template <int DT>
-static kq_fn pick_kq(int mb, int tn, bool zp, bool channel) {
+static kq_fn pick_kq(int mb, int tn, bool zp, bool channel, bool short_groups) {
+  if (tn == 128 && short_groups) return mb == 2 ? pick_kq_short<DT, 2>(zp) : mb == 3 ? pick_kq_short<DT, 3>(zp) : mb == 4 ? pick_kq_short<DT, 4>(zp) : nullptr;
   switch (tn == 128 ? -mb : mb) {
     case -2: return pick_kq<DT, 2, 8, 1>(zp, channel);
     case -3: return pick_kq<DT, 3, 8, 1>(zp, channel);
@@ -480,11 +495,12 @@ int launch_kq(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
   const int parts = priv ? 8 : pl.mb == 4 ? 4 : 2, wn = pl.tn / 128;
   const int period = priv ? 4 : 4 * parts;  // splits are whole multiples of so many k-steps
   const bool f16 = a->dtype == DT_F16;
-  const kq_fn fn = f16 ? pick_kq<DT_F16>(pl.mb, pl.tn, zp, channel) : pick_kq<DT_BF16>(pl.mb, pl.tn, zp, channel);
+  const bool short_groups = !channel && pl.group_ksteps < 4;
+  const kq_fn fn = f16 ? pick_kq<DT_F16>(pl.mb, pl.tn, zp, channel, short_groups) : pick_kq<DT_BF16>(pl.mb, pl.tn, zp, channel, short_groups);
   if ((a->wtype != W4A16_WTYPE_U4B8 && a->wtype != W4A16_WTYPE_U4) || (a->flags & (W4A16_F_ZP_FLOAT | W4A16_F_MOE)) ||
       pl.gm == GM_GIDX || pl.use_perm || pl.splits < 1 || (int64_t)pl.kps * pl.splits < pl.total_ksteps ||
       pl.kps * (pl.splits - 1) >= pl.total_ksteps || pl.kps % period != 0 || pl.total_ksteps % period != 0 ||
-      (pl.tn != 256 && !priv) || !fn || (priv && !channel && pl.group_ksteps < 4) || (priv && (a->lda < 0 || a->lda * 2 * pl.bm >= (1LL << 31))))
+      (pl.tn != 256 && !priv) || !fn || (priv && (a->lda < 0 || a->lda * 2 * pl.bm >= (1LL << 31))))
     return fail(W4A16_EINVAL, "unsupported kernel variant");
   const int smem = kq_smem(pl.mb, parts, wn);
   KParams p = make_kparams(a, pl);
