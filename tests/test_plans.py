@@ -115,3 +115,10 @@ def test_shapes_of_the_k_split_tiles(plan):
     assert {(mb, 128, True, "uint4", "short") for mb in (2, 3)} <= kernels
     assert {(tn, bf16, channel) for tn in (128, 256) for bf16 in (False, True) for channel in (False, True)} <= second_passes
     assert any(m <= 128 and tn == 256 for s in kq.PINNED.values() for (m, _, _), (_, tn, _) in s.items())
+
+
+def test_64_row_kernel_of_the_constants_test(plan):
+    import test_gpu_group_constants as gc
+    for dtype, fmt in gc.TYPES:
+        for group in (32, 64, 128, 256, -1):
+            assert plan(*gc.DENSE, dtype, fmt, group)["kind"] == 3

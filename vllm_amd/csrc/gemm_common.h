@@ -69,12 +69,12 @@ __device__ __forceinline__ uint32_t pack_f16(float lo, float hi) {
 }
 
 // Per-lane dequantisation constants of one Marlin word position w (two columns: half 0 / half 1).
-//  fp16:  value = (1024+q) - zl  |  (1024+16q)/16 - zh , then * s         (all packed-half ops;
+//  fp16:  value = (1024+q) - (1024+z)  |  (64+q) - (64+z) , then * s         (all packed-half ops;
 //         every step is exact except the final multiply, so the operand equals
 //         half(q - z) * half(s) rounded once — the reference's w_ref)
-//  bf16:  the nibbles are turned into the same exact fp16 pairs, (1024+q) and (1024+16q), and one mixed-precision
+//  bf16:  the nibbles are turned into the same exact fp16 pairs, (1024+q) and (64+q), and one mixed-precision
 //         FMA per value (v_fma_mix_f32: fp16 x fp32 + fp32 -> fp32) gives (q - z) * s in fp32:
-//         fma(1024+q, s, -(1024+z) s)  |  fma(1024+16q, s/16, -(64+z) s).  The constants are exact in fp32 (at most
+//         fma(1024+q, s, -(1024+z) s)  |  fma(64+q, s, -(64+z) s).  The constants are exact in fp32 (at most
 //         11 + 8 bits) and so is the result (at most 5 + 8 bits), which v_cvt_pk_bf16_f32 then rounds once:
 //         bf16_rne((q - z) * s), the reference's w_ref.
 template <int DT>
@@ -90,77 +90,109 @@ template <>
 struct ColConst<DT_BF16> {
   float s0, s1;  // scale of half 0 / half 1
   float c0, c1;  // -(1024+z)*s
-  float h0, h1;  // s/16
   float d0, d1;  // -(64+z)*s
 };
 
-// raw: (s_half0, s_half1) packed 16-bit pair as loaded; z0/z1: integer zero points (8 for uint4b8)
-template <int DT, bool UNIT_SCALE>
-__device__ __forceinline__ ColConst<DT> make_col_const(uint32_t s_pair, uint32_t z0, uint32_t z1) {
+constexpr uint32_t ZERO_U4B8 = 0x00080008u;  // the zero-point pair of uint4b8
+// word of the lane's eight zero points -> the pair of word position w
+__device__ __forceinline__ uint32_t zero_pair(uint32_t zq, int w) { return (zq >> (4 * w)) & 0x000f000fu; }
+
+// s_pair: (s_half0, s_half1) packed 16-bit pair as loaded; z_pair: their integer zero points, one in each half
+// MIXED (no scale): every value takes one mixed FMA by a factor kept in a register; a factor known to be one makes it a conversion and an
+// addition
+template <int DT, bool UNIT_SCALE, bool MIXED = true>
+__device__ __forceinline__ ColConst<DT> make_col_const(uint32_t s_pair, uint32_t z_pair) {
   ColConst<DT> cc;
+  // 1024+z and 64+z are exact fp16 integers: 0x6400 | z  and  0x5400 + (z << 4) (ulp of 64.. is 1/16)
+  const uint32_t z1024 = 0x64006400u | z_pair;
   if constexpr (DT == DT_F16) {
     cc.s = UNIT_SCALE ? 0x3c003c00u : s_pair;
-    // 1024+z and 64+z are exact fp16 integers: 0x6400 | z  and  0x5400 + (z << 4) (ulp of 64.. is 1/16)
-    cc.zl = 0x64006400u | z0 | (z1 << 16);
-    cc.zh = 0x54005400u + ((z0 << 4) | (z1 << 20));
+    cc.zl = z1024;
+    cc.zh = 0x54005400u + (z_pair << 4);
   } else {
-    cc.s0 = UNIT_SCALE ? 1.0f : bf16_lo_f32(s_pair);
-    cc.s1 = UNIT_SCALE ? 1.0f : bf16_hi_f32(s_pair);
-    // 1024+z as fp32 bits: 2^10 has its ulp at 2^-13, so z sits at bit 13 of the mantissa
-    const float t0 = __builtin_bit_cast(float, 0x44800000u | (z0 << 13));
-    const float t1 = __builtin_bit_cast(float, 0x44800000u | (z1 << 13));
-    cc.c0 = -t0 * cc.s0;
-    cc.c1 = -t1 * cc.s1;
-    cc.h0 = cc.s0 * 0.0625f;
-    cc.h1 = cc.s1 * 0.0625f;
+    float one = 1.0f;
+    if (UNIT_SCALE && MIXED) asm("" : "+s"(one));
+    cc.s0 = UNIT_SCALE ? one : bf16_lo_f32(s_pair);
+    cc.s1 = UNIT_SCALE ? one : bf16_hi_f32(s_pair);
+    cc.c0 = __builtin_fmaf((float)as_h2(z1024).x, -cc.s0, 0.0f);  // (one mixed FMA each)
+    cc.c1 = __builtin_fmaf((float)as_h2(z1024).y, -cc.s1, 0.0f);
     cc.d0 = __builtin_fmaf(960.0f, cc.s0, cc.c0);
     cc.d1 = __builtin_fmaf(960.0f, cc.s1, cc.c1);
   }
   return cc;
 }
 
+// ---- One register (J = 0..7) of the operands made from a Marlin word pair, in three steps that each depend on the one before.
+// J < 4: register J of the operand of column half 0, else J - 4 of half 1; J & 3 < 2: from the word of k-tile 2ks, else of 2ks + 1.
+// A kernel issues the steps of three consecutive registers between the same MFMAs (see gemm_kq.hip), so that no VALU instruction waits
+// for the one in front of it.
+//   piece_halves  nibbles 2 HF + ODD and that + 4 of the word: the exact fp16 pair 1024 + q (even J) or 64 + q (odd J)
+//   piece_value   fp16: q - z; bf16: (q - z) * s in fp32
+//   piece_finish  fp16: times s; bf16: the pack
+template <int DT>
+struct PieceValue;
+template <>
+struct PieceValue<DT_F16> {
+  f16x2 v;
+};
+template <>
+struct PieceValue<DT_BF16> {
+  float f0, f1;
+};
+
+template <int J>
+__device__ __forceinline__ uint32_t piece_halves(uint32_t x) {
+  constexpr bool HIGH = J & 1;
+  // keep the exponent pattern in a VGPR so that (x & mask) | EX is one v_and_or_b32
+  uint32_t EX = HIGH ? 0x54005400u : 0x64006400u;
+  asm("" : "+v"(EX));
+  const uint32_t y = (J >> 2) ? (x >> 8) : x;
+  return (y & (HIGH ? 0x00f000f0u : 0x000f000fu)) | EX;
+}
+template <int DT, int J>
+__device__ __forceinline__ PieceValue<DT> piece_value(uint32_t halves, const ColConst<DT>& cc) {
+  constexpr int HF = J >> 2, ODD = J & 1;
+  const f16x2 v = as_h2(halves);
+  PieceValue<DT> r;
+  if constexpr (DT == DT_F16) {
+    const f16x2 z = as_h2(ODD ? cc.zh : cc.zl);
+    r.v = v - (HF ? f16x2{z.y, z.y} : f16x2{z.x, z.x});
+  } else {
+    const float m = HF ? cc.s1 : cc.s0;
+    const float a = ODD ? (HF ? cc.d1 : cc.d0) : (HF ? cc.c1 : cc.c0);
+    r.f0 = __builtin_fmaf((float)v.x, m, a);
+    r.f1 = __builtin_fmaf((float)v.y, m, a);
+  }
+  return r;
+}
+template <int DT, bool UNIT_SCALE, int J>
+__device__ __forceinline__ uint32_t piece_finish(const PieceValue<DT>& p, const ColConst<DT>& cc) {
+  if constexpr (DT == DT_F16) {
+    const f16x2 s = as_h2(cc.s);
+    return as_u32(UNIT_SCALE ? p.v : p.v * ((J >> 2) ? f16x2{s.y, s.y} : f16x2{s.x, s.x}));
+  } else {
+    return pack_bf16(p.f0, p.f1);
+  }
+}
+// f(std::integral_constant<int, P>) for the N registers of a k-step
+template <int N, int P = 0, typename F>
+__device__ __forceinline__ void for_each_piece(const F& f) {
+  f(std::integral_constant<int, P>{});
+  if constexpr (P + 1 < N) for_each_piece<N, P + 1>(f);
+}
+
 // xa, xb: word w of the lane's 128-bit loads from k-tile 2ks and 2ks+1.
 // o0 / o1: MFMA B operand (8 values in the lane's K order) for column half 0 / half 1.
 template <int DT, bool UNIT_SCALE>
-__device__ __forceinline__ void dequant_pair(uint32_t xa, uint32_t xb, const ColConst<DT>& cc, u32x4& o0,
-                                             u32x4& o1) {
-  if constexpr (DT == DT_F16) {
-    const uint32_t MLO = 0x000f000fu, MHI = 0x00f000f0u;
-    // keep the exponent pattern in a VGPR so that (x & mask) | EX is one v_and_or_b32
-    uint32_t EX = 0x64006400u;
-    asm("" : "+v"(EX));
-    const f16x2 sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-    const f16x2 s = as_h2(cc.s), zl = as_h2(cc.zl), zh = as_h2(cc.zh);
-    const f16x2 s0 = {s.x, s.x}, s1 = {s.y, s.y};
-    const f16x2 zl0 = {zl.x, zl.x}, zl1 = {zl.y, zl.y};
-    const f16x2 zh0 = {zh.x, zh.x}, zh1 = {zh.y, zh.y};
-    auto lo = [&](uint32_t x, f16x2 z, f16x2 sc) {
-      const f16x2 v = as_h2((x & MLO) | EX) - z;
-      return as_u32(UNIT_SCALE ? v : v * sc);
-    };
-    auto hi = [&](uint32_t x, f16x2 z, f16x2 sc) {
-      const f16x2 v = as_h2((x & MHI) | EX) * sixteenth - z;
-      return as_u32(UNIT_SCALE ? v : v * sc);
-    };
-    const uint32_t ya = xa >> 8, yb = xb >> 8;
-    o0 = u32x4{lo(xa, zl0, s0), hi(xa, zh0, s0), lo(xb, zl0, s0), hi(xb, zh0, s0)};
-    o1 = u32x4{lo(ya, zl1, s1), hi(ya, zh1, s1), lo(yb, zl1, s1), hi(yb, zh1, s1)};
-  } else {
-    // nibble j of a word: j=0 (k0,n0) 1 (k0+8,n0) 2 (k0,n0+8) 3 (k0+8,n0+8) 4..7 same with k0+1
-    uint32_t EX = 0x64006400u;
-    asm("" : "+v"(EX));
-    auto lo = [&](uint32_t x, float sf, float cf) {   // nibbles 0 and 4 of x: 1024+q
-      const f16x2 v = as_h2((x & 0x000f000fu) | EX);
-      return pack_bf16(__builtin_fmaf((float)v.x, sf, cf), __builtin_fmaf((float)v.y, sf, cf));
-    };
-    auto hi = [&](uint32_t x, float hf, float df) {   // nibbles 1 and 5 of x: 1024+16q
-      const f16x2 v = as_h2((x & 0x00f000f0u) | EX);
-      return pack_bf16(__builtin_fmaf((float)v.x, hf, df), __builtin_fmaf((float)v.y, hf, df));
-    };
-    const uint32_t ya = xa >> 8, yb = xb >> 8;
-    o0 = u32x4{lo(xa, cc.s0, cc.c0), hi(xa, cc.h0, cc.d0), lo(xb, cc.s0, cc.c0), hi(xb, cc.h0, cc.d0)};
-    o1 = u32x4{lo(ya, cc.s1, cc.c1), hi(ya, cc.h1, cc.d1), lo(yb, cc.s1, cc.c1), hi(yb, cc.h1, cc.d1)};
-  }
+__device__ __forceinline__ void dequant_pair(uint32_t xa, uint32_t xb, const ColConst<DT>& cc, u32x4& o0, u32x4& o1) {
+  auto piece = [&](auto j_tag, uint32_t x) {
+    constexpr int J = decltype(j_tag)::value;
+    return piece_finish<DT, UNIT_SCALE, J>(piece_value<DT, J>(piece_halves<J>(x), cc), cc);
+  };
+  o0 = u32x4{piece(std::integral_constant<int, 0>{}, xa), piece(std::integral_constant<int, 1>{}, xa),
+             piece(std::integral_constant<int, 2>{}, xb), piece(std::integral_constant<int, 3>{}, xb)};
+  o1 = u32x4{piece(std::integral_constant<int, 4>{}, xa), piece(std::integral_constant<int, 5>{}, xa),
+             piece(std::integral_constant<int, 6>{}, xb), piece(std::integral_constant<int, 7>{}, xb)};
 }
 
 // Float zero points (HQQ; fp16 only): the B operand is fma(q, s, -zs) with zs = half(zp * s) rounded once, as the
@@ -220,57 +252,6 @@ __device__ __forceinline__ float ubyte_f32(uint32_t x) {
   if constexpr (N == 2) asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(f) : "v"(x));
   if constexpr (N == 3) asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(f) : "v"(x));
   return f;
-}
-
-// bf16, the two steps of one operand register apart (the prefill kernel issues them between different MFMAs):
-// the exact fp16 pair of nibbles 2*HF + ODD and that + 4 of x, then the two mixed FMAs and the pack.
-template <int HF, int ODD>
-__device__ __forceinline__ uint32_t bf16_piece_halves(uint32_t x) {
-  uint32_t EX = 0x64006400u;
-  asm("" : "+v"(EX));
-  const uint32_t y = HF ? (x >> 8) : x;
-  return (y & (ODD ? 0x00f000f0u : 0x000f000fu)) | EX;
-}
-template <int HF, int ODD>
-__device__ __forceinline__ void bf16_piece_fma(uint32_t halves, const ColConst<DT_BF16>& cc, float& f0, float& f1) {
-  const f16x2 v = as_h2(halves);
-  const float m = ODD ? (HF ? cc.h1 : cc.h0) : (HF ? cc.s1 : cc.s0);
-  const float a = ODD ? (HF ? cc.d1 : cc.d0) : (HF ? cc.c1 : cc.c0);
-  f0 = __builtin_fmaf((float)v.x, m, a);
-  f1 = __builtin_fmaf((float)v.y, m, a);
-}
-template <int HF, int ODD>
-__device__ __forceinline__ uint32_t bf16_piece_pack(uint32_t halves, const ColConst<DT_BF16>& cc) {
-  float f0, f1;
-  bf16_piece_fma<HF, ODD>(halves, cc, f0, f1);
-  return pack_bf16(f0, f1);
-}
-
-// One register (J = 0..7) of what dequant_pair produces: J < 4 -> o0[J], else o1[J - 4].  Lets a caller spread
-// the dequantisation of a Marlin word pair between MFMAs a few instructions at a time.
-template <int DT, bool UNIT_SCALE, int J>
-__device__ __forceinline__ uint32_t dequant_piece(uint32_t xa, uint32_t xb, const ColConst<DT>& cc) {
-  constexpr int HF = J >> 2, Q = J & 3;
-  const uint32_t x = (Q < 2) ? xa : xb;
-  if constexpr (DT == DT_F16) {
-    uint32_t EX = 0x64006400u;
-    asm("" : "+v"(EX));
-    const uint32_t y = HF ? (x >> 8) : x;
-    const f16x2 s = as_h2(cc.s);
-    const f16x2 sc = HF ? f16x2{s.y, s.y} : f16x2{s.x, s.x};
-    f16x2 v;
-    if constexpr ((Q & 1) == 0) {
-      const f16x2 z = as_h2(cc.zl);
-      v = as_h2((y & 0x000f000fu) | EX) - (HF ? f16x2{z.y, z.y} : f16x2{z.x, z.x});
-    } else {
-      const f16x2 z = as_h2(cc.zh);
-      const f16x2 sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-      v = as_h2((y & 0x00f000f0u) | EX) * sixteenth - (HF ? f16x2{z.y, z.y} : f16x2{z.x, z.x});
-    }
-    return as_u32(UNIT_SCALE ? v : v * sc);
-  } else {
-    return bf16_piece_pack<HF, Q & 1>(bf16_piece_halves<HF, Q & 1>(x), cc);
-  }
 }
 
 // 8-bit weights (uint8b128: stored byte = value + 128).  A lane's Marlin word holds the bytes of one column for

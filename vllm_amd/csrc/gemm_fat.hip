@@ -201,12 +201,7 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
     return v[2 * (w & 1) + half];
   };
   auto col_const = [&](const Stage& s, int w) {
-    uint32_t z0 = 8, z1 = 8;
-    if (ZP) {
-      z0 = (s.zq >> (4 * w)) & 0xf;
-      z1 = (s.zq >> (4 * w + 16)) & 0xf;
-    }
-    return make_col_const<DT, UNIT>(CHANNEL ? 0u : s.sc[w], z0, z1);
+    return make_col_const<DT, UNIT>(CHANNEL ? 0u : s.sc[w], ZP ? zero_pair(s.zq, w) : ZERO_U4B8);
   };
 
   f32x4 acc[FB_MB][4][2];
@@ -275,14 +270,14 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
     // result of the one issued just before it
     constexpr bool PIPE = (CONSTS && DT == DT_BF16);
     uint32_t ph = 0;
-    float pf0 = 0.f, pf1 = 0.f;
-    auto stage_a = [&](auto p_tag) {  // piece P: nibbles -> (1024+q | 1024+16q) fp16 pair
-      constexpr int P = decltype(p_tag)::value, w = P >> 3, J = P & 7, HF = J >> 2, Q = J & 3;
-      if constexpr (DT == DT_BF16) ph = bf16_piece_halves<HF, Q & 1>((Q < 2) ? nxt.b0[w] : nxt.b1[w]);
+    PieceValue<DT_BF16> pv = {0.f, 0.f};
+    auto stage_a = [&](auto p_tag) {  // piece P: nibbles -> (1024+q | 64+q) fp16 pair
+      constexpr int P = decltype(p_tag)::value, w = P >> 3, J = P & 7;
+      ph = piece_halves<J>((J & 3) < 2 ? nxt.b0[w] : nxt.b1[w]);
     };
     auto stage_b = [&](auto p_tag) {  // (q - z) * s in fp32, exact
-      constexpr int P = decltype(p_tag)::value, w = P >> 3, HF = (P & 7) >> 2, Q = P & 3;
-      if constexpr (DT == DT_BF16) bf16_piece_fma<HF, Q & 1>(ph, ccs[w], pf0, pf1);
+      constexpr int P = decltype(p_tag)::value, w = P >> 3, J = P & 7;
+      if constexpr (DT == DT_BF16) pv = piece_value<DT, J>(ph, ccs[w]);
     };
     if constexpr (PIPE) {
       stage_a(std::integral_constant<int, 0>{});
@@ -303,7 +298,7 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
         uint32_t r;
         if constexpr (PIPE) {
           constexpr int P = 8 * w + J;
-          r = pack_bf16(pf0, pf1);
+          r = pack_bf16(pv.f0, pv.f1);
           if constexpr (P + 1 < 32) stage_b(std::integral_constant<int, P + 1>{});
           if constexpr (P + 2 < 32) stage_a(std::integral_constant<int, P + 2>{});
         } else if constexpr (ZPF)
@@ -311,7 +306,7 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
         else if constexpr (FP4 != 0)
           r = ((J & 3) < 2) ? dequant_piece_fp4<DT, J>(xa, fs.a0, fs.a1) : dequant_piece_fp4<DT, J>(xb, fs.b0, fs.b1);
         else if constexpr (BITS == 4)
-          r = dequant_piece<DT, UNIT, J>(xa, xb, cc);
+          r = piece_finish<DT, UNIT, J>(piece_value<DT, J>(piece_halves<J>((J & 3) < 2 ? xa : xb), cc), cc);
         else
           r = dequant_piece8<DT, UNIT, FP8, J>(word8(nxt, w, (J & 3) >> 1, 0), word8(nxt, w, (J & 3) >> 1, 1),
                                                CHANNEL ? 0u : nxt.sc[w]);

@@ -69,9 +69,9 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   // HOIST: the dequantisation constants of the four word positions are kept for the k-step whose operands are being built.  A loop
   // iteration covers four k-steps (128 rows of K, aligned: every K part starts at a multiple of four k-steps), so with groups of
   // 128 rows or more, or one scale per column, they are rebuilt once per iteration instead of once per k-step.  (Not where the registers
-  // are short: 64-row tiles keep them in the 128-column form only, and there not in bf16 or with zero points: 12 to 38 would spill.)
+  // are short: 64-row tiles keep them in the 128-column form only, and there not in bf16 with grouped scales: 12 to 28 would spill.)
   constexpr bool ONCE = PRIV && !SHORT;
-  constexpr bool HOIST = KQ_MB > 4 || (ONCE && (KQ_MB < 4 || CHANNEL || (DT == DT_F16 && !ZP)));
+  constexpr bool HOIST = KQ_MB > 4 || (ONCE && (KQ_MB < 4 || CHANNEL || DT == DT_F16));
   constexpr bool UNIT = CHANNEL;
   extern __shared__ __align__(16) unsigned char smem[];
   int* s_crow = (int*)(smem + KQ_SMEM - KQ_BM * 4);
@@ -203,13 +203,7 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
     s.b1 = bp[(int64_t)(2 * ks + 1) * b_row];
   };
   auto col_const = [&](const Stage& s, int w) {
-    uint32_t z0 = 8, z1 = 8;
-    const uint32_t zq = ONCE ? zq_now : s.zq;
-    if (ZP) {
-      z0 = (zq >> (4 * w)) & 0xf;
-      z1 = (zq >> (4 * w + 16)) & 0xf;
-    }
-    return make_col_const<DT, UNIT>(CHANNEL ? 0u : ONCE ? sc_now[w] : s.sc[w], z0, z1);
+    return make_col_const<DT, UNIT>(CHANNEL ? 0u : ONCE ? sc_now[w] : s.sc[w], ZP ? zero_pair(ONCE ? zq_now : s.zq, w) : ZERO_U4B8);
   };
 
   f32x4 acc[KQ_MB][4][2];
@@ -249,57 +243,62 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   __syncthreads();
 
   // One k-step: per Marlin word w, 2 MB MFMAs on ob[w & 1]; after each MFMA (MB = 8: pair of MFMAs) one register of the following word's
-  // operands (word w + 1 of this k-step, or word 0 of the next k-step `nxt`) is dequantised into ob[(w + 1) & 1].
+  // operands (word w + 1 of this k-step, or word 0 of the next k-step `nxt`) is finished into ob[(w + 1) & 1].  A register is made in three
+  // dependent steps; behind an MFMA stand the last of one register, the second of the next and the first of the one after that, none of
+  // which waits for another (in one chain: 12 % of the loop at six such instructions per MFMA and two wavefronts per SIMD).
   // The scheduling barriers keep the compiler from regrouping this into MFMA-only and VALU-only blocks.
   auto kstep = [&](int buf, int kk, const Stage& cur, const Stage& nxt, auto refresh_tag) {
+    constexpr bool REFRESH = decltype(refresh_tag)::value;
     const u32x4* abase = (const u32x4*)(lds + buf * (KQ_ABUF / 4) + kk * kq_kstep(KQ_MB)) + lane;
     u32x4 af[KQ_MB];
 #pragma unroll
     for (int mb = 0; mb < KQ_MB; ++mb) af[mb] = abase[mb * 64];
-    auto word = [&](auto w_tag) {
-      constexpr int w = decltype(w_tag)::value;
-      constexpr int wn2 = (w + 1) & 3;
-      const Stage& src = w == 3 ? nxt : cur;
-      ColConst<DT> cc_word;
-      if constexpr (ONCE && w == 3 && decltype(refresh_tag)::value) next_scales();
-      if constexpr (!HOIST) {
-        if constexpr (ONCE) asm volatile("" : "+v"(sc_now), "+v"(zq_now));  // (or the compiler keeps all four words' constants)
-        cc_word = col_const(src, wn2);
-      } else if constexpr (w == 3 && decltype(refresh_tag)::value) {  // the words of `cur` are done: constants of `nxt`
-#pragma unroll
-        for (int ww = 0; ww < 4; ++ww) ccs[ww] = col_const(nxt, ww);
-      }
-      const ColConst<DT>& cc = HOIST ? ccs[wn2] : cc_word;
-      const uint32_t xa = src.b0[wn2], xb = src.b1[wn2];
-      auto step = [&](auto j_tag) {
-        constexpr int J = decltype(j_tag)::value;
-#pragma unroll
-        for (int i = J * KQ_MB / 4; i < (J + 1) * KQ_MB / 4; ++i) {
-          if constexpr (KQ_MB < 4)
-            mfma_inplace_v<DT>(acc[i >> 1][w][i & 1], af[i >> 1], ob[w & 1][i & 1]);
-          else
-            mfma_inplace<DT>(acc[i >> 1][w][i & 1], af[i >> 1], ob[w & 1][i & 1]);
-        }
-        const uint32_t r = dequant_piece<DT, UNIT, J>(xa, xb, cc);
-        if constexpr (J < 4)
-          ob[wn2 & 1][0][J] = r;
-        else
-          ob[wn2 & 1][1][J - 4] = r;
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      step(std::integral_constant<int, 0>{});
-      step(std::integral_constant<int, 1>{});
-      step(std::integral_constant<int, 2>{});
-      step(std::integral_constant<int, 3>{});
-      step(std::integral_constant<int, 4>{});
-      step(std::integral_constant<int, 5>{});
-      step(std::integral_constant<int, 6>{});
-      step(std::integral_constant<int, 7>{});
+    ColConst<DT> ccw[2];  // !HOIST: of the word being made and of the one behind it
+    if constexpr (!HOIST) {
+      if constexpr (ONCE) asm volatile("" : "+v"(sc_now), "+v"(zq_now));  // (or the compiler keeps all four words' constants)
+      ccw[0] = col_const(cur, 1);
+    }
+    // register P of the k-step: J = P & 7 of the word behind word P >> 3
+    auto consts = [&](auto p_tag) -> const ColConst<DT>& {
+      constexpr int W = decltype(p_tag)::value >> 3;
+      return HOIST ? ccs[(W + 1) & 3] : ccw[W & 1];
     };
-    word(std::integral_constant<int, 0>{});
-    word(std::integral_constant<int, 1>{});
-    word(std::integral_constant<int, 2>{});
-    word(std::integral_constant<int, 3>{});
+    uint32_t halves = 0;
+    PieceValue<DT> value;
+    auto make_halves = [&](auto p_tag) {
+      constexpr int P = decltype(p_tag)::value, W = P >> 3, J = P & 7;
+      const Stage& src = W == 3 ? nxt : cur;
+      halves = piece_halves<J>((J & 3) < 2 ? src.b0[(W + 1) & 3] : src.b1[(W + 1) & 3]);
+    };
+    make_halves(std::integral_constant<int, 0>{});
+    value = piece_value<DT, 0>(halves, consts(std::integral_constant<int, 0>{}));
+    make_halves(std::integral_constant<int, 1>{});
+    auto step = [&](auto p_tag) {
+      constexpr int P = decltype(p_tag)::value, w = P >> 3, J = P & 7, wn2 = (w + 1) & 3;
+#pragma unroll
+      for (int i = J * KQ_MB / 4; i < (J + 1) * KQ_MB / 4; ++i) {
+        if constexpr (KQ_MB < 4)
+          mfma_inplace_v<DT>(acc[i >> 1][w][i & 1], af[i >> 1], ob[w & 1][i & 1]);
+        else
+          mfma_inplace<DT>(acc[i >> 1][w][i & 1], af[i >> 1], ob[w & 1][i & 1]);
+      }
+      ob[wn2 & 1][J >> 2][J & 3] = piece_finish<DT, UNIT, J>(value, consts(p_tag));
+      // the constants the next registers want: of `nxt` where the k-step ends a group, each as soon as the old ones have been used
+      if constexpr (w == 2 && J == 4 && ONCE && REFRESH) next_scales();
+      if constexpr (HOIST) {
+        if constexpr (REFRESH && w == 2 && J == 4) ccs[0] = col_const(nxt, 0);
+        if constexpr (REFRESH && w == 3 && J == 1) ccs[1] = col_const(nxt, 1);
+        if constexpr (REFRESH && w == 3 && J == 3) ccs[2] = col_const(nxt, 2);
+        if constexpr (REFRESH && w == 3 && J == 5) ccs[3] = col_const(nxt, 3);
+      } else if constexpr (w < 3 && J == 4) {
+        if constexpr (ONCE) asm volatile("" : "+v"(sc_now), "+v"(zq_now));
+        ccw[wn2 & 1] = col_const(w == 2 ? nxt : cur, (w + 2) & 3);
+      }
+      if constexpr (P + 1 < 32) value = piece_value<DT, (P + 1) & 7>(halves, consts(std::integral_constant<int, P + 1>{}));
+      if constexpr (P + 2 < 32) make_halves(std::integral_constant<int, P + 2>{});
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    for_each_piece<32>(step);
   };
 
   // ---- main loop: two chunks (four k-steps = the weight ring) per iteration; the K parts of a workgroup run the same count,

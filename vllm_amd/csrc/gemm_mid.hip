@@ -9,6 +9,12 @@
 //   weights      each wavefront streams its column pair global -> registers (128-bit loads, four k-steps in
 //                flight) and dequantises each Marlin word right before its 8 MFMAs, one operand register per MFMA
 //                (scale applied per element: the B operand equals the reference's half(q - z) * half(s)).
+//                What bounds the loop is VALU issue: 4 cycles of a SIMD each, 12 to 16 more per MFMA.  So scales and zero points of groups of
+//                128 rows and more come once per loop iteration (128 K rows) and the constants made of them stay in registers
+//                (mid_once_kernel); and a register's three dependent steps stand between three MFMAs (see gemm_kq.hip).  Other VALU
+//                instructions per MFMA, before and now: bf16 with zero points 6.2 -> 4.65 (groups of 32 and 64: 5.5), uint4b8 5.35 -> 4.55,
+//                fp16 3.4 -> 3.4, and 120 wait instructions fewer per iteration.  128 experts of 2048 x 768, top-8, 601 tokens, bf16 AWQ:
+//                GEMM1 90 -> 77.5 us, GEMM2 44 -> 39.7.  Dense, 300 to 512 rows, weights not cached: 0.98 of the time in the mean.
 //   activations  the workgroup stages 64 rows x 64 K (two k-steps) into LDS, double buffered, in MFMA fragment
 //                order (one conflict-free ds_read_b128 per operand); MoE rows are gathered through sorted_token_ids
 //                while staging.  One barrier per two k-steps.
@@ -38,13 +44,16 @@ constexpr int MD_SMEM = (2 * MD_ABUF > MD_SLABS ? 2 * MD_ABUF : MD_SLABS) + MD_B
 // BITS = 8: uint8b128 or (FP8) float8_e4m3fn weights in the 8-bit Marlin layout; their stages hold twice the weight
 // registers, which still fits the two-workgroups-per-compute-unit budget (the grouped variants spill 2-9 registers).
 // ZPF: uint4 weights with fp16 zero points laid out like the scales (HQQ; dense only).
-template <int DT, bool ZP, bool CHANNEL, bool MOE, int FP4 = 0, int BITS = 4, bool FP8 = false, bool ZPF = false>
-__global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
+// ONCE: integer 4-bit weights with scale groups of 128 rows or more, or one scale per column (mid_once_kernel).
+template <int DT, bool ZP, bool CHANNEL, bool MOE, int FP4, int BITS, bool FP8, bool ZPF, bool ONCE>
+__device__ __forceinline__ void mid_tile(const KParams& p) {
   static_assert(!ZPF || (DT == DT_F16 && !ZP && !CHANNEL && !MOE && BITS == 4 && FP4 == 0), "float zero points: fp16 uint4 grouped, dense");
   static_assert(FP4 == 0 || (!ZP && !CHANNEL && BITS == 4), "fp4 weights: grouped scale records, no zero points");
   static_assert(BITS == 4 || (BITS == 8 && !ZP), "8-bit weights have no zero points");
   static_assert(!FP8 || BITS == 8, "fp8 weights use the 8-bit layout");
+  static_assert(!ONCE || (BITS == 4 && FP4 == 0 && !ZPF), "integer 4-bit weights");
   constexpr bool UNIT = CHANNEL;
+  constexpr bool PIPE = BITS == 4 && FP4 == 0 && !ZPF;  // see kstep
   extern __shared__ __align__(16) unsigned char smem[];
   int* s_crow = (int*)(smem + MD_SMEM - MD_BM * 8);
   float* s_tw = (float*)(smem + MD_SMEM - MD_BM * 4);
@@ -177,12 +186,20 @@ __global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
     uint32_t zq;
   };
   Stage st[MD_D];
+  // ONCE: scales and zero points come once per loop iteration, with its first k-step, and the four words' constants are kept
+  u32x4 sc128 = {0, 0, 0, 0};
+  uint32_t zq128 = 0;
+  auto issue_scales = [&](int ks) {
+    const int gi = CHANNEL ? 0 : min(ks_b + ks, ks_e - 1) >> p.group_shift;
+    if (!CHANNEL) sc128 = sp[(int64_t)gi * s_row];
+    if (ZP) zq128 = zp[(int64_t)gi * s_row];
+  };
   auto issue = [&](Stage& s, int ks) {  // ks: relative to ks_b
     ks = min(ks_b + ks, ks_e - 1);
     int gi = 0;
     if (!CHANNEL) gi = ks >> p.group_shift;  // the host only picks this kernel for power-of-two group sizes
-    if (!CHANNEL) s.sc = sp[(int64_t)gi * s_row];
-    if (ZP) s.zq = zp[(int64_t)gi * s_row];
+    if (!CHANNEL && !ONCE) s.sc = sp[(int64_t)gi * s_row];
+    if (ZP && !ONCE) s.zq = zp[(int64_t)gi * s_row];
     if (FP4 == 2) s.zq = ks & 1;  // which half of the two-k-step scale record
     if (ZPF) s.zf = zfp[(int64_t)gi * s_row];
     s.b0 = bp[(int64_t)(2 * ks) * b_row];
@@ -212,12 +229,7 @@ __global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
     return r;
   };
   auto col_const = [&](const Stage& s, int w) {
-    uint32_t z0 = 8, z1 = 8;
-    if (ZP) {
-      z0 = (s.zq >> (4 * w)) & 0xf;
-      z1 = (s.zq >> (4 * w + 16)) & 0xf;
-    }
-    return make_col_const<DT, UNIT>(CHANNEL ? 0u : s.sc[w], z0, z1);
+    return make_col_const<DT, UNIT>(CHANNEL ? 0u : ONCE ? sc128[w] : s.sc[w], ZP ? zero_pair(ONCE ? zq128 : s.zq, w) : ZERO_U4B8);
   };
 
   f32x4 acc[MD_MB][4][2];
@@ -233,11 +245,13 @@ __global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
 
   // ---- prologue
   load_a(0);
+  if constexpr (ONCE) issue_scales(0);
 #pragma unroll
   for (int j = 0; j < MD_D; ++j) issue(st[j], j);
   store_a(0);
   // B operands of two Marlin words: the one whose MFMAs are being issued and the one being dequantised
   u32x4 ob[2][2];
+  ColConst<DT> ccs[4];
   if constexpr (ZPF) {
     dequant_pair_zpf(st[0].b0[0], st[0].b1[0], st[0].sc[0], as_u32(as_h2(st[0].zf[0]) * as_h2(st[0].sc[0])), ob[0][0],
                      ob[0][1]);
@@ -251,24 +265,57 @@ __global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
     dequant_pair8<DT, UNIT>(word8(st[0], 0, 0, 0), word8(st[0], 0, 0, 1), word8(st[0], 0, 1, 0), word8(st[0], 0, 1, 1),
                             CHANNEL ? 0u : st[0].sc[0], ob[0][0], ob[0][1]);
   } else {
-    const ColConst<DT> cc = col_const(st[0], 0);
-    dequant_pair<DT, UNIT>(st[0].b0[0], st[0].b1[0], cc, ob[0][0], ob[0][1]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      if (ONCE || w == 0) ccs[w] = col_const(st[0], w);
+    dequant_pair<DT, UNIT>(st[0].b0[0], st[0].b1[0], ccs[0], ob[0][0], ob[0][1]);
   }
   __syncthreads();
 
   // One k-step: per Marlin word w, 8 MFMAs on ob[w & 1]; after each MFMA one register of the following word's
   // operands (word w + 1 of this k-step, or word 0 of the next k-step `nxt`) is dequantised into ob[(w + 1) & 1].
   // The scheduling barriers keep the compiler from regrouping this into MFMA-only and VALU-only blocks.
-  auto kstep = [&](int buf, int kk, const Stage& cur, const Stage& nxt) {
+  auto kstep = [&](int buf, int kk, const Stage& cur, const Stage& nxt, auto refresh_tag) {
     const u32x4* abase = (const u32x4*)(lds + buf * (MD_ABUF / 4)) + (kk * MD_MB) * 64 + lane;
     u32x4 af[MD_MB];
 #pragma unroll
     for (int mb = 0; mb < MD_MB; ++mb) af[mb] = abase[mb * 64];
+    if constexpr (PIPE) {
+      constexpr bool REFRESH = decltype(refresh_tag)::value;
+      if constexpr (!ONCE) ccs[1] = col_const(cur, 1);
+      uint32_t halves = 0;
+      PieceValue<DT> value;
+      auto make_halves = [&](auto p_tag) {  // register P of the k-step: J = P & 7 of the word behind word P >> 3
+        constexpr int P = decltype(p_tag)::value, W = P >> 3, J = P & 7;
+        const Stage& src = W == 3 ? nxt : cur;
+        halves = piece_halves<J>((J & 3) < 2 ? src.b0[(W + 1) & 3] : src.b1[(W + 1) & 3]);
+      };
+      make_halves(std::integral_constant<int, 0>{});
+      value = piece_value<DT, 0>(halves, ccs[1]);
+      make_halves(std::integral_constant<int, 1>{});
+      for_each_piece<32>([&](auto p_tag) {
+        constexpr int P = decltype(p_tag)::value, w = P >> 3, J = P & 7, wn = (w + 1) & 3;
+        mfma_inplace<DT>(acc[J >> 1][w][J & 1], af[J >> 1], ob[w & 1][J & 1]);
+        ob[wn & 1][J >> 2][J & 3] = piece_finish<DT, UNIT, J>(value, ccs[wn]);
+        // the constants the next registers want, each as soon as the old ones have been used
+        if constexpr (ONCE) {
+          if constexpr (REFRESH && w == 2 && J == 4) ccs[0] = col_const(nxt, 0);
+          if constexpr (REFRESH && w == 3 && J == 1) ccs[1] = col_const(nxt, 1);
+          if constexpr (REFRESH && w == 3 && J == 3) ccs[2] = col_const(nxt, 2);
+          if constexpr (REFRESH && w == 3 && J == 5) ccs[3] = col_const(nxt, 3);
+        } else if constexpr (w < 3 && J == 4) {
+          ccs[(w + 2) & 3] = col_const(w == 2 ? nxt : cur, (w + 2) & 3);
+        }
+        if constexpr (P + 1 < 32) value = piece_value<DT, (P + 1) & 7>(halves, ccs[(((P + 1) >> 3) + 1) & 3]);
+        if constexpr (P + 2 < 32) make_halves(std::integral_constant<int, P + 2>{});
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      return;
+    }
     auto word = [&](auto w_tag) {
       constexpr int w = decltype(w_tag)::value;
       constexpr int wn = (w + 1) & 3;
       const Stage& src = w == 3 ? nxt : cur;
-      const ColConst<DT> cc = col_const(src, wn);
       const Fp4Scales fs = fp4_scales(src, wn);
       uint32_t zs = 0;
       if constexpr (ZPF) zs = as_u32(as_h2(src.zf[wn]) * as_h2(src.sc[wn]));
@@ -281,11 +328,9 @@ __global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
           r = dequant_piece_zpf<J>(xa, xb, src.sc[wn], zs);
         else if constexpr (FP4 != 0)
           r = ((J & 3) < 2) ? dequant_piece_fp4<DT, J>(xa, fs.a0, fs.a1) : dequant_piece_fp4<DT, J>(xb, fs.b0, fs.b1);
-        else if constexpr (BITS == 8)
+        else
           r = dequant_piece8<DT, UNIT, FP8, J>(word8(src, wn, (J & 3) >> 1, 0), word8(src, wn, (J & 3) >> 1, 1),
                                                CHANNEL ? 0u : src.sc[wn]);
-        else
-          r = dequant_piece<DT, UNIT, J>(xa, xb, cc);
         if constexpr (J < 4)
           ob[wn & 1][0][J] = r;
         else
@@ -313,17 +358,18 @@ __global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
     const int ks0 = 2 * c0;
     // chunk c0 in buffer 0
     load_a(c0 + 1);
-    kstep(0, 0, st[0], st[1]);
+    kstep(0, 0, st[0], st[1], std::false_type{});
+    if constexpr (ONCE) issue_scales(ks0 + 4);
     issue(st[0], ks0 + 4);
-    kstep(0, 1, st[1], st[2]);
+    kstep(0, 1, st[1], st[2], std::false_type{});
     issue(st[1], ks0 + 5);
     store_a(1);
     __syncthreads();
     // chunk c0+1 in buffer 1
     load_a(c0 + 2);
-    kstep(1, 0, st[2], st[3]);
+    kstep(1, 0, st[2], st[3], std::false_type{});
     issue(st[2], ks0 + 6);
-    kstep(1, 1, st[3], st[0]);
+    kstep(1, 1, st[3], st[0], std::true_type{});
     issue(st[3], ks0 + 7);
     store_a(0);
     __syncthreads();
@@ -437,6 +483,15 @@ __global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
     }
     __builtin_amdgcn_wave_barrier();
   }
+}
+
+template <int DT, bool ZP, bool CHANNEL, bool MOE, int FP4 = 0, int BITS = 4, bool FP8 = false, bool ZPF = false>
+__global__ __launch_bounds__(256, 2) void mid_kernel(const KParams p) {
+  mid_tile<DT, ZP, CHANNEL, MOE, FP4, BITS, FP8, ZPF, false>(p);
+}
+template <int DT, bool ZP, bool CHANNEL, bool MOE>
+__global__ __launch_bounds__(256, 2) void mid_once_kernel(const KParams p) {
+  mid_tile<DT, ZP, CHANNEL, MOE, 0, 4, false, false, true>(p);
 }
 
 // Second pass of a split-K launch of mid_kernel (BM = 64) or of the prefill kernel on MoE blocks (BM = 128): out tile = sum over
@@ -557,10 +612,14 @@ __global__ __launch_bounds__(256) void mid_reduce_kernel(const KParams p) {
 
 typedef void (*mid_fn)(const KParams);
 
+template <int DT, bool MOE, bool ZP>
+static mid_fn pick_mid3(bool channel, bool once) {
+  if (channel) return mid_once_kernel<DT, ZP, true, MOE>;
+  return once ? mid_once_kernel<DT, ZP, false, MOE> : mid_kernel<DT, ZP, false, MOE>;
+}
 template <int DT, bool MOE>
-static mid_fn pick_mid2(bool zp, bool channel) {
-  if (zp) return channel ? mid_kernel<DT, true, true, MOE> : mid_kernel<DT, true, false, MOE>;
-  return channel ? mid_kernel<DT, false, true, MOE> : mid_kernel<DT, false, false, MOE>;
+static mid_fn pick_mid2(bool zp, bool channel, bool once) {
+  return zp ? pick_mid3<DT, MOE, true>(channel, once) : pick_mid3<DT, MOE, false>(channel, once);
 }
 template <int DT, bool MOE>
 static mid_fn pick_mid8(bool fp8, bool channel) {
@@ -585,6 +644,7 @@ int launch_fat_reduce(const w4a16_gemm_args* a, const Plan& pl, const KParams& p
 int launch_mid(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
   const bool zp = a->b_zeros != nullptr, channel = pl.gm == GM_CHANNEL;
   const bool moe = (a->flags & W4A16_F_MOE) != 0;
+  const bool once = pl.group_ksteps >= 4;  // scale groups of 128 rows at least
   mid_fn fn, red;
   if (a->flags & W4A16_F_ZP_FLOAT) {
     if (a->dtype != DT_F16 || channel || moe) return fail(W4A16_EINVAL, "unsupported kernel variant");
@@ -610,10 +670,10 @@ int launch_mid(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
     red = a->dtype == DT_F16 ? (moe ? pick_reduce<DT_F16, true>(false) : pick_reduce<DT_F16, false>(false))
                              : (moe ? pick_reduce<DT_BF16, true>(false) : pick_reduce<DT_BF16, false>(false));
   } else if (a->dtype == DT_F16) {
-    fn = moe ? pick_mid2<DT_F16, true>(zp, channel) : pick_mid2<DT_F16, false>(zp, channel);
+    fn = moe ? pick_mid2<DT_F16, true>(zp, channel, once) : pick_mid2<DT_F16, false>(zp, channel, once);
     red = moe ? pick_reduce<DT_F16, true>(channel) : pick_reduce<DT_F16, false>(channel);
   } else {
-    fn = moe ? pick_mid2<DT_BF16, true>(zp, channel) : pick_mid2<DT_BF16, false>(zp, channel);
+    fn = moe ? pick_mid2<DT_BF16, true>(zp, channel, once) : pick_mid2<DT_BF16, false>(zp, channel, once);
     red = moe ? pick_reduce<DT_BF16, true>(channel) : pick_reduce<DT_BF16, false>(channel);
   }
   KParams p = make_kparams(a, pl);

@@ -263,12 +263,7 @@ __global__ __launch_bounds__(NW * 64, 2) void skinny_kernel(const KParams p) {
     } else if constexpr (HOIST) {
       dequant_pair<DT, unit>(s.b0[w], s.b1[w], ccs[w], o0, o1);
     } else if constexpr (BITS == 4) {
-      uint32_t z0 = 8, z1 = 8;
-      if (ZP) {
-        z0 = (s.zq >> (4 * w)) & 0xf;
-        z1 = (s.zq >> (4 * w + 16)) & 0xf;
-      }
-      const ColConst<DT> cc = make_col_const<DT, unit>(unit ? 0u : s.sc[w], z0, z1);
+      const ColConst<DT> cc = make_col_const<DT, unit, GM != GM_GIDX>(unit ? 0u : s.sc[w], ZP ? zero_pair(s.zq, w) : ZERO_U4B8);
       dequant_pair<DT, unit>(s.b0[w], s.b1[w], cc, o0, o1);
     } else {
       const u32x4& la = (w < 2) ? s.b0 : s.b0h;
@@ -433,7 +428,7 @@ __global__ __launch_bounds__(NW * 64, 2) void skinny_kernel(const KParams p) {
         ccs_gi = s.gi;
 #pragma unroll
         for (int w = 0; w < 4; ++w)
-          ccs[w] = make_col_const<DT, UNIT>(UNIT ? 0u : s.sc[w], ZP ? (s.zq >> (4 * w)) & 0xf : 8, ZP ? (s.zq >> (4 * w + 16)) & 0xf : 8);
+          ccs[w] = make_col_const<DT, UNIT>(UNIT ? 0u : s.sc[w], ZP ? zero_pair(s.zq, w) : ZERO_U4B8);
       }
     }
     auto plain_word = [&](auto w_tag) {
