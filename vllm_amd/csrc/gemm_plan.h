@@ -15,7 +15,7 @@ struct Plan {
   int xcd_map;
   int kind;  // 0: skinny kernel, 1: decode kernel, 2: prefill ("fat") kernel, 3: 64-row ("mid") kernel,
              // 5: in-workgroup K split (gemm_kq.hip): 64 x 256 tiles in K quarters (mb = 4), 80 .. 128 x 256 in halves (mb = 5 .. 8), 32 .. 64 x 128
-             // in eighths (mb = 2 .. 4, tn = 128)
+             // in eighths (mb = 2 .. 4, tn = 128), 6: 8-bit matrix unit, 7: the same on prepared weights
   int tn;    // tile width in columns (128; the decode kernel also has 64)
   int nw = 8;  // 16-row tiles (decode kernel, general kernel with one m-block): wavefronts per workgroup (8 or 4)
   int strip0 = 0;      // 64-row kernel / K-split kernel: first 512- / 256-column strip handled by the launch
@@ -23,8 +23,8 @@ struct Plan {
   int tail_strips = 0; // prefill plan: trailing 512-column strips handed to another kernel (0 = none)
   int tail_kind = 3;   // ... which one: 3 = 64-row kernel, 5 = tall tiles with the K halves inside the workgroup
   int tail_mb = 8;     // ... of so many m-blocks
-  int ks = 1;          // 8-bit-unit kernel (kind 6): K parts inside a workgroup
-  int64_t x8_bytes = 0;  // 8-bit-unit kernel: the activations split in two 8-bit terms, behind the other scratch
+  int ks = 1;          // 8-bit-unit kernels: K parts inside a workgroup
+  int64_t x8_bytes = 0;  // 8-bit-unit kernels: the activations split in two 8-bit terms (and the prepared weights), behind the other scratch
   int64_t ctmp_bytes;  // fp32 split-K partials
   int64_t atmp_bytes;  // column-permuted copy of A (act-order), after the partials; MoE: one row per sorted slot
 };
@@ -41,6 +41,7 @@ int launch_decode(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_fat(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_mid(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int64_t x8_scratch_bytes(int64_t rows, int64_t k);
+int64_t x8_weight_bytes(int64_t k, int64_t n);
 int launch_x8(const w4a16_gemm_args* a, const Plan& pl, void* scratch, hipStream_t stream);
 int launch_kq(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 

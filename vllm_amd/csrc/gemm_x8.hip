@@ -35,6 +35,10 @@
 //            contiguously, 64 in rows of 64 bytes (the first layout tried: 128 x 256 tiles with K halves 937 us, 815 with this one).
 //            Weights global -> registers, one step ahead, spread over the step (a wavefront whose load finds the queue full stands
 //            still).  Through LDS they cost more there than they save in the memory pipe (128 rows: 108 -> 114 us).
+//   prepared Zero points make a weight 16 instructions of eight, which a long launch pays once per 128 rows of A: x8_weights_kernel writes the e4m3
+//            numbers once, in operand order (4096 x 28672: 40 us, 176 MB moved at 4.4 TB/s), and x8_prepared_kernel loads them; 2.3 other VALU
+//            instructions per MFMA are left, the folds.  4096 x 28672 at 4096 rows 786 -> 694 us, 14336 x 4096 at 3000 rows 350 -> 307; the GEMM
+//            alone is at 1.51 to 1.59 PFLOP/s, near what the power limit leaves of the MFMAs (1.65).  uint4b8 gains 3 % at most and stays.
 //   bound    4096 x 28672 bf16, weights not cached, 16-bit kernels and this one: at 4096 rows uint4b8 799 -> 731 us, zero points 812 -> 811; at
 //            1024 rows 225 -> 201 and 226 -> 222; at 203 rows 68.5 -> 58.6 and 67.9 -> 61.8.  Long launches: matrix pipe 54 % (48 % with zero
 //            points) of the cycles at 2.1 GHz, 5.3 (6.8) other VALU instructions per MFMA of twice a 16-bit one's time, a third of which it
@@ -62,8 +66,12 @@ constexpr int X8_TABLES = 16 * 16;  // behind it, with zero points: a table for 
 
 constexpr int X8_WIDE = 13;         // binades from a step's largest value at which what the two terms leave out is added
 
+// prepared weights of one step: 8 KB for each unit, two units for every column pair (whose second n-tile may be missing)
+__host__ __device__ constexpr int64_t x8_weight_step(int64_t n) { return (n + 127) / 128 * 16384; }
+
 struct X8Params {
   KParams k;
+  const unsigned char* w8;   // prepared weights (x8_weights_kernel), or null
   const unsigned char* rec;  // [K / 128][rows / 16][fragment 4][K group 4][row 16][16 bytes]: a fragment is one contiguous KB
   const uint32_t* scl;       // [K / 128][rows]
   int rows;                  // see x8_rows
@@ -287,8 +295,8 @@ __device__ __forceinline__ uint32_t x8_table(int z, int dword) {
   return r;
 }
 
-template <bool ZP, bool CHANNEL, int MB, int KS, int WN>
-__global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) {
+template <bool ZP, bool CHANNEL, int MB, int KS, int WN, bool PREP>
+__device__ __forceinline__ void x8_tile(const X8Params& xp) {
   const KParams& p = xp.k;
   constexpr int BM = 16 * MB, BN = WN * 64;
   constexpr int NL = MB * 4 / WN;  // 1 KB fragments staged per wavefront and step
@@ -323,6 +331,7 @@ __global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) 
 
   const uint16_t* Sc = (const uint16_t*)p.S;
   const uint16_t* bias = (const uint16_t*)p.bias;
+  const int u_mem = wave_on ? u : 0;
   const int nt = !wave_on ? 0 : ((2 * cp + h) * 64 < p.N ? 2 * cp + h : 0);
   // byte offsets of the lane; everything else in an address is uniform
   const uint32_t b_off = (uint32_t)(nt * 128 + (4 * c + g) * 4 + wsel) * 4;
@@ -367,25 +376,32 @@ __global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) 
   uint32_t zraw = 0;
   u32x4 tab[2] = {};
   unsigned char* tables = smem + x8_smem(MB, KS, WN);
-  if (ZP && t < X8_TABLES / 4) ((uint32_t*)tables)[t] = x8_table(t >> 2, t & 3);  // (complete after the first sync_stage)
+  if (ZP && !PREP && t < X8_TABLES / 4) ((uint32_t*)tables)[t] = x8_table(t >> 2, t & 3);  // (complete after the first sync_stage)
   auto load_b = [&](int i, int kt) {
     raw[kt] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(b_res, b_off, (uint32_t)((gb + i) * 8 + kt) * b_row, 0));
   };
   auto load_s = [&](int i) {
     const uint32_t grp = CHANNEL ? 0 : (uint32_t)(4 * (gb + i)) >> p.group_shift;
     if (!CHANNEL) sraw = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(s_res, s_off(), grp * p.N * 2, 0));
-    if (ZP) zraw = __builtin_amdgcn_raw_buffer_load_b32(z_res, z_off(), grp * (p.N / 2), 0);
+    if (ZP && !PREP) zraw = __builtin_amdgcn_raw_buffer_load_b32(z_res, z_off(), grp * (p.N / 2), 0);
+  };
+  // prepared weights: piece q of step i, 16 bytes of operand q >> 1
+  const uint64_t w8_step = x8_weight_step(p.N);
+  auto load_w8 = [&](int i, int q, i32x8 (&o)[4]) {
+    const u32x4 v = *(const u32x4*)(xp.w8 + (uint64_t)(gb + i) * w8_step + (uint64_t)u_mem * 8192 + q * 1024 + lane * 16);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[q >> 1][4 * (q & 1) + e] = (int)v[e];
   };
   // tables of word w's two columns, from the loaded word of zero points
   auto zeros = [&](int w) {
-    if (ZP) {
+    if (ZP && !PREP) {
       const uint32_t z = zraw >> (4 * (wsel + w));
       tab[0] = *(const u32x4*)(tables + (z & 15u) * 16);
       tab[1] = *(const u32x4*)(tables + (z >> 16 & 15u) * 16);
     }
   };
   // k-tile kt of word w (0 or 1 of the wavefront's two) -> its dword of the two operands
-  auto dequant = [&](int w, int kt, i32x8 (&o)[2]) {
+  auto dequant = [&](int w, int kt, auto& o) {
     int o0, o1;
     if constexpr (ZP)
       x8_weights(raw[kt][w], tab[0], tab[1], o0, o1);
@@ -399,7 +415,7 @@ __global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) 
   for (int m = 0; m < MB; ++m)
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[m][i] = f32x4{0, 0, 0, 0};
-  i32x8 bx[2], by[2], b23[2], ah, al;
+  i32x8 bx[4], by[4], b23[2], ah, al;  // (elements 2 and 3 of the first two: prepared weights, whose b23 is not used)
   f32x4 T[2][2] = {};
   constexpr float UNIT = ZP ? 64.f : 256.f;  // of the weights' e4m3 numbers
   float sc[4] = {UNIT, UNIT, UNIT, UNIT};
@@ -438,17 +454,23 @@ __global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) 
   };
 
 #define X8_SB __builtin_amdgcn_sched_barrier(0)
-  auto step = [&](int i, int buf, i32x8 (&b01)[2], i32x8 (&n01)[2]) {
+  auto step = [&](int i, int buf, i32x8 (&b01)[4], i32x8 (&n01)[4]) {
+    const i32x8 &b2 = PREP ? b01[2] : b23[0], &b3 = PREP ? b01[3] : b23[1];
     constexpr int FROM = MB > 3 ? MB - 3 : 1, PER = (8 + MB - FROM - 1) / (MB - FROM);  // next step's word 0: spread over the last row blocks
     // The next step's loads, spread over the step: a wavefront whose load finds the memory pipeline's queue full stands still with
     // its MFMAs.  u: 2 m + word; the weight registers are free from u = 1 on and wanted from m = FROM on.
     const int nx = min(i + 1, steps - 1);
     auto loads = [&](int u) {
-      constexpr int LAST = 2 * FROM - 1, WPER = (8 + LAST - 1) / LAST, SPER = (NL + LAST - 1) / LAST;
+      constexpr int LAST = PREP ? 2 * MB - 2 : 2 * FROM - 1, WPER = (8 + LAST - 1) / LAST, SPER = (NL + LAST - 1) / LAST;
       if (u == 1) load_s(nx), stage_meta(nx, buf ^ 1);
 #pragma unroll
       for (int q = 0; q < WPER; ++q)
-        if ((u - 1) * WPER + q < 8) load_b(nx, (u - 1) * WPER + q);
+        if ((u - 1) * WPER + q < 8) {
+          if constexpr (PREP)
+            load_w8(nx, (u - 1) * WPER + q, n01);
+          else
+            load_b(nx, (u - 1) * WPER + q);
+        }
 #pragma unroll
       for (int q = 0; q < SPER; ++q)
         if ((u - 1) * SPER + q < NL) stage_frag(nx, buf ^ 1, (u - 1) * SPER + q);
@@ -460,25 +482,26 @@ __global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) 
       X8_SB;
       mfma_lo(0, 0, b01[0]);
       fold(m > 0 ? m - 1 : MB - 1, 1, 0);  // (zeros in front of the first step)
-      if (m == 0) dequant(1, 0, b23), dequant(1, 1, b23);
+      if (m == 0 && !PREP) dequant(1, 0, b23), dequant(1, 1, b23);
       X8_SB;
       mfma_lo(0, 1, b01[1]);
       fold(m > 0 ? m - 1 : MB - 1, 1, 1);
-      if (m == 0) dequant(1, 2, b23), dequant(1, 3, b23);
+      if (m == 0 && !PREP) dequant(1, 2, b23), dequant(1, 3, b23);
       X8_SB;
       mfma_hi(0, 0, b01[0]);
-      if (m == 0) scales(1), dequant(1, 4, b23), dequant(1, 5, b23);
+      if (m == 0) scales(1);
+      if (m == 0 && !PREP) dequant(1, 4, b23), dequant(1, 5, b23);
       X8_SB;
       mfma_hi(0, 1, b01[1]);
       if (m + 1 < MB) meta(buf, m + 1);
-      if (m == 0) {
+      if (m == 0 && !PREP) {
         dequant(1, 6, b23), dequant(1, 7, b23);
         X8_SB;
       }
       if (m > 0) loads(2 * m);
 #pragma unroll
       for (int q = 0; q < PER; ++q)
-        if (m >= FROM && (m - FROM) * PER + q < 8) dequant(0, (m - FROM) * PER + q, n01);
+        if (!PREP && m >= FROM && (m - FROM) * PER + q < 8) dequant(0, (m - FROM) * PER + q, n01);
       X8_SB;
       // columns of word 1
       loads(2 * m + 1);
@@ -488,16 +511,16 @@ __global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) 
         meta(buf ^ 1, 0);
         X8_SB;
       }
-      mfma_lo(1, 0, b23[0]);
+      mfma_lo(1, 0, b2);
       fold(m, 0, 0);
       X8_SB;
-      mfma_lo(1, 1, b23[1]);
+      mfma_lo(1, 1, b3);
       fold(m, 0, 1);
       X8_SB;
       frag(m + 1 < MB ? buf : buf ^ 1, m + 1 < MB ? m + 1 : 0, 1, al);
-      mfma_hi(1, 0, b23[0]);
+      mfma_hi(1, 0, b2);
       X8_SB;
-      mfma_hi(1, 1, b23[1]);
+      mfma_hi(1, 1, b3);
       any |= sl;
       sl = sl_n;
       X8_SB;
@@ -514,14 +537,20 @@ __global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) 
     for (int q = 0; q < NL; ++q) stage_frag(0, 0, q);
     stage_meta(0, 0);
 #pragma unroll
-    for (int kt = 0; kt < 8; ++kt) load_b(0, kt);
+    for (int kt = 0; kt < 8; ++kt) {
+      if constexpr (PREP)
+        load_w8(0, kt, bx);
+      else
+        load_b(0, kt);
+    }
     load_s(0);
   }
   sync_stage();
   if (steps > 0) {
     zeros(0);
 #pragma unroll
-    for (int kt = 0; kt < 8; ++kt) dequant(0, kt, bx);
+    for (int kt = 0; kt < 8; ++kt)
+      if (!PREP) dequant(0, kt, bx);
     zeros(1);
     meta(0, 0);
     sl = sl_n;
@@ -567,6 +596,7 @@ __global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) 
 #pragma unroll
     for (int kt = 0; kt < 8; ++kt) load_b(gi - gb, kt);
     load_s(gi - gb);
+    if (ZP && PREP) zraw = __builtin_amdgcn_raw_buffer_load_b32(z_res, z_off(), (CHANNEL ? 0 : (uint32_t)(4 * gi) >> p.group_shift) * (p.N / 2), 0);
 #pragma unroll
     for (int half = 0; half < 2; ++half) {  // (64 K rows at a time, or registers spill)
       u32x4 w[2][4];  // [32 K rows][column]
@@ -734,6 +764,49 @@ __global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) 
   }
 }
 
+template <bool ZP, bool CHANNEL, int MB, int KS, int WN>
+__global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) {
+  x8_tile<ZP, CHANNEL, MB, KS, WN, false>(xp);
+}
+template <bool CHANNEL>
+__global__ __launch_bounds__(512, 2) void x8_prepared_kernel(const X8Params xp) {
+  x8_tile<true, CHANNEL, 8, 1, 8, true>(xp);
+}
+
+// Prepared weights: the e4m3 numbers (q - z) * 2^-6 in the order in which a wavefront takes its operands: [K / 128][unit of 64 columns][16-byte
+// piece 8][lane][16 bytes].  A wavefront: the two units of a column pair in one step.
+__global__ __launch_bounds__(256) void x8_weights_kernel(const uint32_t* B, const uint32_t* Z, int N, int group_shift, bool channel, unsigned char* w8) {
+  __shared__ __align__(16) uint32_t tables[X8_TABLES / 4];
+  const int t = threadIdx.x, lane = t & 63, c = lane & 7, h = (lane >> 3) & 1, g = lane >> 4;
+  if (t < X8_TABLES / 4) tables[t] = x8_table(t >> 2, t & 3);
+  __syncthreads();
+  const int cp = blockIdx.x * 4 + (t >> 6), step = blockIdx.y;
+  if (cp * 128 >= N) return;
+  const int nt = (2 * cp + h) * 64 < N ? 2 * cp + h : 2 * cp;
+  u32x4 x[8];
+#pragma unroll
+  for (int kt = 0; kt < 8; ++kt) x[kt] = __builtin_nontemporal_load((const u32x4*)(B + (int64_t)(step * 8 + kt) * (2 * N) + nt * 128 + (4 * c + g) * 4));
+  const uint32_t z = Z[(int64_t)(channel ? 0 : (4 * step) >> group_shift) * (N >> 3) + nt * 8 + c];
+  unsigned char* out = w8 + step * x8_weight_step(N) + cp * 16384 + lane * 16;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const u32x4 t0 = *(const u32x4*)(tables + (z >> (4 * w) & 15u) * 4), t1 = *(const u32x4*)(tables + (z >> (4 * w + 16) & 15u) * 4);
+    i32x8 o[2];
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt) {
+      int o0, o1;
+      x8_weights(x[kt][w], t0, t1, o0, o1);
+      o[0][kt] = o0, o[1][kt] = o1;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        *(u32x4*)(out + (w >> 1) * 8192 + ((2 * (w & 1) + i) * 2 + q) * 1024) =
+            u32x4{(uint32_t)o[i][4 * q], (uint32_t)o[i][4 * q + 1], (uint32_t)o[i][4 * q + 2], (uint32_t)o[i][4 * q + 3]};
+  }
+}
+
 // Second pass of a launch with K also split across workgroups: adds the fp32 partial tiles in split order.
 template <bool CHANNEL>
 __global__ __launch_bounds__(256) void x8_reduce_kernel(const KParams p, int bm, int bn) {
@@ -776,7 +849,10 @@ int64_t x8_scratch_bytes(int64_t rows, int64_t k) {
   return r * g * 256 + (r * g * 4 + 255) / 256 * 256;
 }
 
-static x8_fn pick_x8_shape(int mb, int ks, int tn, bool zp, bool channel) {
+int64_t x8_weight_bytes(int64_t k, int64_t n) { return k / X8_G * x8_weight_step(n); }
+
+static x8_fn pick_x8_shape(int mb, int ks, int tn, bool zp, bool channel, bool prep) {
+  if (prep) return ks != 1 || mb != 8 || tn != 512 || !zp ? nullptr : channel ? x8_prepared_kernel<true> : x8_prepared_kernel<false>;
   if (ks == 1 && mb == 8) return tn == 512 ? pick_x8<8, 1, 8>(zp, channel) : tn == 256 ? pick_x8<8, 1, 4>(zp, channel) : nullptr;
   if (ks != 2 || tn != 256) return nullptr;
   switch (mb) {
@@ -789,8 +865,8 @@ static x8_fn pick_x8_shape(int mb, int ks, int tn, bool zp, bool channel) {
 }
 
 int launch_x8(const w4a16_gemm_args* a, const Plan& pl, void* scratch, hipStream_t stream) {
-  const bool zp = a->b_zeros != nullptr, channel = pl.gm == GM_CHANNEL;
-  const x8_fn fn = pick_x8_shape(pl.mb, pl.ks, pl.tn, zp, channel);
+  const bool zp = a->b_zeros != nullptr, channel = pl.gm == GM_CHANNEL, prep = pl.kind == 7;
+  const x8_fn fn = pick_x8_shape(pl.mb, pl.ks, pl.tn, zp, channel, prep);
   if (!fn || a->dtype != DT_BF16 || (a->wtype != W4A16_WTYPE_U4B8 && a->wtype != W4A16_WTYPE_U4) ||
       (a->flags & (W4A16_F_ZP_FLOAT | W4A16_F_MOE)) || pl.gm == GM_GIDX || pl.use_perm || pl.splits < 1 || pl.kps % 4 != 0)
     return fail(W4A16_EINVAL, "unsupported kernel variant");
@@ -803,6 +879,14 @@ int launch_x8(const w4a16_gemm_args* a, const Plan& pl, void* scratch, hipStream
   xp.rec = base;
   xp.scl = (const uint32_t*)(base + r * groups * 256);
   xp.rows = (int)r;
+  xp.w8 = nullptr;
+  if (prep) {
+    unsigned char* w8 = base + x8_scratch_bytes(a->size_m, a->size_k);
+    xp.w8 = w8;
+    hipLaunchKernelGGL(x8_weights_kernel, dim3((unsigned)ceil_div(a->size_n, 512), (unsigned)groups), dim3(256), 0,
+                       stream, xp.k.B, xp.k.Z, xp.k.N, xp.k.group_shift, channel, w8);
+    W4A16_HIP(hipGetLastError());
+  }
   // (steps per workgroup: few rows fill the chip only with one)
   const int sg = (r / 16) * groups >= 16 * num_cus() ? 4 : 1;
   hipLaunchKernelGGL((sg == 4 ? x8_split_kernel<4> : x8_split_kernel<1>), dim3((unsigned)(r / 16), (unsigned)ceil_div(groups, sg)), dim3(256), 0,
