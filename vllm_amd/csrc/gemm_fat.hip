@@ -74,7 +74,8 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
       j = d.F + part;
     }
   }
-  const int mt = j % mtiles, nt4 = j / mtiles;
+  int mt = j % mtiles, nt4 = j / mtiles;
+  if (MOE) chunked_tile(j, mtiles, p.ncp, mt, nt4);
   const int cp = nt4 * 4 + wv;                 // column pair of this wavefront
   const bool wave_on = cp * 128 < p.N;         // N not a multiple of 512: trailing wavefronts only help staging
   const int row0 = mt * FB_BM;

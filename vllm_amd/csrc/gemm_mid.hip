@@ -510,6 +510,7 @@ __global__ __launch_bounds__(256) void mid_reduce_kernel(const KParams p) {
     if (d.S == 1 || tile >= d.R) return;
     const int j = d.F + tile;
     mt = j % live, nt4 = p.strip0 + j / live, nsplit = d.S;
+    if (BM == 128) chunked_tile(j, live, p.ncp, mt, nt4);
   }
   const int row0 = mt * BM;
   const uint16_t* Sc = (const uint16_t*)p.S;
