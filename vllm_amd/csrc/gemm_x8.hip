@@ -82,19 +82,31 @@ __host__ __device__ constexpr int64_t x8_rows(int64_t m) { return (m + 15) / 16 
 // ------------------------------------------------------------------------------------------------ activations
 // A workgroup: 16 rows, wavefront w rows 4 w .. 4 w + 3, X8_SG steps one after the other (their loads are issued together).
 // Lane bits: 0 odd half of a k-tile, 1 which four k-tiles, 2-3 row, 4-5 k-tile.
-template <int X8_SG>
-__global__ __launch_bounds__(256) void x8_split_kernel(const uint16_t* a, int64_t lda, int rows, int stride, int groups, unsigned char* rec,
-                                                       uint32_t* scl) {
+// MoE: row r is that of slot r, read through sorted_ids (slots without a token: zeros), or the slot's own where the rows were gathered; rows behind
+// the last live block of 128 are never read, and not written.
+struct X8Slots {
+  const int32_t *ids, *ntpp;
+  int n_sorted, c_rows, top_k, by_slot;
+};
+template <int X8_SG, bool MOE>
+__device__ __forceinline__ void x8_split(const uint16_t* a, int64_t lda, int rows, int stride, int groups, unsigned char* rec, uint32_t* scl,
+                                         const X8Slots& slots) {
+  if (MOE && (int)blockIdx.x * 16 >= (*slots.ntpp + 127) / 128 * 128) return;
   const int lane = threadIdx.x & 63;
   const int odd = lane & 1, j = (lane >> 1) & 1, rr = lane >> 4;
   const int row = blockIdx.x * 16 + (threadIdx.x >> 6) * 4 + ((lane >> 2) & 3);
   const int group0 = blockIdx.y * X8_SG;
+  int64_t src = row < rows ? row : -1;
+  if constexpr (MOE) {
+    const int id = row < slots.n_sorted ? slots.ids[row] : -1;
+    src = (unsigned)id >= (unsigned)slots.c_rows ? -1 : slots.by_slot ? row : id / slots.top_k;
+  }
   __shared__ __align__(16) unsigned char sh[X8_SG * 4096];
   u32x4 xs[X8_SG];
 #pragma unroll
   for (int q = 0; q < X8_SG; ++q) {
     xs[q] = u32x4{0, 0, 0, 0};
-    if (group0 + q < groups && row < rows) xs[q] = *(const u32x4*)(a + row * lda + (group0 + q) * X8_G + (4 * j + rr) * 16 + odd * 8);
+    if (group0 + q < groups && src >= 0) xs[q] = *(const u32x4*)(a + src * lda + (group0 + q) * X8_G + (4 * j + rr) * 16 + odd * 8);
   }
 #pragma unroll
   for (int q = 0; q < X8_SG; ++q) {
@@ -185,6 +197,16 @@ __global__ __launch_bounds__(256) void x8_split_kernel(const uint16_t* a, int64_
   for (int q = 0; q < X8_SG; ++q)
     if (group0 + q < groups)
       *(u32x4*)(rec + ((int64_t)(group0 + q) * stride + blockIdx.x * 16) * 256 + threadIdx.x * 16) = *(const u32x4*)(sh + q * 4096 + threadIdx.x * 16);
+}
+
+template <int X8_SG>
+__global__ __launch_bounds__(256) void x8_split_kernel(const uint16_t* a, int64_t lda, int rows, int stride, int groups, unsigned char* rec,
+                                                       uint32_t* scl) {
+  x8_split<X8_SG, false>(a, lda, rows, stride, groups, rec, scl, X8Slots{});
+}
+__global__ __launch_bounds__(256) void x8_split_slots_kernel(const uint16_t* a, int64_t lda, int stride, int groups, unsigned char* rec, uint32_t* scl,
+                                                             const X8Slots slots) {
+  x8_split<4, true>(a, lda, 0, stride, groups, rec, scl, slots);
 }
 
 // ------------------------------------------------------------------------------------------------ GEMM
@@ -295,7 +317,7 @@ __device__ __forceinline__ uint32_t x8_table(int z, int dword) {
   return r;
 }
 
-template <bool ZP, bool CHANNEL, int MB, int KS, int WN, bool PREP>
+template <bool ZP, bool CHANNEL, int MB, int KS, int WN, bool PREP, bool MOE = false>
 __device__ __forceinline__ void x8_tile(const X8Params& xp) {
   const KParams& p = xp.k;
   constexpr int BM = 16 * MB, BN = WN * 64;
@@ -309,10 +331,26 @@ __device__ __forceinline__ void x8_tile(const X8Params& xp) {
   const int c = lane & 7, h = (lane >> 3) & 1, g = lane >> 4;
   const int G = p.K / X8_G;
 
-  const int mtiles = (p.M + BM - 1) / BM, nsplit = p.splits;
+  int mtiles = (p.M + BM - 1) / BM, nsplit = p.splits;
   int j = blockIdx.x, split = 0, slot = 0;
   int gb = 0, ge = G;
-  if (nsplit > 1) {
+  if constexpr (MOE) {  // (as the prefill kernel: K pieces of the last round's tiles, whole tiles in runs for every XCD)
+    static_assert(BM == FB_BM && KS == 1 && BN == 512, "the tiles of the prefill kernel and of its second pass");
+    zero_fill_side_job(p);
+    mtiles = min((*p.ntpp + BM - 1) / BM, (p.n_sorted + BM - 1) / BM);
+    if (mtiles == 0) return;
+    const TailSplit d = tail_split(mtiles * p.ncp, p.dyn_slots, p.total_ksteps, FB_MIN_SPLIT);
+    nsplit = 1;
+    if (j < d.F) {
+      if ((d.F & 7) == 0) j = (j & 7) * (d.F >> 3) + (j >> 3);
+    } else {
+      const int u = j - d.F;
+      if (u >= d.R * d.S) return;
+      slot = u % d.R, split = u / d.R, nsplit = d.S;
+      gb = split * d.kps / 4, ge = min(gb + d.kps / 4, G);
+      j = d.F + slot;
+    }
+  } else if (nsplit > 1) {
     const int tiles = mtiles * p.ncp, per = p.ksteps_per_split / 4;
     split = j / tiles;
     j -= split * tiles;
@@ -324,15 +362,26 @@ __device__ __forceinline__ void x8_tile(const X8Params& xp) {
   gb += part * max_steps;
   ge = min(gb + max_steps, ge);
   const int steps = ge - gb;  // the last part may have fewer (or none)
-  const int mt = j % mtiles, strip = p.strip0 + j / mtiles;
+  int mt = j % mtiles, strip = p.strip0 + j / mtiles;
+  if (MOE) chunked_tile(j, mtiles, p.ncp, mt, strip);
   const int row0 = mt * BM;
   const int u = strip * WN + wn, cp = u >> 1, wsel = (u & 1) * 2;
   const bool wave_on = cp * 128 < p.N;
 
+  const uint32_t* Bq = p.B;
   const uint16_t* Sc = (const uint16_t*)p.S;
   const uint16_t* bias = (const uint16_t*)p.bias;
+  if constexpr (MOE) {
+    const int e = p.expert_ids[mt];
+    if (e < 0) return;  // expert of another rank
+    Bq += e * p.b_estride;
+    Sc += e * p.s_estride;
+    if (bias) bias += e * p.n_estride;
+  }
   const int u_mem = wave_on ? u : 0;
-  const int nt = !wave_on ? 0 : ((2 * cp + h) * 64 < p.N ? 2 * cp + h : 0);
+  // (fused SiLU-and-mul: gate n-tile cp paired with the up n-tile of the same output columns, N / 128 + cp)
+  const bool act = MOE && p.act;
+  const int nt = !wave_on ? 0 : act ? (h ? (p.N >> 7) + cp : cp) : ((2 * cp + h) * 64 < p.N ? 2 * cp + h : 0);
   // byte offsets of the lane; everything else in an address is uniform
   const uint32_t b_off = (uint32_t)(nt * 128 + (4 * c + g) * 4 + wsel) * 4;
   // (nt * 64 + 8 c + 2 wsel) * 2 of the scales; two instructions per step for a register of the loop's 256
@@ -344,7 +393,7 @@ __device__ __forceinline__ void x8_tile(const X8Params& xp) {
   const uint32_t b_row = (uint32_t)p.N * 8;  // bytes of one k-tile
   // buffer resources: 32-bit offsets, nothing per lane but the lane's own (the host checks the sizes)
   const int b_bytes = (int)((uint32_t)(p.K / 16) * b_row), sg = CHANNEL ? 1 : (4 * G) >> p.group_shift;
-  const auto b_res = __builtin_amdgcn_make_buffer_rsrc((void*)p.B, 0, b_bytes, 0x00020000);
+  const auto b_res = __builtin_amdgcn_make_buffer_rsrc((void*)Bq, 0, b_bytes, 0x00020000);
   const auto s_res = __builtin_amdgcn_make_buffer_rsrc((void*)Sc, 0, sg * p.N * 2, 0x00020000);
   const auto z_res = __builtin_amdgcn_make_buffer_rsrc((void*)p.Z, 0, sg * (p.N / 2), 0x00020000);
 
@@ -531,6 +580,15 @@ __device__ __forceinline__ void x8_tile(const X8Params& xp) {
     }
   };
 
+  // MoE: C row (-1: none) and routing weight of every row of the tile
+  int* s_crow = (int*)(smem + x8_smem(MB, KS, WN));
+  float* s_tw = (float*)(s_crow + BM);
+  if (MOE && t < BM) {
+    const int id = row0 + t < p.n_sorted ? p.sorted_ids[row0 + t] : -1, dst = (unsigned)id < (unsigned)p.c_rows ? id : -1;
+    s_crow[t] = dst;
+    if (p.mul_topk) s_tw[t] = dst >= 0 ? p.topk_w[dst] : 0.f;
+  }
+
   // ---- prologue and main loop: one step (128 K rows) per barrier
   if (steps > 0) {
 #pragma unroll
@@ -583,6 +641,13 @@ __device__ __forceinline__ void x8_tile(const X8Params& xp) {
     __builtin_memcpy(&late, (const void*)args, sizeof(late));
   }
 
+  // the row of A behind row r of the tile (one that has a token)
+  auto a_row = [&](int r) {
+    int64_t src = row0 + r;
+    if (MOE && !late.k.a_by_slot) src = s_crow[r] / late.k.top_k;
+    return (const uint16_t*)late.k.A + src * late.k.lda;
+  };
+
   // ---- wide steps: what the two terms of the flagged rows leave out, by the 16-bit unit, behind the loop (activations from A, weights as
   // the integers q - z).  A row's result depends on that row alone, and a wavefront on nothing that others do here.
   auto add_rest = [&](int gi) {
@@ -618,8 +683,7 @@ __device__ __forceinline__ void x8_tile(const X8Params& xp) {
         if (!__any(mine)) continue;
         u32x4 a[2] = {};
         if (mine) {
-          const uint32_t* src =
-              (const uint32_t*)((const uint16_t*)late.k.A + (int64_t)(row0 + 16 * m + (lane & 15)) * late.k.lda + gi * X8_G + 64 * half) + g;
+          const uint32_t* src = (const uint32_t*)(a_row(16 * m + (lane & 15)) + gi * X8_G + 64 * half) + g;
 #pragma unroll
           for (int q = 0; q < 8; ++q) a[q >> 2][q & 3] = src[4 * q];
 #pragma unroll
@@ -705,22 +769,53 @@ __device__ __forceinline__ void x8_tile(const X8Params& xp) {
   const int ncol = 64 * (2 * cp + lh) + 16 * wsel + (lc & 31);
   const bool col_ok = wave_on && ncol < late.k.N;
   float cs[4] = {1.f, 1.f, 1.f, 1.f}, bs[4] = {0.f, 0.f, 0.f, 0.f};
-  if (col_ok) {
-    const int base = ncol & ~31, cl = ncol & 31;
+  auto col_consts = [&](int col, float* sc_out, float* b_out) {
+    const int base = col & ~31, cl = col & 31;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      if (CHANNEL) cs[i] = bf16_lo_f32(Sc[base + single_perm_pos(cl + i)]);
-      if (bias) bs[i] = bf16_lo_f32(bias[base + single_perm_pos(cl + i)]);
+      if (CHANNEL) sc_out[i] = bf16_lo_f32(Sc[base + single_perm_pos(cl + i)]);
+      if (bias) b_out[i] = bf16_lo_f32(bias[base + single_perm_pos(cl + i)]);
     }
+  };
+  // fused SiLU-and-mul (unsplit): lane -> row (lane >> 3) + 8 i, gate columns ac .. ac + 3 of the slab's first 32 and the up columns of the same outputs
+  const bool act_now = act && nsplit == 1;
+  const int ac = (lane & 7) * 4, ocol = 64 * cp + 16 * wsel + ac;
+  float cu[4] = {1.f, 1.f, 1.f, 1.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
+  if (act_now) {
+    if (wave_on) {
+      col_consts(ocol, cs, bs);
+      col_consts((late.k.N >> 1) + ocol, cu, bu);
+    }
+  } else if (col_ok && !act) {
+    col_consts(ncol, cs, bs);
   }
+  auto finish_act = [&](int r, f32x4 v, f32x4 w) {
+    const int crow = s_crow[r];
+    if (crow < 0) return;
+    const float tw = late.k.mul_topk ? s_tw[r] : 1.f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      v[q] = (v[q] * cs[q] + bs[q]) * tw;
+      w[q] = (w[q] * cu[q] + bu[q]) * tw;
+    }
+    store_row4_silu_mul<DT_BF16>(late.k, crow, ocol, v, w);
+  };
   auto finish = [&](int r, f32x4 v) {  // r: row of the tile
+    if (MOE && s_crow[r] < 0) return;
     if (nsplit > 1) {
       *(f32x4*)(late.k.ctmp + (((int64_t)slot * nsplit + split) * BM + r) * BN + (ncol - strip * BN)) = v;
       return;
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[q] = v[q] * cs[q] + bs[q];
-    store_row4<DT_BF16, false>(late.k, row0 + r, ncol, v);
+    if constexpr (MOE) {
+      if (late.k.mul_topk) {
+        const float tw = s_tw[r];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] *= tw;
+      }
+    }
+    store_row4<DT_BF16, MOE>(late.k, MOE ? s_crow[r] : row0 + r, ncol, v);
   };
 #pragma unroll
   for (int m = 0; m < MS; m += 2) {
@@ -731,6 +826,16 @@ __device__ __forceinline__ void x8_tile(const X8Params& xp) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) slab[(16 * e + 4 * g + r) * X8_RS + 40 * h + 8 * i + c] = acc[m + e][i][r];
     __builtin_amdgcn_wave_barrier();
+    if (MOE && act_now) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float* at = slab + ((lane >> 3) + 8 * i) * X8_RS + ac;
+        const f32x4 v = *(const f32x4*)at, w = *(const f32x4*)(at + 40);
+        if (wave_on) finish_act(16 * m + (lane >> 3) + 8 * i, v, w);
+      }
+      __builtin_amdgcn_wave_barrier();
+      continue;
+    }
     f32x4 v[2 * 4];
 #pragma unroll
     for (int i = 0; i < 8; ++i)
@@ -738,15 +843,20 @@ __device__ __forceinline__ void x8_tile(const X8Params& xp) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int r = (m0 + m) * 16 + (lane >> 4) + 4 * i;
-      if ((i < 4 || m + 1 < MS) && r < BM && col_ok && row0 + r < late.k.M) finish(r, v[i]);
+      if ((i < 4 || m + 1 < MS) && r < BM && col_ok && (MOE || row0 + r < late.k.M)) finish(r, v[i]);
     }
     __builtin_amdgcn_wave_barrier();
   }
   if (wave_on && __any((any >> 16 & 1u) != 0)) {
     // rows with infinities, four at a time: 16 lanes have those of theirs that the same lanes have stored above
     const uint32_t* flags = late.scl + row0;
-    const int rows = min(min(BM, (m0 + MS) * 16), late.k.M - row0);  // of the tile, in front of the part's end
+    const int rows = MOE ? BM : min(min(BM, (m0 + MS) * 16), late.k.M - row0);  // of the tile, in front of the part's end
     const int n_in = 128 * cp + 16 * wsel + (lc & 31);          // (lanes whose columns are behind the matrix look along)
+    // (lanes of gate columns finish what those eight behind them have of the up columns; the stores above came from other lanes)
+    if (MOE && act_now) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const int n_act = (lh ? late.k.N >> 1 : 0) + 64 * cp + 16 * wsel + (lc & 31);
+    const uint32_t* b_late = late.k.B;
+    if constexpr (MOE) b_late += late.k.expert_ids[mt] * late.k.b_estride;
 #pragma unroll 1
     for (int r0 = m0 * 16; r0 < rows; r0 += 64) {
       uint32_t f = 0;
@@ -756,9 +866,17 @@ __device__ __forceinline__ void x8_tile(const X8Params& xp) {
 #pragma unroll 1
       for (; hit; hit &= hit - 1) {
         const int r = r0 + __builtin_ctzll(hit);
-        const f32x4 v = x8_infinite_row<ZP, CHANNEL>((const uint16_t*)late.k.A + (int64_t)(row0 + r) * late.k.lda, flags + r, late.rows, gb0, ge0, late.k.B, Sc,
-                                                     late.k.Z, late.k.N, late.k.group_shift, col_ok ? ncol : n_in);
-        if (col_ok) finish(r, v);
+        const f32x4 v = x8_infinite_row<ZP, CHANNEL>(a_row(r), flags + r, late.rows, gb0, ge0, b_late, Sc, late.k.Z, late.k.N, late.k.group_shift,
+                                                     act ? n_act : col_ok ? ncol : n_in);
+        if (MOE && act_now) {
+          f32x4 w;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) w[q] = __shfl(v[q], (lane + 8) & 63);
+          // (ac, ocol and their constants are those of lanes 0 .. 7)
+          if (lh == 0) finish_act(r, v, w);
+        } else if (col_ok) {
+          finish(r, v);
+        }
       }
     }
   }
@@ -767,6 +885,10 @@ __device__ __forceinline__ void x8_tile(const X8Params& xp) {
 template <bool ZP, bool CHANNEL, int MB, int KS, int WN>
 __global__ __launch_bounds__(64 * KS * WN, 2) void x8_kernel(const X8Params xp) {
   x8_tile<ZP, CHANNEL, MB, KS, WN, false>(xp);
+}
+template <bool CHANNEL>
+__global__ __launch_bounds__(512, 2) void x8_moe_kernel(const X8Params xp) {
+  x8_tile<false, CHANNEL, 8, 1, 8, false, true>(xp);
 }
 template <bool CHANNEL>
 __global__ __launch_bounds__(512, 2) void x8_prepared_kernel(const X8Params xp) {
@@ -906,6 +1028,37 @@ int launch_x8(const w4a16_gemm_args* a, const Plan& pl, void* scratch, hipStream
     W4A16_HIP(hipGetLastError());
   }
   return 0;
+}
+
+int64_t x8_moe_scratch_bytes(int64_t n_sorted, int64_t k) {
+  const int64_t r = (n_sorted + 127) / 128 * 128, g = k / X8_G;
+  return r * g * 256 + (r * g * 4 + 255) / 256 * 256;
+}
+
+// MoE blocks of 128 slots, uint4b8: the prefill kernel's tiles, plan and second pass
+int launch_x8_moe(const w4a16_gemm_args* a, const Plan& pl, void* scratch, hipStream_t stream) {
+  const bool channel = pl.gm == GM_CHANNEL;
+  if (a->dtype != DT_BF16 || a->wtype != W4A16_WTYPE_U4B8 || !(a->flags & W4A16_F_MOE) || pl.gm == GM_GIDX || pl.bm != 128 || pl.tn != 512 ||
+      pl.splits != 1 || pl.dyn_slots <= 0 || pl.total_ksteps % 4 != 0 || (!channel && pl.group_ksteps % 4 != 0))
+    return fail(W4A16_EINVAL, "unsupported kernel variant");
+  if (pl.tiles <= 0) return 0;
+  X8Params xp{};
+  xp.k = make_kparams(a, pl);
+  const int groups = (int)(a->size_k / X8_G), rows = pl.mtiles * 128;
+  unsigned char* base = (unsigned char*)scratch;
+  xp.rec = base;
+  xp.scl = (const uint32_t*)(base + (int64_t)rows * groups * 256);
+  xp.rows = rows;
+  const X8Slots slots = {xp.k.sorted_ids, xp.k.ntpp, xp.k.n_sorted, xp.k.c_rows, xp.k.top_k, xp.k.a_by_slot};
+  hipLaunchKernelGGL(x8_split_slots_kernel, dim3((unsigned)(rows / 16), (unsigned)ceil_div(groups, 4)), dim3(256), 0, stream, (const uint16_t*)a->a, a->lda,
+                     rows, groups, base, (uint32_t*)xp.scl, slots);
+  W4A16_HIP(hipGetLastError());
+  const x8_fn fn = channel ? x8_moe_kernel<true> : x8_moe_kernel<false>;
+  const int smem = x8_smem(8, 1, 8) + 128 * 8;
+  W4A16_HIP(allow_dynamic_lds((const void*)fn, smem));
+  hipLaunchKernelGGL(fn, dim3((unsigned)(pl.tiles + mid_tail_pieces(pl.tiles, pl.dyn_slots))), dim3(512), smem, stream, xp);
+  W4A16_HIP(hipGetLastError());
+  return launch_fat_reduce(a, pl, xp.k, stream);
 }
 
 }  // namespace w4a16

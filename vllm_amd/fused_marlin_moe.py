@@ -53,9 +53,15 @@ def _tall_from(quant_type: ScalarType, k: int, n: int, w1_scale, w2_scale, is_k_
         with k * n >= 4096 * 8192       0.95 - 1.02    0.93 - 0.98    from 192
       fp16 uint4b8, others              1.02 - 1.11    0.93 - 1.12    never (mean 1.05 / 1.01): the cheapest dequantisation
 
+    bf16 uint4b8 with groups of whole 128 rows or one scale per column runs blocks of 128 on the 8-bit matrix unit (gemm_x8.hip), which takes
+    0.90 - 1.00 of the prefill kernel's time (nine expert shapes of 2048 x 1408 to 6144 x 10752, 96 to 1024 slots; 1.04 at most), and against
+    blocks of 64 0.83 - 1.00 from 192 slots with both K >= 4096, 0.86 - 0.99 with 4096 x 2048, 3584 x 2560 and 7168 x 2048 (channel-wise
+    0.92 - 1.02 from 384), 0.95 - 1.02 with 2048 x 8192 and 1.06 - 1.13 with 2048 x 1408.  So its line is at k >= 3072, n >= 2048, k * n >=
+    4096 * 2048.
+
     The spread inside a row is how the tiles fill their last round.  With a K below 4096 the sides cross: 64 experts of 2048 x 1408
     1.02 - 1.17, 32 of 4096 x 2048 0.94 - 1.05, while bf16 gains on 16 of 2048 x 8192 and 64 of 7168 x 2048 (0.89 - 0.94)."""
-    if quant_type not in (scalar_types.uint4, scalar_types.uint4b8) or not is_k_full or min(k, n) < 4096 or k % 128 or n % 128:
+    if quant_type not in (scalar_types.uint4, scalar_types.uint4b8) or not is_k_full or k < 3072 or n < 2048 or k % 128 or n % 128:
         return 0
     rows = []  # K rows per scale row
     for kk, g in ((k, w1_scale.size(1)), (n, w2_scale.size(1))):
@@ -63,6 +69,9 @@ def _tall_from(quant_type: ScalarType, k: int, n: int, w1_scale, w2_scale, is_k_
             return 0
         rows.append(kk // g)
     fp16, fine, channel = w1_scale.dtype == torch.float16, min(rows) < 128, rows[0] == k or rows[1] == n
+    if min(k, n) < 4096:
+        on_x8 = not fp16 and quant_type == scalar_types.uint4b8 and not fine
+        return 0 if not on_x8 or k * n < 4096 * 2048 else 384 if channel else 192
     if fp16 and quant_type == scalar_types.uint4b8:
         return 0 if fine or channel else 192 if k * n >= 4096 * 8192 else 384
     return 384 if fine or (fp16 and channel) else 192
