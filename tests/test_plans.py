@@ -28,8 +28,8 @@ def plan(tmp_path_factory):
                    check=True, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
     probe = ctypes.CDLL(out).plan_probe
 
-    def call(m, k, n, dtype, fmt, group, act_order=False, more_scratch=True):
-        """`dtype`: a torch dtype; operands are never read."""
+    def call(m, k, n, dtype, fmt, group, act_order=False, more_scratch=True, moe_slots=0):
+        """`dtype`: a torch dtype; operands are never read.  moe_slots: MoE blocks of 64 and so many sorted slots."""
         a = _lib.GemmArgs()
         a.struct_size = ctypes.sizeof(_lib.GemmArgs)
         a.dtype = _lib.DTYPE_BF16 if dtype == torch.bfloat16 else _lib.DTYPE_F16
@@ -42,6 +42,10 @@ def plan(tmp_path_factory):
         if act_order:
             a.g_idx = a.perm = 4096
         a.size_m, a.size_n, a.size_k, a.num_groups = m, n, k, 1 if group == -1 else k // group
+        if moe_slots:
+            a.flags |= _lib.F_MOE
+            a.lda, a.moe_block_size, a.top_k, a.n_sorted = k, 64, 1, moe_slots
+            a.sorted_token_ids = a.expert_ids = a.num_tokens_past_padded = 4096
         a.workspace_len = 1024  # what marlin_make_workspace_new makes on this GPU
         res = (ctypes.c_int32 * len(FIELDS))()
         assert probe(ctypes.byref(a), int(more_scratch), res) == 0
@@ -133,3 +137,26 @@ def test_prepared_weights(plan):
         assert (p["kind"], p["ks"], p["mb"], p["tn"], p["splits"]) == (7, 1, 8, 512, 1), (k, n, m, group, p)
         assert plan(m, k, n, torch.bfloat16, "uint4", group, more_scratch=False)["kind"] != 7
         assert plan(m, k, n, torch.float16, "uint4", group)["kind"] != 7
+
+
+def test_moe_blocks_of_64(plan):
+    """256-column tiles until 512-column ones number 9/4 (fp16) or 3 (bf16) of the compute units; operands of 2 GiB and more run on the 64-row kernel."""
+    import torch
+    for dtype in (torch.float16, torch.bfloat16):
+        for fmt in ("uint4", "uint4b8"):
+            for group in (32, 128, -1):
+                blocks = 72 if dtype == torch.float16 else 96      # 8 strips to a block
+                for slots, k, n, kind, tn in [
+                        (64, 128, 64, 8, 256),
+                        (64 * (blocks - 1), 2048, 4096, 8, 256),
+                        (64 * (blocks - 1) + 1, 2048, 4096, 8, 512),
+                        (64 * 96, 4096, 3648, 8, 512),
+                        (64 * 8, 65536, 65536 - 64, 8, 512),       # an expert just under 2 GiB of weights
+                        (64 * 8, 65536, 65536, 3, 512)]:
+                    got = plan(min(slots, 4096), k, n, dtype, fmt, group, moe_slots=slots)
+                    assert (got["kind"], got["tn"], got["splits"]) == (kind, tn, 1), (slots, k, n, group, got)
+    rows = (1 << 31) // (2 * 4096)
+    assert plan(rows - 1, 4096, 512, torch.bfloat16, "uint4", 128, moe_slots=rows)["kind"] == 8
+    assert plan(rows, 4096, 512, torch.bfloat16, "uint4", 128, moe_slots=rows)["kind"] == 3
+    # act-order: the gathered rows, one for each slot, are what the kernel reads
+    assert plan(rows - 1, 4096, 512, torch.bfloat16, "uint4b8", 128, act_order=True, moe_slots=rows)["kind"] == 3

@@ -54,7 +54,7 @@ struct KParams {
 // round, and a second pass adds the pieces: F tiles run whole, the R = L - F tail tiles as R * S pieces of kps k-steps
 // (a multiple of 4, at least 32).  The 64-row kernel only from S = min_split = 3 on: a tail of more than slots / 3 tiles already
 // runs with fewer workgroups per compute unit, hence faster, and halving it gains less than the partial tiles cost; the
-// prefill kernel (blocks of 128 slots, one workgroup per compute unit) from 2 on.  Both passes derive the same numbers from L.
+// prefill kernel (blocks of 128 slots, one workgroup per compute unit) from 2 on.  (gemm_slots.hip has a line of its own.)  Both passes derive the same numbers from L.
 constexpr int TAIL_MIN_KSTEPS = 32;
 struct TailSplit {
   int F, R, S, kps;

@@ -16,7 +16,7 @@ struct Plan {
   int kind;  // 0: skinny kernel, 1: decode kernel, 2: prefill ("fat") kernel, 3: 64-row ("mid") kernel,
              // 5: in-workgroup K split (gemm_kq.hip): 64 x 256 tiles in K quarters (mb = 4), 80 .. 128 x 256 in halves (mb = 5 .. 8), 32 .. 64 x 128
              // in eighths (mb = 2 .. 4, tn = 128), 6: 8-bit matrix unit, 7: the same on prepared weights,
-             // 9: the same on MoE blocks of 128 slots
+             // 8: MoE blocks of 64 slots, integer 4-bit weights (gemm_slots.hip, tn = 256 or 512), 9: the 8-bit unit on MoE blocks of 128 slots
   int tn;    // tile width in columns (128; the decode kernel also has 64)
   int nw = 8;  // 16-row tiles (decode kernel, general kernel with one m-block): wavefronts per workgroup (8 or 4)
   int strip0 = 0;      // 64-row kernel / K-split kernel: first 512- / 256-column strip handled by the launch
@@ -46,6 +46,7 @@ int64_t x8_weight_bytes(int64_t k, int64_t n);
 int64_t x8_moe_scratch_bytes(int64_t n_sorted, int64_t k);
 int launch_x8_moe(const w4a16_gemm_args* a, const Plan& pl, void* scratch, hipStream_t stream);
 int launch_x8(const w4a16_gemm_args* a, const Plan& pl, void* scratch, hipStream_t stream);
+int launch_slots(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_kq(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 
 }  // namespace w4a16
