@@ -13,7 +13,12 @@
 // MFMA work per byte of weights is 64x the decode kernel's; the bound is the matrix pipe, and the VALU work
 // of dequantisation (about 105 instructions per 64 MFMAs for fp16) is interleaved with them: the MFMAs run
 // word-major (16 per Marlin word), and as soon as a word's operands are dead the next k-step's word is
-// dequantised into the same registers.
+// dequantised into the same registers.  One wavefront per SIMD has nothing to hide a wait behind, so (1) the A operands of a k-step are
+// read from LDS during the last word of the one before; (2) a register's three dependent steps stand between three MFMA pairs; (3) scales and
+// zero points of groups of 128 rows and more come once per 128 rows (ONCE), shorter groups have a loop of their own: with both loops in one
+// kernel the registers did not reach.  Dense 4096 x 28672 and 5120 x 13824, 512 to 4096 rows: groups of 32 and 64 0.92 - 0.98 of the time (fp16
+// uint4b8, 1501 rows: 337 -> 323 us), of 128 0.98 - 1.00, channel-wise level; MoE blocks of 128, three expert shapes: 0.98 in the mean, short
+// groups 0.96.
 // MoE blocks of 128 sorted slots run here too when experts are large and full (_tall_from in fused_marlin_moe.py): the 64-row kernel dequantises
 // every weight once per 64 rows (8 experts of 4096 x 14336, top-2, 4096 tokens, bf16: GEMM1 2129 -> 1815 us, GEMM2 1011 -> 874).
 // Requirements (host-checked; otherwise the skinny kernel runs): K % 128 == 0, no per-row g_idx.
@@ -34,8 +39,9 @@ constexpr int FB_SMEM = (2 * FB_ABUF > FB_SLABS ? 2 * FB_ABUF : FB_SLABS) + FB_B
 // FP4 = 1 / 2: float4_e2m1f weights (4-bit layout) with NVFP4 / MXFP4 scale records, one 16-byte record per lane and
 // k-step / two k-steps (the host sets the group to 1 / 2 k-steps); NVFP4's global scale is applied to the accumulator.
 // ZPF: uint4 weights with fp16 zero points laid out like the scales (HQQ): operand = fma(q, s, -half(zp * s)).
+// ONCE: integer 4-bit weights with groups of 128 rows at least, or one scale per column.
 // MOE: blocks of 128 sorted token slots (integer 4-bit weights); rows are gathered through sorted_token_ids while staging.
-template <int DT, bool ZP, bool CHANNEL, int BITS = 4, bool FP8 = false, int FP4 = 0, bool ZPF = false, bool MOE = false>
+template <int DT, bool ZP, bool CHANNEL, int BITS = 4, bool FP8 = false, int FP4 = 0, bool ZPF = false, bool MOE = false, bool ONCE = false>
 __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
   static_assert(!ZPF || (DT == DT_F16 && !ZP && !CHANNEL && BITS == 4 && FP4 == 0), "float zero points: fp16 uint4 grouped");
   static_assert(BITS == 4 || (BITS == 8 && !ZP), "8-bit weights have no zero points");
@@ -170,9 +176,9 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
   auto issue = [&](Stage& s, int ks) {
     ks = min(ks_b + ks, ks_e - 1);
     int gi = 0;
-    if (!CHANNEL) gi = ks >> p.group_shift;  // the host only picks this kernel for power-of-two group sizes
-    if (!CHANNEL) s.sc = sp[(int64_t)gi * s_row];
-    if (ZP) s.zq = zp[(int64_t)gi * s_row];
+    if (!CHANNEL && !ONCE) gi = ks >> p.group_shift;  // the host only picks this kernel for power-of-two group sizes
+    if (!CHANNEL && !ONCE) s.sc = sp[(int64_t)gi * s_row];
+    if (ZP && !ONCE) s.zq = zp[(int64_t)gi * s_row];
     if (FP4 == 2) s.zq = ks & 1;  // which half of the two-k-step scale record
     if (ZPF) s.zf = zfp[(int64_t)gi * s_row];
     s.b0 = bp[(int64_t)(2 * ks) * b_row];
@@ -181,6 +187,14 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
       s.b0h = bp[(int64_t)(2 * ks) * b_row + 1];
       s.b1h = bp[(int64_t)(2 * ks + 1) * b_row + 1];
     }
+  };
+  // groups of 128 rows at least: scales and zero points once per loop iteration
+  u32x4 sc128 = {0, 0, 0, 0};
+  uint32_t zq128 = 0;
+  auto issue_scales = [&](int ks) {
+    const int gi = CHANNEL ? 0 : min(ks_b + ks, ks_e - 1) >> p.group_shift;
+    if (!CHANNEL) sc128 = sp[(int64_t)gi * s_row];
+    if (ZP) zq128 = zp[(int64_t)gi * s_row];
   };
   struct Fp4Scales { float a0, a1, b0, b1; };
   auto fp4_scales = [&](const Stage& s, int w) {
@@ -202,7 +216,7 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
     return v[2 * (w & 1) + half];
   };
   auto col_const = [&](const Stage& s, int w) {
-    return make_col_const<DT, UNIT>(CHANNEL ? 0u : s.sc[w], ZP ? zero_pair(s.zq, w) : ZERO_U4B8);
+    return make_col_const<DT, UNIT>(CHANNEL ? 0u : ONCE ? sc128[w] : s.sc[w], ZP ? zero_pair(ONCE ? zq128 : s.zq, w) : ZERO_U4B8);
   };
 
   f32x4 acc[FB_MB][4][2];
@@ -218,6 +232,7 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
 
   // ---- prologue
   load_a(0);
+  if constexpr (ONCE) issue_scales(0);
 #pragma unroll
   for (int j = 0; j < FB_D; ++j) issue(st[j], j);
   store_a(0);
@@ -256,58 +271,59 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
   // one register of the next k-step's operands (3-5 VALU instructions) is dequantised into ob[CUR ^ 1]; the
   // scheduling barriers keep the compiler from regrouping that into MFMA-only and VALU-only blocks, which would
   // leave the matrix pipe idle during the VALU blocks.
-  auto kstep = [&](auto cur_tag, int buf, int kk, const Stage& nxt, auto refresh_tag) {
-    constexpr int CUR = decltype(cur_tag)::value;
-    const u32x4* abase = (const u32x4*)(lds + buf * (FB_ABUF / 4)) + (kk * FB_MB) * 64 + lane;
-    u32x4 af[FB_MB];
+  // The A operands of the next k-step are read from LDS during the last word, each right behind the last MFMA that uses its registers: a whole
+  // word of MFMAs covers the reads.  With the chunk's second k-step (CUR) that is the next chunk, which is therefore stored two words, and the
+  // workgroup's barrier passed one word, before the end.
+  auto a_frags = [&](int buf, int kk) { return (const u32x4*)(lds + buf * (FB_ABUF / 4)) + (kk * FB_MB) * 64 + lane; };
+  u32x4 af[FB_MB];
 #pragma unroll
-    for (int mb = 0; mb < FB_MB; ++mb) af[mb] = abase[mb * 64];
+  for (int mb = 0; mb < FB_MB; ++mb) af[mb] = a_frags(0, 0)[mb * 64];
+  auto kstep = [&](auto cur_tag, int buf, const Stage& nxt, auto refresh_tag) __attribute__((always_inline)) {
+    constexpr int CUR = decltype(cur_tag)::value;
+    const u32x4* anext = CUR ? a_frags(buf ^ 1, 0) : a_frags(buf, 1);
     if constexpr (CONSTS && decltype(refresh_tag)::value) {
 #pragma unroll
       for (int w = 0; w < 4; ++w) ccs[w] = col_const(nxt, w);
     }
-    // bf16 integer weights: the three dependent stages of one operand register (nibbles -> exact fp16 pair, two
-    // mixed FMAs, one pack) are spread over three consecutive MFMA pairs, so that no VALU instruction reads the
-    // result of the one issued just before it
-    constexpr bool PIPE = (CONSTS && DT == DT_BF16);
+    // integer weights: the three dependent stages of one operand register (nibbles -> exact fp16 pair, minus the zero point (bf16: times the scale
+    // too, in fp32), times the scale (bf16: the pack)) are spread over three consecutive MFMA pairs, so that no VALU
+    // instruction reads the result of the one issued just before it
     uint32_t ph = 0;
-    PieceValue<DT_BF16> pv = {0.f, 0.f};
+    PieceValue<DT> pv;
     auto stage_a = [&](auto p_tag) {  // piece P: nibbles -> (1024+q | 64+q) fp16 pair
       constexpr int P = decltype(p_tag)::value, w = P >> 3, J = P & 7;
       ph = piece_halves<J>((J & 3) < 2 ? nxt.b0[w] : nxt.b1[w]);
     };
-    auto stage_b = [&](auto p_tag) {  // (q - z) * s in fp32, exact
+    auto stage_b = [&](auto p_tag) {
       constexpr int P = decltype(p_tag)::value, w = P >> 3, J = P & 7;
-      if constexpr (DT == DT_BF16) pv = piece_value<DT, J>(ph, ccs[w]);
+      pv = piece_value<DT, J>(ph, ccs[w]);
     };
-    if constexpr (PIPE) {
+    if constexpr (CONSTS) {
       stage_a(std::integral_constant<int, 0>{});
       stage_b(std::integral_constant<int, 0>{});
       stage_a(std::integral_constant<int, 1>{});
     }
-    auto word = [&](auto w_tag) {
+    auto word = [&](auto w_tag) __attribute__((always_inline)) {
       constexpr int w = decltype(w_tag)::value;
-      const ColConst<DT>& cc = ccs[w];
       const Fp4Scales fs = fp4_scales(nxt, w);
       uint32_t zs = 0;
       if constexpr (ZPF) zs = as_u32(as_h2(nxt.zf[w]) * as_h2(nxt.sc[w]));
       const uint32_t xa = nxt.b0[w], xb = nxt.b1[w];
-      auto step = [&](auto j_tag) {
+      auto step = [&](auto j_tag) __attribute__((always_inline)) {
         constexpr int J = decltype(j_tag)::value;
         mfma_inplace<DT>(acc[J][w][0], af[J], ob[CUR][w][0]);
         mfma_inplace<DT>(acc[J][w][1], af[J], ob[CUR][w][1]);
         uint32_t r;
-        if constexpr (PIPE) {
+        if constexpr (w == 3) af[J] = anext[J * 64];
+        if constexpr (CONSTS) {
           constexpr int P = 8 * w + J;
-          r = pack_bf16(pv.f0, pv.f1);
+          r = piece_finish<DT, UNIT, J>(pv, ccs[w]);
           if constexpr (P + 1 < 32) stage_b(std::integral_constant<int, P + 1>{});
           if constexpr (P + 2 < 32) stage_a(std::integral_constant<int, P + 2>{});
         } else if constexpr (ZPF)
           r = dequant_piece_zpf<J>(xa, xb, nxt.sc[w], zs);
         else if constexpr (FP4 != 0)
           r = ((J & 3) < 2) ? dequant_piece_fp4<DT, J>(xa, fs.a0, fs.a1) : dequant_piece_fp4<DT, J>(xb, fs.b0, fs.b1);
-        else if constexpr (BITS == 4)
-          r = piece_finish<DT, UNIT, J>(piece_value<DT, J>(piece_halves<J>((J & 3) < 2 ? xa : xb), cc), cc);
         else
           r = dequant_piece8<DT, UNIT, FP8, J>(word8(nxt, w, (J & 3) >> 1, 0), word8(nxt, w, (J & 3) >> 1, 1),
                                                CHANNEL ? 0u : nxt.sc[w]);
@@ -328,47 +344,40 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
     };
     word(std::integral_constant<int, 0>{});
     word(std::integral_constant<int, 1>{});
+    if constexpr (CUR) {
+      store_a(buf ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     word(std::integral_constant<int, 2>{});
+    if constexpr (CUR) {
+      __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);
+    }
     word(std::integral_constant<int, 3>{});
   };
   const std::integral_constant<int, 0> even{};
   const std::integral_constant<int, 1> odd{};
 
   // ---- main loop: two chunks (four k-steps = the weight ring) per iteration.  The last k-step of an iteration
-  // dequantises the first k-step of the next 128 rows of K: the constants are rebuilt there, and in the other three
-  // k-steps too when a group is shorter than 128 rows.
-  auto main_loop = [&](auto every_tag) {
-    const std::true_type refresh{};
+  // dequantises the first k-step of the next 128 rows of K: the constants are rebuilt there,
+  // and in the other three k-steps too when a group is shorter than 128 rows.
+  const std::bool_constant<!ONCE && !(CONSTS && CHANNEL)> every{};
 #pragma unroll 1
-    for (int c0 = 0; c0 < nchunks; c0 += 2) {
-      const int ks0 = 2 * c0;
-      // chunk c0 in buffer 0
-      load_a(c0 + 1);
-      kstep(even, 0, 0, st[1], every_tag);
-      issue(st[0], ks0 + 4);
-      kstep(odd, 0, 1, st[2], every_tag);
-      issue(st[1], ks0 + 5);
-      store_a(1);
-      __syncthreads();
-      // chunk c0+1 in buffer 1
-      load_a(c0 + 2);
-      kstep(even, 1, 0, st[3], every_tag);
-      issue(st[2], ks0 + 6);
-      kstep(odd, 1, 1, st[0], refresh);
-      issue(st[3], ks0 + 7);
-      store_a(0);
-      __syncthreads();
-    }
-  };
-  if constexpr (!CONSTS) {
-    main_loop(std::true_type{});
-  } else if constexpr (CHANNEL) {
-    main_loop(std::false_type{});
-  } else {
-    if (p.group_shift < 2)
-      main_loop(std::true_type{});
-    else
-      main_loop(std::false_type{});
+  for (int c0 = 0; c0 < nchunks; c0 += 2) {
+    const int ks0 = 2 * c0;
+    // chunk c0 in buffer 0
+    load_a(c0 + 1);
+    kstep(even, 0, st[1], every);
+    if constexpr (ONCE) issue_scales(ks0 + 4);
+    issue(st[0], ks0 + 4);
+    kstep(odd, 0, st[2], every);
+    issue(st[1], ks0 + 5);
+    // chunk c0+1 in buffer 1
+    load_a(c0 + 2);
+    kstep(even, 1, st[3], every);
+    issue(st[2], ks0 + 6);
+    kstep(odd, 1, st[0], std::true_type{});
+    issue(st[3], ks0 + 7);
   }
 
   // ------------------------------------------------------------------------------ epilogue
@@ -471,15 +480,15 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
 
 typedef void (*fat_fn)(const KParams);
 
-template <int DT>
-static fat_fn pick_fat2(bool zp, bool channel) {
-  if (zp) return channel ? fat_kernel<DT, true, true> : fat_kernel<DT, true, false>;
-  return channel ? fat_kernel<DT, false, true> : fat_kernel<DT, false, false>;
+template <int DT, bool ZP, bool MOE>
+static fat_fn pick_fat3(bool channel, bool once) {
+  if (channel) return fat_kernel<DT, ZP, true, 4, false, 0, false, MOE, true>;
+  return once ? fat_kernel<DT, ZP, false, 4, false, 0, false, MOE, true> : fat_kernel<DT, ZP, false, 4, false, 0, false, MOE, false>;
 }
-template <int DT>
-static fat_fn pick_fat_moe(bool zp, bool channel) {
-  if (zp) return channel ? fat_kernel<DT, true, true, 4, false, 0, false, true> : fat_kernel<DT, true, false, 4, false, 0, false, true>;
-  return channel ? fat_kernel<DT, false, true, 4, false, 0, false, true> : fat_kernel<DT, false, false, 4, false, 0, false, true>;
+template <int DT, bool MOE>
+static fat_fn pick_fat2(bool zp, bool channel, bool once) {
+  if (zp) return pick_fat3<DT, true, MOE>(channel, once);
+  return pick_fat3<DT, false, MOE>(channel, once);
 }
 template <int DT>
 static fat_fn pick_fat8(bool fp8, bool channel) {
@@ -489,12 +498,12 @@ static fat_fn pick_fat8(bool fp8, bool channel) {
 
 int launch_fat(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
   const bool zp = a->b_zeros != nullptr, channel = pl.gm == GM_CHANNEL;
-  const bool moe = (a->flags & W4A16_F_MOE) != 0;
+  const bool moe = (a->flags & W4A16_F_MOE) != 0, once = pl.group_ksteps >= 4;
   fat_fn fn;
   if (moe) {
     if ((a->flags & W4A16_F_ZP_FLOAT) || (a->wtype != W4A16_WTYPE_U4B8 && a->wtype != W4A16_WTYPE_U4) || pl.dyn_slots <= 0)
       return fail(W4A16_EINVAL, "unsupported kernel variant");
-    fn = a->dtype == DT_F16 ? pick_fat_moe<DT_F16>(zp, channel) : pick_fat_moe<DT_BF16>(zp, channel);
+    fn = a->dtype == DT_F16 ? pick_fat2<DT_F16, true>(zp, channel, once) : pick_fat2<DT_BF16, true>(zp, channel, once);
   } else if (a->flags & W4A16_F_ZP_FLOAT) {
     if (a->dtype != DT_F16 || channel) return fail(W4A16_EINVAL, "unsupported kernel variant");
     fn = fat_kernel<DT_F16, false, false, 4, false, 0, true>;
@@ -508,7 +517,7 @@ int launch_fat(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
     if (zp) return fail(W4A16_EINVAL, "unsupported kernel variant");
     fn = a->dtype == DT_F16 ? pick_fat8<DT_F16>(fp8, channel) : pick_fat8<DT_BF16>(fp8, channel);
   } else {
-    fn = a->dtype == DT_F16 ? pick_fat2<DT_F16>(zp, channel) : pick_fat2<DT_BF16>(zp, channel);
+    fn = a->dtype == DT_F16 ? pick_fat2<DT_F16, false>(zp, channel, once) : pick_fat2<DT_BF16, false>(zp, channel, once);
   }
   KParams p = make_kparams(a, pl);
   if (pl.tiles <= 0) return 0;
