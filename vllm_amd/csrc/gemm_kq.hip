@@ -59,7 +59,9 @@ constexpr int kq_smem(int MB, int Q, int WN) {
   return (stage > slabs ? stage : slabs) + 16 * MB * 4;                     // + C row of each tile row
 }
 
-// SHORT: private parts with groups below 128 rows, whose scales and constants come with every k-step
+// SHORT: private parts and tall tiles with groups below 128 rows, whose scales and constants come with every k-step.  (Tall tiles had both loops in
+// one kernel, 40 to 80 registers more, and scales in every k-step for every group: 80 to 112 rows, groups of 32 and 64 0.90 - 0.97 of the
+// time, of 128 0.96 - 1.00, reading A early included; 14336 x 4096 at 1501 rows, fp16, groups of 128: 166 -> 160 us.)
 template <int DT, bool ZP, bool CHANNEL, int MB = 4, int Q = 4, int WN = 2, bool SHORT = false>
 __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   static_assert((MB == 4 && Q == 4 && WN == 2) || (MB > 4 && MB <= 8 && Q == 2 && WN == 2) || (MB >= 2 && MB <= 4 && Q == 8 && WN == 1),
@@ -70,8 +72,13 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   // iteration covers four k-steps (128 rows of K, aligned: every K part starts at a multiple of four k-steps), so with groups of
   // 128 rows or more, or one scale per column, they are rebuilt once per iteration instead of once per k-step.  (Not where the registers
   // are short: 64-row tiles keep them in the 128-column form only, and there not in bf16 with grouped scales: 12 to 28 would spill.)
-  constexpr bool ONCE = PRIV && !SHORT;
-  constexpr bool HOIST = KQ_MB > 4 || (ONCE && (KQ_MB < 4 || CHANNEL || DT == DT_F16));
+  constexpr bool ONCE = !SHORT && (PRIV || KQ_MB > 4);
+  constexpr bool HOIST = KQ_MB > 4 || (PRIV && ONCE && (KQ_MB < 4 || CHANNEL || DT == DT_F16));
+  // EARLY: the A operands of the next k-step are read from LDS during this one's last word, and the next chunk is stored and the barrier passed
+  // before that; 80 to 112 rows then load chunks two ahead, being stored half a k-step sooner.  Time over reading at the start of the k-step:
+  // 64 x 256 0.99, 80 to 112 rows 0.98 (fp16 uint4b8 0.97, channel-wise 0.99); 128 rows, whose words are longer, 1.015, private parts, which have
+  // two wavefronts to a SIMD and no barrier, 1.00 - 1.02: these two don't.
+  constexpr bool EARLY = !PRIV && KQ_MB < 8;
   constexpr bool UNIT = CHANNEL;
   extern __shared__ __align__(16) unsigned char smem[];
   int* s_crow = (int*)(smem + KQ_SMEM - KQ_BM * 4);
@@ -128,6 +135,7 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   //  behind it)
   constexpr int AR = PRIV ? 8 : 16, AN = KQ_BM / AR;           // rows per load instruction, loads per chunk
   constexpr int NH = PRIV && KQ_MB == 4 ? 2 : 1, AH = AN / NH;  // (64 rows: the chunk in two halves, for its registers)
+  constexpr int AD = EARLY && KQ_MB > 4 ? 2 : 1;                // chunks in flight
   const int tq = wn * 64 + lane;
   const int piece = tq & 7;
   const uint16_t* arow[PRIV ? 1 : AN];
@@ -147,26 +155,26 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   // K pairs 8*pp + 2j (pp = piece & 3), which belong to lane (j*16 + row%16), dword pp, of k-step piece >> 2.
   uint32_t* lds = (uint32_t*)smem + q * (2 * KQ_ABUF / 4);
   const int a_wr0 = (piece >> 2) * kq_kstep(KQ_MB) + (tq >> 3) * 4 + (piece & 3);
-  u32x4 areg[AH];
+  u32x4 areg[AD][AH];
   // (chunk and k-step indices are clamped instead of guarded: the last iteration re-reads its own data, which
   //  keeps the main loop free of branches)
-  auto load_a = [&](int chunk, int half) {  // chunk: relative to ks_b
+  auto load_a = [&](int chunk, int half, int slot = 0) {  // chunk: relative to ks_b
     chunk = min(ks_b / 2 + chunk, ks_e / 2 - 1);
 #pragma unroll
     for (int i = 0; i < AH; ++i) {
       if constexpr (PRIV)
-        areg[i] = *(const u32x4*)(abase + (int64_t)chunk * 128 + aoff[half * AH + i]);
+        areg[slot][i] = *(const u32x4*)(abase + (int64_t)chunk * 128 + aoff[half * AH + i]);
       else
-        areg[i] = *(const u32x4*)(arow[i] + chunk * 64);
+        areg[slot][i] = *(const u32x4*)(arow[i] + chunk * 64);
     }
   };
-  auto store_a = [&](int buf, int half) {
+  auto store_a = [&](int buf, int half, int slot = 0) {
     uint32_t* dst = lds + buf * (KQ_ABUF / 4) + a_wr0;
 #pragma unroll
     for (int i = 0; i < AH; ++i) {
       const int r = AR * (half * AH + i);  // (row (tq >> 3) + r: m-block r / 16, AR = 8: upper half of it for odd loads)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) dst[(r / 16) * 256 + (r % 16) * 4 + j * 64] = areg[i][j];
+      for (int j = 0; j < 4; ++j) dst[(r / 16) * 256 + (r % 16) * 4 + j * 64] = areg[slot][i][j];
     }
   };
   // (a wavefront's LDS accesses are executed in order; that they stay in this order is for the compiler to know)
@@ -223,6 +231,7 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
 #pragma unroll
     for (int hf = 0; hf < NH; ++hf) {
       load_a(0, hf);
+      if constexpr (AD == 2) load_a(1, 0, 1);
       if (hf == 0) {
         if constexpr (ONCE) issue_scales(0);
 #pragma unroll
@@ -247,12 +256,20 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   // dependent steps; behind an MFMA stand the last of one register, the second of the next and the first of the one after that, none of
   // which waits for another (in one chain: 12 % of the loop at six such instructions per MFMA and two wavefronts per SIMD).
   // The scheduling barriers keep the compiler from regrouping this into MFMA-only and VALU-only blocks.
-  auto kstep = [&](int buf, int kk, const Stage& cur, const Stage& nxt, auto refresh_tag) {
-    constexpr bool REFRESH = decltype(refresh_tag)::value;
-    const u32x4* abase = (const u32x4*)(lds + buf * (KQ_ABUF / 4) + kk * kq_kstep(KQ_MB)) + lane;
-    u32x4 af[KQ_MB];
+  // (EARLY: each operand right behind the last MFMA that uses its registers)
+  auto a_frags = [&](int buf, int kk) { return (const u32x4*)(lds + buf * (KQ_ABUF / 4) + kk * kq_kstep(KQ_MB)) + lane; };
+  u32x4 af[KQ_MB];
+  if constexpr (EARLY) {
 #pragma unroll
-    for (int mb = 0; mb < KQ_MB; ++mb) af[mb] = abase[mb * 64];
+    for (int mb = 0; mb < KQ_MB; ++mb) af[mb] = a_frags(0, 0)[mb * 64];
+  }
+  auto kstep = [&](int buf, auto kk_tag, const Stage& cur, const Stage& nxt, auto refresh_tag) __attribute__((always_inline)) {
+    constexpr bool REFRESH = decltype(refresh_tag)::value, KK = decltype(kk_tag)::value;
+    const u32x4* anext = KK ? a_frags(buf ^ 1, 0) : a_frags(buf, 1);
+    if constexpr (!EARLY) {
+#pragma unroll
+      for (int mb = 0; mb < KQ_MB; ++mb) af[mb] = a_frags(buf, KK)[mb * 64];
+    }
     ColConst<DT> ccw[2];  // !HOIST: of the word being made and of the one behind it
     if constexpr (!HOIST) {
       if constexpr (ONCE) asm volatile("" : "+v"(sc_now), "+v"(zq_now));  // (or the compiler keeps all four words' constants)
@@ -273,14 +290,18 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
     make_halves(std::integral_constant<int, 0>{});
     value = piece_value<DT, 0>(halves, consts(std::integral_constant<int, 0>{}));
     make_halves(std::integral_constant<int, 1>{});
-    auto step = [&](auto p_tag) {
+    auto step = [&](auto p_tag) __attribute__((always_inline)) {
       constexpr int P = decltype(p_tag)::value, w = P >> 3, J = P & 7, wn2 = (w + 1) & 3;
+      if constexpr (EARLY && KK && P == 16) store_a(buf ^ 1, NH - 1, buf ? 0 : AD - 1);
+      if constexpr (EARLY && KK && P == 24) loop_barrier();
 #pragma unroll
       for (int i = J * KQ_MB / 4; i < (J + 1) * KQ_MB / 4; ++i) {
         if constexpr (KQ_MB < 4)
           mfma_inplace_v<DT>(acc[i >> 1][w][i & 1], af[i >> 1], ob[w & 1][i & 1]);
         else
           mfma_inplace<DT>(acc[i >> 1][w][i & 1], af[i >> 1], ob[w & 1][i & 1]);
+        if constexpr (EARLY && w == 3)
+          if (i & 1) af[i >> 1] = anext[(i >> 1) * 64];
       }
       ob[wn2 & 1][J >> 2][J & 3] = piece_finish<DT, UNIT, J>(value, consts(p_tag));
       // the constants the next registers want: of `nxt` where the k-step ends a group, each as soon as the old ones have been used
@@ -300,42 +321,37 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
     };
     for_each_piece<32>(step);
   };
+  auto end_chunk = [&](int buf) {
+    if constexpr (!EARLY) {
+      store_a(buf ^ 1, NH - 1);
+      loop_barrier();
+    }
+  };
 
   // ---- main loop: two chunks (four k-steps = the weight ring) per iteration; the K parts of a workgroup run the same count,
   // but private ones, which may have one iteration more or fewer, or none.  The
   // last k-step of an iteration builds the first operands of the next 128 rows of K: the constants are rebuilt there,
   // and in the other three k-steps too when a group is shorter than 128 rows.
-  auto main_loop = [&](auto every_tag) {
-    const std::true_type refresh{};
+  const std::bool_constant<HOIST && !ONCE> every{};
+  const std::true_type refresh{};
 #pragma unroll 1
-    for (int c0 = 0; c0 < nchunks; c0 += 2) {
-      const int ks0 = 2 * c0;
-      load_a(c0 + 1, 0);
-      kstep(0, 0, st[0], st[1], every_tag);
-      if constexpr (ONCE) issue_scales(ks0 + 4);
-      issue(st[0], ks0 + 4);
-      if constexpr (NH == 2) store_a(1, 0), load_a(c0 + 1, 1);
-      kstep(0, 1, st[1], st[2], every_tag);
-      issue(st[1], ks0 + 5);
-      store_a(1, NH - 1);
-      loop_barrier();
-      load_a(c0 + 2, 0);
-      kstep(1, 0, st[2], st[3], every_tag);
-      issue(st[2], ks0 + 6);
-      if constexpr (NH == 2) store_a(0, 0), load_a(c0 + 2, 1);
-      kstep(1, 1, st[3], st[0], refresh);
-      issue(st[3], ks0 + 7);
-      store_a(0, NH - 1);
-      loop_barrier();
-    }
-  };
-  if constexpr (CHANNEL || !HOIST || PRIV) {
-    main_loop(std::false_type{});
-  } else {
-    if (p.group_shift < 2)
-      main_loop(std::true_type{});
-    else
-      main_loop(std::false_type{});
+  for (int c0 = 0; c0 < nchunks; c0 += 2) {
+    const int ks0 = 2 * c0;
+    load_a(c0 + AD, 0);
+    kstep(0, std::false_type{}, st[0], st[1], every);
+    if constexpr (ONCE) issue_scales(ks0 + 4);
+    issue(st[0], ks0 + 4);
+    if constexpr (NH == 2) store_a(1, 0), load_a(c0 + 1, 1);
+    kstep(0, std::true_type{}, st[1], st[2], every);
+    issue(st[1], ks0 + 5);
+    end_chunk(0);
+    load_a(c0 + AD + 1, 0, AD - 1);
+    kstep(1, std::false_type{}, st[2], st[3], every);
+    issue(st[2], ks0 + 6);
+    if constexpr (NH == 2) store_a(0, 0), load_a(c0 + 2, 1);
+    kstep(1, std::true_type{}, st[3], st[0], refresh);
+    issue(st[3], ks0 + 7);
+    end_chunk(1);
   }
 
   // ------------------------------------------------------------------------------ epilogue
@@ -469,6 +485,11 @@ static kq_fn pick_kq(bool zp, bool channel) {
   if (zp) return channel ? kq_kernel<DT, true, true, MB, Q, WN> : kq_kernel<DT, true, false, MB, Q, WN>;
   return channel ? kq_kernel<DT, false, true, MB, Q, WN> : kq_kernel<DT, false, false, MB, Q, WN>;
 }
+template <int DT, int MB>
+static kq_fn pick_kq_tall(bool zp, bool channel, bool short_groups) {
+  if (short_groups) return zp ? kq_kernel<DT, true, false, MB, 2, 2, true> : kq_kernel<DT, false, false, MB, 2, 2, true>;
+  return pick_kq<DT, MB, 2, 2>(zp, channel);
+}
 // (64-row tiles with zero points would spill)
 template <int DT, int MB>
 static kq_fn pick_kq_short(bool zp) {
@@ -486,10 +507,10 @@ static kq_fn pick_kq(int mb, int tn, bool zp, bool channel, bool short_groups) {
     case -3: return pick_kq<DT, 3, 8, 1>(zp, channel);
     case -4: return pick_kq<DT, 4, 8, 1>(zp, channel);
     case 4: return pick_kq<DT, 4, 4, 2>(zp, channel);
-    case 5: return pick_kq<DT, 5, 2, 2>(zp, channel);
-    case 6: return pick_kq<DT, 6, 2, 2>(zp, channel);
-    case 7: return pick_kq<DT, 7, 2, 2>(zp, channel);
-    case 8: return pick_kq<DT, 8, 2, 2>(zp, channel);
+    case 5: return pick_kq_tall<DT, 5>(zp, channel, short_groups);
+    case 6: return pick_kq_tall<DT, 6>(zp, channel, short_groups);
+    case 7: return pick_kq_tall<DT, 7>(zp, channel, short_groups);
+    case 8: return pick_kq_tall<DT, 8>(zp, channel, short_groups);
     default: return nullptr;
   }
 }
