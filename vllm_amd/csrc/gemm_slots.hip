@@ -246,12 +246,24 @@ __global__ __launch_bounds__(256, W == 2 ? 3 : 2) void slots_kernel(const KParam
     // One k-step: per word, 2 LIVE MFMAs on ob[w & 1], column half 0 first (its registers are free for the next word's half 1); between them the
     // eight registers of the following word's operands (word w + 1 of this k-step, or word 0 of the next k-step `nxt`) are made into
     // ob[(w + 1) & 1], in three dependent steps each, of which three consecutive registers are at one step each (see gemm_kq.hip).
-    auto kstep = [&](int buf, int kk, const Stage& cur, const Stage& nxt, auto refresh_tag) {
-      constexpr bool REFRESH = decltype(refresh_tag)::value;
-      const u32x4* abase = (const u32x4*)(lds + buf * (SL_ABUF / 4) + kk * SL_KSTEP) + lane;
-      u32x4 af[LIVE];
+    auto a_frags = [&](int buf, int kk) { return (const u32x4*)(lds + buf * (SL_ABUF / 4) + kk * SL_KSTEP) + lane; };
+    // EARLY: the A operands of the next k-step are read during this one's last word, each behind the last MFMA that uses its registers, and the next
+    // chunk is stored and the barrier passed before that.  Layers of 64 to 192 slots per expert 0.97 of the time; with one or two m-blocks a
+    // word is over before the reads are (1.00).
+    constexpr bool EARLY = LIVE > 2;
+    u32x4 af[LIVE];
+    if constexpr (EARLY) {
 #pragma unroll
-      for (int mb = 0; mb < LIVE; ++mb) af[mb] = abase[mb * 64];
+      for (int mb = 0; mb < LIVE; ++mb) af[mb] = a_frags(0, 0)[mb * 64];
+    }
+    // store_tag: the half chunk that the chunk's second k-step stores, 0 in its first
+    auto kstep = [&](int buf, auto store_tag, const Stage& cur, const Stage& nxt, auto refresh_tag) __attribute__((always_inline)) {
+      constexpr bool REFRESH = decltype(refresh_tag)::value, KK = decltype(store_tag)::value > 0;
+      const u32x4* anext = KK ? a_frags(buf ^ 1, 0) : a_frags(buf, 1);
+      if constexpr (!EARLY) {
+#pragma unroll
+        for (int mb = 0; mb < LIVE; ++mb) af[mb] = a_frags(buf, KK)[mb * 64];
+      }
       if constexpr (!ONCE) ccs[1] = col_const(cur, 1);
       uint32_t halves = 0;
       PieceValue<DT> value;
@@ -263,11 +275,15 @@ __global__ __launch_bounds__(256, W == 2 ? 3 : 2) void slots_kernel(const KParam
       make_halves(std::integral_constant<int, 0>{});
       value = piece_value<DT, 0>(halves, ccs[1]);
       make_halves(std::integral_constant<int, 1>{});
-      for_each_piece<8 * W>([&](auto p_tag) {
+      for_each_piece<8 * W>([&](auto p_tag) __attribute__((always_inline)) {
         constexpr int P = decltype(p_tag)::value, w = P >> 3, J = P & 7, NW = (w + 1) % W;
+        if constexpr (EARLY && KK && P == 8 * W - 12) store_a(store_tag);
+        if constexpr (EARLY && KK && P == 8 * W - 4) __syncthreads();
 #pragma unroll
-        for (int i = J * LIVE / 4; i < (J + 1) * LIVE / 4; ++i)
+        for (int i = J * LIVE / 4; i < (J + 1) * LIVE / 4; ++i) {
           mfma_inplace_v<DT>(acc[i % LIVE][w][i / LIVE], af[i % LIVE], ob[w & 1][i / LIVE]);
+          if (EARLY && w == W - 1 && i >= LIVE) af[i % LIVE] = anext[(i % LIVE) * 64];
+        }
         ob[NW & 1][J >> 2][J & 3] = piece_finish<DT, UNIT, J>(value, ccs[NW]);
         // the constants the next registers want, each as soon as the old ones have been used
         if constexpr (ONCE) {
@@ -284,29 +300,34 @@ __global__ __launch_bounds__(256, W == 2 ? 3 : 2) void slots_kernel(const KParam
       });
     };
 
+    auto end_chunk = [&](auto store_tag) {
+      if constexpr (!EARLY) {
+        store_a(store_tag);
+        __syncthreads();
+      }
+    };
+
     // ---- main loop: two chunks (four k-steps = the weight ring) per iteration
 #pragma unroll 1
     for (int c0 = 0; c0 < nchunks; c0 += 2) {
       const int ks0 = 2 * c0;
       load_a(c0, HALF_CHUNK(AD + 1));
-      kstep(0, 0, st[0], st[1], std::false_type{});
+      kstep(0, HALF_CHUNK(0), st[0], st[1], std::false_type{});
       if constexpr (ONCE) issue_scales(ks0 + 4);
       issue(st[0], ks0 + 4);
       store_a(HALF_CHUNK(2));
       load_a(c0, HALF_CHUNK(AD + 2));
-      kstep(0, 1, st[1], st[2], std::false_type{});
+      kstep(0, HALF_CHUNK(3), st[1], st[2], std::false_type{});
       issue(st[1], ks0 + 5);
-      store_a(HALF_CHUNK(3));
-      __syncthreads();
+      end_chunk(HALF_CHUNK(3));
       load_a(c0, HALF_CHUNK(AD + 3));
-      kstep(1, 0, st[2], st[3], std::false_type{});
+      kstep(1, HALF_CHUNK(0), st[2], st[3], std::false_type{});
       issue(st[2], ks0 + 6);
       store_a(HALF_CHUNK(4));
       load_a(c0, HALF_CHUNK(AD + 4));
-      kstep(1, 1, st[3], st[0], std::true_type{});
+      kstep(1, HALF_CHUNK(5), st[3], st[0], std::true_type{});
       issue(st[3], ks0 + 7);
-      store_a(HALF_CHUNK(5));
-      __syncthreads();
+      end_chunk(HALF_CHUNK(5));
     }
 #undef HALF_CHUNK
 
