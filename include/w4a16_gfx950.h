@@ -157,7 +157,8 @@ enum {
 
 /* Bytes of scratch (c_tmp) a call with these operands may use (0 = none): fp32 split-K partials, the gathered copy of A
  * (act-order), and A in two 8-bit terms (dense bf16 problems of more than 128 rows that run on the 8-bit matrix unit:
- * 2 bytes per element).  With c_tmp = NULL a call falls back to a plan without the terms and without the K splits that
+ * 2 bytes per element; with zero points and enough rows the signed weights too, K * N bytes with N rounded up to 128;
+ * MoE blocks of 128 slots: 2 bytes per slot and element).  With c_tmp = NULL a call falls back to a plan without the terms and without the K splits that
  * are only taken for speed.
  * The reference allocates the equivalent inside the op (gptq_marlin.cu:751-763). */
 int64_t w4a16_gemm_scratch_bytes(const w4a16_gemm_args* args);
@@ -171,7 +172,7 @@ int w4a16_marlin_gemm(const w4a16_gemm_args* args, void* stream);
  * tiles, the column-gathered copy of A (act-order) and the arrival counters live in a buffer of
  * W4A16_STATIC_SCRATCH_BYTES (+ 16 KiB of counters) inside the library's own device memory: resident on every GPU of
  * every process that loads the library, whether or not this entry point is ever called, until the process ends.
- * Where only A in 8-bit terms or a K split taken for speed would exceed it, the call runs on a plan without them.  A
+ * Where only signed weights, A in 8-bit terms or a K split taken for speed would exceed it, the call runs on a plan without them.  A
  * problem that needs more scratch than that all the same fails with W4A16_EINVAL and a message; nothing is launched
  * then.  The call allocates and frees nothing.  All calls on one GPU share that GPU's buffer: calls that overlap in time
  * on one GPU (two streams, two host threads) race and must be serialised by the caller.  Inputs and the output are the caller's, as in w4a16_marlin_gemm, and results are identical to those of
