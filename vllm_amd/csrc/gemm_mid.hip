@@ -1,5 +1,6 @@
 // W4A16 GEMM for gfx950 with 64-row tiles: C[M,N] = A[M,K] * dequant(Bq)[K,N] (+bias), dense (64 < M, too few
-// rows or tiles for the 128-row prefill kernel) and MoE blocks of 64 sorted token slots
+// rows or tiles for the 128-row prefill kernel) and MoE blocks of 64 sorted token slots (integer 4-bit weights only with an operand of 2 GiB or
+// more: gemm_slots.hip has the others, at 0.87 of the time)
 // (the counterpart of the reference's thread_m_blocks = 4 configurations, csrc/moe/marlin_moe_wna16/ops.cu:451-512).
 //
 //   workgroup tile 64 rows x 512 columns, 4 wavefronts, each owning 64 rows x 128 columns (one column pair):

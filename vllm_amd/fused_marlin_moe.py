@@ -80,8 +80,8 @@ def _tall_from(quant_type: ScalarType, k: int, n: int, w1_scale, w2_scale, is_k_
 def pick_block_size(tokens: int, topk: int, num_experts: int, expert_bytes: int = 1 << 30, tall_from: int = 0) -> int:
     """Token slots per expert block, from the average expert's share of the slots (the quantity the reference's rule
     uses, fused_marlin_moe.py:279-282), fitted to the kernels behind each size on MI355X: blocks of 16 slots run on the
-    weight-streaming kernel, whose cost is one pass over the expert's weights per block; blocks of 64 on the 64-row
-    kernel, which costs about two such passes per block, so it wins once an expert fills more than one and a quarter
+    weight-streaming kernel, whose cost is one pass over the expert's weights per block; blocks of 64 on 64-row
+    tiles, which cost about two such passes per block, so they win once an expert fills more than one and a quarter
     blocks of 16 (sooner for experts of a few MB, where the per-block fixed costs count).  Blocks of 8 never beat 16,
     and 32 / 48 lost their niche (few, large experts) when the 64-row kernel began to split K for a thin last round (48 was timed
     as four row blocks; on tiles of three it has not been).
