@@ -10,8 +10,11 @@
 // same weights) do what four bf16 MFMAs did, in the same 64 cycles; the step's sums are then scaled in fp32, acc = fma(s, sum, acc), so no
 // weight is rounded.  Where an outlier leaves eight neighbours of its row and step more than 13 binades below it, what the terms leave out
 // of that row is added by the 16-bit unit behind the loop ("wide" steps): otherwise a term's error is below 2^-9 of the largest of eight
-// neighbours, no more than rounding their weights to bf16 costs.  4096 x 28672 at 203 rows, 59 us: one wide step of one row 64, one feature
-// 1000 times the others 59, 10^5 times 73 (one wide step in every row), eight of them 152, one in every step 430.
+// neighbours, no more than rounding their weights to bf16 costs.  A column whose weights at the large values are zero sees the small ones alone, so
+// a step is also wide where a value loses bits and fewer than 32 of the 128 are within 13 binades of the largest (sparse rows; 2^13 with 1 and 2^-12
+// side by side: the 2^-12 was lost).  With 32 and more, only a column whose weights are zero at all of them shows the loss: 2^-23 of the
+// largest value.  (Normal activations have 120 and more there; the test costs no time that shows.)  4096 x 28672 at 203 rows, 59 us: one wide step of
+// one row 64, one feature 1000 times the others 59, 10^5 times 73 (one wide step in every row), eight of them 152, one in every step 430.
 //   Measured on the unit: subnormals are kept; lane l holds row / column l & 15 and the 32 bytes of K block l >> 4, one scale byte
 // per row serves the whole step when all four lanes of the row carry it; products of eight neighbouring bytes are added with the bits
 // below 2^-14 of the largest cut off, these sums then in fp32.  What counts as large is the sum of the two exponents, a subnormal's being
@@ -65,6 +68,8 @@ __host__ __device__ constexpr int x8_smem(int mb, int ks, int wn) {
 constexpr int X8_TABLES = 16 * 16;  // behind it, with zero points: a table for each
 
 constexpr int X8_WIDE = 13;         // binades from a step's largest value at which what the two terms leave out is added
+constexpr int X8_EXACT = 14;        // binades from it down to which the two terms leave nothing out
+constexpr int X8_FEW = 32;          // and it is added, too, where fewer values than this are within X8_WIDE
 
 // prepared weights of one step: 8 KB for each unit, two units for every column pair (whose second n-tile may be missing)
 __host__ __device__ constexpr int64_t x8_weight_step(int64_t n) { return (n + 127) / 128 * 16384; }
@@ -148,7 +153,22 @@ __device__ __forceinline__ void x8_split(const uint16_t* a, int64_t lda, int row
     }
     // wide step: eight neighbours below 2^-X8_WIDE of the row's largest value (not zeros: those are exact), see x8_rest
     const bool wide = mine != 0 && (int)mine < (int)m - (X8_WIDE << 7);
-    if (__ballot(wide) >> (lane & 12) & 0x000f000f000f000full) flags |= 4u;
+    const uint64_t row_lanes = 0x000f000f000f000full << (lane & 12);
+    if (__ballot(wide) & row_lanes) flags |= 4u;
+    // ... or a value that loses bits in a step with few large ones: a column whose weights at those are zero has nothing else to show
+    u16x2 least = {0xffff, 0xffff};  // of the lane's magnitudes that are not zero, less one
+#pragma unroll
+    for (int i = 0; i < 4; ++i) least = __builtin_elementwise_min(least, __builtin_bit_cast(u16x2, x[i] & 0x7fff7fffu) - u16x2{1, 1});
+    const uint64_t lossy = __ballot((int)min((uint32_t)least.x, (uint32_t)least.y) + 1 < ((int)(m >> 7) - X8_EXACT) << 7);
+    if (lossy) {
+      int large = 0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int mag = (int)(x[i >> 1] >> (16 * (i & 1)) & 0x7fffu);
+        large += __popcll(__ballot(mag >= (int)m - (X8_WIDE << 7)) & row_lanes);
+      }
+      if (large < X8_FEW && (lossy & row_lanes)) flags |= 4u;
+    }
     const int e = max((int)(m >> 7) - 134, -122);  // |a| * 2^-e < 256
     const float inv = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);
     uint32_t hi01 = 0, hi23 = 0, lo01 = 0, lo23 = 0;
