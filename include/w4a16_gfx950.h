@@ -149,17 +149,21 @@ enum {
                                    c is [size_m * top_k, d] and receives silu(gate) * up, rounded exactly as
                                    silu_and_mul does on the rounded GEMM result (each of gate, up, silu, product
                                    rounded once to the activation type) */
-  W4A16_F_SUM_TOPK = 128        /* MoE only: c is [size_m / sum_top_k, size_n], zero on entry (zero_fill of an earlier
+  W4A16_F_SUM_TOPK = 128,       /* MoE only: c is [size_m / sum_top_k, size_n], zero on entry (zero_fill of an earlier
                                    launch on the same stream can do that); every result row i, rounded to the
                                    activation type, is added to c[i / sum_top_k] with packed 16-bit atomic adds.
                                    sum_top_k <= 2 (a sum of two rounded terms does not depend on their order) */
+  W4A16_F_LESS_SCRATCH = 256    /* plan as if there were no scratch but for what the problem cannot do without: no 8-bit terms or
+                                   prepared weights, no K splits taken for speed; w4a16_gemm_scratch_bytes answers for that plan.
+                                   For callers whose allocation of the larger one failed */
 };
 
 /* Bytes of scratch (c_tmp) a call with these operands may use (0 = none): fp32 split-K partials, the gathered copy of A
  * (act-order), and A in two 8-bit terms (dense bf16 problems of more than 128 rows that run on the 8-bit matrix unit:
- * 2 bytes per element; with zero points and enough rows the signed weights too, K * N bytes with N rounded up to 128;
- * MoE blocks of 128 slots: 2 bytes per slot and element).  With c_tmp = NULL a call falls back to a plan without the terms and without the K splits that
- * are only taken for speed.
+ * 2 bytes per element; with zero points and enough rows the signed weights too, K * N bytes with N rounded up to 128, at most
+ * 512 MiB; MoE blocks of 128 slots: 2 bytes per slot and element, at most 512 MiB).  Problems that would need more run on the
+ * 16-bit unit or without prepared weights.  With c_tmp = NULL, or with W4A16_F_LESS_SCRATCH, a call falls back to a plan without
+ * the terms and without the K splits that are only taken for speed.
  * The reference allocates the equivalent inside the op (gptq_marlin.cu:751-763). */
 int64_t w4a16_gemm_scratch_bytes(const w4a16_gemm_args* args);
 

@@ -28,8 +28,8 @@ def plan(tmp_path_factory):
                    check=True, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
     probe = ctypes.CDLL(out).plan_probe
 
-    def call(m, k, n, dtype, fmt, group, act_order=False, more_scratch=True, moe_slots=0):
-        """`dtype`: a torch dtype; operands are never read.  moe_slots: MoE blocks of 64 and so many sorted slots."""
+    def call(m, k, n, dtype, fmt, group, act_order=False, more_scratch=True, moe_slots=0, moe_block=64):
+        """`dtype`: a torch dtype; operands are never read.  moe_slots: MoE blocks of `moe_block` and so many sorted slots."""
         a = _lib.GemmArgs()
         a.struct_size = ctypes.sizeof(_lib.GemmArgs)
         a.dtype = _lib.DTYPE_BF16 if dtype == torch.bfloat16 else _lib.DTYPE_F16
@@ -44,7 +44,7 @@ def plan(tmp_path_factory):
         a.size_m, a.size_n, a.size_k, a.num_groups = m, n, k, 1 if group == -1 else k // group
         if moe_slots:
             a.flags |= _lib.F_MOE
-            a.lda, a.moe_block_size, a.top_k, a.n_sorted = k, 64, 1, moe_slots
+            a.lda, a.moe_block_size, a.top_k, a.n_sorted = k, moe_block, 1, moe_slots
             a.sorted_token_ids = a.expert_ids = a.num_tokens_past_padded = 4096
         a.workspace_len = 1024  # what marlin_make_workspace_new makes on this GPU
         res = (ctypes.c_int32 * len(FIELDS))()
@@ -160,3 +160,14 @@ def test_moe_blocks_of_64(plan):
     assert plan(rows, 4096, 512, torch.bfloat16, "uint4", 128, moe_slots=rows)["kind"] == 3
     # act-order: the gathered rows, one for each slot, are what the kernel reads
     assert plan(rows - 1, 4096, 512, torch.bfloat16, "uint4b8", 128, act_order=True, moe_slots=rows)["kind"] == 3
+
+
+def test_extra_scratch_has_a_bound(plan):
+    """Prepared weights and the terms of MoE rows take 512 MiB at most; problems beyond that run without them."""
+    import torch
+    assert plan(4096, 8192, 65536, torch.bfloat16, "uint4", 128)["kind"] == 7
+    assert plan(4096, 8192, 65536 + 64, torch.bfloat16, "uint4", 128)["kind"] != 7
+    slots = 504 * 128                       # rows of 4096 x 2 bytes and 32 scale words
+    assert plan(4096, 4096, 2048, torch.bfloat16, "uint4b8", 128, moe_slots=slots, moe_block=128)["kind"] == 9
+    assert plan(4096, 4096, 2048, torch.bfloat16, "uint4b8", 128, moe_slots=slots + 1, moe_block=128)["kind"] == 2
+    assert plan(4096, 4096, 2048, torch.bfloat16, "uint4b8", 128, more_scratch=False, moe_slots=8192, moe_block=128)["kind"] == 2

@@ -15,7 +15,7 @@ WTYPE_U4B8, WTYPE_U4, WTYPE_U8B128, WTYPE_FE4M3, WTYPE_FE2M1 = 0, 1, 2, 3, 4
 DTYPE_F16, DTYPE_BF16, DTYPE_F32 = 0, 1, 2
 ABI_VERSION = 3  # W4A16_ABI_VERSION of include/w4a16_gfx950.h this mirror was written against
 F_IS_K_FULL, F_USE_ATOMIC_ADD, F_USE_FP32_REDUCE, F_MUL_TOPK_WEIGHTS, F_MOE, F_ZP_FLOAT = 1, 2, 4, 8, 16, 32
-F_SILU_AND_MUL, F_SUM_TOPK = 64, 128
+F_SILU_AND_MUL, F_SUM_TOPK, F_LESS_SCRATCH = 64, 128, 256
 
 c_void_p, c_i64, c_i32, c_u32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_uint32
 

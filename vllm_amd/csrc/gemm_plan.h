@@ -41,6 +41,9 @@ int launch_skinny(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_decode(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_fat(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_mid(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
+// What a plan may ask for beyond partial tiles and copies of A that other plans need too: prepared weights, and the terms of MoE rows (two bytes for
+// each slot and element, where the 16-bit kernels read A in place).  8 experts of 4096 x 14336, top-2, 4096 tokens: 251 MiB; 8192 x 57344: 448.
+constexpr int64_t X8_EXTRA_MAX = 512LL << 20;
 int64_t x8_scratch_bytes(int64_t rows, int64_t k);
 int64_t x8_weight_bytes(int64_t k, int64_t n);
 int64_t x8_moe_scratch_bytes(int64_t n_sorted, int64_t k);

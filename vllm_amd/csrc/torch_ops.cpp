@@ -160,16 +160,23 @@ Tensor permute_cols(const Tensor& A, const Tensor& perm) {
 }
 
 // -------------------------------------------------------------------------------------------------------- GEMM
-// Scratch comes from torch's caching allocator: stream-ordered reuse, given back when `tmp` goes.
+// Scratch comes from torch's caching allocator: stream-ordered reuse, given back when `tmp` goes.  Where the GPU has no room for what the fastest
+// plan asks for, the call runs on the one that needs least.
 void run_gemm(w4a16_gemm_args& args, const Tensor& a) {
   OnDevice on(a);
-  const int64_t need = w4a16_gemm_scratch_bytes(&args);
-  if (need < 0) check_rc((int)need);
+  auto scratch = [&]() {
+    const int64_t need = w4a16_gemm_scratch_bytes(&args);
+    if (need < 0) check_rc((int)need);
+    return need > 0 ? at::empty({need / 4}, a.options().dtype(at::kFloat)) : Tensor();
+  };
   Tensor tmp;
-  if (need > 0) {
-    tmp = at::empty({need / 4}, a.options().dtype(at::kFloat));
-    args.c_tmp = (float*)tmp.mutable_data_ptr();
+  try {
+    tmp = scratch();
+  } catch (const c10::OutOfMemoryError&) {
+    args.flags |= W4A16_F_LESS_SCRATCH;
+    tmp = scratch();
   }
+  if (tmp.defined()) args.c_tmp = (float*)tmp.mutable_data_ptr();
   check_rc(w4a16_marlin_gemm(&args, stream_of(a)));
 }
 
