@@ -1,4 +1,4 @@
-"""64-row tiles (gemm_mid.hip): dequantisation constants made once per 128 rows of K (groups of 128 rows and more, one scale per column) and with
+"""64-row tiles (dense: gemm_mid.hip; MoE: gemm_slots.hip, and gemm_mid.hip in test_gpu_moe_beyond_limits.py): dequantisation constants made once per 128 rows of K (groups of 128 rows and more, one scale per column) and with
 every k-step (shorter groups).  A row of A with a single one picks one row of the weights: the result is that row, bit for bit, for every
 group boundary, word position and half of a column tile."""
 import pytest

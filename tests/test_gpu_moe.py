@@ -170,7 +170,7 @@ def test_moe_gemm_equals_oracle(dev, m, topk, e, bs, variant, mul):
 
 
 def test_moe_gemm_split_k_blocks_of_64(dev):
-    """Enough rows for blocks of 64 but fewer than 256 tiles: the 64-row kernel splits K and runs its reduction pass."""
+    """Enough rows for blocks of 64 but fewer tiles than workgroups, K = 2048: tiles of 256 columns, none of them cut along K (gemm_slots.hip)."""
     import vllm_amd.ops as ops
     from vllm_amd.marlin_utils import marlin_make_workspace_new
     from vllm_amd.moe_align_block_size import moe_align_block_size
@@ -198,10 +198,10 @@ def test_moe_gemm_split_k_blocks_of_64(dev):
 
 @pytest.mark.parametrize("m,foreign", [(300, False), (300, True), (1200, False), (8300, False)])
 def test_moe_gemm_tail_tiles_split_on_the_device(dev, m, foreign):
-    """Blocks of 64 with a long K: the 64-row kernel cuts the tiles of its last, partly filled round of resident
-    workgroups along K, by a number of pieces it derives from the live block count on the device, and a second pass adds
-    the pieces.  24 live tiles -> 4 pieces each; 80 -> 4; about 520 -> 512 whole tiles and a few split ones; with blocks
-    of experts held by another rank (left untouched) among them."""
+    """Blocks of 64 with a long K: the tiles of the last, partly filled round of resident workgroups (three to a compute unit
+    with tiles of 256 columns, gemm_slots.hip) are cut along K, by a number of pieces derived from the live block count on
+    the device, and a second pass adds the pieces.  About 48 and 160 live tiles -> 4 pieces each; about 1050 -> 768 whole
+    tiles and the others in two; with blocks of experts held by another rank (left untouched) among them."""
     import vllm_amd.ops as ops
     from vllm_amd.marlin_utils import marlin_make_workspace_new
     from vllm_amd.moe_align_block_size import moe_align_block_size

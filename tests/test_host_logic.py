@@ -228,3 +228,22 @@ def test_moe_blocks_of_128_by_weight_type():
     assert tall_from(st.uint4b8, bf16, 96, k=4608, n=4608) == 0
     assert pick_block_size(768, 2, 8, tall_from=192) == 128 and pick_block_size(767, 2, 8, tall_from=192) == 64
     assert pick_block_size(4096, 2, 8, tall_from=0) == 64
+
+
+def test_moe_blocks_of_128_with_a_short_k():
+    """Below a K of 4096 only what the 8-bit unit takes, bf16 uint4b8 with groups of whole 128 rows, from k = 3072, n = 2048 and 4096 * 2048 weights on."""
+    import torch
+    from vllm_amd.fused_marlin_moe import _tall_from
+    from vllm_amd.scalar_type import scalar_types as st
+
+    def tall_from(k, n, wtype=st.uint4b8, dtype=torch.bfloat16, group=128):
+        scale = lambda kk: torch.empty(1, 1 if group == -1 else kk // group, 1, dtype=dtype)  # noqa: E731
+        return _tall_from(wtype, k, n, scale(k), scale(n), True)
+
+    for k, n in [(4096, 2048), (3584, 2560), (7168, 2048), (3072, 2816), (3072, 14336)]:
+        assert tall_from(k, n) == tall_from(k, n, group=256) == 192 and tall_from(k, n, group=-1) == 384
+        for group in (32, 64):
+            assert tall_from(k, n, group=group) == 0
+        assert tall_from(k, n, dtype=torch.float16) == tall_from(k, n, st.uint4) == tall_from(k, n, st.uint4, torch.float16) == 0
+    for k, n in [(3072, 2048), (3072, 2688), (4096, 1920), (2944, 8192), (2048, 8192)]:
+        assert tall_from(k, n) == 0

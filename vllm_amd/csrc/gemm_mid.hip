@@ -14,8 +14,8 @@
 //                128 rows and more come once per loop iteration (128 K rows) and the constants made of them stay in registers
 //                (mid_once_kernel); and a register's three dependent steps stand between three MFMAs (see gemm_kq.hip).  Other VALU
 //                instructions per MFMA, before and now: bf16 with zero points 6.2 -> 4.65 (groups of 32 and 64: 5.5), uint4b8 5.35 -> 4.55,
-//                fp16 3.4 -> 3.4, and 120 wait instructions fewer per iteration.  128 experts of 2048 x 768, top-8, 601 tokens, bf16 AWQ:
-//                GEMM1 90 -> 77.5 us, GEMM2 44 -> 39.7.  Dense, 300 to 512 rows, weights not cached: 0.98 of the time in the mean.
+//                fp16 3.4 -> 3.4, and 120 wait instructions fewer per iteration.  Dense, 300 to 512 rows, weights not
+//                cached: 0.98 of the time in the mean.
 //   activations  the workgroup stages 64 rows x 64 K (two k-steps) into LDS, double buffered, in MFMA fragment
 //                order (one conflict-free ds_read_b128 per operand); MoE rows are gathered through sorted_token_ids
 //                while staging.  One barrier per two k-steps.
