@@ -42,25 +42,30 @@ def _tall_from(quant_type: ScalarType, k: int, n: int, w1_scale, w2_scale, is_k_
     """Slots per expert from which blocks of 128 slots (the prefill kernel) should run both GEMMs [., k] x [k, 2n] and
     [., n] x [n, k]; 0: never.  The kernel takes integer 4-bit weights, whole power-of-two groups, K a multiple of 128.  It
     dequantises every weight once per 128 rows instead of once per 64, but keeps one workgroup per compute unit, so every tile
-    pays for its start and its epilogue.  Time over that with blocks of 64, 8-32 experts of 4096 x 4096 to 6144 x 10752:
+    pays for its start and its epilogue.  Time of whole layers over that with blocks of 64, run back to back, 8 experts of 4096 x 14336, 16 of
+    6144 x 10752, 5120 x 8192 and 4096 x 4096, even and skewed routing (range, mean):
 
-                                      192-256 slots  384-1024 slots
-      bf16 or zero points, group 128    0.84 - 1.03    0.83 - 1.02    from 192
-      bf16, channel-wise                0.88 - 0.99    0.84 - 0.96    from 192
-      fp16 zero points, channel-wise    0.96 - 1.02    0.92 - 1.05    from 384 (mean 0.99 / 0.97)
-      bf16 or zero points, group 32/64  0.95 - 1.07    0.90 - 1.07    from 384 (mean 1.02 / 0.97)
-      fp16 uint4b8, group 128           0.95 - 1.07    0.95 - 1.07    from 384 (mean 1.02 / 0.99)
-        with k * n >= 4096 * 8192       0.95 - 1.02    0.93 - 0.98    from 192
-      fp16 uint4b8, others              1.02 - 1.11    0.93 - 1.12    never (mean 1.05 / 1.01): the cheapest dequantisation
+                                      192-256 slots      384-768 slots
+      bf16 uint4b8, group 128         0.91 - 1.14  0.98  0.87 - 1.02  0.93   from 192 (8-bit matrix unit)
+      bf16 uint4b8, channel-wise      0.93 - 1.17  1.01  0.90 - 1.06  0.96   from 192 (8-bit matrix unit)
+      bf16 uint4b8, group 32          0.92 - 1.18  1.00  0.89 - 1.04  0.94   from 384
+      bf16 zero points, group 128     0.95 - 1.20  1.03  0.91 - 1.06  0.96   from 192
+      bf16 zero points, channel-wise  0.97 - 1.25  1.06  0.92 - 1.11  0.99   from 192
+      fp16 zero points, group 128     0.96 - 1.17  1.05  0.94 - 1.04  0.99   from 192
+      fp16 zero points, group 32      0.95 - 1.14  1.02  0.92 - 1.03  0.97   from 384
+      fp16 zero points, channel-wise  1.01 - 1.23  1.10  1.01 - 1.10  1.05   from 384
+      fp16 uint4b8, group 128         0.98 - 1.20  1.07  0.96 - 1.07  1.01   from 384, with k * n >= 4096 * 8192 from 192
+      fp16 uint4b8, others            0.97 - 1.22  1.08  0.96 - 1.10  1.03   never: the cheapest dequantisation
 
-    bf16 uint4b8 with groups of whole 128 rows or one scale per column runs blocks of 128 on the 8-bit matrix unit (gemm_x8.hip), which takes
-    0.90 - 1.00 of the prefill kernel's time (nine expert shapes of 2048 x 1408 to 6144 x 10752, 96 to 1024 slots; 1.04 at most), and against
-    blocks of 64 0.83 - 1.00 from 192 slots with both K >= 4096, 0.86 - 0.99 with 4096 x 2048, 3584 x 2560 and 7168 x 2048 (channel-wise
-    0.92 - 1.02 from 384), 0.95 - 1.02 with 2048 x 8192 and 1.06 - 1.13 with 2048 x 1408.  So its line is at k >= 3072, n >= 2048, k * n >=
-    4096 * 2048.
+    The lines were drawn against blocks of 64 on the 512-column tiles of gemm_mid.hip; gemm_slots.hip, which has them now, takes 0.87 of that time, so
+    that at 192 to 256 slots only bf16 uint4b8 still gains.
 
-    The spread inside a row is how the tiles fill their last round.  With a K below 4096 the sides cross: 64 experts of 2048 x 1408
-    1.02 - 1.17, 32 of 4096 x 2048 0.94 - 1.05, while bf16 gains on 16 of 2048 x 8192 and 64 of 7168 x 2048 (0.89 - 0.94)."""
+    bf16 uint4b8 with groups of whole 128 rows or one scale per column runs blocks of 128 on the 8-bit matrix unit (gemm_x8.hip), whose results are the
+    closer ones (weights unrounded).  With a K below 4096, 192 / 256 / 384 / 768 slots, group 128: 64 experts of 7168 x 2048 1.03 / 0.99 / 0.99 / 0.94,
+    64 of 3584 x 2560 1.04 / 1.03 / 1.01 / 0.98, 32 of 3072 x 3072 1.06 / 1.03 / 1.04 / 0.96, 32 of 4096 x 2048 1.08 / 1.10 / 1.03 / 1.00; 8 of 2048 x 8192
+    1.07 / 1.01 / 1.07 / 1.01 and 64 of 2048 x 1408 1.21 / 1.20 / 1.18 / 1.07 are left out: its line is at k >= 3072, n >= 2048, k * n >= 4096 * 2048.
+
+    The spread inside a row is how the tiles fill their last round."""
     if quant_type not in (scalar_types.uint4, scalar_types.uint4b8) or not is_k_full or k < 3072 or n < 2048 or k % 128 or n % 128:
         return 0
     rows = []  # K rows per scale row
@@ -79,10 +84,12 @@ def _tall_from(quant_type: ScalarType, k: int, n: int, w1_scale, w2_scale, is_k_
 
 def pick_block_size(tokens: int, topk: int, num_experts: int, expert_bytes: int = 1 << 30, tall_from: int = 0) -> int:
     """Token slots per expert block, from the average expert's share of the slots (the quantity the reference's rule
-    uses, fused_marlin_moe.py:279-282), fitted to the kernels behind each size on MI355X: blocks of 16 slots run on the
-    weight-streaming kernel, whose cost is one pass over the expert's weights per block; blocks of 64 on 64-row
-    tiles, which cost about two such passes per block, so they win once an expert fills more than one and a quarter
-    blocks of 16 (sooner for experts of a few MB, where the per-block fixed costs count).  Blocks of 8 never beat 16,
+    uses, fused_marlin_moe.py:279-282): blocks of 16 slots run on the weight-streaming kernel, whose cost is one pass over the expert's
+    weights per block and which multiplies unrounded weights (groups of 64 rows and more); blocks of 64 on 64-row tiles, which cost about two such passes per
+    block when the line was drawn, one and a quarter blocks of 16 per expert (sooner for experts of a few MB, where the per-block fixed costs
+    count).  With gemm_slots.hip they cost less: time on blocks of 16 over 64, whole layers of 12 expert shapes, at 10 / 14 / 18 / 20 slots per expert
+    0.9 / 1.0 / 1.15 / 1.2 (128 experts of 2048 x 768 1.06 / 1.17 / 1.31 / 1.30, 16 of 1024 x 2048 0.72 - 0.77), by type from 0.95 (bf16, group 128) to 1.10 (bf16, group 32) at 14.
+    The line stays: moving it down would round the weights of calls that have them exact.  Blocks of 8 never beat 16,
     and 32 / 48 lost their niche (few, large experts) when the 64-row kernel began to split K for a thin last round (48 was timed
     as four row blocks; on tiles of three it has not been).
     tall_from: blocks of 128 from so many slots per expert (see _tall_from); 0: never."""
