@@ -72,12 +72,12 @@ def test_dense(dev, fmt, k, n, m):
 def test_moe_blocks_of_128(dev):
     import vllm_amd.ops as ops
     from vllm_amd.scalar_type import scalar_types
-    moe = Moe(dev, 8192, 3136, [9000, 40, 3000], 128)
+    moe = Moe(dev, 8192, 192, [9000, 40, 3000], 128)
     a = torch.randn(moe.tokens, moe.k, generator=torch.Generator(device=dev).manual_seed(5), device=dev).bfloat16()
     full = moe.gemm(a)
     s, x, t = moe.routing
     c = torch.full_like(full, 7)
-    with Limit(100 << 20):  # (the tail tiles' pieces take 64)
+    with Limit(100 << 20):  # (the tail tiles' pieces take 48)
         ops.moe_wna16_marlin_gemm(a, c, moe.w, None, moe.s, None, None, moe.g_idx, moe.perm, moe.workspace, s, x, t, moe.weights, moe_block_size=128,
                                   top_k=1, mul_topk_weights=True, is_ep=False, b_q_type=scalar_types.uint4b8, size_m=moe.tokens, size_n=moe.n,
                                   size_k=moe.k, is_k_full=True, use_atomic_add=False, use_fp32_reduce=True, is_zp_float=False)

@@ -62,11 +62,11 @@ class Moe:
 
 CASES = [
     # k, n, tokens of each expert, group, foreign, act-order
-    (256, 3136, [1], 128, False, False),                                # one live row block
-    (4096, 3072, [300, 40, 0, 129, 127, 128], 128, True, False),        # all tiles cut along K
-    (2048, 3136, [700, 5, 333], 256, False, False),
+    (256, 192, [1], 128, False, False),                                 # one live tile
+    (4096, 1024, [300, 40, 0, 129, 127, 128], 128, True, False),        # all tiles cut along K
+    (2048, 576, [700, 5, 333], 256, False, False),
     (1024, 4160, [128, 1, 260], -1, False, False),                      # last strip one n-tile
-    (512, 3200, [150, 33], 128, False, True),
+    (512, 640, [150, 33], 128, False, True),
     (1024, 16448, [1100, 130, 17, 250], 128, False, False),             # whole tiles in front of cut ones
     (1024, 33344, [300, 1000, 20, 13], -1, False, False),               # more row blocks than a chunk of the tile order
 ]
@@ -130,7 +130,7 @@ def test_fused_layer_equals_separate_launches(dev, monkeypatch, tokens, group, s
     import vllm_amd.fused_marlin_moe as fm
     from vllm_amd.scalar_type import scalar_types
     monkeypatch.setattr(fm, "pick_block_size", lambda *a, **kw: 128)
-    e, hidden, inter, topk = 4, 3072, 1536, 2
+    e, hidden, inter, topk = 4, 512, 384, 2
     w = [[_layer(k, n, "uint4b8", group, dev, seed=10 * j + i) for i in range(e)] for j, (k, n) in enumerate(((hidden, 2 * inter), (inter, hidden)))]
     w1, s1, w2, s2 = (torch.stack([layer[j] for layer in x]) for x in w for j in (0, 1))
     g = torch.Generator(device=dev).manual_seed(3)

@@ -58,7 +58,7 @@ def test_prepared_weights(dev, workspace, k, n, m):
 
 @pytest.mark.parametrize("group", [128, -1])
 def test_moe_blocks_of_128(dev, group):
-    moe = Moe(dev, 1024, 3136, [300, 40, 0, 129, 127, 128], group)
+    moe = Moe(dev, 1024, 576, [300, 40, 0, 129, 127, 128], group)
     a = _rows(moe.tokens, moe.k, dev)
     out = moe.gemm(a, False)
     for e in range(moe.e):

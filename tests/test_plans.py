@@ -168,23 +168,21 @@ def test_extra_scratch_has_a_bound(plan):
     assert plan(4096, 8192, 65536, torch.bfloat16, "uint4", 128)["kind"] == 7
     assert plan(4096, 8192, 65536 + 64, torch.bfloat16, "uint4", 128)["kind"] != 7
     slots = 504 * 128                       # rows of 4096 x 2 bytes and 32 scale words
-    assert plan(4096, 4096, 3072, torch.bfloat16, "uint4b8", 128, moe_slots=slots, moe_block=128)["kind"] == 9
-    assert plan(4096, 4096, 3072, torch.bfloat16, "uint4b8", 128, moe_slots=slots + 1, moe_block=128)["kind"] == 2
-    assert plan(4096, 4096, 3072, torch.bfloat16, "uint4b8", 128, more_scratch=False, moe_slots=8192, moe_block=128)["kind"] == 2
+    assert plan(4096, 4096, 2048, torch.bfloat16, "uint4b8", 128, moe_slots=slots, moe_block=128)["kind"] == 9
+    assert plan(4096, 4096, 2048, torch.bfloat16, "uint4b8", 128, moe_slots=slots + 1, moe_block=128)["kind"] == 2
+    assert plan(4096, 4096, 2048, torch.bfloat16, "uint4b8", 128, more_scratch=False, moe_slots=8192, moe_block=128)["kind"] == 2
 
 
 def test_moe_blocks_of_128(plan):
-    """bf16 uint4b8 with groups of whole 128 rows or one scale per column and 3072 columns runs on the 8-bit unit, everything else on the prefill
-    kernel."""
+    """bf16 uint4b8 with groups of whole 128 rows or one scale per column runs on the 8-bit unit, everything else on the prefill kernel."""
     import torch
     for dtype in (torch.float16, torch.bfloat16):
         for fmt in ("uint4", "uint4b8"):
             for group in (32, 64, 128, 256, -1):
-                for slots, k, n in [(128, 256, 3072), (9208, 4096, 28672), (9208, 14336, 4096)]:
+                for slots, k, n in [(128, 256, 64), (9208, 4096, 28672), (9208, 14336, 4096)]:
                     x8 = dtype == torch.bfloat16 and fmt == "uint4b8" and group not in (32, 64)
                     assert plan(128, k, n, dtype, fmt, group, moe_slots=slots, moe_block=128)["kind"] == (9 if x8 else 2), (dtype, fmt, group, k)
-    assert plan(128, 4096, 3072, torch.bfloat16, "uint4b8", 128, act_order=True, moe_slots=9208, moe_block=128)["kind"] == 9
-    assert plan(128, 4096, 3008, torch.bfloat16, "uint4b8", 128, moe_slots=9208, moe_block=128)["kind"] == 2
+    assert plan(128, 4096, 4096, torch.bfloat16, "uint4b8", 128, act_order=True, moe_slots=9208, moe_block=128)["kind"] == 9
     assert plan(128, 65536, 65536 - 64, torch.bfloat16, "uint4b8", 128, moe_slots=128, moe_block=128)["kind"] == 9
     assert plan(128, 65536, 65536, torch.bfloat16, "uint4b8", 128, moe_slots=128, moe_block=128)["kind"] == 2  # 2 GiB of an expert's weights
 
@@ -199,13 +197,5 @@ def test_moe_beyond_limits(plan):
                 assert plan(m, k, bl.N, dtype, fmt, group, moe_slots=990)["kind"] == 3
     k, ids = bl.LONG_IDS
     for group in (128, 256, -1):
-        for slots in (990, ids):
-            assert plan(1000, k, bl.N, torch.bfloat16, "uint4b8", group, moe_slots=slots, moe_block=128)["kind"] == 2
-
-
-def test_shapes_of_the_8_bit_unit_on_moe(plan):
-    """Every case of test_gpu_x8_moe.py runs there."""
-    import test_gpu_x8_moe as xm
-    import torch
-    for k, n, counts, group, _, act in xm.CASES:
-        assert plan(sum(counts), k, n, torch.bfloat16, "uint4b8", group, act_order=act, moe_slots=sum(counts) + 127 * len(counts), moe_block=128)["kind"] == 9
+        assert plan(1000, k, bl.N, torch.bfloat16, "uint4b8", group, moe_slots=ids, moe_block=128)["kind"] == 2
+        assert plan(1000, k, bl.N, torch.bfloat16, "uint4b8", group, moe_slots=ids - 128, moe_block=128)["kind"] == 9
