@@ -675,7 +675,7 @@ def main():
             "bound": "mfma", "achieved": pf_flops / pf_sec / 1e12, "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": pf_flops / pf_sec / 1e12 / MFMA_PEAK_TFLOPS, "traffic": None,
             "kernel": "w4a16::fat_kernel<bf16, zero points, grouped> (qkv also runs its last 512-column strips on "
-                      "w4a16::kq_kernel, gate_up runs on w4a16::x8_kernel)", "launches": sum(v["launches_timed"] for v in pf.values()),
+                      "w4a16::kq_kernel, gate_up runs on w4a16::x8_prepared_kernel)", "launches": sum(v["launches_timed"] for v in pf.values()),
             "flops_per_launch_avg": pf_flops / 4, "avg_launch_us": pf_sec / 4 * 1e6,
             "workload": "llama3-8b linears at M=4096, bf16, AWQ uint4 + uint4 zero points g128 (qkv, o, gate_up, down), "
                         "time-weighted over the four layers",

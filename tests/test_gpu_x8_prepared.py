@@ -10,8 +10,9 @@ from test_gpu_x8 import _c_args, _layer, _rel, _run
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(512, 28672, 3500), (256, 20544, 4090), (384, 16448, 3060)]  # (K, N, M); the last strips of the latter two are one n-tile
-WEIGHTS = [(128, s) for s in SHAPES] + [(256, SHAPES[0]), (-1, SHAPES[0]), (-1, SHAPES[1])]
+SHAPES = [(512, 28672, 2040), (256, 8256, 4000), (384, 16448, 2010)]  # (K, N, M); the last strips of the latter two are one n-tile
+PINNED = [(512, 28672, 3500), (256, 20544, 4090), (384, 16448, 3060)]  # the same, with prepared weights (test_plans.py); those above run without
+WEIGHTS = [(g, shapes[i]) for shapes in (SHAPES, PINNED) for g, i in ((128, 0), (128, 1), (128, 2), (256, 0), (-1, 0), (-1, 1))]
 OVER_STATIC = (512, 131072, 2040)  # whose prepared weights exceed the static entry point's buffer
 
 

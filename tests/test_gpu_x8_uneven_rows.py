@@ -7,7 +7,7 @@ import torch
 
 from test_gpu_x8 import LARGE, SPLIT, _layer, _run
 from test_gpu_x8_moe import Moe
-from test_gpu_x8_prepared import SHAPES as PREPARED
+from test_gpu_x8_prepared import PINNED as PREPARED
 
 pytestmark = pytest.mark.gpu
 

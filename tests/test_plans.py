@@ -129,10 +129,10 @@ def test_64_row_kernel_of_the_constants_test(plan):
 
 
 def test_prepared_weights(plan):
-    """The shapes of test_gpu_x8_prepared.py have their weights prepared; without room for them they run on other kernels."""
+    """The pinned shapes of test_gpu_x8_prepared.py have their weights prepared; without room for them they run on other kernels."""
     import test_gpu_x8_prepared as xp
     import torch
-    for (k, n, m), group in [(s, g) for g, s in xp.WEIGHTS] + [(xp.OVER_STATIC, 128)]:
+    for (k, n, m), group in [(s, g) for g, s in xp.WEIGHTS if s in xp.PINNED] + [(xp.OVER_STATIC, 128)]:
         p = plan(m, k, n, torch.bfloat16, "uint4", group)
         assert (p["kind"], p["ks"], p["mb"], p["tn"], p["splits"]) == (7, 1, 8, 512, 1), (k, n, m, group, p)
         assert plan(m, k, n, torch.bfloat16, "uint4", group, more_scratch=False)["kind"] != 7
