@@ -332,7 +332,10 @@ __global__ __launch_bounds__(DNW * 64, 2) void decode_kernel(const uint32_t* eB,
   if (nst >= DD) {
 #pragma unroll
     for (int j = 0; j < DD; ++j) issue(st[j], w_b + j);
+    Pace pace;
+    if constexpr (!MOE) pace.start(nst);
     for (; done + 2 * DD <= nst; done += DD) {
+      if constexpr (!MOE) pace.round(done);
 #pragma unroll
       for (int j = 0; j < DD; ++j) {
         consume(st[j]);
@@ -346,6 +349,7 @@ __global__ __launch_bounds__(DNW * 64, 2) void decode_kernel(const uint32_t* eB,
     for (int j = 0; j < DD; ++j)
       if (j < nst) issue(st[j], w_b + j);
   }
+  if constexpr (!MOE) __builtin_amdgcn_s_setprio(0);
 #pragma unroll 1
   for (; done < nst; done += DD) {
 #pragma unroll

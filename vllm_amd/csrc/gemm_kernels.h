@@ -31,6 +31,7 @@ struct KParams {
   int xcd_map;
   int tn;        // tile width in columns (128, or 64 for the narrow decode tiles)
   int strip0;    // 64-row kernel / K-split kernel: first 512- / 256-column strip of this launch (it may finish what the prefill kernel left)
+  int resident;  // MoE blocks of 64 slots: workgroups that run at a time
   int dyn_slots; // 64-row kernel, MoE: > 0 = the K split is chosen on the device from the number of live blocks (tail_split)
   // MoE
   const int32_t* sorted_ids;
@@ -269,6 +270,7 @@ inline KParams make_kparams(const w4a16_gemm_args* a, const Plan& pl) {
   p.tn = pl.tn;
   p.strip0 = pl.strip0;
   p.dyn_slots = pl.dyn_slots;
+  p.resident = pl.resident;
   p.sorted_ids = a->sorted_token_ids;
   p.expert_ids = a->expert_ids;
   p.ntpp = a->num_tokens_past_padded;
@@ -323,6 +325,35 @@ __device__ __forceinline__ void mfma_inplace_v(f32x4& acc, const u32x4& a, const
   else
     asm(W4A16_MFMA_PRE "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
 }
+
+// The wavefronts of a SIMD share its issue slots oldest first: where they do not wait for each other, the oldest runs ahead, and the youngest ends
+// alone, with nobody to fill its waits (three workgroups of a compute unit that start together on tiles of 64 x 256 with K = 2048 ended after 48, 54
+// and 70 us).  So a wavefront's priority falls with its progress: those behind catch up with those in front, and all end together.  Levels at 1/4, 1/2 and
+// 3/4 or 1/2, 13/16 and 15/16 measure the same within 1 %.  Only for wavefronts that end a launch: where others follow, staggered ends are what lets one
+// workgroup's start and end run under another's loop (MoE blocks of 64 slots with the levels in every round: 0.92 - 0.98 of the speed).
+//   Time before over now, weights not cached or repeated alike: MoE blocks of 64 slots, ten layers 1.016 (128 experts of 2048 x 768, top-8, 601 tokens 123.2
+// -> 118.7 us); private K parts 1.01 - 1.05 (4096 x 6144 at 203 rows, bf16, 19.4 -> 18.8); 16-row tiles, dense, 1.00 - 1.05 (4096 x 6144 at 37 rows, bf16
+// with zero points, 10.25 -> 9.75), in MoE 0.99: those don't.
+struct Pace {
+  int at, n, level;
+  __device__ __forceinline__ void start(int rounds, bool last = true) {
+    __builtin_amdgcn_s_setprio(3);
+    n = rounds, at = last ? rounds * 3 / 8 : 0x7fffffff, level = 3;
+  }
+  __device__ __forceinline__ void round(int i) {  // at the start of round i, uniform
+    if (i < at) return;
+    if (level == 3) {
+      __builtin_amdgcn_s_setprio(2);
+      at = n * 11 / 16, level = 2;
+    } else if (level == 2) {
+      __builtin_amdgcn_s_setprio(1);
+      at = n * 7 / 8, level = 1;
+    } else {
+      __builtin_amdgcn_s_setprio(0);
+      at = 0x7fffffff;
+    }
+  }
+};
 
 constexpr int RED_RS = 148;  // row stride (floats) of the 128-column reduction slab (4 mod 16: conflict-free)
 

@@ -334,9 +334,12 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   // and in the other three k-steps too when a group is shorter than 128 rows.
   const std::bool_constant<HOIST && !ONCE> every{};
   const std::true_type refresh{};
+  Pace pace;
+  if constexpr (PRIV) pace.start(nchunks);
 #pragma unroll 1
   for (int c0 = 0; c0 < nchunks; c0 += 2) {
     const int ks0 = 2 * c0;
+    if constexpr (PRIV) pace.round(c0);
     load_a(c0 + AD, 0);
     kstep(0, std::false_type{}, st[0], st[1], every);
     if constexpr (ONCE) issue_scales(ks0 + 4);

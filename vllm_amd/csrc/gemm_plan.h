@@ -20,6 +20,7 @@ struct Plan {
   int tn;    // tile width in columns (128; the decode kernel also has 64)
   int nw = 8;  // 16-row tiles (decode kernel, general kernel with one m-block): wavefronts per workgroup (8 or 4)
   int strip0 = 0;      // 64-row kernel / K-split kernel: first 512- / 256-column strip handled by the launch
+  int resident = 0;    // MoE blocks of 64 slots: workgroups that run at a time
   int dyn_slots = 0;   // 64-row kernel, MoE: resident workgroups that the device-side K split of the tail tiles fills
   int tail_strips = 0; // prefill plan: trailing 512-column strips handed to another kernel (0 = none)
   int tail_kind = 3;   // ... which one: 3 = 64-row kernel, 5 = tall tiles with the K halves inside the workgroup

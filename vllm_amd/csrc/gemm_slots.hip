@@ -307,10 +307,13 @@ __global__ __launch_bounds__(256, W == 2 ? 3 : 2) void slots_kernel(const KParam
       }
     };
 
+    Pace pace;
+    pace.start(nchunks, (int)blockIdx.x + p.resident >= d.F + d.R * d.S);
     // ---- main loop: two chunks (four k-steps = the weight ring) per iteration
 #pragma unroll 1
     for (int c0 = 0; c0 < nchunks; c0 += 2) {
       const int ks0 = 2 * c0;
+      pace.round(c0);
       load_a(c0, HALF_CHUNK(AD + 1));
       kstep(0, HALF_CHUNK(0), st[0], st[1], std::false_type{});
       if constexpr (ONCE) issue_scales(ks0 + 4);
