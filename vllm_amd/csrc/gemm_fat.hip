@@ -454,11 +454,19 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
       __builtin_amdgcn_wave_barrier();
       continue;
     }
+    // (a row's read and store in one round would wait for each read by itself)
+    f32x4 rows[8];
+    int crows[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int r16 = (lane >> 5) + 2 * i;
-      const int crow = MOE ? s_crow[mb * 16 + r16] : row0 + mb * 16 + r16;
-      f32x4 v = *(const f32x4*)(slab + r16 * RED_RS + fpos);
+      crows[i] = MOE ? s_crow[mb * 16 + r16] : row0 + mb * 16 + r16;
+      rows[i] = *(const f32x4*)(slab + r16 * RED_RS + fpos);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r16 = (lane >> 5) + 2 * i, crow = crows[i];
+      f32x4 v = rows[i];
       if (!fcol_ok || (MOE ? crow < 0 : crow >= p.M)) continue;
       if (MOE && nsplit > 1) {
         // a K piece: the fp32 partial tile [row 128][column 512] goes to scratch; the pass launched behind finishes the rows

@@ -9,7 +9,7 @@
 //                in the 64-row kernel (B operand = the reference's half(q - z) * half(s)).
 //   activations  each K-quarter stages its own 64 rows x 64 K chunk into LDS in MFMA fragment order (its two
 //                wavefronts share it), double buffered; one workgroup barrier per two k-steps.
-//   epilogue     the four quarters' partial tiles are added through LDS, one 16-row block at a time.
+//   epilogue     the four quarters' partial tiles are added through LDS, two 16-row blocks at a time.
 //   split-K      with fewer tiles than compute units (129..~1000 rows of a narrow layer) K is also cut across
 //                workgroups, in splits of whole multiples of 512 K rows: the workgroup writes its 64 x 256 fp32 partial
 //                tile (already summed over its quarters) to scratch with plain 128-bit stores and kq_reduce_kernel,
@@ -54,9 +54,12 @@ constexpr int KQ_D = 4;      // weight k-steps in flight per wavefront
 // 2 k-steps x 4 dwords, then hit 64 different ones (128-row tiles without: 4096 x 4096 at 1024 rows 41.4 us, 41.6 with, and three spills)
 constexpr int kq_kstep(int MB) { return MB * 256 + (MB < 8 ? 32 : 0); }
 constexpr int kq_abuf(int MB) { return 2 * kq_kstep(MB) * 4; }  // one A buffer of one K part: 2 k-steps
+constexpr int KQ_ME = 2;   // m-blocks per round of the epilogue (four and eight K parts)
+constexpr int KQ_RS = 76;  // floats per row of an epilogue slab of 64 columns (40 for the half of either n-tile: conflict-free, 16-byte aligned)
 constexpr int kq_smem(int MB, int Q, int WN) {
-  const int stage = Q * 2 * kq_abuf(MB), slabs = WN * Q * 16 * RED_RS * 4;  // staging rings | the wavefronts' epilogue slabs
-  return (stage > slabs ? stage : slabs) + 16 * MB * 4;                     // + C row of each tile row
+  // staging rings | what the parts hand each other in the epilogue
+  const int stage = Q * 2 * kq_abuf(MB), boxes = Q == 2 ? WN * Q * MB * 4096 : KQ_ME * WN * Q * 16 * RED_RS * 4;
+  return stage > boxes ? stage : boxes;
 }
 
 // SHORT: private parts and tall tiles with groups below 128 rows, whose scales and constants come with every k-step.  (Tall tiles had both loops in
@@ -66,7 +69,7 @@ template <int DT, bool ZP, bool CHANNEL, int MB = 4, int Q = 4, int WN = 2, bool
 __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   static_assert((MB == 4 && Q == 4 && WN == 2) || (MB > 4 && MB <= 8 && Q == 2 && WN == 2) || (MB >= 2 && MB <= 4 && Q == 8 && WN == 1),
                 "64 x 256 in K quarters, 80 .. 128 x 256 in K halves or 32 .. 64 x 128 in K eighths");
-  constexpr int KQ_MB = MB, KQ_BM = 16 * MB, KQ_Q = Q, KQ_ABUF = kq_abuf(MB), KQ_SMEM = kq_smem(MB, Q, WN), KQ_TN = 128 * WN;
+  constexpr int KQ_MB = MB, KQ_BM = 16 * MB, KQ_Q = Q, KQ_ABUF = kq_abuf(MB), KQ_TN = 128 * WN;
   constexpr bool PRIV = (WN == 1);  // a K part is one wavefront: it stages its own activations, nothing in the loop waits for another
   // HOIST: the dequantisation constants of the four word positions are kept for the k-step whose operands are being built.  A loop
   // iteration covers four k-steps (128 rows of K, aligned: every K part starts at a multiple of four k-steps), so with groups of
@@ -81,7 +84,6 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   constexpr bool EARLY = !PRIV && KQ_MB < 8;
   constexpr bool UNIT = CHANNEL;
   extern __shared__ __align__(16) unsigned char smem[];
-  int* s_crow = (int*)(smem + KQ_SMEM - KQ_BM * 4);
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -103,17 +105,6 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   const uint16_t* Sc = (const uint16_t*)p.S;
   const uint32_t* Zp = p.Z;
   const uint16_t* bias = (const uint16_t*)p.bias;
-  // which A row feeds tile row r and which C row receives it (-1: none)
-  auto tile_row_ids = [&](int r, int& src, int& dst) {
-    src = dst = -1;
-    if (row0 + r < p.M) src = dst = row0 + r;
-  };
-  if (t < KQ_BM) {
-    int src, dst;
-    tile_row_ids(t, src, dst);
-    s_crow[t] = dst;
-  }
-
   // ---- weights of this wavefront
   const int nt = (wave_on && (2 * cp + h) * 64 < p.N) ? 2 * cp + h : 0;
   const int64_t b_row = p.N >> 1;
@@ -146,9 +137,8 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
     if constexpr (PRIV) {
       aoff[i] = (uint32_t)min((tq >> 3) + AR * i, p.M - 1 - row0) * ((uint32_t)p.lda * 2) + piece * 16;  // (the host checks the size)
     } else {
-      int src, dst;
-      tile_row_ids((tq >> 3) + AR * i, src, dst);
-      arow[i] = (const uint16_t*)p.A + (int64_t)(src < 0 ? 0 : src) * p.lda + piece * 8;
+      const int src = row0 + (tq >> 3) + AR * i;
+      arow[i] = (const uint16_t*)p.A + (int64_t)(src < p.M ? src : 0) * p.lda + piece * 8;
     }
   }
   // LDS A layout per part: [buffer][k-step 2][m-block][lane 64][4 dwords]; the 16 bytes of (row, piece) are the
@@ -364,18 +354,10 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   // per m-block: every wavefront writes its 16 x 128 partial to its slab [16 rows][RED_RS]; after a barrier the
   // wavefront of K part q adds the Q parts' slabs of its column pair for rows (16 / Q) q .. and finishes them.
   // (the last barrier of the loop, or this one, separates the slabs from the A buffers they overlay)
+  // (the last barrier of the loop, or this one, separates what follows from the A buffers it overlays)
   if constexpr (PRIV) __syncthreads();
-  float* slabs = (float*)smem;
-  float* mine = slabs + wv * (16 * RED_RS);
-  int el = t;  // (taken apart again here: a lane's place kept through the loop would spill in one of the kernels)
-  asm volatile("" : "+v"(el));
-  const int slab_at = 4 * (el >> 4 & 3) * RED_RS + 72 * (el >> 3 & 1) + (el & 7);
-  const int fc4 = (lane & 31) * 4;
-  const int fpos = fc4 + (fc4 >= 64 ? 8 : 0);
-  const int ncol = cp * 128 + fc4;
-  const bool fcol_ok = wave_on && ncol < p.N;
-  float cs[4] = {1.f, 1.f, 1.f, 1.f}, bs[4] = {0.f, 0.f, 0.f, 0.f};
-  if (fcol_ok) {
+  const int ncol0 = cp * 128;
+  auto col_consts = [&](int ncol, float* cs, float* bs) {
     const int base = ncol & ~31, cl = ncol & 31;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -388,39 +370,122 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
         bs[j] = (DT == DT_F16) ? f16_lo_f32(bv) : bf16_lo_f32(bv);
       }
     }
-  }
+  };
+  float cs[4] = {1.f, 1.f, 1.f, 1.f}, bs[4] = {0.f, 0.f, 0.f, 0.f};
+  int el = t;  // (taken apart again here: a lane's place kept through the loop would spill in one of the kernels)
+  asm volatile("" : "+v"(el));
+  if constexpr (KQ_Q == 2) {
+    // Two parts: each hands the other the fragments (m-block, word, column half: 16 rows x 16 columns, four rows to a lane) of two words of the
+    // four and finishes those of the other two, all in one exchange of half the accumulators.  From the loop to the end, 80 rows, four splits: 2.1 us,
+    // 3.7 with every m-block through slabs of both parts and two barriers; 96 rows, unsplit 2.9 and 4.9.  14336 x 4096 at 300 rows, fp16, act-order 51.6 ->
+    // 50.6 us, 4096 x 6144 at 1501 rows 90.7 -> 87.7.
+    float* const boxes = (float*)smem;
+    constexpr int BOX = KQ_MB * 4 * 256;  // floats of a wavefront's box: what it gets
+    float* const to = boxes + (wv ^ WN) * BOX + (el & 63) * 4;
+    float* const box = boxes + wv * BOX;
+    auto word_of = [&](int part, int i) { return 2 * part + (i >> 1); };  // fragment i of an m-block: word, half i & 1
+    const int lc = (el & 15) * 4, lh = lc >> 5, lpos = lh * 40 + (lc & 31);  // 64 columns: 32 of either n-tile
+    const int ncol = ncol0 + 64 * lh + 32 * q + (lc & 31);
+    const bool col_ok = wave_on && ncol < p.N;
+    if (col_ok && p.splits == 1) col_consts(ncol, cs, bs);
+    auto exchange = [&](auto part_tag) __attribute__((always_inline)) {  // (the part as a constant: accumulators are registers)
+      constexpr int PART = decltype(part_tag)::value;
 #pragma unroll
-  for (int mb = 0; mb < KQ_MB; ++mb) {
+      for (int mb = 0; mb < KQ_MB; ++mb)
 #pragma unroll
-    for (int w = 0; w < 4; ++w)
+        for (int i = 0; i < 4; ++i) *(f32x4*)(to + (mb * 4 + i) * 256) = acc[mb][word_of(1 - PART, i)][i & 1];
+      __syncthreads();
+      float* const part_out = p.ctmp + ((((int64_t)(strip * mtiles + mt) * p.splits + split) * WN + wn) * 2 + PART) * (KQ_MB * 1024) + (el & 63) * 4;
+      float* const slab = box;  // [2][16 rows][KQ_RS], over what has been read
+      constexpr int SLAB = 16 * KQ_RS;
+      f32x4 v[KQ_MB][4];
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf)
+      for (int mb = 0; mb < KQ_MB; ++mb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) mine[slab_at + r * RED_RS + 16 * w + 8 * hf] = acc[mb][w][hf][r];
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 8 / KQ_Q; ++i) {
-      const int r16 = (16 / KQ_Q) * q + (lane >> 5) + 2 * i;
-      const int crow = s_crow[mb * 16 + r16];
-      f32x4 v = {0, 0, 0, 0};
-#pragma unroll
-      for (int qq = 0; qq < KQ_Q; ++qq) v += *(const f32x4*)(slabs + (qq * WN + wn) * (16 * RED_RS) + r16 * RED_RS + fpos);
+        for (int i = 0; i < 4; ++i) {
+          const f32x4 got = *(const f32x4*)(box + (mb * 4 + i) * 256 + (el & 63) * 4), own = acc[mb][word_of(PART, i)][i & 1];
+          v[mb][i] = own + got;
+        }
       if (p.splits > 1) {
-        if (crow >= 0)
-          *(f32x4*)(p.ctmp + (((int64_t)(strip * mtiles + mt) * p.splits + split) * KQ_BM + mb * 16 + r16) * KQ_TN +
-                    wn * 128 + fc4) = v;
-      } else if (fcol_ok && crow >= 0) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = v[j] * cs[j] + bs[j];
-        u32x2 o;
-        if constexpr (DT == DT_F16)
-          o = u32x2{pack_f16(v[0], v[1]), pack_f16(v[2], v[3])};
-        else
-          o = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
-        *(u32x2*)((uint16_t*)p.C + (int64_t)crow * p.N + ncol) = o;
+        for (int mb = 0; mb < KQ_MB; ++mb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) *(f32x4*)(part_out + (mb * 4 + i) * 256) = v[mb][i];
+        return;
       }
+      __builtin_amdgcn_wave_barrier();
+      const int at = 4 * (el >> 4 & 3) * KQ_RS + 40 * (el >> 3 & 1) + (el & 7);
+#pragma unroll
+      for (int m0 = 0; m0 < KQ_MB; m0 += 2) {
+#pragma unroll
+        for (int e = 0; e < 2 && m0 + e < KQ_MB; ++e)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) slab[e * SLAB + at + r * KQ_RS + 8 * i] = v[m0 + e][i][r];
+        __builtin_amdgcn_wave_barrier();
+        f32x4 rows[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (i < 4 || m0 + 1 < KQ_MB) rows[i] = *(const f32x4*)(slab + (i >> 2) * SLAB + ((el >> 4 & 3) + 4 * (i & 3)) * KQ_RS + lpos);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int crow = row0 + 16 * m0 + (el >> 4 & 3) + 4 * i;
+          if ((i < 4 || m0 + 1 < KQ_MB) && col_ok && crow < p.M) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) rows[i][j] = rows[i][j] * cs[j] + bs[j];
+            store_row4<DT, false>(p, crow, ncol, rows[i]);
+          }
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+    };
+    if (q == 0)
+      exchange(std::integral_constant<int, 0>{});
+    else
+      exchange(std::integral_constant<int, 1>{});
+  } else {
+    // per two m-blocks: every wavefront writes its 16 x 128 partials to its slabs [16 rows][RED_RS]; after a barrier the
+    // wavefront of K part q adds the Q parts' slabs of its column pair for rows (16 / Q) q .. and finishes them.
+    constexpr int ME = KQ_ME, SLABS = WN * KQ_Q * 16 * RED_RS;
+    float* slabs = (float*)smem;
+    const int slab_at = wv * (16 * RED_RS) + 4 * (el >> 4 & 3) * RED_RS + 72 * (el >> 3 & 1) + (el & 7);
+    const int fc4 = (lane & 31) * 4;
+    const int fpos = fc4 + (fc4 >= 64 ? 8 : 0);
+    const int ncol = ncol0 + fc4;
+    const bool fcol_ok = wave_on && ncol < p.N;
+    if (fcol_ok) col_consts(ncol, cs, bs);
+#pragma unroll
+    for (int m0 = 0; m0 < KQ_MB; m0 += ME) {
+      if (m0 > 0) __syncthreads();
+#pragma unroll
+      for (int e = 0; e < ME && m0 + e < KQ_MB; ++e)
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) slabs[e * SLABS + slab_at + r * RED_RS + 16 * w + 8 * hf] = acc[m0 + e][w][hf][r];
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < ME && m0 + e < KQ_MB; ++e)
+#pragma unroll
+        for (int i = 0; i < 8 / KQ_Q; ++i) {
+          const int mb = m0 + e, r16 = (16 / KQ_Q) * q + (lane >> 5) + 2 * i;
+          const int crow = row0 + mb * 16 + r16;
+          f32x4 v = {0, 0, 0, 0};
+#pragma unroll
+          for (int qq = 0; qq < KQ_Q; ++qq) v += *(const f32x4*)(slabs + e * SLABS + (qq * WN + wn) * (16 * RED_RS) + r16 * RED_RS + fpos);
+          if (p.splits > 1) {
+            if (crow < p.M)
+              *(f32x4*)(p.ctmp + (((int64_t)(strip * mtiles + mt) * p.splits + split) * KQ_BM + mb * 16 + r16) * KQ_TN + wn * 128 + fc4) = v;
+          } else if (fcol_ok && crow < p.M) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = v[j] * cs[j] + bs[j];
+            store_row4<DT, false>(p, crow, ncol, v);
+          }
+        }
     }
-    __syncthreads();
   }
 }
 
@@ -480,6 +545,65 @@ __global__ __launch_bounds__(256) void kq_reduce_kernel(const KParams p, int mb)
   }
 }
 
+// The same behind tall tiles, whose partial tiles are fragments in the order in which their wavefronts hold them: [column pair][K part][m-block]
+// [word of two, column half][lane][row of four].  One workgroup per (tile, m-block), a wavefront for each column pair and part.
+template <int DT, bool CHANNEL>
+__global__ __launch_bounds__(256) void kq_reduce_tall_kernel(const KParams p, int mb) {
+  __shared__ __align__(16) float slabs[4][16 * KQ_RS];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;  // wv: 2 wn + part
+  const int mtiles = (p.M + 16 * mb - 1) / (16 * mb);
+  const int tile = blockIdx.x / mb, m = blockIdx.x % mb;
+  const int mt = tile % mtiles, cp = (p.strip0 + tile / mtiles) * 2 + (wv >> 1);
+  const int lc = (lane & 15) * 4, lh = lc >> 5;
+  const int ncol = cp * 128 + 64 * lh + 32 * (wv & 1) + (lc & 31), row0 = (mt * mb + m) * 16 + (lane >> 4);
+  if (row0 - (lane >> 4) >= p.M || cp * 128 >= p.N) return;
+  const bool col_ok = ncol < p.N;
+  float cs[4] = {1.f, 1.f, 1.f, 1.f}, bs[4] = {0.f, 0.f, 0.f, 0.f};
+  const uint16_t* Sc = (const uint16_t*)p.S;
+  const uint16_t* bias = (const uint16_t*)p.bias;
+  if (col_ok) {
+    const int base = ncol & ~31, cl = ncol & 31;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (CHANNEL) cs[j] = lo_f32<DT>(Sc[base + single_perm_pos(cl + j)]);
+      if (bias) bs[j] = lo_f32<DT>(bias[base + single_perm_pos(cl + j)]);
+    }
+  }
+  const int64_t piece = mb * 4096;  // floats of a partial tile
+  const float* parts = p.ctmp + (int64_t)tile * p.splits * piece + (wv * mb + m) * 1024 + lane * 4;
+  f32x4 v[4] = {};
+  for (int s0 = 0; s0 < p.splits; s0 += 4) {  // (four splits' loads are in flight together)
+    f32x4 a[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[j][i] = *(const f32x4*)(parts + min(s0 + j, p.splits - 1) * piece + i * 256);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (s0 + j < p.splits) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += a[j][i];
+      }
+  }
+  float* slab = slabs[wv];
+  const int at = 4 * (lane >> 4) * KQ_RS + 40 * (lane >> 3 & 1) + (lane & 7);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) slab[at + r * KQ_RS + 8 * i] = v[i][r];
+  __builtin_amdgcn_wave_barrier();
+  f32x4 rows[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) rows[i] = *(const f32x4*)(slab + ((lane >> 4) + 4 * i) * KQ_RS + lh * 40 + (lc & 31));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (!col_ok || row0 + 4 * i >= p.M) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) rows[i][j] = rows[i][j] * cs[j] + bs[j];
+    store_row4<DT, false>(p, row0 + 4 * i, ncol, rows[i]);
+  }
+}
+
 typedef void (*kq_fn)(const KParams);
 typedef void (*kq_reduce_fn)(const KParams, int);
 
@@ -518,7 +642,8 @@ static kq_fn pick_kq(int mb, int tn, bool zp, bool channel, bool short_groups) {
   }
 }
 template <int DT>
-static kq_reduce_fn pick_kq_reduce(int tn, bool channel) {
+static kq_reduce_fn pick_kq_reduce(int tn, int mb, bool channel) {
+  if (mb > 4) return channel ? kq_reduce_tall_kernel<DT, true> : kq_reduce_tall_kernel<DT, false>;
   if (tn == 128) return channel ? kq_reduce_kernel<DT, true, 128> : kq_reduce_kernel<DT, false, 128>;
   return channel ? kq_reduce_kernel<DT, true, 256> : kq_reduce_kernel<DT, false, 256>;
 }
@@ -542,7 +667,7 @@ int launch_kq(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream) {
   hipLaunchKernelGGL(fn, dim3((unsigned)((int64_t)pl.tiles * pl.splits)), dim3(64 * wn * parts), smem, stream, p);
   W4A16_HIP(hipGetLastError());
   if (pl.splits > 1) {
-    const kq_reduce_fn red = f16 ? pick_kq_reduce<DT_F16>(pl.tn, channel) : pick_kq_reduce<DT_BF16>(pl.tn, channel);
+    const kq_reduce_fn red = f16 ? pick_kq_reduce<DT_F16>(pl.tn, pl.mb, channel) : pick_kq_reduce<DT_BF16>(pl.tn, pl.mb, channel);
     hipLaunchKernelGGL(red, dim3((unsigned)pl.tiles * pl.mb), dim3(256), 0, stream, p, pl.mb);
     W4A16_HIP(hipGetLastError());
   }

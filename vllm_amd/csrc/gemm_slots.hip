@@ -338,7 +338,8 @@ __global__ __launch_bounds__(256, W == 2 ? 3 : 2) void slots_kernel(const KParam
     // (the inline-asm MFMAs are opaque to the compiler's hazard logic: let the matrix pipe drain before the
     //  accumulators are read)
     asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
-    // per wavefront and m-block: accumulators -> private LDS slab [16 rows][RS] -> 8-byte row stores.
+    // per wavefront and m-block: accumulators -> private LDS slab [16 rows][RS] -> 8-byte row stores.  All rows of an m-block are read before one is
+    // stored: read and stored one by one, each read was waited for by itself (GEMM2 of 128 experts: 6 us of 40 behind the loop).
     // (the last barrier of the loop separates the slabs from the A buffers they overlay)
     if (!wave_on) return;
     int el = lane;  // (a lane's places are worked out again here: kept through the loop they would spill)
@@ -350,6 +351,7 @@ __global__ __launch_bounds__(256, W == 2 ? 3 : 2) void slots_kernel(const KParam
     constexpr int LR = 8 * W, LA = 4 * W;
     const int lc = (el % LR) * 4, lpos = lc / HALF * (HALF + 8) + lc % HALF, ac = (el % LA) * 4;
     const int ncol = 2 * HALF * u + lc, ocol = HALF * u + ac;
+    const int er = el / LR;  // first row of the lane
     if (!act && ncol >= p.N) el = -1;  // (the second n-tile of the last pair may be missing)
     float cs[4] = {1.f, 1.f, 1.f, 1.f}, bs[4] = {0.f, 0.f, 0.f, 0.f}, cu[4] = {1.f, 1.f, 1.f, 1.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
     auto col_consts = [&](int col, float* sc_out, float* b_out) {
@@ -376,38 +378,50 @@ __global__ __launch_bounds__(256, W == 2 ? 3 : 2) void slots_kernel(const KParam
           for (int r = 0; r < 4; ++r) slab[slab_at + r * RS + 16 * w + 8 * hf] = acc[mb][w][hf][r];
       __builtin_amdgcn_wave_barrier();
       if (act && nsplit == 1) {
+        constexpr int NI = 16 * LA / 64;
+        f32x4 v[NI], up[NI];
+        int crow[NI];
 #pragma unroll
-        for (int i = 0; i < 16 * LA / 64; ++i) {
+        for (int i = 0; i < NI; ++i) {
           const int r16 = el / LA + 64 / LA * i;
-          const int crow = s_crow[mb * 16 + r16];
-          if (crow < 0) continue;
-          f32x4 v = *(const f32x4*)(slab + r16 * RS + ac);
-          f32x4 up = *(const f32x4*)(slab + r16 * RS + ac + HALF + 8);
+          crow[i] = s_crow[mb * 16 + r16];
+          v[i] = *(const f32x4*)(slab + r16 * RS + ac);
+          up[i] = *(const f32x4*)(slab + r16 * RS + ac + HALF + 8);
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            v[j] = v[j] * cs[j] + bs[j];
-            up[j] = up[j] * cu[j] + bu[j];
+            v[i][j] = v[i][j] * cs[j] + bs[j];
+            up[i][j] = up[i][j] * cu[j] + bu[j];
           }
           if (p.mul_topk) {
-            const float tw = s_tw[mb * 16 + r16];
+            const float tw = s_tw[mb * 16 + el / LA + 64 / LA * i];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              v[j] *= tw;
-              up[j] *= tw;
+              v[i][j] *= tw;
+              up[i][j] *= tw;
             }
           }
-          store_row4_silu_mul<DT>(p, crow, ocol, v, up);
+          if (crow[i] >= 0) store_row4_silu_mul<DT>(p, crow[i], ocol, v[i], up[i]);
         }
         __builtin_amdgcn_wave_barrier();
         continue;
       }
+      constexpr int NI = 16 * LR / 64;
+      f32x4 rows[NI];
+      int crows[NI];
 #pragma unroll
-      for (int i = 0; i < 16 * LR / 64; ++i) {
-        if (el < 0) break;
-        const int r16 = el / LR + 64 / LR * i;
-        const int crow = s_crow[mb * 16 + r16];
-        f32x4 v = *(const f32x4*)(slab + r16 * RS + lpos);
-        if (crow < 0) continue;
+      for (int i = 0; i < NI; ++i) {
+        const int r16 = er + 64 / LR * i;
+        crows[i] = s_crow[mb * 16 + r16];
+        rows[i] = *(const f32x4*)(slab + r16 * RS + lpos);
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int r16 = er + 64 / LR * i, crow = crows[i];
+        f32x4 v = rows[i];
+        if (el < 0 || crow < 0) continue;
         if (nsplit > 1) {
           // K is split: the fp32 partial tile [row 64][column TN] goes to scratch; the kernel launched behind this one adds the
           // splits and finishes the rows
