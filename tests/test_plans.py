@@ -199,3 +199,19 @@ def test_moe_beyond_limits(plan):
     for group in (128, 256, -1):
         assert plan(1000, k, bl.N, torch.bfloat16, "uint4b8", group, moe_slots=ids, moe_block=128)["kind"] == 2
         assert plan(1000, k, bl.N, torch.bfloat16, "uint4b8", group, moe_slots=ids - 128, moe_block=128)["kind"] == 9
+
+
+def test_tiles_of_rows_with_unscaled_weights(plan):
+    """The shapes of test_gpu_rows.py run on the tile they are listed with; what the kernel does not take, and what has never run on 16-row tiles, stays."""
+    import torch
+    import test_gpu_rows as rows
+    for (m, k, n, dtype, fmt, group, act), tile in rows.ROWS.items():
+        p = plan(m, k, n, dtype, fmt, group, act)
+        assert (p["kind"], p["mb"], p["splits"], p["tn"]) == (10,) + tile + (64,), (m, k, n, dtype, fmt, group, p)
+        assert plan(16, k, n, dtype, fmt, group, act)["kind"] == 1 and plan(49, k, n, dtype, fmt, group, act)["kind"] != 10
+    for m, k, n, group in [(37, 14336, 4096, 64), (37, 14336 + 64, 4096, -1), (37, 14336, 4096, 32), (37, 4096, 4096, 128), (37, 4096, 28672, 128),
+                           (20, 4096, 64 * 257, 128)]:
+        assert plan(m, k, n, torch.bfloat16, "uint4", group)["kind"] != 10, (m, k, n, group)
+    # no more scratch than the 16-row tiles had, where a caller asks for little
+    p = plan(37, 14336, 4096, torch.bfloat16, "uint4", 128, more_scratch=False)
+    assert p["kind"] in (1, 10) and p["splits"] <= 4

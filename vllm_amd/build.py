@@ -12,7 +12,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libw4a16_gfx950.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 
-SOURCES = ["c_api.hip", "repack.hip", "gemm.hip", "gemm_skinny.hip", "gemm_decode.hip", "gemm_fat.hip", "gemm_mid.hip", "gemm_kq.hip", "gemm_slots.hip", "gemm_x8.hip", "moe_glue.hip"]
+SOURCES = ["c_api.hip", "repack.hip", "gemm.hip", "gemm_skinny.hip", "gemm_decode.hip", "gemm_rows.hip", "gemm_fat.hip", "gemm_mid.hip", "gemm_kq.hip", "gemm_slots.hip", "gemm_x8.hip", "moe_glue.hip"]
 
 # The 16-row kernel takes the values in front of its first loads as leading scalar arguments; with this option the first
 # 14 dwords of a kernel's argument block arrive in SGPRs when a wavefront starts (gfx950 firmware loads them while it

@@ -16,7 +16,8 @@ struct Plan {
   int kind;  // 0: skinny kernel, 1: decode kernel, 2: prefill ("fat") kernel, 3: 64-row ("mid") kernel,
              // 5: in-workgroup K split (gemm_kq.hip): 64 x 256 tiles in K quarters (mb = 4), 80 .. 128 x 256 in halves (mb = 5 .. 8), 32 .. 64 x 128
              // in eighths (mb = 2 .. 4, tn = 128), 6: 8-bit matrix unit, 7: the same on prepared weights,
-             // 8: MoE blocks of 64 slots, integer 4-bit weights (gemm_slots.hip, tn = 256 or 512), 9: the 8-bit unit on MoE blocks of 128 slots
+             // 8: MoE blocks of 64 slots, integer 4-bit weights (gemm_slots.hip, tn = 256 or 512), 9: the 8-bit unit on MoE blocks of 128 slots,
+             // 10: tiles of 32 or 48 rows x 64 columns, unscaled weights (gemm_rows.hip)
   int tn;    // tile width in columns (128; the decode kernel also has 64)
   int nw = 8;  // 16-row tiles (decode kernel, general kernel with one m-block): wavefronts per workgroup (8 or 4)
   int strip0 = 0;      // 64-row kernel / K-split kernel: first 512- / 256-column strip handled by the launch
@@ -39,6 +40,7 @@ int moe_gather_rows(const w4a16_gemm_args* a, void* out, hipStream_t stream);
 inline int64_t mid_tail_pieces(int64_t tiles, int slots) { return tiles * 8 < slots ? tiles * 8 : slots; }
 
 int launch_skinny(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
+int launch_rows(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_decode(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_fat(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
 int launch_mid(const w4a16_gemm_args* a, const Plan& pl, hipStream_t stream);
