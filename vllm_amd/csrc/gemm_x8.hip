@@ -224,6 +224,7 @@ __device__ __forceinline__ void x8_split(const uint16_t* a, int64_t lda, int row
 template <int X8_SG>
 __global__ __launch_bounds__(256) void x8_split_kernel(const uint16_t* a, int64_t lda, int rows, int stride, int groups, unsigned char* rec,
                                                        uint32_t* scl) {
+  asm volatile("" ::"s"(a), "s"(lda), "s"(rows), "s"(stride), "s"(groups), "s"(rec), "s"(scl));  // (the arguments in one turn, not three)
   x8_split<X8_SG, false>(a, lda, rows, stride, groups, rec, scl, X8Slots{});
 }
 __global__ __launch_bounds__(256) void x8_split_slots_kernel(const uint16_t* a, int64_t lda, int stride, int groups, unsigned char* rec, uint32_t* scl,
@@ -1033,7 +1034,9 @@ int launch_x8(const w4a16_gemm_args* a, const Plan& pl, void* scratch, hipStream
   }
   // (steps per workgroup: few rows fill the chip only with one)
   const int sg = (r / 16) * groups >= 16 * num_cus() ? 4 : 1;
-  hipLaunchKernelGGL((sg == 4 ? x8_split_kernel<4> : x8_split_kernel<1>), dim3((unsigned)(r / 16), (unsigned)ceil_div(groups, sg)), dim3(256), 0,
+  // (rows that a tile has; what is behind the last tile is never used)
+  const int64_t blocks = ceil_div((int64_t)pl.mtiles * pl.bm, 16) < r / 16 ? ceil_div((int64_t)pl.mtiles * pl.bm, 16) : r / 16;
+  hipLaunchKernelGGL((sg == 4 ? x8_split_kernel<4> : x8_split_kernel<1>), dim3((unsigned)blocks, (unsigned)ceil_div(groups, sg)), dim3(256), 0,
                      stream, (const uint16_t*)a->a, a->lda, (int)a->size_m, (int)r, groups, (unsigned char*)xp.rec,
                      (uint32_t*)xp.scl);
   W4A16_HIP(hipGetLastError());
