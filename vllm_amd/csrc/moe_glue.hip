@@ -16,91 +16,126 @@ constexpr int ALIGN_THREADS = 1024;
 constexpr int ALIGN_WAVES = ALIGN_THREADS / 64;
 constexpr int ALIGN_MAX_EXPERTS = 1024;
 
-// Every workgroup recomputes the histogram and the scan (numel and E are small), then its 16
-// wavefronts each place the tokens of experts wg*16 + wave, +gridDim*16, ... by ballot ranking.
-__global__ __launch_bounds__(ALIGN_THREADS) void moe_align_kernel(
-    const int32_t* __restrict__ topk_ids, int numel, int num_experts, int block_size,
-    int32_t* __restrict__ sorted_ids, int sorted_len, int32_t* __restrict__ expert_ids, int expert_ids_len,
-    int32_t* __restrict__ num_post_pad) {
-  __shared__ int cnt[ALIGN_MAX_EXPERTS];
-  __shared__ int off[ALIGN_MAX_EXPERTS + 1];
-  const int t = threadIdx.x;
-  for (int e = t; e < num_experts; e += ALIGN_THREADS) cnt[e] = 0;
-  __syncthreads();
-  for (int i = t; i < numel; i += ALIGN_THREADS) {
-    const int e = topk_ids[i];
-    if (e >= 0 && e < num_experts) atomicAdd(&cnt[e], 1);
-  }
-  __syncthreads();
-  if (t < 64) {  // wave 0: exclusive scan of padded counts, 64 experts per round
-    int run = 0;
-    for (int base = 0; base < num_experts; base += 64) {
-      const int e = base + t;
-      const int padded = e < num_experts ? (cnt[e] + block_size - 1) / block_size * block_size : 0;
-      int incl = padded;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int v = __shfl_up(incl, d, 64);
-        if (t >= d) incl += v;
-      }
-      if (e < num_experts) off[e] = run + incl - padded;
-      run += __shfl(incl, 63, 64);
-    }
-    if (t == 0) off[num_experts] = run;
-  }
-  __syncthreads();
-  const int total = off[num_experts];
+// Up to 4 * ALIGN_THREADS * ALIGN_GROUPS ids: a workgroup holds all of them in its registers, every wavefront a contiguous run, asked for once.  Bound by
+// its chain of round trips, which is cut to ids, histogram in LDS, positions and stores: a workgroup counts its own one to four experts in every run by
+// ballots while the histogram fills, and every wavefront adds up the padded counts in front of them by itself (a scan by one wavefront stood behind
+// a barrier of its own); the slots and blocks past the total are written by all workgroups.  The kernels that walked the ids two or three times: 333 ids of
+// 128 experts 3.5 -> 2.8 us, 2000 6.0 -> 3.2, 4808 7.5 -> 4.1, 16384 of 64 8.7 -> 5.8, 65536 of 128 25.8 -> 14.9, 64000 of 8 26.4 -> 22.6
+// (LDS atomics on eight addresses).
+using i32x4 = int32_t __attribute__((ext_vector_type(4)));
+constexpr int ALIGN_GROUPS = 16, ALIGN_OWN = 4;
 
-  if (blockIdx.x == 0) {
-    if (t == 0) *num_post_pad = total;
-    // expert id of every block; blocks past the padded total are zero-filled
-    for (int e = t; e < num_experts; e += ALIGN_THREADS) {
-      const int b0 = off[e] / block_size, b1 = off[e + 1] / block_size;
-      for (int b = b0; b < b1 && b < expert_ids_len; ++b) expert_ids[b] = e;
-    }
-    for (int b = total / block_size + t; b < expert_ids_len; b += ALIGN_THREADS) expert_ids[b] = 0;
-    for (int i = total + t; i < sorted_len; i += ALIGN_THREADS) sorted_ids[i] = numel;
-  }
-
-  const int lane = t & 63, wv = t >> 6;
-  for (int e = blockIdx.x * ALIGN_WAVES + wv; e < num_experts; e += gridDim.x * ALIGN_WAVES) {
-    int pos = off[e];
-    const int end = off[e + 1];
-    if (pos == end) continue;
-    // four independent loads per round trip (the loop is latency-bound: 64 ids per wavefront and load otherwise)
-    for (int base = 0; base < numel; base += 256) {
-      int id[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int i = base + 64 * u + lane;
-        id[u] = i < numel ? topk_ids[i] : -1;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int i = base + 64 * u + lane;
-        const bool hit = id[u] == e;  // (e >= 0: padding ids never match)
-        const unsigned long long m = __ballot(hit);
-        if (hit) {
-          const int rank = __popcll(m & ((1ull << lane) - 1ull));
-          if (pos + rank < sorted_len) sorted_ids[pos + rank] = i;
-        }
-        pos += __popcll(m);
-      }
-    }
-    for (int i = pos + lane; i < end && i < sorted_len; i += 64) sorted_ids[i] = numel;
-  }
+// sum over the wavefront, in every lane (as wave_max below)
+template <int CTRL>
+__device__ __forceinline__ int dpp_add(int x) { return x + __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true); }
+__device__ __forceinline__ int wave_sum(int x) {
+  x = dpp_add<0x111>(x);  // row_shr:1, 2, 4, 8
+  x = dpp_add<0x112>(x);
+  x = dpp_add<0x114>(x);
+  x = dpp_add<0x118>(x);
+  x = dpp_add<0x142>(x);  // row_bcast:15
+  x = dpp_add<0x143>(x);  // row_bcast:31
+  return __builtin_amdgcn_readlane(x, 63);
 }
 
-// The same contract for long id lists (prefill): the kernel above walks all ids once per expert with one wavefront, four
-// dependent 4-byte loads per round trip, and re-reads them with as many round trips for the histogram; here
+template <int THREADS, int R>
+__global__ __launch_bounds__(THREADS) void moe_align_held_kernel(
+    const int32_t* __restrict__ topk_ids, int numel, int num_experts, int block_size, int vec, int32_t* __restrict__ sorted_ids, int sorted_len,
+    int32_t* __restrict__ expert_ids, int expert_ids_len, int32_t* __restrict__ num_post_pad) {
+  constexpr int WAVES = THREADS / 64;
+  __shared__ int cnt[ALIGN_MAX_EXPERTS];
+  __shared__ int run_cnt[ALIGN_OWN][WAVES];
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  // ids of this lane: four consecutive ones of each of R groups; -1 past the end
+  i32x4 v[R];
+  const int i0 = (wv * R * 64 + lane) * 4;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = i0 + r * 256;
+    if (vec && i + 4 <= numel) {
+      v[r] = *(const i32x4*)(topk_ids + i);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[r][q] = i + q < numel ? topk_ids[i + q] : -1;
+    }
+  }
+  for (int e = t; e < num_experts; e += THREADS) cnt[e] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if ((unsigned)v[r][q] < (unsigned)num_experts) atomicAdd(&cnt[v[r][q]], 1);
+  // this workgroup's experts: blockIdx.x, + gridDim.x, ... (at most ALIGN_OWN: host)
+#pragma unroll
+  for (int o = 0; o < ALIGN_OWN; ++o) {
+    const int e = blockIdx.x + o * gridDim.x;
+    if (e >= num_experts) break;
+    int n = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) n += __popcll(__ballot(v[r][q] == e));
+    if (lane == 0) run_cnt[o][wv] = n;
+  }
+  __syncthreads();
+  auto padded = [&](int n) { return (n + block_size - 1) / block_size * block_size; };
+  int before[ALIGN_OWN] = {}, all = 0;  // padded slots of the experts in front of each of this workgroup's, and of all
+  for (int e = lane; e < num_experts; e += 64) {
+    const int n = padded(cnt[e]);
+    all += n;
+#pragma unroll
+    for (int o = 0; o < ALIGN_OWN; ++o) before[o] += e < (int)(blockIdx.x + o * gridDim.x) ? n : 0;
+  }
+  const int total = wave_sum(all);
+#pragma unroll
+  for (int o = 0; o < ALIGN_OWN; ++o) {
+    const int e = blockIdx.x + o * gridDim.x;
+    if (e >= num_experts) break;
+    const int off = wave_sum(before[o]), n = cnt[e], end = off + padded(n);
+    int pos = off + wave_sum(lane < wv ? run_cnt[o][lane] : 0);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      unsigned long long m[4];
+      int in_front = 0, hits = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        m[q] = __ballot(v[r][q] == e);
+        in_front += __builtin_amdgcn_mbcnt_hi((uint32_t)(m[q] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m[q], 0));
+        hits += __popcll(m[q]);
+      }
+      if (hits) {
+        int p = pos + in_front;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (v[r][q] == e) {
+            if (p < sorted_len) sorted_ids[p] = i0 + r * 256 + q;
+            ++p;
+          }
+        }
+      }
+      pos += hits;
+    }
+    for (int i = off + n + t; i < end && i < sorted_len; i += THREADS) sorted_ids[i] = numel;
+    const int b1 = end / block_size;
+    for (int b = off / block_size + t; b < b1 && b < expert_ids_len; b += THREADS) expert_ids[b] = e;
+  }
+  // slots past the total hold numel, blocks past it 0
+  const int at = blockIdx.x * THREADS + t, step = gridDim.x * THREADS;
+  for (int i = total + at; i < sorted_len; i += step) sorted_ids[i] = numel;
+  for (int b = total / block_size + at; b < expert_ids_len; b += step) expert_ids[b] = 0;
+  if (at == 0) *num_post_pad = total;
+}
+
+// The same contract for longer id lists:
 //   * every thread fetches its ids with 16-byte loads, several in flight, for the histogram (LDS atomics: per-expert
 //     ballot counts for the few-expert case, where lanes queue on a few addresses, measured slower);
 //   * the ids of an expert are placed by `spe` wavefronts of a workgroup, each on a contiguous slice of the ids:
 //     count the matches of the slice, exchange the counts through LDS, place from the slice's start position.  A lane
 //     holds four consecutive ids; a match's rank is the matches of the lanes in front plus its own earlier components,
 //     so the order inside an expert stays the order of the ids (stable, deterministic).
-using i32x4 = int32_t __attribute__((ext_vector_type(4)));
 constexpr int ALIGN_ROUND = 8;  // 16-byte loads in flight per lane in the placement passes (2048 ids per wavefront round)
+template <bool VEC>  // topk_ids on 16 bytes
 __global__ __launch_bounds__(ALIGN_THREADS) void moe_align_sliced_kernel(
     const int32_t* __restrict__ topk_ids, int numel, int num_experts, int block_size, int spe,
     int32_t* __restrict__ sorted_ids, int sorted_len, int32_t* __restrict__ expert_ids, int expert_ids_len,
@@ -113,7 +148,11 @@ __global__ __launch_bounds__(ALIGN_THREADS) void moe_align_sliced_kernel(
   for (int e = t; e < num_experts; e += ALIGN_THREADS) cnt[e] = 0;
   __syncthreads();
   const int nvec = numel >> 2;  // whole 16-byte groups; the last numel & 3 ids are handled one by one
-  const i32x4* vids = (const i32x4*)topk_ids;
+  auto load4 = [&](int vi) {
+    if constexpr (VEC) return ((const i32x4*)topk_ids)[vi];
+    const int32_t* at = topk_ids + 4 * vi;
+    return i32x4{at[0], at[1], at[2], at[3]};
+  };
 
   // ---- histogram
   for (int v0 = 0; v0 < nvec; v0 += 4 * ALIGN_THREADS) {
@@ -121,7 +160,7 @@ __global__ __launch_bounds__(ALIGN_THREADS) void moe_align_sliced_kernel(
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int vi = v0 + j * ALIGN_THREADS + t;
-      v[j] = vi < nvec ? vids[vi] : i32x4{-1, -1, -1, -1};
+      v[j] = vi < nvec ? load4(vi) : i32x4{-1, -1, -1, -1};
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -185,7 +224,7 @@ __global__ __launch_bounds__(ALIGN_THREADS) void moe_align_sliced_kernel(
 #pragma unroll
           for (int r = 0; r < ALIGN_ROUND; ++r) {
             const int vi = v0 + 64 * r + lane;
-            v[r] = vi < ve ? vids[vi] : i32x4{-1, -1, -1, -1};
+            v[r] = vi < ve ? load4(vi) : i32x4{-1, -1, -1, -1};
           }
 #pragma unroll
           for (int r = 0; r < ALIGN_ROUND; ++r) {
@@ -497,22 +536,31 @@ extern "C" int w4a16_moe_align_block_size(const int32_t* topk_ids, int64_t numel
   W4A16_CHECK(block_size >= 1, "block_size must be positive");
   W4A16_CHECK(numel >= 0 && numel < (1LL << 30), "bad topk_ids.numel()");
   W4A16_CHECK(sorted_len >= numel, "sorted_token_ids is shorter than topk_ids");
-  if (numel >= 2048 && ((uintptr_t)topk_ids & 15) == 0) {
-    // slices per expert: enough wavefronts for 64 and more workgroups, slices of at least 256 ids
-    int spe = 1;
-    while (spe < ALIGN_WAVES && num_experts * spe < 1024 && numel / (2 * spe) >= 256) spe *= 2;
-    const int64_t turns = ceil_div(num_experts, ALIGN_WAVES / spe);
-    const int grid = (int)(turns < 256 ? turns : 256);
-    moe_align_sliced_kernel<<<grid, ALIGN_THREADS, 0, (hipStream_t)stream>>>(
-        topk_ids, (int)numel, num_experts, block_size, spe, sorted_token_ids, (int)sorted_len, expert_ids,
-        (int)expert_ids_len, num_tokens_post_pad);
+  const int vec = ((uintptr_t)topk_ids & 15) == 0;
+  if (numel <= 4 * ALIGN_THREADS * ALIGN_GROUPS) {
+    const int grid = num_experts < 256 ? num_experts : 256;
+    // (256 threads start 1 us sooner than 1024: 2000 ids 3.2 us against 3.5; 4808 and 8192 ids 4.1 and 4.9 with 1024, 4.2 and 4.8 with 512)
+    const int threads = numel <= 2048 ? 256 : ALIGN_THREADS;
+    const int64_t r = ceil_div(numel, 4 * threads);  // groups per thread
+    const auto fn = threads == 256 ? (r <= 1 ? moe_align_held_kernel<256, 1> : moe_align_held_kernel<256, 2>)
+                    : r <= 1       ? moe_align_held_kernel<ALIGN_THREADS, 1>
+                    : r <= 2       ? moe_align_held_kernel<ALIGN_THREADS, 2>
+                    : r <= 4       ? moe_align_held_kernel<ALIGN_THREADS, 4>
+                    : r <= 8       ? moe_align_held_kernel<ALIGN_THREADS, 8>
+                                   : moe_align_held_kernel<ALIGN_THREADS, ALIGN_GROUPS>;
+    fn<<<grid, threads, 0, (hipStream_t)stream>>>(topk_ids, (int)numel, num_experts, block_size, vec, sorted_token_ids, (int)sorted_len, expert_ids,
+                                                  (int)expert_ids_len, num_tokens_post_pad);
     W4A16_HIP(hipGetLastError());
     return 0;
   }
-  const int grid = (int)ceil_div(num_experts, ALIGN_WAVES);
-  moe_align_kernel<<<grid, ALIGN_THREADS, 0, (hipStream_t)stream>>>(
-      topk_ids, (int)numel, num_experts, block_size, sorted_token_ids, (int)sorted_len, expert_ids,
-      (int)expert_ids_len, num_tokens_post_pad);
+  // slices per expert: enough wavefronts for 64 and more workgroups, slices of at least 256 ids
+  int spe = 1;
+  while (spe < ALIGN_WAVES && num_experts * spe < 1024 && numel / (2 * spe) >= 256) spe *= 2;
+  const int64_t turns = ceil_div(num_experts, ALIGN_WAVES / spe);
+  const int grid = (int)(turns < 256 ? turns : 256);
+  const auto fn = vec ? moe_align_sliced_kernel<true> : moe_align_sliced_kernel<false>;
+  fn<<<grid, ALIGN_THREADS, 0, (hipStream_t)stream>>>(topk_ids, (int)numel, num_experts, block_size, spe, sorted_token_ids, (int)sorted_len, expert_ids,
+                                                      (int)expert_ids_len, num_tokens_post_pad);
   W4A16_HIP(hipGetLastError());
   return 0;
 }
