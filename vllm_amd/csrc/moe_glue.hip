@@ -392,6 +392,40 @@ __device__ __forceinline__ float wave_max(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
 }
 
+// the same of whole numbers: one instruction a step (a lane that has no source reads the lowest number)
+template <int CTRL>
+__device__ __forceinline__ int dpp_imax(int x) { return max(x, __builtin_amdgcn_update_dpp((int)0x80000000, x, CTRL, 0xf, 0xf, false)); }
+__device__ __forceinline__ int wave_imax(int x) {
+  x = dpp_imax<0x111>(x);
+  x = dpp_imax<0x112>(x);
+  x = dpp_imax<0x114>(x);
+  x = dpp_imax<0x118>(x);
+  x = dpp_imax<0x142>(x);
+  x = dpp_imax<0x143>(x);
+  return __builtin_amdgcn_readlane(x, 63);
+}
+// sum over the wavefront, in every lane, pairs 32, 16, ... 1 lanes apart (rotations by 8, 4, 2 and 1 in rows of 16 meet the lane that far apart, or one
+// with the same sum)
+template <int CTRL>
+__device__ __forceinline__ float dpp_rot_add(float x) {
+  const int v = __builtin_bit_cast(int, x);
+  return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float wave_sum_pairs(float x) {
+  auto a = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
+  x = __builtin_bit_cast(float, (int)a[0]) + __builtin_bit_cast(float, (int)a[1]);
+  a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
+  x = __builtin_bit_cast(float, (int)a[0]) + __builtin_bit_cast(float, (int)a[1]);
+  x = dpp_rot_add<0x128>(x);  // row_ror:8, 4, 2, 1
+  x = dpp_rot_add<0x124>(x);
+  x = dpp_rot_add<0x122>(x);
+  return dpp_rot_add<0x121>(x);
+}
+
+// One wavefront per token.  Bound by its chain of dependent instructions: maximum, sum and, per pick, the largest probability and the first lane that holds
+// it.  So the picks compare the probabilities as whole numbers (not negative: the same order; a step of the maximum is one instruction instead of three),
+// the sum stays in the registers, and the loop over the picks has no branch (601 tokens of 128 experts, top-8 3.8 -> 2.9 us, 4096 tokens 5.5 -> 3.9,
+// 1000 of 256 experts, top-16 6.9 -> 5.0, 16 of 8, top-2 2.3 -> 1.9; the same bits).
 template <typename T, int PL>
 __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__ gating, float* __restrict__ weights,
                                                            int32_t* __restrict__ ids, int32_t* __restrict__ src_rows,
@@ -416,43 +450,49 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
     v[i] = e < num_experts ? expf(v[i] - mx) : 0.f;
     sum += v[i];
   }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+  sum = wave_sum_pairs(sum);
   // A row with a NaN or +inf (or nothing but -inf) has no probabilities: every sum of exponentials but that is 1 or more.  It
   // picks experts 0, 1, ... with NaN weights, so that its token's result is NaN and no id is out of range.
   const bool bad = !(sum > 0.f);
+  int pr[PL];  // the probabilities' bits
 #pragma unroll
   for (int i = 0; i < PL; ++i) {
     const int e = lane + 64 * i;
-    v[i] = e < num_experts ? fmaxf(v[i] / sum, 0.f) : -1.f;  // (0 for a NaN) probabilities are >= 0: -1 marks "not a candidate"
+    pr[i] = __builtin_bit_cast(int, e < num_experts ? fmaxf(v[i] / sum, 0.f) : -1.f);  // (0 for a NaN) probabilities are >= 0: -1 marks "not a candidate"
   }
   const int64_t base = (int64_t)tok * topk;
   float selected = 0.f, my_w = 0.f;
   int my_e = 0;
-  for (int k = 0; k < topk; ++k) {
-    float best = v[0];
+  auto pick = [&](int k) {
+    int top = pr[0];
 #pragma unroll
-    for (int i = 1; i < PL; ++i) best = fmaxf(best, v[i]);
-    best = wave_max(best);
+    for (int i = 1; i < PL; ++i) top = max(top, pr[i]);
+    top = wave_imax(top);  // (>= 0: topk <= num_experts)
+    const float best = __builtin_bit_cast(float, top);
     int be = 0x7fffffff;
 #pragma unroll
     for (int i = PL - 1; i >= 0; --i) {
-      const unsigned long long m = __ballot(v[i] == best && v[i] >= 0.f);
-      if (m) be = 64 * i + __builtin_ctzll(m);
+      const unsigned long long m = __ballot(pr[i] == top);
+      be = m ? 64 * i + __builtin_ctzll(m) : be;
     }
     selected += best;
-    if ((k & 63) == lane) {
-      my_w = best;
-      my_e = be;
-      if (topk > 64) {  // more picks than lanes: kept in memory, each by the lane that rescales it
-        weights[base + k] = bad ? __builtin_nanf("") : best;
-        ids[base + k] = be;
+    const bool mine = (k & 63) == lane;
+    my_w = mine ? best : my_w;
+    my_e = mine ? be : my_e;
+#pragma unroll
+    for (int i = 0; i < PL; ++i) pr[i] = lane + 64 * i == be ? __builtin_bit_cast(int, -1.f) : pr[i];
+  };
+  if (topk <= 64) {
+    for (int k = 0; k < topk; ++k) pick(k);
+  } else {
+    for (int k = 0; k < topk; ++k) {
+      pick(k);
+      if ((k & 63) == lane) {  // more picks than lanes: kept in memory, each by the lane that rescales it
+        weights[base + k] = bad ? __builtin_nanf("") : my_w;
+        ids[base + k] = my_e;
         src_rows[base + k] = k * num_tokens + tok;
       }
     }
-#pragma unroll
-    for (int i = 0; i < PL; ++i)
-      if (lane + 64 * i == be) v[i] = -1.f;
   }
   if (bad) my_w = __builtin_nanf("");
   const float denom = renormalize && selected > 0.f ? selected : 1.f;
