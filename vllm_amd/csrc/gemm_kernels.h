@@ -97,7 +97,7 @@ __host__ __device__ inline void chunked_tile(int j, int live, int strips, int& m
 }
 
 // Side job of a launch: the grid clears `zero_n16` 16-byte pieces at `zero_ptr` (the output of a later launch that
-// accumulates with atomic adds).  Every workgroup of the grid calls this first, before any early exit.
+// accumulates with atomic adds).  Every workgroup of the grid calls this once, in front of any exit.
 __device__ __forceinline__ void zero_fill_side_job(const KParams& p, unsigned block, unsigned nblocks) {
   if (p.zero_n16 <= 0) return;
   const int64_t per = (p.zero_n16 + nblocks - 1) / nblocks;

@@ -13,7 +13,8 @@
 //                  and the registers of the addresses.  So both operands stay under 2 GiB (the planner checks; gemm_mid.hip takes the others).
 // Measured, whole layers in a graph (7 expert shapes of 1024 x 2048 to 4096 x 14336, 12 to 192 slots per expert, even and skewed routing, fp16 and
 // bf16, groups of 32 to channel-wise; 945 layers): 0.87 of the time on 512-column tiles of the 64-row kernel in the mean, 0.70 - 0.85 with small
-// experts or few rows, 0.95 - 1.02 with full blocks and many tiles.  128 experts of 2048 x 768, top-8, 601 tokens, bf16 AWQ: layer 124.3 -> 118.8 us.
+// experts or few rows, 0.95 - 1.02 with full blocks and many tiles.  128 experts of 2048 x 768, top-8, 601 tokens, bf16 AWQ: layer 124.3 -> 118.8 us (112 with what came
+// later: scalar loads in front of the loop, rows read together behind it, priorities, and the launches around the GEMMs).
 // Requirements (host-checked): MoE blocks of 64 slots, K % 128 == 0, power-of-two groups or one scale per column, A's columns in weight order.
 #include <type_traits>
 
