@@ -281,6 +281,7 @@ __global__ __launch_bounds__(DNW * 64, 2) void decode_kernel(const uint32_t* eB,
     // A bounce: natural [row][128 B] layout in, MFMA operand (row m, K pairs 8s+2g) out
     *(u32x4*)slab_wr = s.a[0];
     *(u32x4*)(slab_wr + 8 * A_ROW) = s.a[1];
+    lds_lanes_in_order();
     u32x4 af[2];
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {

@@ -96,6 +96,14 @@ __host__ __device__ inline void chunked_tile(int j, int live, int strips, int& m
   }
 }
 
+// Where the lanes of one wavefront hand each other data through LDS: between the stores and the reads of other lanes' data, and between those and the
+// next stores (or a scheduling barrier, which no memory access passes either).  A wavefront's LDS accesses are executed in order; that they stay in
+// the order they are written in is for the compiler to know.  No instructions.
+__device__ __forceinline__ void lds_lanes_in_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Side job of a launch: the grid clears `zero_n16` 16-byte pieces at `zero_ptr` (the output of a later launch that
 // accumulates with atomic adds).  Every workgroup of the grid calls this once, in front of any exit.
 __device__ __forceinline__ void zero_fill_side_job(const KParams& p, unsigned block, unsigned nblocks) {

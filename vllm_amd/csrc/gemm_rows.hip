@@ -111,6 +111,7 @@ __global__ __launch_bounds__(RW_NW * 64, 2) void rows_kernel(const KParams p) {
     // activations: rows of 128 bytes in, MFMA operands (row, K pairs 8 s + 2 g) out
 #pragma unroll
     for (int i = 0; i < 2 * MB; ++i) *(u32x4*)(slab_wr + 8 * i * RW_AROW) = s.a[i];
+    lds_lanes_in_order();
     u32x4 vb;  // operand of the row sums
     if constexpr (HI_TRICK) {
       vb = u32x4{RAW_BIAS_LO, RAW_BIAS_HI, RAW_BIAS_LO, RAW_BIAS_HI};

@@ -327,6 +327,7 @@ __global__ __launch_bounds__(NW * 64, 2) void skinny_kernel(const KParams p) {
     {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) *(u32x4*)(slab_wr + mb * 16 * A_ROW) = s.a[mb];
+    lds_lanes_in_order();
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
       const uint32_t* q = slab_rd + mb * 16 * A_ROW;
@@ -474,6 +475,7 @@ __global__ __launch_bounds__(NW * 64, 2) void skinny_kernel(const KParams p) {
       const int i = done + j;
       if (i < nks) {
         consume(st[j], w_b + i);
+        lds_lanes_in_order();
         if (i + D < nks) {
             issue(st[j], w_b + i + D);
         }
