@@ -9,7 +9,7 @@
 //                in the 64-row kernel (B operand = the reference's half(q - z) * half(s)).
 //   activations  each K-quarter stages its own 64 rows x 64 K chunk into LDS in MFMA fragment order (its two
 //                wavefronts share it), double buffered; one workgroup barrier per two k-steps.
-//   epilogue     the four quarters' partial tiles are added through LDS, two 16-row blocks at a time.
+//   epilogue     the four quarters' partial tiles are added through LDS, one 16-row block at a time.
 //   split-K      with fewer tiles than compute units (129..~1000 rows of a narrow layer) K is also cut across
 //                workgroups, in splits of whole multiples of 512 K rows: the workgroup writes its 64 x 256 fp32 partial
 //                tile (already summed over its quarters) to scratch with plain 128-bit stores and kq_reduce_kernel,
@@ -54,11 +54,12 @@ constexpr int KQ_D = 4;      // weight k-steps in flight per wavefront
 // 2 k-steps x 4 dwords, then hit 64 different ones (128-row tiles without: 4096 x 4096 at 1024 rows 41.4 us, 41.6 with, and three spills)
 constexpr int kq_kstep(int MB) { return MB * 256 + (MB < 8 ? 32 : 0); }
 constexpr int kq_abuf(int MB) { return 2 * kq_kstep(MB) * 4; }  // one A buffer of one K part: 2 k-steps
-constexpr int KQ_ME = 2;   // m-blocks per round of the epilogue (four and eight K parts)
 constexpr int KQ_RS = 76;  // floats per row of an epilogue slab of 64 columns (40 for the half of either n-tile: conflict-free, 16-byte aligned)
 constexpr int kq_smem(int MB, int Q, int WN) {
-  // staging rings | what the parts hand each other in the epilogue
-  const int stage = Q * 2 * kq_abuf(MB), boxes = Q == 2 ? WN * Q * MB * 4096 : KQ_ME * WN * Q * 16 * RED_RS * 4;
+  // staging rings | what the parts hand each other in the epilogue.  64 x 256 and 32 x 128 tiles 74 KB, 48 and 64 x 128 100 and 132, tall ones 80 to 128:
+  // one workgroup to a compute unit, which is what their registers leave room for.  (Four and eight parts with two m-blocks at a time, 148 KB: level, 1.001
+  // of the time in the mean of 90 problems of 49 to 1000 rows, weights not cached, none beyond 1.012 either way.)
+  const int stage = Q * 2 * kq_abuf(MB), boxes = Q == 2 ? WN * Q * MB * 4096 : WN * Q * 16 * RED_RS * 4;
   return stage > boxes ? stage : boxes;
 }
 
@@ -351,9 +352,6 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   // (the inline-asm MFMAs are opaque to the compiler's hazard logic: let the matrix pipe drain before the
   //  accumulators are read)
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
-  // per m-block: every wavefront writes its 16 x 128 partial to its slab [16 rows][RED_RS]; after a barrier the
-  // wavefront of K part q adds the Q parts' slabs of its column pair for rows (16 / Q) q .. and finishes them.
-  // (the last barrier of the loop, or this one, separates the slabs from the A buffers they overlay)
   // (the last barrier of the loop, or this one, separates what follows from the A buffers it overlays)
   if constexpr (PRIV) __syncthreads();
   const int ncol0 = cp * 128;
@@ -445,9 +443,8 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
     else
       exchange(std::integral_constant<int, 1>{});
   } else {
-    // per two m-blocks: every wavefront writes its 16 x 128 partials to its slabs [16 rows][RED_RS]; after a barrier the
-    // wavefront of K part q adds the Q parts' slabs of its column pair for rows (16 / Q) q .. and finishes them.
-    constexpr int ME = KQ_ME, SLABS = WN * KQ_Q * 16 * RED_RS;
+    // per m-block: every wavefront writes its 16 x 128 partial to its slab [16 rows][RED_RS]; after a barrier the wavefront of
+    // K part q adds the Q parts' slabs of its column pair for rows (16 / Q) q .. and finishes them.
     float* slabs = (float*)smem;
     const int slab_at = wv * (16 * RED_RS) + 4 * (el >> 4 & 3) * RED_RS + 72 * (el >> 3 & 1) + (el & 7);
     const int fc4 = (lane & 31) * 4;
@@ -456,35 +453,31 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
     const bool fcol_ok = wave_on && ncol < p.N;
     if (fcol_ok) col_consts(ncol, cs, bs);
 #pragma unroll
-    for (int m0 = 0; m0 < KQ_MB; m0 += ME) {
-      if (m0 > 0) __syncthreads();
+    for (int mb = 0; mb < KQ_MB; ++mb) {
+      if (mb > 0) __syncthreads();
 #pragma unroll
-      for (int e = 0; e < ME && m0 + e < KQ_MB; ++e)
+      for (int w = 0; w < 4; ++w)
 #pragma unroll
-        for (int w = 0; w < 4; ++w)
+        for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-          for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) slabs[e * SLABS + slab_at + r * RED_RS + 16 * w + 8 * hf] = acc[m0 + e][w][hf][r];
+          for (int r = 0; r < 4; ++r) slabs[slab_at + r * RED_RS + 16 * w + 8 * hf] = acc[mb][w][hf][r];
       __syncthreads();
 #pragma unroll
-      for (int e = 0; e < ME && m0 + e < KQ_MB; ++e)
+      for (int i = 0; i < 8 / KQ_Q; ++i) {
+        const int r16 = (16 / KQ_Q) * q + (lane >> 5) + 2 * i;
+        const int crow = row0 + mb * 16 + r16;
+        f32x4 v = {0, 0, 0, 0};
 #pragma unroll
-        for (int i = 0; i < 8 / KQ_Q; ++i) {
-          const int mb = m0 + e, r16 = (16 / KQ_Q) * q + (lane >> 5) + 2 * i;
-          const int crow = row0 + mb * 16 + r16;
-          f32x4 v = {0, 0, 0, 0};
+        for (int qq = 0; qq < KQ_Q; ++qq) v += *(const f32x4*)(slabs + (qq * WN + wn) * (16 * RED_RS) + r16 * RED_RS + fpos);
+        if (p.splits > 1) {
+          if (crow < p.M)
+            *(f32x4*)(p.ctmp + (((int64_t)(strip * mtiles + mt) * p.splits + split) * KQ_BM + mb * 16 + r16) * KQ_TN + wn * 128 + fc4) = v;
+        } else if (fcol_ok && crow < p.M) {
 #pragma unroll
-          for (int qq = 0; qq < KQ_Q; ++qq) v += *(const f32x4*)(slabs + e * SLABS + (qq * WN + wn) * (16 * RED_RS) + r16 * RED_RS + fpos);
-          if (p.splits > 1) {
-            if (crow < p.M)
-              *(f32x4*)(p.ctmp + (((int64_t)(strip * mtiles + mt) * p.splits + split) * KQ_BM + mb * 16 + r16) * KQ_TN + wn * 128 + fc4) = v;
-          } else if (fcol_ok && crow < p.M) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = v[j] * cs[j] + bs[j];
-            store_row4<DT, false>(p, crow, ncol, v);
-          }
+          for (int j = 0; j < 4; ++j) v[j] = v[j] * cs[j] + bs[j];
+          store_row4<DT, false>(p, crow, ncol, v);
         }
+      }
     }
   }
 }
