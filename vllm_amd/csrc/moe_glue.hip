@@ -593,9 +593,9 @@ extern "C" int w4a16_moe_align_block_size(const int32_t* topk_ids, int64_t numel
     W4A16_HIP(hipGetLastError());
     return 0;
   }
-  // slices per expert: enough wavefronts for 64 and more workgroups, slices of at least 256 ids
+  // slices per expert: enough wavefronts for 64 and more workgroups
   int spe = 1;
-  while (spe < ALIGN_WAVES && num_experts * spe < 1024 && numel / (2 * spe) >= 256) spe *= 2;
+  while (spe < ALIGN_WAVES && num_experts * spe < 1024) spe *= 2;
   const int64_t turns = ceil_div(num_experts, ALIGN_WAVES / spe);
   const int grid = (int)(turns < 256 ? turns : 256);
   const auto fn = vec ? moe_align_sliced_kernel<true> : moe_align_sliced_kernel<false>;
