@@ -58,7 +58,7 @@ constexpr int KQ_RS = 76;  // floats per row of an epilogue slab of 64 columns (
 constexpr int kq_smem(int MB, int Q, int WN) {
   // staging rings | what the parts hand each other in the epilogue.  64 x 256 and 32 x 128 tiles 74 KB, 48 and 64 x 128 100 and 132, tall ones 80 to 128:
   // one workgroup to a compute unit, which is what their registers leave room for.  (Four and eight parts with two m-blocks at a time, 148 KB: level, 1.001
-  // of the time in the mean of 90 problems of 49 to 1000 rows, weights not cached, none beyond 1.012 either way.)
+  // of the time in the mean of 90 problems of 80 to 967 rows, weights not cached, none beyond 1.012 either way.)
   const int stage = Q * 2 * kq_abuf(MB), boxes = Q == 2 ? WN * Q * MB * 4096 : WN * Q * 16 * RED_RS * 4;
   return stage > boxes ? stage : boxes;
 }
