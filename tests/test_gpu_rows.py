@@ -1,5 +1,5 @@
-"""Tiles of 32 and 48 rows with unscaled weights (gemm_rows.hip), at the edges of their row counts, with one and several K splits and uneven ones,
-against float64.  tests/test_plans.py pins that these problems run there."""
+"""Tiles of 32 and 48 rows with unscaled weights (gemm_rows.hip), at the edges of their row counts, with one to seven K splits (the last arrival adds four
+at a time) and with a shorter last one, against float64.  tests/test_plans.py pins that these problems run there."""
 import pytest
 import torch
 
@@ -8,21 +8,29 @@ from test_gpu_kq_heights import _layer, _rel, _run, workspace  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 F16, BF16 = torch.float16, torch.bfloat16
-# (m, k, n, dtype, fmt, group, act_order): (m-blocks, splits) of the plan
+# (m, k, n, dtype, fmt, group, act_order): (m-blocks, splits, units of 128 K rows per split) of the plan
 ROWS = {
-    (17, 14336, 4096, BF16, "uint4", 128, False): (2, 4),
-    (32, 14336, 4096, BF16, "uint4", 256, False): (2, 4),
-    (33, 14336, 4096, F16, "uint4", 128, False): (3, 4),
-    (48, 14336, 4096, BF16, "uint4b8", 128, True): (3, 4),
-    (48, 18944, 3584, F16, "uint4b8", 128, False): (3, 4),
-    (20, 18944, 3648, BF16, "uint4", -1, False): (2, 4),
-    (31, 28672, 4096, F16, "uint4b8", -1, False): (2, 4),
-    (17, 28672, 4096, F16, "uint4b8", 128, False): (2, 4),
-    (29, 18944, 3584, F16, "uint4", -1, False): (2, 4),
-    (47, 13824, 5120, BF16, "uint4", 128, False): (3, 3),
-    (48, 4096, 11008, F16, "uint4", 128, False): (3, 1),
-    (40, 4096, 11008, BF16, "uint4b8", -1, False): (3, 1),
-    (37, 5120, 13824, F16, "uint4b8", 128, False): (3, 1),
+    (17, 14336, 4096, BF16, "uint4", 128, False): (2, 4, 28),
+    (32, 14336, 4096, BF16, "uint4", 256, False): (2, 4, 28),
+    (33, 14336, 4096, F16, "uint4", 128, False): (3, 4, 28),
+    (48, 14336, 4096, BF16, "uint4b8", 128, True): (3, 4, 28),
+    (48, 18944, 3584, F16, "uint4b8", 128, False): (3, 4, 37),
+    (20, 18944, 3648, BF16, "uint4", -1, False): (2, 4, 37),
+    (31, 28672, 4096, F16, "uint4b8", -1, False): (2, 4, 56),
+    (17, 28672, 4096, F16, "uint4b8", 128, False): (2, 4, 56),
+    (29, 18944, 3584, F16, "uint4", -1, False): (2, 4, 37),
+    (47, 13824, 5120, BF16, "uint4", 128, False): (3, 3, 36),
+    (48, 4096, 11008, F16, "uint4", 128, False): (3, 1, 32),
+    (40, 4096, 11008, BF16, "uint4b8", -1, False): (3, 1, 32),
+    (37, 5120, 13824, F16, "uint4b8", 128, False): (3, 1, 40),
+    # the last split is shorter
+    (37, 11008, 4096, BF16, "uint4", 128, False): (3, 4, 22),
+    (48, 8064, 6400, BF16, "uint4b8", -1, False): (3, 2, 32),
+    (17, 9344, 7168, BF16, "uint4", 128, False): (2, 2, 37),
+    (32, 25472, 3072, F16, "uint4b8", 128, False): (2, 5, 40),
+    (48, 24192, 3072, BF16, "uint4b8", 128, True): (3, 5, 38),
+    (17, 20736, 2304, F16, "uint4", -1, False): (2, 7, 24),
+    (33, 18560, 2304, BF16, "uint4", 128, False): (3, 7, 21),
 }
 
 

@@ -1,5 +1,5 @@
 """Many back-to-back launches of the paths that add K splits across workgroups (the 16-row kernel's in-kernel
-exchange on o_proj- and down_proj-sized layers at M = 16; the two-pass K split of the 64 x 256 and the 64 x 512 kernels):
+exchange on o_proj- and down_proj-sized layers at M = 16, that of the 32- and 48-row tiles; the two-pass K split of the 64 x 256 and the 64 x 512 kernels):
 every result must equal the first bit for bit, and the workspace counters must be zero at the end.  The launches of a
 burst go out on one stream without host synchronisation in between."""
 import pytest
@@ -14,9 +14,11 @@ CASES = [("o M=16, 16-row kernel", 16, 4096, 4096), ("down M=16, 16-row kernel",
          ("qkv M=4, 16-row kernel", 4, 4096, 6144),
          ("down M=256, 64 x 256 tiles + second pass", 256, 14336, 4096),
          ("gate_up M=192, 64 x 512 tiles + second pass", 192, 4096, 28672)]
+# (tests/test_plans.py pins that these run on tiles of 48 and 32 rows with four K splits)
+ROWS_CASES = [("down M=48, 48-row tiles", 48, 18944, 3584), ("down M=17, 32-row tiles", 17, 28672, 4096)]
 
 
-@pytest.mark.parametrize("name,m,k,n", CASES)
+@pytest.mark.parametrize("name,m,k,n", CASES + ROWS_CASES)
 def test_split_k_paths_are_stable_over_many_launches(dev, name, m, k, n):
     import vllm_amd.ops as ops
     from vllm_amd.marlin_utils import marlin_make_workspace_new

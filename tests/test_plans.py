@@ -10,7 +10,8 @@ from vllm_amd import _lib
 from vllm_amd import build as vbuild
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-FIELDS = ["kind", "mb", "tn", "splits", "kps", "ks", "tail_strips", "tail_kind", "tail_mb", "xcd_map"]
+FIELDS = ["kind", "mb", "tn", "splits", "kps", "ks", "tail_strips", "tail_kind", "tail_mb", "xcd_map",
+          "scratch_kib", "first_scratch_kib", "first_kind"]
 
 
 @pytest.fixture(scope="module")
@@ -205,13 +206,32 @@ def test_tiles_of_rows_with_unscaled_weights(plan):
     """The shapes of test_gpu_rows.py run on the tile they are listed with; what the kernel does not take, and what has never run on 16-row tiles, stays."""
     import torch
     import test_gpu_rows as rows
-    for (m, k, n, dtype, fmt, group, act), tile in rows.ROWS.items():
+    tiles, uneven, splits = set(), set(), set()
+    for (m, k, n, dtype, fmt, group, act), (mb, sp, units) in rows.ROWS.items():
         p = plan(m, k, n, dtype, fmt, group, act)
-        assert (p["kind"], p["mb"], p["splits"], p["tn"]) == (10,) + tile + (64,), (m, k, n, dtype, fmt, group, p)
+        assert (p["kind"], p["mb"], p["splits"], p["kps"], p["tn"]) == (10, mb, sp, 4 * units, 64), (m, k, n, dtype, fmt, group, p)
+        tiles.add((mb, dtype, fmt, group == -1))
+        splits.add((mb, sp))
+        if k // 128 % units:
+            uneven.add((mb, sp))
+        # no more scratch than the 16-row tiles take, where a caller asks for little: with this many splits those keep the problem
+        less = plan(m, k, n, dtype, fmt, group, act, more_scratch=False)
+        assert less["first_kind"] == 1 and less["scratch_kib"] <= less["first_scratch_kib"], (m, k, n, less)
+        assert less["kind"] == (1 if sp > 1 else 10) and (sp == 1 or p["scratch_kib"] > p["first_scratch_kib"]), (m, k, n, less)
         assert plan(16, k, n, dtype, fmt, group, act)["kind"] == 1 and plan(49, k, n, dtype, fmt, group, act)["kind"] != 10
     for m, k, n, group in [(37, 14336, 4096, 64), (37, 14336 + 64, 4096, -1), (37, 14336, 4096, 32), (37, 4096, 4096, 128), (37, 4096, 28672, 128),
                            (20, 4096, 64 * 257, 128)]:
         assert plan(m, k, n, torch.bfloat16, "uint4", group)["kind"] != 10, (m, k, n, group)
-    # no more scratch than the 16-row tiles had, where a caller asks for little
-    p = plan(37, 14336, 4096, torch.bfloat16, "uint4", 128, more_scratch=False)
-    assert p["kind"] in (1, 10) and p["splits"] <= 4
+    assert {(mb, s) for mb in (2, 3) for s in (2, 5, 7)} <= uneven and {(3, 1), (2, 4), (3, 3), (3, 4)} <= splits
+    assert {t[:3] for t in tiles} >= {(3, dt, fmt) for dt in (torch.float16, torch.bfloat16) for fmt in ("uint4", "uint4b8")}
+
+
+def test_static_and_repeated_calls_on_tiles_of_rows(plan):
+    """The calls of test_zz_no_alloc.py and test_gpu_splitk_stress.py that stand for the exchange between K splits of 32- and 48-row tiles."""
+    import test_gpu_splitk_stress as stress
+    import test_zz_no_alloc as static
+    import torch
+    k, n, group, dtype, zp, act, ms = static.ROWS_CASE
+    assert [(p["kind"], p["mb"], p["splits"]) for p in (plan(m, k, n, dtype, "uint4" if zp else "uint4b8", group, act) for m in ms)] == [(10, 3, 4), (10, 2, 4)]
+    got = [plan(m, k, n, torch.float16, "uint4b8", 128) for _, m, k, n in stress.ROWS_CASES]
+    assert [(p["kind"], p["mb"], p["splits"]) for p in got] == [(10, 3, 4), (10, 2, 4)]

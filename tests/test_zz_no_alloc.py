@@ -28,7 +28,9 @@ def _args(lib_mod, a, c, layer_dev, m, n, k, groups, ws, c_tmp, zp, g_idx, perm,
     return args
 
 
+ROWS_CASE = (14336, 4096, 128, torch.bfloat16, True, False, (37, 20))  # tiles of 48 and 32 rows, K split across workgroups
 CASES = [
+    ROWS_CASE,
     # (k, n, group, dtype, zp, act_order, (m_first, m_second))
     (14336, 4096, 128, torch.float16, False, False, (16, 3)),     # decode kernel, K split across workgroups
     (4096, 4096, 128, torch.float16, False, False, (16, 1)),      # decode kernel, small layer
