@@ -63,6 +63,18 @@ constexpr int kq_smem(int MB, int Q, int WN) {
   return stage > boxes ? stage : boxes;
 }
 
+// channel scale and bias of four finished columns starting at `ncol` (scales and bias are stored permuted); 1 and 0 are the caller's
+template <int DT, bool CHANNEL>
+__device__ __forceinline__ void kq_col_consts(const KParams& p, int ncol, float* cs, float* bs) {
+  const uint16_t *Sc = (const uint16_t*)p.S, *bias = (const uint16_t*)p.bias;
+  const int base = ncol & ~31, cl = ncol & 31;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (CHANNEL) cs[j] = lo_f32<DT>(Sc[base + single_perm_pos(cl + j)]);
+    if (bias) bs[j] = lo_f32<DT>(bias[base + single_perm_pos(cl + j)]);
+  }
+}
+
 // SHORT: private parts and tall tiles with groups below 128 rows, whose scales and constants come with every k-step.  (Tall tiles had both loops in
 // one kernel, 40 to 80 registers more, and scales in every k-step for every group: 80 to 112 rows, groups of 32 and 64 0.90 - 0.97 of the
 // time, of 128 0.96 - 1.00, reading A early included; 14336 x 4096 at 1501 rows, fp16, groups of 128: 166 -> 160 us.)
@@ -105,7 +117,6 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   const uint32_t* Bq = p.B;
   const uint16_t* Sc = (const uint16_t*)p.S;
   const uint32_t* Zp = p.Z;
-  const uint16_t* bias = (const uint16_t*)p.bias;
   // ---- weights of this wavefront
   const int nt = (wave_on && (2 * cp + h) * 64 < p.N) ? 2 * cp + h : 0;
   const int64_t b_row = p.N >> 1;
@@ -355,20 +366,6 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
   // (the last barrier of the loop, or this one, separates what follows from the A buffers it overlays)
   if constexpr (PRIV) __syncthreads();
   const int ncol0 = cp * 128;
-  auto col_consts = [&](int ncol, float* cs, float* bs) {
-    const int base = ncol & ~31, cl = ncol & 31;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (CHANNEL) {
-        const uint16_t sv = Sc[base + single_perm_pos(cl + j)];
-        cs[j] = (DT == DT_F16) ? f16_lo_f32(sv) : bf16_lo_f32(sv);
-      }
-      if (bias) {
-        const uint16_t bv = bias[base + single_perm_pos(cl + j)];
-        bs[j] = (DT == DT_F16) ? f16_lo_f32(bv) : bf16_lo_f32(bv);
-      }
-    }
-  };
   float cs[4] = {1.f, 1.f, 1.f, 1.f}, bs[4] = {0.f, 0.f, 0.f, 0.f};
   int el = t;  // (taken apart again here: a lane's place kept through the loop would spill in one of the kernels)
   asm volatile("" : "+v"(el));
@@ -385,7 +382,7 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
     const int lc = (el & 15) * 4, lh = lc >> 5, lpos = lh * 40 + (lc & 31);  // 64 columns: 32 of either n-tile
     const int ncol = ncol0 + 64 * lh + 32 * q + (lc & 31);
     const bool col_ok = wave_on && ncol < p.N;
-    if (col_ok && p.splits == 1) col_consts(ncol, cs, bs);
+    if (col_ok && p.splits == 1) kq_col_consts<DT, CHANNEL>(p, ncol, cs, bs);
     auto exchange = [&](auto part_tag) __attribute__((always_inline)) {  // (the part as a constant: accumulators are registers)
       constexpr int PART = decltype(part_tag)::value;
 #pragma unroll
@@ -451,7 +448,7 @@ __global__ __launch_bounds__(64 * WN * Q) void kq_kernel(const KParams p) {
     const int fpos = fc4 + (fc4 >= 64 ? 8 : 0);
     const int ncol = ncol0 + fc4;
     const bool fcol_ok = wave_on && ncol < p.N;
-    if (fcol_ok) col_consts(ncol, cs, bs);
+    if (fcol_ok) kq_col_consts<DT, CHANNEL>(p, ncol, cs, bs);
 #pragma unroll
     for (int mb = 0; mb < KQ_MB; ++mb) {
       if (mb > 0) __syncthreads();
@@ -495,23 +492,8 @@ __global__ __launch_bounds__(256) void kq_reduce_kernel(const KParams p, int mb)
   const int fc4 = (t % (KQ_TN / 4)) * 4;
   const int ncol = (p.strip0 + strip) * KQ_TN + fc4;
   if (ncol >= p.N) return;
-  const uint16_t* Sc = (const uint16_t*)p.S;
-  const uint16_t* bias = (const uint16_t*)p.bias;
   float cs[4] = {1.f, 1.f, 1.f, 1.f}, bs[4] = {0.f, 0.f, 0.f, 0.f};
-  {
-    const int base = ncol & ~31, cl = ncol & 31;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (CHANNEL) {
-        const uint16_t sv = Sc[base + single_perm_pos(cl + j)];
-        cs[j] = (DT == DT_F16) ? f16_lo_f32(sv) : bf16_lo_f32(sv);
-      }
-      if (bias) {
-        const uint16_t bv = bias[base + single_perm_pos(cl + j)];
-        bs[j] = (DT == DT_F16) ? f16_lo_f32(bv) : bf16_lo_f32(bv);
-      }
-    }
-  }
+  kq_col_consts<DT, CHANNEL>(p, ncol, cs, bs);
   const float* parts = p.ctmp + (int64_t)tile * p.splits * (KQ_BM * KQ_TN) + fc4;
 #pragma unroll
   for (int i = 0; i < 16 / TR; ++i) {
@@ -552,16 +534,7 @@ __global__ __launch_bounds__(256) void kq_reduce_tall_kernel(const KParams p, in
   if (row0 - (lane >> 4) >= p.M || cp * 128 >= p.N) return;
   const bool col_ok = ncol < p.N;
   float cs[4] = {1.f, 1.f, 1.f, 1.f}, bs[4] = {0.f, 0.f, 0.f, 0.f};
-  const uint16_t* Sc = (const uint16_t*)p.S;
-  const uint16_t* bias = (const uint16_t*)p.bias;
-  if (col_ok) {
-    const int base = ncol & ~31, cl = ncol & 31;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (CHANNEL) cs[j] = lo_f32<DT>(Sc[base + single_perm_pos(cl + j)]);
-      if (bias) bs[j] = lo_f32<DT>(bias[base + single_perm_pos(cl + j)]);
-    }
-  }
+  if (col_ok) kq_col_consts<DT, CHANNEL>(p, ncol, cs, bs);
   const int64_t piece = mb * 4096;  // floats of a partial tile
   const float* parts = p.ctmp + (int64_t)tile * p.splits * piece + (wv * mb + m) * 1024 + lane * 4;
   f32x4 v[4] = {};
