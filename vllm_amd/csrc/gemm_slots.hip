@@ -327,8 +327,9 @@ __global__ __launch_bounds__(256, W == 2 ? 3 : 2) void slots_kernel(const KParam
     Pace pace;
     pace.start(nchunks, (int)blockIdx.x + p.resident >= d.F + d.R * d.S);
     // ---- main loop: two chunks (four k-steps = the weight ring) per iteration.  The last iteration stands behind it and asks for nothing: as part of the
-    // loop it read its own data again, and the epilogue's registers waited for that (ten layers of 8 to 128 experts 0.99 of the time in two runs,
-    // 32 experts of 3072 x 1024, 600 tokens 107.6 -> 103.2 us, 128 of 2048 x 768, 601 tokens 110.2 -> 109.4, 1300 tokens level).
+    // loop it read its own data again, and the epilogue's registers waited for that: 1.011 of the time in the mean of 45 layers of 8 to 128 experts, 0.972 to
+    // 1.039 (both GEMMs, weights not cached; 128 experts of 2048 x 768, 601 tokens level, 1300 tokens 177.5 -> 173.5 us, 32 of 3072 x 1024, 600 tokens
+    // 93.1 -> 91.0).
     auto round = [&](int c0, auto end_tag) __attribute__((always_inline)) {
       constexpr bool END = decltype(end_tag)::value;
       const int ks0 = 2 * c0;
