@@ -166,8 +166,8 @@ __device__ __forceinline__ void store_row4_silu_mul(const KParams& p, int crow, 
 // non-coherent line), 8 bytes at a time.  The writer waits for its stores (s_waitcnt) before it counts
 // itself as arrived; the reader is whoever sees the last arrival.
 //
-// Why the last arriver reads complete partial tiles, instruction by instruction (16-row kernels, gemm_decode.hip /
-// gemm_skinny.hip epilogue):
+// Why the last arriver reads complete partial tiles, instruction by instruction (epilogues of gemm_decode.hip, gemm_rows.hip
+// and gemm_skinny.hip):
 //   1. every thread of a writing workgroup issues its partial sums as `global_store_dwordx2 ... sc1`: the store is
 //      performed at the device-coherent level, not left dirty in the XCD's L2;
 //   2. `s_waitcnt vmcnt(0)` (__builtin_amdgcn_s_waitcnt(0)) in every thread: vmcnt only drops when the memory system has
@@ -343,7 +343,8 @@ __device__ __forceinline__ void mfma_inplace_v(f32x4& acc, const u32x4& a, const
 // -> 118.7 us); private K parts 1.01 - 1.05 (4096 x 6144 at 203 rows, bf16, 19.4 -> 18.8); 16-row tiles, dense, 1.00 - 1.05 (4096 x 6144 at 37 rows, bf16
 // with zero points, 10.25 -> 9.75), in MoE 0.99: those don't.
 //   The levels hold for the whole SIMD: a kernel of another stream that shares it and sets none runs at 0, so it gets the issue slots that these
-// wavefronts leave until they have fallen to 0 themselves (7/8 of their loop; tiles of MoE rounds that others follow stay at 3 to their end).
+// wavefronts leave until they have fallen to 0 themselves (7/8 of their loop; loops of a few rounds end at 1 or 2, tiles of MoE rounds that others
+// follow at 3, and keep that to their end).
 struct Pace {
   int at, n, level;
   __device__ __forceinline__ void start(int rounds, bool last = true) {
